@@ -84,6 +84,11 @@ SIGNATURES = {
     "ds_conv2d_tiled_fused_i32": (_c_int, [_ptr] * 8 + [_c_int] * 18 + [_ptr, _size, _ptr]),
     "ds_conv2d_tiled_fused_pair_workspace_bytes": (_size, [_c_int] * 6 + [_fcp, _fcp]),
     "ds_conv2d_tiled_fused_pair_i32": (_c_int, [_ptr] + [_c_int] * 7 + [_fcp, _fcp, _ptr, _size, _ptr]),
+    "ds_mfma_weight_bytes": (_size, [_c_int] * 6),
+    "ds_mfma_tile_weights_i32": (_c_int, [_ptr, _ptr] + [_c_int] * 7 + [_ptr]),
+    "ds_mfma_input_bytes": (_size, [_c_int] * 7),
+    "ds_mfma_prepare": (_c_int, [_ptr, _c_int, _ptr] + [_c_int] * 13 + [_ptr]),
+    "ds_mfma_conv2d": (_c_int, [_ptr] * 9 + [_c_int] * 23 + [_ptr]),
     "ds_quantize_f32_i32": (_c_int, [_ptr, _ptr, _c_i64, _c_int, _c_int, _c_int, _ptr]),
     "ds_quantize_pad_f32_i32": (_c_int, [_ptr, _ptr] + [_c_int] * 9 + [_ptr]),
     "ds_quantize_transpose_f32_i32": (_c_int, [_ptr, _ptr] + [_c_int] * 6 + [_ptr]),

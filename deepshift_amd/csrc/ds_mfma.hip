@@ -1,0 +1,976 @@
+// Shift convolutions and shift GEMMs on the matrix cores (int8 MFMA, int32 accumulation), exact modulo 2^32.
+//
+// A term sgn * (x >> s) is not linear in x, but it is a short sum of products of 8-bit numbers.  With x written in
+// 7-bit digits, x = d0 + 2^7 d1 + 2^14 d2 + 2^21 d3 + 2^28 d4 (d0, d1 in 0..127, the others balanced), and
+// s = 7 q + r, 0 <= r < 7:
+//     x >> s = (d_q >> r) + sum_{i > q} d_i * 2^(6-r) * 2^(7(i-q-1)+1)
+//     64 * (d_q >> r) = sum_j (bit j of d_q, in place) * [r <= j] 2^(6-r)
+// i.e. bit masks of a digit (one AND per four activations) times weight planes that hold 0 or a signed power of two
+// up to 64 -- all of them int8 -- plus products of whole digits with the full weight plane of their q.  A weight is
+// stored as up to four selector bytes, one per group of four shifts, from which one v_perm_b32 per four weights makes
+// any plane; 12 selects the constant 0.  Fields of up to 14 take 18 products of int8 per term, of up to 6 nine, of up
+// to 3 six; activations of 8 bits take one product per distinct shift (x >> s, selected by +-1).  The matrix cores do
+// 1024 such products per clock and SIMD, so 18 per term end at 139 Tpair/s, where the vector kernels' one instruction
+// per term ends at 39.3.  Measured, 64 -> 64 channels, 3 x 3, 64 images of 56 x 56, shifts to 14: 115 us (65 Tpair/s)
+// and 21 us for the layout pass, against 300 us; shifts to 2 on 8-bit activations, 512 -> 512 channels, 128 images of
+// 7 x 7: 66 us (223 Tpair/s).  A pure loop of v_mfma_i32_32x32x32_i8 reaches 0.7 of the nominal rate (47 clocks of
+// 2.4 GHz for 32): what is left between the two is the vector work that makes the planes, in part under the MFMAs.
+//
+// Activations are laid out first (ds_mfma_prepare): [image][row][32-channel block][digit][column][32 channels], so that
+// the 32 pixels x 32 channels of one operand are 1 KiB in a row; d3 and d4 are written, and read, only for rows in
+// which one of them is not zero (|x| >= 16 in 16.16).
+#include "ds_common.h"
+#include "ds_epilogue.h"
+
+namespace ds {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+constexpr int kDigits = 5;          // 7-bit digits of an int32 activation
+constexpr int kMfmaMaxK = 1 << 17;  // 64 * 127 * K stays within int32
+
+// Which products a launch forms (MfmaMode): the widest shift that occurs, and the activations' width.
+enum { kI32S15 = 0, kI32S7 = 1, kI32S4 = 2, kI8S8 = 3, kI8S4 = 4, kI8S3 = 5 };
+__host__ __device__ constexpr int mode_groups(int mode)
+{
+    return mode == kI32S15 ? 4 : (mode == kI32S7 || mode == kI8S8) ? 2 : 1;
+}
+__host__ __device__ constexpr bool mode_i8(int mode) { return mode >= kI8S8; }
+
+// The reduction in blocks of 32 activation bytes that lie side by side: 32 channels of one tap, or, where a pixel has
+// at most 16 channels, 32 / cp taps of one filter row (cp channels each).
+struct MfmaGeom {
+    int cp, cb, taps, fwg, kb, ntiles;
+};
+inline MfmaGeom mfma_geom(int N, int C, int FH, int FW)
+{
+    MfmaGeom g;
+    g.cp = C <= 4 ? 4 : C <= 8 ? 8 : C <= 16 ? 16 : 32;
+    if (FH * FW == 1) g.cp = 32;
+    g.cb = ceil_div(C, g.cp);
+    g.taps = 32 / g.cp;
+    g.fwg = ceil_div(FW, g.taps);
+    g.kb = g.cb * FH * g.fwg;
+    g.ntiles = ceil_div(N, 64) * 2;
+    return g;
+}
+inline size_t mfma_blob_corr(const MfmaGeom &g, int mode) { return (size_t)g.ntiles * g.kb * mode_groups(mode) * 1024; }
+
+// One thread per (channel tile, block, lane): the 16 selector bytes per group of its fragment.
+__global__ __launch_bounds__(256) void mfma_tile_kernel(const int32_t *__restrict__ w_ref, v4i *__restrict__ blob, int N,
+                                                        int C, int FH, int FW, int bits, int mode, int cp, int cb,
+                                                        int taps, int fwg, int kb, long total)
+{
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= total) return;
+    const int lane = (int)(t & 63);
+    const long tile_kb = t >> 6;
+    const int b = (int)(tile_kb % kb), tile = (int)(tile_kb / kb);
+    const int fg = b % fwg, fh = b / fwg % FH, c0 = b / fwg / FH * cp;
+    const int n = tile * 32 + (lane & 31);
+    const int K = C * FH * FW, num = codes_per_word(bits), comm = ceil_div(K, num);
+    const int groups = mode_groups(mode);
+    uint32_t sel[4][4];
+    for (int g = 0; g < 4; ++g)
+        for (int w = 0; w < 4; ++w) sel[g][w] = 0x0c0c0c0cu;
+    for (int i = 0; i < 16; ++i) {
+        const int kk = (lane >> 5) * 16 + i;
+        const int c = c0 + kk % cp, fw = fg * taps + kk / cp;
+        if (n >= N || c >= C || fw >= FW) continue;
+        const int k = (c * FH + fh) * FW + fw;
+        const uint32_t code = (uint32_t)w_ref[(long)n * comm + k / num] >> ((k % num) * (bits + 1));
+        uint32_t s = code & ((1u << bits) - 1u);
+        const uint32_t neg = ((code >> bits) & 1u) ? 0u : 4u;
+        if (s >= 32) continue;  // a zero weight
+        uint32_t g, l;
+        if (mode_i8(mode)) {
+            s = s < 7 ? s : 7;
+            g = s >> 2;
+            l = s & 3;
+        } else {
+            g = s < 4 ? 0 : s < 7 ? 1 : s < 11 ? 2 : 3;
+            l = s - (g == 0 ? 0 : g == 1 ? 4 : g == 2 ? 7 : 11);
+        }
+        if (g >= (uint32_t)groups || l > 3) continue;  // the caller vouches that it does not occur
+        const int at = (i & 3) * 8;
+        sel[g][i >> 2] = (sel[g][i >> 2] & ~(255u << at)) | ((l | neg) << at);
+    }
+    for (int g = 0; g < groups; ++g) {
+        v4i v;
+        for (int w = 0; w < 4; ++w) v[w] = (int)sel[g][w];
+        blob[(tile_kb * groups + g) * 64 + lane] = v;
+    }
+}
+
+// Per channel, what the +128 on the shifted 8-bit activations adds: sum_k sgn * 2^(7-s) over s >= 1.
+__global__ __launch_bounds__(64) void mfma_corr_kernel(const int32_t *__restrict__ w_ref, int32_t *__restrict__ corr, int N,
+                                                       int K, int bits)
+{
+    const int n = blockIdx.x, num = codes_per_word(bits), comm = ceil_div(K, num);
+    int sum = 0;
+    if (n < N)
+        for (int k = threadIdx.x; k < K; k += 64) {
+            const uint32_t code = (uint32_t)w_ref[(long)n * comm + k / num] >> ((k % num) * (bits + 1));
+            uint32_t s = code & ((1u << bits) - 1u);
+            if (s == 0 || s >= 32) continue;
+            s = s < 7 ? s : 7;
+            const int v = 1 << (7 - s);
+            sum += ((code >> bits) & 1u) ? v : -v;
+        }
+    for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o);
+    if (threadIdx.x == 0) corr[n] = sum;
+}
+
+// ---------------------------------------------------------------------------------------------
+// activations -> operand layout
+// ---------------------------------------------------------------------------------------------
+
+// Layout of the prepared activations, shared by the pass that writes them and the contraction.
+struct MfmaX {
+    int Hp, Wp, cp, cb, digits;
+    int dstride, cbstride, rstride;  // bytes between digits, 32-channel blocks, rows
+    int fy, cbf;                     // flag bytes per row, channel blocks that each of them covers
+    long rows;
+    size_t planes;                   // bytes of the digits; the flags follow
+};
+inline MfmaX mfma_x(int Nb, int C, int Hp, int Wp, const MfmaGeom &g, bool i8)
+{
+    MfmaX x;
+    x.Hp = Hp;
+    x.Wp = Wp;
+    x.cp = g.cp;
+    x.cb = g.cb;
+    x.digits = i8 ? 1 : kDigits;
+    x.dstride = Wp * g.cp;
+    x.cbstride = x.dstride * x.digits;
+    x.rstride = x.cbstride * g.cb;
+    x.rows = (long)Nb * Hp;
+    // enough workgroups to fill the chip: a row's channel blocks are shared out over up to eight of them
+    int fy = 1;
+    while (fy < 8 && x.rows * fy < 1024 && g.cb >= 2 * fy) fy *= 2;
+    x.cbf = ceil_div(g.cb, fy);
+    x.fy = ceil_div(g.cb, x.cbf);
+    // a block of several taps may read up to 32 bytes past the last pixel
+    x.planes = align_up((size_t)x.rows * x.rstride + 64, 256);
+    return x;
+}
+
+enum { kSrcF32 = 0, kSrcI32 = 1, kSrcI8 = 2 };
+
+struct PrepArgs {
+    const void *x;
+    int8_t *dst;
+    uint8_t *flags;
+    MfmaX lay;
+    int C, H, W, ph, pw;
+    int M, K;        // rows of a matrix: image n holds rows 64 n .. 64 n + 63, C = K
+    int vec;         // a matrix whose rows can be read four values at a time
+    QuantSpec spec;
+};
+
+template <int SRC>
+__device__ __forceinline__ int32_t prep_value(const void *x, size_t i, const QuantSpec &spec)
+{
+    if (SRC == kSrcF32) return quantize_one(((const float *)x)[i], spec);
+    if (SRC == kSrcI32) return ((const int32_t *)x)[i];
+    return ((const int8_t *)x)[i];
+}
+
+__device__ __forceinline__ void digits_of(int32_t v, int32_t d[kDigits])
+{
+    const int32_t b = v >> 14;
+    d[0] = v & 127;
+    d[1] = (v >> 7) & 127;
+    d[2] = (int32_t)((uint32_t)b << 25) >> 25;
+    const int32_t c = (b - d[2]) >> 7;
+    d[3] = (int32_t)((uint32_t)c << 25) >> 25;
+    d[4] = (c - d[3]) >> 7;
+}
+
+// Workgroup (row, part): CH channels of one pixel per thread and step, two threads side by side for the halves of a
+// 32-channel block, so that loads run along the row and stores are contiguous.  Bound by memory: 4 bytes read and 3
+// written per element (5 where a digit d3 or d4 of the row is not zero: a second sweep writes those).
+template <int SRC, bool I8, bool MATRIX, int CH>
+__global__ __launch_bounds__(256) void mfma_prepare_kernel(PrepArgs a)
+{
+    const MfmaX &L = a.lay;
+    const int row = blockIdx.x, part = blockIdx.y;
+    const int n = row / L.Hp, hp = row - n * L.Hp, h = hp - a.ph;
+    const int halves = CH == 16 && L.cp == 32 ? 2 : 1;
+    const int cb0 = part * L.cbf, cb1 = cb0 + L.cbf < L.cb ? cb0 + L.cbf : L.cb;
+    const int items = (cb1 - cb0) * L.Wp * halves;
+    int8_t *dst = a.dst + (size_t)row * L.rstride;
+    const bool row_in = MATRIX || (unsigned)h < (unsigned)a.H;
+    int high = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+        for (int t = threadIdx.x; t < items; t += 256) {
+            const int half = halves == 2 ? t & 1 : 0;
+            const int tw = halves == 2 ? t >> 1 : t;
+            const int cbi = tw / L.Wp, wp = tw - cbi * L.Wp, cb = cb0 + cbi;
+            const int c0 = cb * L.cp + half * CH;
+            int32_t v[CH];
+            if (MATRIX) {
+                const int m = n * 64 + wp;
+                const size_t base = (size_t)m * a.K + c0;
+                if (a.vec && m < a.M && c0 + CH <= a.K) {
+                    // rows and base aligned: four values per load
+#pragma unroll
+                    for (int q = 0; q < CH / 4; ++q) {
+                        const v4i r = *(const v4i *)((const int32_t *)a.x + base + 4 * q);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            v[4 * q + i] = SRC == kSrcF32 ? quantize_one(__int_as_float(r[i]), a.spec) : r[i];
+                    }
+                } else
+#pragma unroll
+                for (int i = 0; i < CH; ++i)
+                    v[i] = (m < a.M && c0 + i < a.K) ? prep_value<SRC>(a.x, base + i, a.spec) : 0;
+            } else {
+                const int w = wp - a.pw;
+                const bool in = row_in && (unsigned)w < (unsigned)a.W;
+                const size_t base = ((size_t)n * a.C + c0) * a.H * a.W + (size_t)h * a.W + w;
+                const size_t plane = (size_t)a.H * a.W;
+#pragma unroll
+                for (int i = 0; i < CH; ++i)
+                    v[i] = (in && c0 + i < a.C) ? prep_value<SRC>(a.x, base + i * plane, a.spec) : 0;
+            }
+            int8_t *o = dst + (size_t)cb * L.cbstride + wp * L.cp + half * CH;
+            constexpr int D = I8 ? 1 : kDigits;
+            uint32_t words[D][CH / 4];
+#pragma unroll
+            for (int q = 0; q < CH / 4; ++q) {
+#pragma unroll
+                for (int d = 0; d < D; ++d) words[d][q] = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    int32_t dg[kDigits];
+                    if (I8)
+                        dg[0] = v[q * 4 + i];
+                    else
+                        digits_of(v[q * 4 + i], dg);
+#pragma unroll
+                    for (int d = 0; d < D; ++d) words[d][q] |= ((uint32_t)dg[d] & 255u) << (8 * i);
+                }
+            }
+            const int lo = pass == 0 ? 0 : 3, hi = I8 ? 1 : pass == 0 ? 3 : 5;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (d >= lo && d < hi)
+#pragma unroll
+                    for (int q = 0; q < CH / 4; ++q) ((uint32_t *)(o + (size_t)d * L.dstride))[q] = words[d][q];
+                if (d >= 3)
+#pragma unroll
+                    for (int q = 0; q < CH / 4; ++q) high |= words[d][q] != 0;
+            }
+        }
+        if (I8) return;
+        if (pass == 0) {
+            high = __syncthreads_or(high);
+            if (threadIdx.x == 0) a.flags[(size_t)row * L.fy + part] = high ? 1 : 0;
+            if (!high) return;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// the contraction
+// ---------------------------------------------------------------------------------------------
+
+struct MfmaArgs {
+    const int8_t *x;
+    const uint8_t *flags;
+    const int8_t *blob;
+    const int32_t *corr, *bias;
+    int32_t *y;                 // int32 sums, or
+    float *out;                 // the float result and / or
+    void *q;                    // the next layer's input
+    const float *scale, *shift, *residual;
+    MfmaX lay;
+    int N, KB, FH, fwg, tapstep;
+    int OH, OW, sh, sw, crop_h, crop_w;
+    uint32_t pixels;
+    int ks, tc, ctiles, ptiles;   // K parts, channel tiles per workgroup, workgroups along channels and pixels
+    long ostride_n;
+    int ostride_c;
+    int matrix;                 // pixels are matrix rows
+    int relu, q_bytes, qHp, qWp, qph, qpw;
+    float inv;
+    QuantSpec qspec;
+    FastDiv by_image, by_row, by_ctiles;
+};
+
+__device__ __forceinline__ v4i perm4(uint32_t neg, uint32_t pos, v4i sel)
+{
+    v4i r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (int)__builtin_amdgcn_perm(neg, pos, (uint32_t)sel[i]);
+    return r;
+}
+__device__ __forceinline__ v4i and4(v4i v, uint32_t m)
+{
+    v4i r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = v[i] & (int)m;
+    return r;
+}
+__device__ __forceinline__ v4i or4(v4i a, v4i b)
+{
+    v4i r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = a[i] | b[i];
+    return r;
+}
+
+// Look-up words of the weight planes: byte l = the value of the group's l-th shift, for positive and negative weights.
+constexpr uint32_t kPosLo = 0x08102040u, kNegLo = 0xf8f0e0c0u;   // r = 0..3: 64, 32, 16, 8
+constexpr uint32_t kPosHi = 0x00010204u, kNegHi = 0x00fffefcu;   // r = 4..6: 4, 2, 1
+constexpr uint32_t kPos14 = 0x40000000u, kNeg14 = 0xc0000000u;   // s = 14, the last of its group: 64
+__host__ __device__ constexpr uint32_t low_bytes(uint32_t v, int n) { return n >= 4 ? v : v & ((1u << (8 * n)) - 1u); }
+
+template <int MODE, int MT, int NT>
+struct Operands {
+    static constexpr int G = mode_groups(MODE), D = mode_i8(MODE) ? 1 : 3;
+    v4i sel[MT][G];
+    v4i dig[NT][D];
+};
+
+template <int MT, int NT>
+__device__ __forceinline__ void product(v16i (&acc)[MT][NT], const v4i (&w)[MT], const v4i (&b)[NT])
+{
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int p = 0; p < NT; ++p) acc[m][p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[m], b[p], acc[m][p], 0, 0, 0);
+}
+
+// The seven bit products of digit q: adds to an, leaves the full weight plane 2^(6-r) in w.
+template <int MODE, int MT, int NT>
+__device__ __forceinline__ void bit_products(const Operands<MODE, MT, NT> &o, int q, v16i (&an)[MT][NT], v4i (&w)[MT])
+{
+    v4i b[NT], w3[MT];
+#pragma unroll
+    for (int j = 0; j < 7; ++j) {
+        // shifts of at most 3: bits 3 to 6 meet the same weights
+        if (MODE == kI32S4 && j > 3) break;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            if (j <= 3) {
+                w[m] = perm4(low_bytes(kNegLo, j + 1), low_bytes(kPosLo, j + 1), o.sel[m][2 * q]);
+                w3[m] = w[m];
+            } else if constexpr (Operands<MODE, MT, NT>::G > 1) {
+                w[m] = or4(w3[m], perm4(low_bytes(kNegHi, j - 3), low_bytes(kPosHi, j - 3), o.sel[m][2 * q + 1]));
+            }
+        }
+        const uint32_t mask = MODE == kI32S4 && j == 3 ? 0x78787878u : 0x01010101u << j;
+#pragma unroll
+        for (int p = 0; p < NT; ++p) b[p] = and4(o.dig[p][q], mask);
+        product<MT, NT>(an, w, b);
+    }
+}
+
+template <int MODE, int MT, int NT>
+__device__ __forceinline__ void digit_product(const Operands<MODE, MT, NT> &o, int d, v16i (&acc)[MT][NT], const v4i (&w)[MT])
+{
+    v4i b[NT];
+#pragma unroll
+    for (int p = 0; p < NT; ++p) b[p] = o.dig[p][d];
+    product<MT, NT>(acc, w, b);
+}
+
+template <int MODE, int MT, int NT>
+__device__ __forceinline__ void block_i8(const Operands<MODE, MT, NT> &o, v16i (&acc)[MT][NT])
+{
+    constexpr int S = MODE == kI8S8 ? 8 : MODE == kI8S4 ? 4 : 3;
+    v4i b[NT], u[NT], w[MT];
+#pragma unroll
+    for (int p = 0; p < NT; ++p)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[p][i] = o.dig[p][0][i] ^ (int)0x80808080;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+            w[m] = perm4(0xffu << (8 * (s & 3)), 0x01u << (8 * (s & 3)), o.sel[m][s >> 2]);
+#pragma unroll
+        for (int p = 0; p < NT; ++p) {
+            if (s == 0)
+                b[p] = o.dig[p][0];
+            else
+#pragma unroll
+                for (int i = 0; i < 4; ++i) b[p][i] = (int)(((uint32_t)u[p][i] >> s) & ((0xffu >> s) * 0x01010101u));
+        }
+        product<MT, NT>(acc, w, b);
+    }
+}
+
+// Position in the reduction: blocks run over (32-channel block, filter row, group of taps), the last fastest.
+struct KPos {
+    int cb, fh, fg, off;
+};
+
+template <int MODE, int MT, int NT>
+__device__ __forceinline__ void load_digits(const MfmaArgs &a, Operands<MODE, MT, NT> &o, int from, int to, const KPos &k,
+                                            const uint32_t (&px)[NT])
+{
+    const int8_t *xb = a.x + k.off;
+#pragma unroll
+    for (int d = 0; d < Operands<MODE, MT, NT>::D; ++d)
+        if (d >= from && d < to)
+#pragma unroll
+            for (int p = 0; p < NT; ++p) o.dig[p][d] = *(const v4i *)(xb + d * a.lay.dstride + px[p]);
+}
+template <int MODE, int MT, int NT>
+__device__ __forceinline__ void load_selectors(Operands<MODE, MT, NT> &o, int from, int to, const int8_t *w, int wtile, int kb)
+{
+    constexpr int G = Operands<MODE, MT, NT>::G;
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+        if (g >= from && g < to)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) o.sel[m][g] = *(const v4i *)(w + (size_t)m * wtile + (kb * G + g) * 1024);
+}
+template <int MODE, int MT, int NT>
+__device__ __forceinline__ void load_block(const MfmaArgs &a, Operands<MODE, MT, NT> &o, const int8_t *w, int wtile, int kb,
+                                           const KPos &k, const uint32_t (&px)[NT])
+{
+    load_selectors<MODE, MT, NT>(o, 0, 4, w, wtile, kb);
+    load_digits<MODE, MT, NT>(a, o, 0, 3, k, px);
+}
+
+__device__ __forceinline__ void k_start(const MfmaArgs &a, KPos &k, int kb)
+{
+    const int per = a.FH * a.fwg;
+    k.cb = kb / per;
+    const int rest = kb - k.cb * per;
+    k.fh = rest / a.fwg;
+    k.fg = rest - k.fh * a.fwg;
+    k.off = k.cb * a.lay.cbstride + k.fh * a.lay.rstride + k.fg * a.tapstep;
+}
+__device__ __forceinline__ void k_next(const MfmaArgs &a, KPos &k)
+{
+    k.off += a.tapstep;
+    if (++k.fg == a.fwg) {
+        k.fg = 0;
+        k.off += a.lay.rstride - a.fwg * a.tapstep;
+        if (++k.fh == a.FH) {
+            k.fh = 0;
+            ++k.cb;
+            k.off += a.lay.cbstride - a.FH * a.lay.rstride;
+        }
+    }
+}
+
+// Digits d3 and d4 of the rows that have any: what they add to the sums, modulo 2^32.
+template <int MODE, int MT, int NT>
+__device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[64], int lane, const int8_t *w, int wtile,
+                                            int kb0, int kb1, const uint32_t (&px)[NT], const uint32_t (&row)[NT])
+{
+    constexpr int G = mode_groups(MODE);
+#pragma unroll
+    for (int i = 0; i < MT * NT * 16; ++i) slot[i][lane] = 0;
+    for (int d = 3; d <= 4; ++d) {
+#pragma unroll 1
+        for (int q = 0; q < (MODE == kI32S15 ? 3 : 1); ++q) {
+            v16i acc[MT][NT] = {};
+            KPos k;
+            k_start(a, k, kb0);
+#pragma unroll 1
+            for (int kb = kb0; kb < kb1; ++kb, k_next(a, k)) {
+                v4i b[NT], wv[MT];
+#pragma unroll
+                for (int p = 0; p < NT; ++p) {
+                    const bool on = a.flags[(size_t)(row[p] + k.fh) * a.lay.fy + k.cb / a.lay.cbf] != 0;
+                    b[p] = v4i{0, 0, 0, 0};
+                    if (on) b[p] = *(const v4i *)(a.x + k.off + d * a.lay.dstride + px[p]);
+                }
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    const int8_t *s = w + (size_t)m * wtile + kb * G * 1024;
+                    if (q == 2) {
+                        wv[m] = perm4(kNeg14, kPos14, *(const v4i *)(s + 3 * 1024));
+                    } else {
+                        wv[m] = perm4(kNegLo, kPosLo, *(const v4i *)(s + (G > 2 ? 2 * q : 0) * 1024));
+                        if (G > 1)
+                            wv[m] = or4(wv[m], perm4(kNegHi, kPosHi, *(const v4i *)(s + (G > 2 ? 2 * q + 1 : 1) * 1024)));
+                    }
+                }
+                product<MT, NT>(acc, wv, b);
+            }
+            const int by = 7 * (d - q - 1) + 1;
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int p = 0; p < NT; ++p)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        slot[(m * NT + p) * 16 + i][lane] += (int)((uint32_t)acc[m][p][i] << by);
+        }
+    }
+}
+
+struct PixelAt {
+    uint32_t n, oh, ow;
+};
+__device__ __forceinline__ PixelAt pixel_at(const MfmaArgs &a, uint32_t p)
+{
+    PixelAt r;
+    r.n = div_by(p, a.by_image);
+    const uint32_t rem = p - r.n * a.by_image.d;
+    r.oh = div_by(rem, a.by_row);
+    r.ow = rem - r.oh * a.by_row.d;
+    return r;
+}
+
+// What follows the sums of R x 4 channels (R groups of four, 8 apart) at one pixel: the per-channel constants, then the
+// residuals, are all asked for before the first value is stored (one wait each, not one per value).
+template <int R>
+struct ChannelTail {
+    int32_t add[R * 4];
+    float scale[R * 4], shift[R * 4];
+};
+template <int R>
+__device__ __forceinline__ void load_tail(const MfmaArgs &a, ChannelTail<R> &t, int ch0)
+{
+#pragma unroll
+    for (int i = 0; i < R * 4; ++i) {
+        const int ch = ch0 + 8 * (i >> 2) + (i & 3), c = ch < a.N ? ch : a.N - 1;
+        t.add[i] = (a.bias ? a.bias[c] : 0) - (a.corr ? a.corr[c] : 0);
+        t.scale[i] = a.scale ? a.scale[c] : 1.0f;
+        t.shift[i] = a.shift ? a.shift[c] : 0.0f;
+    }
+}
+struct OutAt {
+    size_t i;         // of channel 0 in y / out / residual
+    size_t j;         // of channel 0 in q
+    bool in;
+};
+__device__ __forceinline__ OutAt out_at(const MfmaArgs &a, const PixelAt &at, uint32_t p)
+{
+    OutAt o;
+    o.in = p < a.pixels;
+    o.i = a.matrix ? (size_t)p * a.N : (size_t)at.n * a.ostride_n + (at.oh * a.OW + at.ow);
+    o.j = ((size_t)at.n * a.N * a.qHp + at.oh + a.qph) * a.qWp + at.ow + a.qpw;
+    return o;
+}
+template <int R>
+__device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail<R> &t, const int32_t (&sum)[R * 4], int ch0,
+                                           const OutAt &o)
+{
+    const int qplane = a.qHp * a.qWp;
+    float res[R * 4];
+    if (a.residual) {
+#pragma unroll
+        for (int i = 0; i < R * 4; ++i) {
+            const int ch = ch0 + 8 * (i >> 2) + (i & 3);
+            res[i] = o.in && ch < a.N ? a.residual[o.i + (size_t)ch * a.ostride_c] : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < R * 4; ++i) {
+        const int ch = ch0 + 8 * (i >> 2) + (i & 3);
+        if (!o.in || ch >= a.N) continue;
+        const int32_t v = sum[i] + t.add[i];
+        const size_t at = o.i + (size_t)ch * a.ostride_c;
+        if (a.y) {
+            a.y[at] = v;
+            continue;
+        }
+        const float f = affine_one(v, a.inv, t.scale[i], t.shift[i], a.residual ? &res[i] : nullptr, a.relu);
+        if (a.out) a.out[at] = f;
+        if (a.q) {
+            const int32_t qv = quantize_one(f, a.qspec);
+            if (a.q_bytes == 1)
+                ((int8_t *)a.q)[o.j + (size_t)ch * qplane] = (int8_t)qv;
+            else
+                ((int32_t *)a.q)[o.j + (size_t)ch * qplane] = qv;
+        }
+    }
+}
+
+// Four waves per workgroup; a wave owns MT * 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
+// parts of a tile lie in one workgroup and meet in LDS).  No operand passes through LDS: activations and selectors are
+// fragments in memory already, each a contiguous KiB.
+template <int MODE, int MT, int NT>
+__global__ __launch_bounds__(256, 2) void mfma_kernel(MfmaArgs a)
+{
+    __shared__ int32_t part[4][MT * NT * 16][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // workgroups are dealt to the eight XCDs in turn: give each XCD neighbouring tiles
+    uint32_t wg = blockIdx.x;
+    const uint32_t per = gridDim.x >> 3;
+    if (wg < per * 8) wg = (wg & 7) * per + (wg >> 3);
+    const uint32_t pt = div_by_uniform(wg, a.by_ctiles);
+    const int ct = (int)(wg - pt * a.ctiles);
+    const int kpart = wave % a.ks, t = wave / a.ks;
+    const int pw = 4 / a.ks / a.tc;   // pixel tiles per workgroup
+    const int c0 = (ct * a.tc + t % a.tc) * MT * 32;
+    const uint32_t p0 = ((uint32_t)pt * pw + t / a.tc) * (NT * 32);
+    const int kb0 = (int)((long)a.KB * kpart / a.ks), kb1 = (int)((long)a.KB * (kpart + 1) / a.ks);
+
+    constexpr int G = mode_groups(MODE);
+    const int wtile = a.KB * G * 1024;
+    const bool live = c0 < a.N && p0 < a.pixels;
+    uint32_t pix[NT], px[NT], row[NT];
+#pragma unroll
+    for (int p = 0; p < NT; ++p) {
+        pix[p] = p0 + p * 32 + (lane & 31);
+        const uint32_t clamped = pix[p] < a.pixels ? pix[p] : a.pixels - 1;
+        const PixelAt at = pixel_at(a, clamped);
+        row[p] = at.n * a.lay.Hp + at.oh * a.sh + a.crop_h;
+        px[p] = row[p] * a.lay.rstride + (at.ow * a.sw + a.crop_w) * a.lay.cp + (lane >> 5) * 16;
+    }
+    v16i total[MT][NT] = {};
+    if (live && kb0 < kb1) {
+        const int8_t *wl = a.blob + (size_t)(c0 >> 5) * wtile + lane * 16;
+        bool high = false;
+        if constexpr (!mode_i8(MODE)) {
+            const uint32_t r0 = __builtin_amdgcn_readfirstlane(row[0]);
+            const uint32_t r1 = __builtin_amdgcn_readlane(row[NT - 1], 31) + a.FH;
+            int any = 0;
+            for (uint32_t i = r0 * a.lay.fy + lane; i < r1 * a.lay.fy; i += 64) any |= a.flags[i];
+            high = __any(any);
+            if (high) high_digits<MODE, MT, NT>(a, part[wave], lane, wl, wtile, kb0, kb1, px, row);
+        }
+        v16i acc[MT][NT] = {};
+        Operands<MODE, MT, NT> o0;
+        KPos k;
+        k_start(a, k, kb0);
+        int kb = kb0;
+        load_block<MODE, MT, NT>(a, o0, wl, wtile, kb, k, px);
+        if constexpr (mode_i8(MODE)) {
+            Operands<MODE, MT, NT> o1;
+            while (true) {
+                if (kb + 1 < kb1) {
+                    k_next(a, k);
+                    load_block<MODE, MT, NT>(a, o1, wl, wtile, kb + 1, k, px);
+                }
+                block_i8<MODE, MT, NT>(o0, acc);
+                if (++kb >= kb1) break;
+                if (kb + 1 < kb1) {
+                    k_next(a, k);
+                    load_block<MODE, MT, NT>(a, o0, wl, wtile, kb + 1, k, px);
+                }
+                block_i8<MODE, MT, NT>(o1, acc);
+                if (++kb >= kb1) break;
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int p = 0; p < NT; ++p) total[m][p] = acc[m][p];
+        } else {
+            // every operand is loaded again as soon as its last product is issued: the loads of the next block are
+            // in flight during this one's remaining products, with one set of registers
+            v16i a0[MT][NT] = {}, a1[MT][NT] = {};
+            while (true) {
+                v4i w[MT];
+                const bool more = kb + 1 < kb1;
+                if (more) k_next(a, k);
+                const int kn = more ? kb + 1 : kb;
+                bit_products<MODE, MT, NT>(o0, 0, acc, w);
+                if constexpr (MODE == kI32S15) {
+                    load_selectors<MODE, MT, NT>(o0, 0, 2, wl, wtile, kn);
+                    load_digits<MODE, MT, NT>(a, o0, 0, 1, k, px);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                digit_product<MODE, MT, NT>(o0, 1, a0, w);
+                digit_product<MODE, MT, NT>(o0, 2, a1, w);
+                if constexpr (MODE == kI32S15) {
+                    bit_products<MODE, MT, NT>(o0, 1, acc, w);
+                    load_selectors<MODE, MT, NT>(o0, 2, 3, wl, wtile, kn);
+                    load_digits<MODE, MT, NT>(a, o0, 1, 2, k, px);
+                    __builtin_amdgcn_sched_barrier(0);
+                    digit_product<MODE, MT, NT>(o0, 2, a0, w);
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) w[m] = perm4(kNeg14, kPos14, o0.sel[m][3]);
+                    digit_product<MODE, MT, NT>(o0, 2, acc, w);
+                    load_selectors<MODE, MT, NT>(o0, 3, 4, wl, wtile, kn);
+                    load_digits<MODE, MT, NT>(a, o0, 2, 3, k, px);
+                } else {
+                    load_block<MODE, MT, NT>(a, o0, wl, wtile, kn, k, px);
+                }
+                if (!more) break;
+                ++kb;
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int p = 0; p < NT; ++p)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        total[m][p][i] = (acc[m][p][i] >> 6) + (int)((uint32_t)a0[m][p][i] << 1) +
+                                         (int)((uint32_t)a1[m][p][i] << 8);
+            if (high)
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int p = 0; p < NT; ++p)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) total[m][p][i] += part[wave][(m * NT + p) * 16 + i][lane];
+        }
+    }
+    const int chl = c0 + 4 * (lane >> 5);
+    if (a.ks == 1) {
+        if (!live) return;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            ChannelTail<4> t;
+            load_tail<4>(a, t, chl + m * 32);
+#pragma unroll
+            for (int p = 0; p < NT; ++p) {
+                int32_t v[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] = total[m][p][i];
+                store_tail<4>(a, t, v, chl + m * 32, out_at(a, pixel_at(a, pix[p]), pix[p]));
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int p = 0; p < NT; ++p)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) part[wave][(m * NT + p) * 16 + i][lane] = total[m][p][i];
+    __syncthreads();
+    if (!live) return;
+    // the ks waves of a tile share its epilogue, in halves of 32 x 32 values
+    const int units = MT * NT * 2 / a.ks;
+    for (int u = kpart * units; u < (kpart + 1) * units; ++u) {
+        const int m = u / (NT * 2), p = (u >> 1) % NT;
+        const int ch = chl + m * 32 + (u & 1) * 16;
+        ChannelTail<2> tl;
+        load_tail<2>(a, tl, ch);
+        int32_t v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            v[i] = 0;
+            for (int s = 0; s < a.ks; ++s) v[i] += part[t * a.ks + s][u * 8 + i][lane];
+        }
+        const uint32_t pp = p0 + p * 32 + (lane & 31);
+        store_tail<2>(a, tl, v, ch, out_at(a, pixel_at(a, pp), pp));
+    }
+}
+
+// The padding of the next layer's input.
+template <typename Q>
+__global__ __launch_bounds__(256) void mfma_border_kernel(Q *__restrict__ q, int planes, int Hp, int Wp, int ph, int pw)
+{
+    const int rows = 2 * ph * Wp, side = 2 * pw * (Hp - 2 * ph), per = rows + side;
+    const long total = (long)planes * per;
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long)gridDim.x * 256) {
+        const long plane = i / per;
+        int r = (int)(i - plane * per), h, w;
+        if (r < rows) {
+            h = r / Wp;
+            w = r - h * Wp;
+            if (h >= ph) h += Hp - 2 * ph;
+        } else {
+            r -= rows;
+            h = r / (2 * pw);
+            w = r - h * 2 * pw;
+            h += ph;
+            if (w >= pw) w += Wp - 2 * pw;
+        }
+        q[(plane * Hp + h) * Wp + w] = 0;
+    }
+}
+
+template <int MODE, int MT, int NT>
+static int launch_mfma(MfmaArgs &a, hipStream_t st)
+{
+    const int waves = device_cus() * 8;
+    const int ctiles32 = ceil_div(a.N, MT * 32);
+    const long tiles = (long)ctiles32 * ceil_div((int)a.pixels, NT * 32);
+    // fewer tiles than three for every wave slot: the waves of a workgroup share tiles along the reduction
+    a.ks = tiles >= 3L * waves ? 1 : tiles >= 3L * waves / 2 ? 2 : 4;
+    while (a.ks > 1 && a.KB < 2 * a.ks) a.ks >>= 1;
+    a.tc = (a.ks <= 2 && ctiles32 > 1) ? 2 : 1;
+    a.ctiles = ceil_div(ctiles32, a.tc);
+    a.ptiles = ceil_div((int)a.pixels, NT * 32 * (4 / a.ks / a.tc));
+    a.by_ctiles = fast_div((uint32_t)a.ctiles);
+    hipLaunchKernelGGL((mfma_kernel<MODE, MT, NT>), dim3((unsigned)(a.ctiles * a.ptiles)), dim3(256), 0, st, a);
+    return launch_status();
+}
+
+template <int SRC, bool I8>
+static int launch_prepare(const PrepArgs &a, bool matrix, hipStream_t st)
+{
+    const dim3 grid((unsigned)a.lay.rows, (unsigned)a.lay.fy);
+    if (matrix)
+        hipLaunchKernelGGL((mfma_prepare_kernel<SRC, I8, true, 16>), grid, dim3(256), 0, st, a);
+    else if (a.lay.cp >= 16)
+        hipLaunchKernelGGL((mfma_prepare_kernel<SRC, I8, false, 16>), grid, dim3(256), 0, st, a);
+    else if (a.lay.cp == 8)
+        hipLaunchKernelGGL((mfma_prepare_kernel<SRC, I8, false, 8>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((mfma_prepare_kernel<SRC, I8, false, 4>), grid, dim3(256), 0, st, a);
+    return launch_status();
+}
+
+// The mode of a layer, or -1: the largest shift among its non-zero weights and the activations' width decide.
+static int mode_of(int max_shift, int x_bytes)
+{
+    if (max_shift < 0 || max_shift > 31) return -1;
+    if (x_bytes == 1) return max_shift <= 2 ? kI8S3 : max_shift <= 3 ? kI8S4 : kI8S8;
+    if (x_bytes != 4) return -1;
+    return max_shift <= 3 ? kI32S4 : max_shift <= 6 ? kI32S7 : max_shift <= 14 ? kI32S15 : -1;
+}
+
+}  // namespace ds
+
+using namespace ds;
+
+DS_EXPORT size_t ds_mfma_weight_bytes(int N, int C, int FH, int FW, int max_shift, int x_bytes)
+{
+    const int mode = mode_of(max_shift, x_bytes);
+    if (mode < 0 || N <= 0 || C <= 0 || FH <= 0 || FW <= 0) return 0;
+    if ((double)C * FH * FW > kMfmaMaxK) return 0;
+    const MfmaGeom g = mfma_geom(N, C, FH, FW);
+    if ((double)g.kb * mode_groups(mode) * 1024 > (double)(1u << 30)) return 0;   // 32-bit offsets within a tile
+    return mfma_blob_corr(g, mode) + (size_t)g.ntiles * 32 * 4;
+}
+
+DS_EXPORT int ds_mfma_tile_weights_i32(const int32_t *w_ref, void *blob, int N, int C, int FH, int FW, int bits,
+                                       int max_shift, int x_bytes, ds_stream_t stream)
+{
+    if (!w_ref || !blob) return DS_EINVAL;
+    if (bits < 1 || bits > 6) return DS_EBITS;
+    if (ds_mfma_weight_bytes(N, C, FH, FW, max_shift, x_bytes) == 0) return DS_EINVAL;
+    const int mode = mode_of(max_shift, x_bytes);
+    const MfmaGeom g = mfma_geom(N, C, FH, FW);
+    hipStream_t st = (hipStream_t)stream;
+    const long total = (long)g.ntiles * g.kb * 64;
+    hipLaunchKernelGGL(mfma_tile_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, w_ref, (v4i *)blob, N, C,
+                       FH, FW, bits, mode, g.cp, g.cb, g.taps, g.fwg, g.kb, total);
+    int rc = launch_status();
+    if (rc != DS_OK || !mode_i8(mode)) return rc;
+    hipLaunchKernelGGL(mfma_corr_kernel, dim3((unsigned)(g.ntiles * 32)), dim3(64), 0, st, w_ref,
+                       (int32_t *)((char *)blob + mfma_blob_corr(g, mode)), N, C * FH * FW, bits);
+    return launch_status();
+}
+
+// Bytes of the prepared activations of a padded Nb x C x Hp x Wp input (a matrix of M rows and K columns: Nb =
+// ceil(M / 64), C = K, Hp = 1, Wp = 64); 0 where this path does not serve the layer.
+DS_EXPORT size_t ds_mfma_input_bytes(int Nb, int C, int Hp, int Wp, int FH, int FW, int x_bytes)
+{
+    if (Nb <= 0 || C <= 0 || Hp <= 0 || Wp <= 0 || FH <= 0 || FW <= 0 || (x_bytes != 1 && x_bytes != 4)) return 0;
+    if (Hp < FH || Wp < FW || (double)Nb * Hp > 2147483647.0) return 0;
+    const MfmaGeom g = mfma_geom(1, C, FH, FW);
+    const double bytes = (double)Nb * Hp * Wp * g.cb * g.cp * (x_bytes == 1 ? 1 : kDigits);
+    if (bytes > 2.0e9 || (double)Nb * C * Hp * Wp > 2.0e9) return 0;
+    const MfmaX x = mfma_x(Nb, C, Hp, Wp, g, x_bytes == 1);
+    return x.planes + align_up((size_t)x.rows * x.fy, 256);
+}
+
+DS_EXPORT int ds_mfma_prepare(const void *x, int source, void *dst, int Nb, int C, int H, int W, int ph, int pw, int FH,
+                              int FW, int matrix_rows, int x_bytes, int mode, int I, int F, ds_stream_t stream)
+{
+    if (!x || !dst || ph < 0 || pw < 0) return DS_EINVAL;
+    const bool matrix = matrix_rows > 0;
+    if (matrix && (H != 1 || W != 64 || ph || pw || Nb != ceil_div(matrix_rows, 64))) return DS_EINVAL;
+    if (source < kSrcF32 || source > kSrcI8 || (source == kSrcI32 && x_bytes != 4) || (source == kSrcI8 && x_bytes != 1))
+        return DS_EINVAL;
+    const int Hp = H + 2 * ph, Wp = W + 2 * pw;
+    if (ds_mfma_input_bytes(Nb, C, Hp, Wp, FH, FW, x_bytes) == 0) return DS_EINVAL;
+    PrepArgs a{};
+    const MfmaGeom g = mfma_geom(1, C, FH, FW);
+    a.lay = mfma_x(Nb, C, Hp, Wp, g, x_bytes == 1);
+    a.x = x;
+    a.dst = (int8_t *)dst;
+    a.flags = (uint8_t *)dst + a.lay.planes;
+    a.C = C;
+    a.H = H;
+    a.W = W;
+    a.ph = ph;
+    a.pw = pw;
+    a.M = matrix_rows;
+    a.K = C;
+    a.vec = matrix && source != kSrcI8 && C % 4 == 0 && (uintptr_t)x % 16 == 0;
+    a.spec = make_spec(I, F, mode);
+    hipStream_t st = (hipStream_t)stream;
+    if (source == kSrcI8) return launch_prepare<kSrcI8, true>(a, matrix, st);
+    if (source == kSrcI32) return launch_prepare<kSrcI32, false>(a, matrix, st);
+    return x_bytes == 1 ? launch_prepare<kSrcF32, true>(a, matrix, st) : launch_prepare<kSrcF32, false>(a, matrix, st);
+}
+
+DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32_t *bias, int32_t *y, float *out, void *q,
+                             const float *scale, const float *shift, const float *residual, int Nb, int C, int Hp, int Wp,
+                             int O, int FH, int FW, int sh, int sw, int crop_h, int crop_w, int prep_FH, int prep_FW,
+                             int matrix_rows, int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw,
+                             int q_bytes, ds_stream_t stream)
+{
+    const int border_kept = q_bytes & DS_Q_BORDER_KEPT;
+    q_bytes &= 0xff;
+    if (!prepared || !blob || (!y && !out && !q) || (y && (out || q))) return DS_EINVAL;
+    if (sh <= 0 || sw <= 0 || crop_h < 0 || crop_w < 0 || ph < 0 || pw < 0) return DS_EINVAL;
+    if (q && q_bytes != 1 && q_bytes != 4) return DS_EINVAL;
+    const int mode = mode_of(max_shift, x_bytes);
+    if (mode < 0 || ds_mfma_weight_bytes(O, C, FH, FW, max_shift, x_bytes) == 0) return DS_EINVAL;
+    if (ds_mfma_input_bytes(Nb, C, Hp, Wp, prep_FH, prep_FW, x_bytes) == 0) return DS_EINVAL;
+    const MfmaGeom g = mfma_geom(O, C, FH, FW);
+    if (g.cp != mfma_geom(O, C, prep_FH, prep_FW).cp) return DS_EINVAL;   // prepared for another grouping of taps
+    const int Hc = Hp - 2 * crop_h, Wc = Wp - 2 * crop_w;
+    if (Hc < FH || Wc < FW) return DS_EINVAL;
+    MfmaArgs a{};
+    a.lay = mfma_x(Nb, C, Hp, Wp, g, x_bytes == 1);
+    a.x = (const int8_t *)prepared;
+    a.flags = (const uint8_t *)prepared + a.lay.planes;
+    a.blob = (const int8_t *)blob;
+    a.corr = mode_i8(mode) ? (const int32_t *)((const char *)blob + mfma_blob_corr(g, mode)) : nullptr;
+    a.bias = bias;
+    a.y = y;
+    a.out = out;
+    a.q = q;
+    a.scale = scale;
+    a.shift = shift;
+    a.residual = residual;
+    a.N = O;
+    a.KB = g.kb;
+    a.FH = FH;
+    a.fwg = g.fwg;
+    a.tapstep = g.taps * g.cp;
+    a.sh = sh;
+    a.sw = sw;
+    a.crop_h = crop_h;
+    a.crop_w = crop_w;
+    a.OH = (Hc - FH) / sh + 1;
+    a.OW = (Wc - FW) / sw + 1;
+    const double pixels = (double)Nb * a.OH * a.OW;
+    if (pixels > 1.0e9 || (double)O * pixels > 8.0e9) return DS_EINVAL;
+    a.matrix = matrix_rows > 0;
+    a.pixels = a.matrix ? (uint32_t)matrix_rows : (uint32_t)pixels;
+    if (a.matrix && ((double)matrix_rows > pixels || q)) return DS_EINVAL;
+    a.ostride_c = a.matrix ? 1 : a.OH * a.OW;
+    a.ostride_n = (long)a.ostride_c * O;
+    a.relu = relu;
+    a.q_bytes = q_bytes;
+    a.qph = ph;
+    a.qpw = pw;
+    a.qHp = a.OH + 2 * ph;
+    a.qWp = a.OW + 2 * pw;
+    a.inv = ldexpf(1.0f, -F_in);
+    a.qspec = make_spec(I, F, DS_Q_ROUND_TO_FIXED);
+    a.by_image = fast_div((uint32_t)(a.OH * a.OW));
+    a.by_row = fast_div((uint32_t)a.OW);
+    hipStream_t st = (hipStream_t)stream;
+    if (q && !border_kept && (ph || pw)) {
+        const long cells = (long)Nb * O * (2L * ph * a.qWp + 2L * pw * a.OH);
+        const unsigned blocks = (unsigned)((cells + 255) / 256 < 4096 ? (cells + 255) / 256 : 4096);
+        if (q_bytes == 1)
+            hipLaunchKernelGGL((mfma_border_kernel<int8_t>), dim3(blocks), dim3(256), 0, st, (int8_t *)q, Nb * O, a.qHp,
+                               a.qWp, ph, pw);
+        else
+            hipLaunchKernelGGL((mfma_border_kernel<int32_t>), dim3(blocks), dim3(256), 0, st, (int32_t *)q, Nb * O, a.qHp,
+                               a.qWp, ph, pw);
+    }
+    switch (mode) {
+    case kI32S15: return launch_mfma<kI32S15, 1, 2>(a, st);
+    case kI32S7: return launch_mfma<kI32S7, 1, 2>(a, st);
+    case kI32S4: return launch_mfma<kI32S4, 1, 2>(a, st);
+    case kI8S8: return launch_mfma<kI8S8, 2, 2>(a, st);
+    case kI8S4: return launch_mfma<kI8S4, 2, 2>(a, st);
+    default: return launch_mfma<kI8S3, 2, 2>(a, st);
+    }
+}

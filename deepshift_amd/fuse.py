@@ -181,6 +181,39 @@ class FusedShortcutPair(nn.Module):
             spec["want_float"] = want_float
         return spec
 
+    def _on_matrix_cores(self, xq, cwa, cwb, residual_first, residual_shortcut):
+        """Both convolutions from one preparation of the input, or ``None`` where the matrix-core kernels have no
+        form for them (they group the taps of layers with few channels by the filter's size)."""
+        a, b = self.first, self.shortcut
+        if xq.shape[1] <= 16 or xq.numel() == 0:
+            return None
+        blobs = []
+        for fused, cw in ((a, cwa), (b, cwb)):
+            conv = fused.conv
+            top = kernels.mfma_shift(cw, 4)
+            blob = None if top is None else kernels._mfma_of(cw, top, 4, conv.out_channels, conv.in_channels,
+                                                            *conv.kernel_size)
+            if blob is None:
+                return None
+            blobs.append((top, blob))
+        prepared = kernels.mfma_prepare(xq, 0, a.conv.kernel_size, 4)
+        if prepared is None:
+            return None
+        results = []
+        for (top, blob), fused, cw, crop, residual in zip(blobs, (a, b), (cwa, cwb), ((0, 0), tuple(a.conv.padding)),
+                                                          (residual_first, residual_shortcut)):
+            conv = fused.conv
+            want_float, spec = True, None
+            if fused.emit is not None:
+                want_float = fused.emit[3]
+                spec = tuple(fused.emit[:3]) + (fused.emit[4] if len(fused.emit) == 5 else torch.int32,)
+            bias = conv._fixed_bias.get(conv.bias, conv.act_integer_bits, conv.act_fraction_bits, round_to_fixed=True)
+            out, q = kernels.mfma_conv2d(prepared, blob, bias, conv.out_channels, conv.kernel_size, conv.stride, top, crop,
+                                         a.conv.act_fraction_bits, fused.scale, fused.shift, residual, fused.relu, spec,
+                                         want_float, conv.__dict__.setdefault("_handoff_buffers", {}))
+            results.append(self._result(fused, out, q))
+        return tuple(results)
+
     @staticmethod
     def _result(fused, out, q):
         if fused.emit is None:
@@ -193,6 +226,9 @@ class FusedShortcutPair(nn.Module):
         if not _pairable_weights(cwa, cwb) or xq.dtype != torch.int32:
             raise RuntimeError("the weights of a paired shortcut changed in a way that needs another kernel; "
                                "fuse the model again")
+        both = self._on_matrix_cores(xq, cwa, cwb, residual_first, residual_shortcut)
+        if both is not None:
+            return both
         (oa, qa), (ob, qb) = kernels.conv2d_tiled_fused_pair(
             xq, a.conv.stride, a.conv.act_fraction_bits,
             self._spec(a, cwa, (0, 0), residual_first), self._spec(b, cwb, tuple(a.conv.padding), residual_shortcut))

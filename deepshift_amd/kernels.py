@@ -578,6 +578,21 @@ def linear_chain_status(ws_cache):
     return 0
 
 
+def linear_forward(x2d, conc_weight, bias, N, integer_bits, fraction_bits, round_to_fixed, relu=False):
+    """float32 ``[M, K]`` -> float32 ``[M, N]`` of a LinearShift layer from its packed weights, on whichever kernel
+    serves the size best: one launch for small problems, the matrix cores for others they have a form for, else
+    :func:`linear_layer` (same results)."""
+    M, K = x2d.shape
+    # the one-launch kernel's time grows with K whatever M is (1 x 4096 x 4096: 128 us against 51 here), and with the
+    # pairs (512 x 512 x 512: 21 against 25 us, 128 x 2048 x 1000: 42 against 30)
+    if not (small_linear_serves(M, K, N) and K <= 2048 and M * K * N <= 1 << 27):
+        route = mfma_route(x2d, 0, conc_weight, N, (1, 1), 4, integer_bits, fraction_bits, round_to_fixed)
+        if route is not None:
+            return mfma_conv2d(route[0], route[1], bias, N, (1, 1), 1, route[2], 0, fraction_bits, relu=relu)[0]
+    return linear_layer(x2d, _tiled_of(conc_weight, N, K), bias, N, kernel_bits(conc_weight), conc_weight.base,
+                        integer_bits, fraction_bits, round_to_fixed, relu)
+
+
 def linear_layer(x2d, tiled, bias, N, bits, base, integer_bits, fraction_bits, round_to_fixed, relu=False):
     """float32 ``[M, K]`` -> float32 ``[M, N]`` through the kernel path of a LinearShift layer: one
     launch for small problems, conversion + tiled GEMM + dequantisation otherwise (same results).
@@ -610,6 +625,9 @@ def linear(input, shift, sign, bias=None, conc_weight=None, use_cuda=True):
     N = shift.size(0)
     if bias is not None:
         bias = _require_device_i32("bias", bias)
+    y = _mfma_linear(input, conc_weight, bias, N)
+    if y is not None:
+        return y
     tiled = _tiled_of(conc_weight, N, K)
     ldx = (M + 63) // 64 * 64
     xT = torch.empty([K, ldx], dtype=torch.int32, device=input.device)
@@ -786,7 +804,10 @@ def conv2d_paired(x_padded, paired, bias, O, kernel_size, stride, field_bits, x_
     """Shift convolution on an already padded int8 NCHW input and the blob of
     :func:`tile_weights_paired`; the int32 result of :func:`conv2d_tiled` on the same values.
     ``x_bound``: a bound on ``|x|`` that the caller vouches for (128 always holds); a smaller one lets
-    the kernel widen its 16-bit sums less often."""
+    the kernel widen its 16-bit sums less often.  Activations that :func:`mfma_prepare` laid out go to the matrix
+    cores, with the blob and the ``max_shift`` of :func:`mfma_route` as ``paired`` and ``field_bits``."""
+    if isinstance(x_padded, Prepared):
+        return mfma_conv2d(x_padded, paired, bias, O, kernel_size, stride, field_bits)
     if x_padded.dtype != torch.int8 or not x_padded.is_cuda or x_padded.dim() != 4:
         raise TypeError("x_padded must be a 4-D int8 GPU tensor")
     x_padded = x_padded.contiguous()
@@ -812,7 +833,11 @@ def conv2d_paired_fused(x_padded, paired, bias, O, kernel_size, stride, field_bi
     result ``act(y / 2**F * scale[c] + shift[c] + residual)`` (``None`` unless ``want_float``) and, with
     ``emit = (padding, integer_bits, fraction_bits, dtype)``, the next shift convolution's round-to-fixed,
     zero padded input.  Bit-identical to :func:`conv2d_paired` followed by :func:`requantize_affine_pad`
-    / :func:`dequantize_affine`; no pre-fill, no atomics, the int32 sums are never stored."""
+    / :func:`dequantize_affine`; no pre-fill, no atomics, the int32 sums are never stored.  Prepared
+    activations as for :func:`conv2d_paired`."""
+    if isinstance(x_padded, Prepared):
+        return mfma_conv2d(x_padded, paired, bias, O, kernel_size, stride, field_bits, 0, fraction_bits_in, scale, shift,
+                           residual, relu, emit, want_float, q_cache)
     if x_padded.dtype != torch.int8 or not x_padded.is_cuda or x_padded.dim() != 4:
         raise TypeError("x_padded must be a 4-D int8 GPU tensor")
     x_padded = x_padded.contiguous()
@@ -864,6 +889,169 @@ def conv2d_paired_fused(x_padded, paired, bias, O, kernel_size, stride, field_bi
     return out, q
 
 
+# ---------------------------------------------------------------------------------------------
+# the matrix-core kernels
+# ---------------------------------------------------------------------------------------------
+
+_MFMA_SRC = {torch.float32: 0, torch.int32: 1, torch.int8: 2}
+
+
+def mfma_shift(conc_weight, x_bytes):
+    """The ``max_shift`` argument of the matrix-core entry points for this layer, or ``None`` if they do not serve
+    it: base 0, a known largest shift, and for int32 activations one of at most 14."""
+    if conc_weight is None or conc_weight.base != 0:
+        return None
+    top = getattr(conc_weight, "max_field", None)
+    if top is None or top < 0 or top > (14 if x_bytes == 4 else 31):
+        return None
+    return int(top)
+
+
+def _mfma_of(conc_weight, max_shift, x_bytes, N, C, FH=1, FW=1):
+    """The matrix-core blob of a ConcWeight, built once and cached on the object; ``None``: no such form."""
+    data = conc_weight.data
+    key = (data.data_ptr(), data._version, N, C, FH, FW, max_shift, conc_weight.bits)
+    cache = conc_weight.__dict__.setdefault("_mfma", {})
+    cached = cache.get(x_bytes)
+    if cached is None or cached[0] != key:
+        nbytes = _lib.lib().ds_mfma_weight_bytes(N, C, FH, FW, max_shift, x_bytes)
+        blob = None
+        if nbytes:
+            packed = _require_device_i32("packed", data)
+            num = 32 // (conc_weight.bits + 1)
+            want = N * ((C * FH * FW + num - 1) // num)
+            if packed.numel() != want:
+                raise ValueError("packed weight has %d words, expected %d" % (packed.numel(), want))
+            blob = torch.empty(nbytes, dtype=torch.uint8, device=data.device)
+            _lib.call("ds_mfma_tile_weights_i32", _lib.ptr(packed), _lib.ptr(blob), N, C, FH, FW,
+                      int(conc_weight.bits), max_shift, x_bytes, _lib.current_stream(data.device))
+        cached = cache[x_bytes] = (key, blob)
+    return cached[1]
+
+
+def mfma_route(x, padding, conc_weight, O, kernel_size, x_bytes, integer_bits=16, fraction_bits=16,
+               round_to_fixed=True):
+    """``(prepared activations, blob, max_shift)`` of a layer that the matrix-core kernels serve, else ``None``."""
+    if x.numel() == 0 or x.data_ptr() % 4:
+        return None
+    max_shift = mfma_shift(conc_weight, x_bytes)
+    if max_shift is None:
+        return None
+    C = x.shape[1]
+    blob = _mfma_of(conc_weight, max_shift, x_bytes, O, C, *_pair(kernel_size))
+    if blob is None:
+        return None
+    prepared = mfma_prepare(x, padding, kernel_size, x_bytes, integer_bits, fraction_bits, round_to_fixed)
+    return None if prepared is None else (prepared, blob, max_shift)
+
+
+def _mfma_conv_serves(Nb, C, Hp, Wp, O, kernel_size, stride, x_bytes=4):
+    """Whether the output has anything in it, its offsets fit, and the matrix cores are the faster place: with int32
+    activations and at most 16 channels on both sides, half of every 32-channel tile is padding (256 x 16 x 32 x 32 -> 16:
+    74 us against 54 on the two-instruction kernel, 17 -> 17 channels are even)."""
+    FH, FW = _pair(kernel_size)
+    sh, sw = _pair(stride)
+    if Hp < FH or Wp < FW or sh <= 0 or sw <= 0 or O == 0 or (x_bytes == 4 and O <= 16 and C <= 16):
+        return False
+    pixels = Nb * ((Hp - FH) // sh + 1) * ((Wp - FW) // sw + 1)
+    return 0 < pixels <= 10 ** 9 and pixels * O <= 8 * 10 ** 9
+
+
+def _mfma_linear(x, conc_weight, bias, N):
+    if x.shape[0] * N == 0:
+        return None
+    route = mfma_route(x, 0, conc_weight, N, (1, 1), 4)
+    return None if route is None else mfma_conv2d(route[0], route[1], bias, N, (1, 1), 1, route[2])
+
+
+class Prepared:
+    """Activations in the operand layout of the matrix-core kernels (:func:`mfma_prepare`)."""
+
+    def __init__(self, data, dims, filt, rows, x_bytes):
+        self.data = data        # uint8, the digits and the row flags
+        self.dims = dims        # (Nb, C, Hp, Wp)
+        self.filter = filt      # the filter size it was grouped for
+        self.rows = rows        # rows of a matrix, 0 for images
+        self.x_bytes = x_bytes
+
+
+def mfma_prepare(x, padding, kernel_size, x_bytes, integer_bits=16, fraction_bits=16, round_to_fixed=True):
+    """float32 / int32 / int8 NCHW images, or a float32 / int32 matrix [M, K], -> :class:`Prepared`, or ``None``
+    where the matrix-core kernels do not serve the size."""
+    x = x.contiguous()
+    ph, pw = _pair(padding)
+    FH, FW = _pair(kernel_size)
+    if x.dim() == 2:
+        rows, C = x.shape
+        Nb, H, W = (rows + 63) // 64, 1, 64
+    else:
+        rows = 0
+        Nb, C, H, W = x.shape
+    nbytes = _lib.lib().ds_mfma_input_bytes(Nb, C, H + 2 * ph, W + 2 * pw, FH, FW, x_bytes)
+    if not nbytes:
+        return None
+    data = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    _lib.call("ds_mfma_prepare", _lib.ptr(x), _MFMA_SRC[x.dtype], _lib.ptr(data), Nb, C, H, W, ph, pw, FH, FW, rows,
+              x_bytes, _lib.DS_Q_ROUND_TO_FIXED if round_to_fixed else _lib.DS_Q_CAST, int(integer_bits),
+              int(fraction_bits), _lib.current_stream(x.device))
+    return Prepared(data, (Nb, C, H + 2 * ph, W + 2 * pw), (FH, FW), rows, x_bytes)
+
+
+def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0, fraction_bits_in=None, scale=None,
+                shift=None, residual=None, relu=False, emit=None, want_float=True, q_cache=None):
+    """The layer from prepared activations.  ``fraction_bits_in`` None: int32 sums (with ``bias``).  Otherwise what
+    :func:`conv2d_tiled_fused` returns for the same arguments.  A prepared matrix gives ``[M, O]``."""
+    Nb, C, Hp, Wp = prepared.dims
+    FH, FW = _pair(kernel_size)
+    sh, sw = _pair(stride)
+    ch, cw = _pair(crop)
+    OH, OW = (Hp - 2 * ch - FH) // sh + 1, (Wp - 2 * cw - FW) // sw + 1
+    dev = prepared.data.device
+    if bias is not None:
+        bias = _require_device_i32("bias", bias)
+    shape = (prepared.rows, O) if prepared.rows else (Nb, O, OH, OW)
+    for name, t in (("scale", scale), ("shift", shift)):
+        if t is not None and (t.dtype != torch.float32 or t.numel() != O or not t.is_contiguous()):
+            raise ValueError("%s must be a contiguous float32 tensor of %d elements" % (name, O))
+    if residual is not None:
+        if tuple(residual.shape) != shape or residual.dtype != torch.float32:
+            raise ValueError("residual must be float32 with the shape of the output")
+        residual = residual.contiguous()
+    y = out = q = None
+    ph, pw, I, Fq, qb = 0, 0, 16, 16, 4
+    if fraction_bits_in is None:
+        y = torch.empty(shape, dtype=torch.int32, device=dev)
+    else:
+        if emit is None and not want_float:
+            raise ValueError("nothing to produce")
+        if want_float:
+            out = torch.empty(shape, dtype=torch.float32, device=dev)
+        if emit is not None:
+            padding, I, Fq, dtype = emit
+            ph, pw = _pair(padding)
+            qb = 1 if dtype == torch.int8 else 4
+            qshape = (Nb, O, OH + 2 * ph, OW + 2 * pw)
+            if q_cache is not None and (ph or pw):
+                q = _kept_padded_buffer(q_cache, qshape, dtype, dev)
+                qb |= _lib.DS_Q_BORDER_KEPT
+            else:
+                q = torch.empty(qshape, dtype=dtype, device=dev)
+    M = prepared.rows or Nb * OH * OW
+    keep = (prepared.data, blob, bias, y, out, q, scale, shift, residual)
+
+    def launch():
+        _lib.call("ds_mfma_conv2d", *[_lib.ptr(t) for t in keep], Nb, C, Hp, Wp, O, FH, FW, sh, sw, ch, cw,
+                  prepared.filter[0], prepared.filter[1], prepared.rows, max_shift, prepared.x_bytes,
+                  int(fraction_bits_in or 0), int(bool(relu)), int(I), int(Fq), ph, pw, qb, _lib.current_stream(dev))
+
+    kind = "linear" if prepared.rows else "conv"
+    with _Timed(kind, M, C * FH * FW, O, dev):
+        launch()
+    if _REPLAY_SINK is not None and fraction_bits_in is not None:
+        _REPLAY_SINK.append((kind, M, C * FH * FW, O, launch))
+    return y if fraction_bits_in is None else (out, q)
+
+
 def conv2d(input, shift, sign, bias=None, conc_weight=None, stride=1, padding=0, dilation=1,
            groups=1, use_cuda=True):
     """Shift convolution with the contract of the reference's ``kernels.conv2d`` (kernels.py:28-67).
@@ -887,6 +1075,10 @@ def conv2d(input, shift, sign, bias=None, conc_weight=None, stride=1, padding=0,
         raise ValueError("filter has %d input channels, input has %d" % (Cw, C))
     if bias is not None:
         bias = _require_device_i32("bias", bias)
+    if _mfma_conv_serves(Nb, C, H + 2 * ph, W + 2 * pw, O, (FH, FW), stride):
+        route = mfma_route(input, (ph, pw), conc_weight, O, (FH, FW), 4)
+        if route is not None:
+            return mfma_conv2d(route[0], route[1], bias, O, (FH, FW), stride, route[2])
     if ph or pw:
         xp = torch.empty([Nb, C, H + 2 * ph, W + 2 * pw], dtype=torch.int32, device=input.device)
         _lib.call("ds_pad_i32", _lib.ptr(input), _lib.ptr(xp), Nb, C, H, W, ph, pw,

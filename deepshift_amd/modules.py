@@ -170,9 +170,7 @@ class LinearShift(_PackedWeightsMixin, nn.Module):
             return out.reshape(*lead, self.out_features)
         conc_weight = self.packed_weights()
         bias = self._fixed_bias.get(self.bias, I, Fb, round_to_fixed=False)
-        tiled = kernels._tiled_of(conc_weight, self.out_features, self.in_features)
-        out = kernels.linear_layer(x2d, tiled, bias, self.out_features, kernels.kernel_bits(conc_weight),
-                                   conc_weight.base, I, Fb, round_to_fixed=False, relu=relu)
+        out = kernels.linear_forward(x2d, conc_weight, bias, self.out_features, I, Fb, round_to_fixed=False, relu=relu)
         return out.reshape(*lead, self.out_features)
 
     def forward(self, input):
@@ -321,6 +319,59 @@ def _small_for_int8(module, input_shape, field_bits):
     return tiles * groups < 8192
 
 
+def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, prequantized, emit, pool):
+    """:func:`conv_kernel_forward` on the matrix cores, or ``None`` where they have no form for the layer."""
+    I, Fb = module.act_integer_bits, module.act_fraction_bits
+    padding = (0, 0) if prequantized else module.padding
+    if prequantized:
+        x_bytes = input.element_size()
+    else:
+        x_bytes = 1 if I >= 2 and I + Fb <= 8 else 4
+        input = input.float()
+        if module.padding_mode == 'circular':
+            input = _circular_pad(input, padding)
+            padding = (0, 0)
+    Nb, C, H, W = input.shape
+    if not input.is_cuda or not kernels._mfma_conv_serves(Nb, C, H + 2 * padding[0], W + 2 * padding[1], module.out_channels,
+                                                         module.kernel_size, module.stride, x_bytes):
+        return None
+    route = kernels.mfma_route(input, padding, conc_weight, module.out_channels, module.kernel_size, x_bytes, I, Fb)
+    if route is None:
+        return None
+    prepared, blob, max_shift = route
+    bias = module._fixed_bias.get(module.bias, I, Fb, round_to_fixed=True)
+    int8_entry = x_bytes == 1 and kernels.paired_fields(conc_weight, module.out_channels, I, Fb)
+    if pool is not None:
+        sums = kernels.conv2d_paired if int8_entry else kernels.mfma_conv2d
+        out = sums(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift)
+        return _pooled(out, Fb, scale, shift, residual, relu, pool, emit)
+    want_float, spec = True, None
+    if emit is not None:
+        want_float = emit[3]
+        spec = tuple(emit[:3]) + (emit[4] if len(emit) == 5 else torch.int32,)
+    # the consumers' padded input lives in a buffer of this layer whose border is zeroed once
+    cache = module.__dict__.setdefault("_handoff_buffers", {})
+    fused = kernels.conv2d_paired_fused if int8_entry else kernels.mfma_conv2d
+    f, q = fused(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift, 0, Fb, scale,
+                 shift, residual, relu, spec, want_float, cache)
+    if emit is None:
+        return f
+    return (f, q) if want_float else q
+
+
+def _pooled(out, Fb, scale, shift, residual, relu, pool, emit):
+    """The pass behind a convolution whose ReLU is followed by a max pooling."""
+    if residual is not None:
+        raise ValueError("a fused max pooling cannot follow a residual add")
+    if emit is None:
+        return kernels.requantize_affine_maxpool(out, Fb, scale, shift, relu, pool)[0]
+    next_padding, next_I, next_F, want_float = emit[:4]
+    dtype = emit[4] if len(emit) == 5 else torch.int32
+    f, q = kernels.requantize_affine_maxpool(out, Fb, scale, shift, relu, pool, next_padding, next_I, next_F, want_float,
+                                             dtype)
+    return (f, q) if want_float else q
+
+
 def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, residual=None, relu=False,
                         prequantized=False, emit=None, pool=None, input_nonneg=False):
     """Fixed-point shift convolution of a float NCHW input (modules.py:152-162,317-337).
@@ -343,6 +394,9 @@ def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, resi
         raise NotImplementedError("the shift kernel supports dilation=1 and groups=1 only")
     I, Fb = module.act_integer_bits, module.act_fraction_bits
     # formats of at most 8 bits on narrow shift fields: int8 activations, two pixels per register
+    result = _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, prequantized, emit, pool)
+    if result is not None:
+        return result
     fields = kernels.paired_fields(conc_weight, module.out_channels, I, Fb)
     if prequantized:
         xq = input
@@ -405,18 +459,11 @@ def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, resi
             return (f, q) if want_float else q
         out = kernels.conv2d_tiled(xq, tiled, bias, module.out_channels, module.kernel_size,
                                    module.stride, kbits, conc_weight.base)
+    if pool is not None:
+        return _pooled(out, Fb, scale, shift, residual, relu, pool, emit)
     emit_dtype = torch.int32
     if emit is not None and len(emit) == 5:
         emit, emit_dtype = emit[:4], emit[4]
-    if pool is not None:
-        if residual is not None:
-            raise ValueError("a fused max pooling cannot follow a residual add")
-        if emit is None:
-            return kernels.requantize_affine_maxpool(out, Fb, scale, shift, relu, pool)[0]
-        next_padding, next_I, next_F, want_float = emit
-        f, q = kernels.requantize_affine_maxpool(out, Fb, scale, shift, relu, pool, next_padding,
-                                                 next_I, next_F, want_float, emit_dtype)
-        return (f, q) if want_float else q
     if emit is not None:
         next_padding, next_I, next_F, want_float = emit
         f, q = kernels.requantize_affine_pad(out, Fb, scale, shift, residual, relu, next_padding,

@@ -97,9 +97,7 @@ class LinearShiftQ(_PackedQMixin, nn.Module):
             return out.reshape(*lead, self.out_features)
         conc_weight = self.packed_weights()
         bias = self._fixed_bias.get(self.bias, I, Fb, round_to_fixed=True)
-        tiled = kernels._tiled_of(conc_weight, self.out_features, self.in_features)
-        out = kernels.linear_layer(x2d, tiled, bias, self.out_features, kernels.kernel_bits(conc_weight),
-                                   conc_weight.base, I, Fb, round_to_fixed=True, relu=relu)
+        out = kernels.linear_forward(x2d, conc_weight, bias, self.out_features, I, Fb, round_to_fixed=True, relu=relu)
         return out.reshape(*lead, self.out_features)
 
     def forward(self, input):

@@ -394,6 +394,31 @@ int ds_conv2d_tiled_fused_pair_i32(const int32_t *x_padded, int Nb, int C, int H
                                    int F_in, const ds_fused_conv *a, const ds_fused_conv *b, void *workspace,
                                    size_t workspace_bytes, ds_stream_t stream);
 
+/* ---- shift layers on the matrix cores (int8 MFMA, exact modulo 2^32) ----
+ * ds_mfma_weight_bytes / ds_mfma_tile_weights_i32: reference-format words (fields of `bits`, base 0) -> the blob of
+ * these kernels.  max_shift: the largest shift among the non-zero weights (the caller vouches for it); x_bytes: 4 for
+ * int32 activations (max_shift <= 14), 1 for activations of at most 8 bits.  0 / DS_EINVAL: no such form.
+ * ds_mfma_input_bytes / ds_mfma_prepare: a padded Nb x C x Hp x Wp input (Hp = H + 2 ph, Wp = W + 2 pw) in the
+ * operand layout.  source: 0 float32 NCHW, converted with (mode, I, F) as ds_quantize_f32_i32 does (x_bytes 1:
+ * round-to-fixed formats of at most 8 bits), 1 int32 NCHW, 2 int8 NCHW, all unpadded.  matrix_rows > 0: x is a
+ * row-major matrix of that many rows and C columns instead, with Nb = ceil(rows / 64), H = 1, W = 64, no padding.
+ * FH, FW: the filter that will read it (layers of at most 16 channels group taps).  dst: 16-byte aligned.
+ * ds_mfma_conv2d: the layer, from prepared activations: either y (int32 sums + bias) or out / q as
+ * ds_conv2d_tiled_fused_i32 writes them (q_bytes | DS_Q_BORDER_KEPT: the padding of q is zero already).  crop_h,
+ * crop_w: rows / columns of the prepared tensor outside the convolution's window.  prep_FH, prep_FW: the filter given to
+ * ds_mfma_prepare. */
+size_t ds_mfma_weight_bytes(int N, int C, int FH, int FW, int max_shift, int x_bytes);
+int ds_mfma_tile_weights_i32(const int32_t *w_ref, void *blob, int N, int C, int FH, int FW, int bits, int max_shift,
+                             int x_bytes, ds_stream_t stream);
+size_t ds_mfma_input_bytes(int Nb, int C, int Hp, int Wp, int FH, int FW, int x_bytes);
+int ds_mfma_prepare(const void *x, int source, void *dst, int Nb, int C, int H, int W, int ph, int pw, int FH, int FW,
+                    int matrix_rows, int x_bytes, int mode, int I, int F, ds_stream_t stream);
+int ds_mfma_conv2d(const void *prepared, const void *blob, const int32_t *bias, int32_t *y, float *out, void *q,
+                   const float *scale, const float *shift, const float *residual, int Nb, int C, int Hp, int Wp, int O,
+                   int FH, int FW, int sh, int sw, int crop_h, int crop_w, int prep_FH, int prep_FW, int matrix_rows,
+                   int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw, int q_bytes,
+                   ds_stream_t stream);
+
 /* ---- fixed-point conversion ------------------------------------------------------------ */
 
 /* Replaces utils.round_to_fixed (utils.py:7-21) + the (x * 2**F).int() cast (modules.py:25,153)

@@ -1,0 +1,142 @@
+"""GPU: the matrix-core kernels (ds_mfma_*) against the CPU oracle, bit for bit: every mode (largest shift x width of the
+activations) at the edges of its tiles -- channels, pixels, reduction blocks, taps grouped for few channels, crops -- with
+activations over the whole range of their type, and the epilogue against the separate passes."""
+import numpy as np
+import pytest
+import torch
+
+from deepshift_amd import kernels, modules, utils
+from tests.conftest import random_codes
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def _weights(rng, shape, top, ternary):
+    s, sign = random_codes(rng, (shape[0], int(np.prod(shape[1:]))), max_s=top)
+    s.flat[0], sign.flat[0] = top, -1
+    if ternary:
+        sign[rng.random(sign.shape) < 0.3] = 0
+        sign.flat[0] = -1
+    s, sign = s.reshape(shape), sign.reshape(shape)
+    cw = utils.compress_bits(_dev(-s.astype(np.float32)), _dev(sign.astype(np.float32)))
+    assert cw.max_field == top
+    return s, sign, cw
+
+
+def _activations(rng, shape, x_bytes, spread):
+    if x_bytes == 1:
+        return rng.integers(-128, 128, size=shape).astype(np.int8)
+    x = rng.integers(-spread, spread, size=shape).astype(np.int32)
+    if spread > 1 << 20:
+        # rows with and without high digits, and the ends of the range
+        x[..., : shape[-1] // 2] &= 0xfffff
+        x[0] >>= 12
+        x.flat[-1], x.flat[0], x.flat[x.size // 2] = 2 ** 31 - 1, -2 ** 31, -2 ** 27
+    return x
+
+
+# (Nb, C, H, W, O, k, stride, pad)
+SHAPES = [(2, 64, 12, 12, 64, 3, 1, 1), (3, 24, 13, 9, 40, 5, 2, 2), (1, 3, 33, 31, 17, 7, 2, 3), (2, 33, 7, 9, 33, 1, 1, 0),
+          (2, 9, 11, 10, 65, 3, 1, 1), (5, 7, 6, 5, 20, 2, 1, 0), (1, 130, 5, 5, 70, 3, 2, 1), (1, 1, 4, 4, 32, 3, 1, 1),
+          (9, 40, 8, 8, 129, 1, 2, 0)]
+MODES = [(14, 4), (11, 4), (6, 4), (5, 4), (3, 4), (1, 4), (14, 1), (31, 1), (7, 1), (3, 1), (2, 1)]
+
+
+@pytest.mark.parametrize("spread", [1 << 20, 2 ** 31 - 1], ids=["low", "full"])
+@pytest.mark.parametrize("top,x_bytes", MODES, ids=lambda v: str(v))
+def test_convolutions_match_the_oracle(oracle, rng, top, x_bytes, spread):
+    if x_bytes == 1 and spread > 1 << 20:
+        pytest.skip("8-bit activations have one range")
+    for i, (Nb, C, H, W, O, k, st, pad) in enumerate(SHAPES):
+        print(top, x_bytes, spread, SHAPES[i], flush=True)
+        s, sign, cw = _weights(rng, (O, C, k, k), top, ternary=i % 2 == 1)
+        x = _activations(rng, (Nb, C, H, W), x_bytes, spread)
+        bias = rng.integers(-2 ** 31, 2 ** 31 - 1, size=O).astype(np.int32)
+        route = kernels.mfma_route(_dev(x), (pad, pad), cw, O, (k, k), x_bytes)
+        assert route is not None
+        got = kernels.mfma_conv2d(route[0], route[1], _dev(bias), O, (k, k), (st, st), route[2])
+        xp = np.pad(x.astype(np.int32), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+        want = oracle.conv2d(xp, -s.astype(np.int32), sign.astype(np.int32), bias, (st, st))
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 7, 3), (63, 33, 31), (64, 64, 64), (65, 129, 70), (200, 1000, 130)])
+def test_matrices_match_the_oracle(oracle, rng, M, K, N):
+    for top in (14, 6, 3):
+        s, sign, cw = _weights(rng, (N, K), top, ternary=False)
+        x = _activations(rng, (M, K), 4, 2 ** 31 - 1)
+        bias = rng.integers(-2 ** 20, 2 ** 20, size=N).astype(np.int32)
+        want = oracle.linear(x, -s.astype(np.int32), sign.astype(np.int32), bias)
+        got = kernels.linear(_dev(x), _dev(s), _dev(sign), _dev(bias), cw)
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+        # rows that start at an odd element: four-wide loads are off
+        base = torch.empty(M * K + 1, dtype=torch.int32, device=DEV)
+        base[1:] = _dev(x).reshape(-1)
+        route = kernels.mfma_route(base[1:].view(M, K), 0, cw, N, (1, 1), 4)
+        got = kernels.mfma_conv2d(route[0], route[1], _dev(bias), N, (1, 1), 1, route[2])
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("x_bytes", [4, 1])
+@pytest.mark.parametrize("Nb,C,H,O,k,st", [(2, 32, 14, 40, 3, 1), (1, 64, 7, 96, 1, 1), (40, 32, 28, 64, 3, 2)])
+def test_epilogue_matches_the_separate_passes(rng, x_bytes, Nb, C, H, O, k, st):
+    pad = k // 2
+    F_in, spec = (16, ((1, 1), 16, 16, torch.int32)) if x_bytes == 4 else (5, ((1, 1), 3, 5, torch.int8))
+    s, sign, cw = _weights(rng, (O, C, k, k), 14, ternary=False)
+    x = _dev(_activations(rng, (Nb, C, H, H), x_bytes, 1 << 18))
+    prepared, blob, top = kernels.mfma_route(x, (pad, pad), cw, O, (k, k), x_bytes)
+    y = kernels.mfma_conv2d(prepared, blob, None, O, (k, k), (st, st), top)
+    scale, shift = (torch.rand(O, device=DEV) + 0.5), torch.randn(O, device=DEV)
+    for residual in (None, torch.randn(y.shape, device=DEV)):
+        for relu in (False, True):
+            want = kernels.requantize_affine_pad(y, F_in, scale, shift, residual, relu, *spec[:3], True, spec[3])
+            cache = {}
+            for q_cache in (None, cache, cache):
+                out, q = kernels.mfma_conv2d(prepared, blob, None, O, (k, k), (st, st), top, 0, F_in, scale, shift, residual,
+                                             relu, spec, True, q_cache)
+                assert torch.equal(out, want[0]) and torch.equal(q, want[1])
+                del q
+
+
+def test_a_cropped_window_reads_the_centre(oracle, rng):
+    """A 1 x 1 convolution on the tensor that was padded for a 3 x 3."""
+    s, sign, cw = _weights(rng, (64, 64, 1, 1), 14, ternary=False)
+    x = _activations(rng, (3, 64, 9, 9), 4, 1 << 24)
+    xp = np.pad(x, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    blob = kernels._mfma_of(cw, 14, 4, 64, 64, 1, 1)
+    got = kernels.mfma_conv2d(kernels.mfma_prepare(_dev(xp), 0, (3, 3), 4), blob, None, 64, (1, 1), (2, 2), 14, (1, 1))
+    want = oracle.conv2d(x, -s.astype(np.int32), sign.astype(np.int32), None, (2, 2))
+    np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+def test_layers_without_a_form_keep_their_kernels(oracle, rng):
+    """Shifts past 14 on int32 activations, left shifts: the plane and two-instruction kernels."""
+    for top in (15, 20):
+        s, sign, cw = _weights(rng, (64, 64, 3, 3), top, ternary=False)
+        assert kernels.mfma_shift(cw, 4) is None and kernels.mfma_shift(cw, 1) == top
+        x = _activations(rng, (1, 64, 6, 6), 4, 1 << 24)
+        got = kernels.conv2d(_dev(x), _dev(s), _dev(sign), None, cw, 1, 1)
+        xp = np.pad(x, ((0, 0), (0, 0), (1, 1), (1, 1)))
+        np.testing.assert_array_equal(got.cpu().numpy(), oracle.conv2d(xp, -s.astype(np.int32), sign.astype(np.int32), None,
+                                                                       (1, 1)))
+    assert kernels.mfma_shift(utils.ConcWeight(None, -2, 4, max_field=3), 4) is None
+    assert kernels.mfma_shift(utils.ConcWeight(None, 0, 4), 4) is None
+
+
+@pytest.mark.parametrize("I,F", [(16, 16), (3, 5)])
+def test_modules_match_the_float_path(I, F):
+    """A plain module against its float form on values of the layer's grid small enough for float32 sums to be exact."""
+    torch.manual_seed(0)
+    layer = modules.Conv2dShift(20, 36, 3, padding=1, use_kernel=True, act_integer_bits=I, act_fraction_bits=F).to(DEV)
+    layer.shift.data = torch.randint(-3, 1, layer.shift.shape, device=DEV).float()
+    layer.sign.data = torch.randint(0, 2, layer.sign.shape, device=DEV).float() * 2 - 1
+    layer.bias.data.zero_()
+    x = torch.randint(-3, 4, (2, 20, 9, 9), device=DEV).float()
+    with torch.no_grad():
+        want = torch.nn.functional.conv2d(x, layer.sign * 2.0 ** layer.shift, padding=1)
+        assert torch.equal(layer(x), want)
