@@ -15,6 +15,7 @@ DS_SMALL_RELU = 0x100
 DS_BITS_ZERO_TOP = 0x100
 DS_BITS_TOP_UNUSED = 0x200
 DS_Q_BORDER_KEPT = 0x100
+DS_Q_OPERANDS = 0x200
 DS_CHAIN_ONE_LAUNCH = 0x200
 DS_CHAIN_LAUNCH_PER_LAYER = 0x400
 DS_CHAIN_CONTROL_BYTES = 12288
@@ -88,7 +89,7 @@ SIGNATURES = {
     "ds_mfma_tile_weights_i32": (_c_int, [_ptr, _ptr] + [_c_int] * 7 + [_ptr]),
     "ds_mfma_input_bytes": (_size, [_c_int] * 7),
     "ds_mfma_prepare": (_c_int, [_ptr, _c_int, _ptr] + [_c_int] * 13 + [_ptr]),
-    "ds_mfma_conv2d": (_c_int, [_ptr] * 9 + [_c_int] * 23 + [_ptr]),
+    "ds_mfma_conv2d": (_c_int, [_ptr] * 9 + [_c_int] * 28 + [_ptr]),
     "ds_quantize_f32_i32": (_c_int, [_ptr, _ptr, _c_i64, _c_int, _c_int, _c_int, _ptr]),
     "ds_quantize_pad_f32_i32": (_c_int, [_ptr, _ptr] + [_c_int] * 9 + [_ptr]),
     "ds_quantize_transpose_f32_i32": (_c_int, [_ptr, _ptr] + [_c_int] * 6 + [_ptr]),

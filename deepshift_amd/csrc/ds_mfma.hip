@@ -131,6 +131,8 @@ struct MfmaX {
     int Hp, Wp, cp, cb, digits;
     int dstride, cbstride, rstride;  // bytes between digits, 32-channel blocks, rows
     int fy, cbf;                     // flag bytes per row, channel blocks that each of them covers
+    int tiles, th, tw, tph, tpw;     // written by a convolution: one flag per 32 of its th x tw pixels and 16 channels
+    int c16;
     long rows;
     size_t planes;                   // bytes of the digits; the flags follow
 };
@@ -153,6 +155,8 @@ inline MfmaX mfma_x(int Nb, int C, int Hp, int Wp, const MfmaGeom &g, bool i8)
     x.fy = ceil_div(g.cb, x.cbf);
     // a block of several taps may read up to 32 bytes past the last pixel
     x.planes = align_up((size_t)x.rows * x.rstride + 64, 256);
+    x.tiles = 0;
+    x.c16 = ceil_div(C, 16);
     return x;
 }
 
@@ -294,6 +298,8 @@ struct MfmaArgs {
     long ostride_n;
     int ostride_c;
     int matrix;                 // pixels are matrix rows
+    MfmaX qlay;                 // q in the operand layout of the next layer (qlay.planes != 0)
+    uint8_t *qflags;
     int relu, q_bytes, qHp, qWp, qph, qpw;
     float inv;
     QuantSpec qspec;
@@ -461,54 +467,6 @@ __device__ __forceinline__ void k_next(const MfmaArgs &a, KPos &k)
     }
 }
 
-// Digits d3 and d4 of the rows that have any: what they add to the sums, modulo 2^32.
-template <int MODE, int MT, int NT>
-__device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[64], int lane, const int8_t *w, int wtile,
-                                            int kb0, int kb1, const uint32_t (&px)[NT], const uint32_t (&row)[NT])
-{
-    constexpr int G = mode_groups(MODE);
-#pragma unroll
-    for (int i = 0; i < MT * NT * 16; ++i) slot[i][lane] = 0;
-    for (int d = 3; d <= 4; ++d) {
-#pragma unroll 1
-        for (int q = 0; q < (MODE == kI32S15 ? 3 : 1); ++q) {
-            v16i acc[MT][NT] = {};
-            KPos k;
-            k_start(a, k, kb0);
-#pragma unroll 1
-            for (int kb = kb0; kb < kb1; ++kb, k_next(a, k)) {
-                v4i b[NT], wv[MT];
-#pragma unroll
-                for (int p = 0; p < NT; ++p) {
-                    const bool on = a.flags[(size_t)(row[p] + k.fh) * a.lay.fy + k.cb / a.lay.cbf] != 0;
-                    b[p] = v4i{0, 0, 0, 0};
-                    if (on) b[p] = *(const v4i *)(a.x + k.off + d * a.lay.dstride + px[p]);
-                }
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    const int8_t *s = w + (size_t)m * wtile + kb * G * 1024;
-                    if (q == 2) {
-                        wv[m] = perm4(kNeg14, kPos14, *(const v4i *)(s + 3 * 1024));
-                    } else {
-                        wv[m] = perm4(kNegLo, kPosLo, *(const v4i *)(s + (G > 2 ? 2 * q : 0) * 1024));
-                        if (G > 1)
-                            wv[m] = or4(wv[m], perm4(kNegHi, kPosHi, *(const v4i *)(s + (G > 2 ? 2 * q + 1 : 1) * 1024)));
-                    }
-                }
-                product<MT, NT>(acc, wv, b);
-            }
-            const int by = 7 * (d - q - 1) + 1;
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-#pragma unroll
-                for (int p = 0; p < NT; ++p)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        slot[(m * NT + p) * 16 + i][lane] += (int)((uint32_t)acc[m][p][i] << by);
-        }
-    }
-}
-
 struct PixelAt {
     uint32_t n, oh, ow;
 };
@@ -520,6 +478,103 @@ __device__ __forceinline__ PixelAt pixel_at(const MfmaArgs &a, uint32_t p)
     r.oh = div_by(rem, a.by_row);
     r.ow = rem - r.oh * a.by_row.d;
     return r;
+}
+
+// Whether the 16 bytes that a lane reads at tap (fh, fg) of channel block cb have digits d3 and d4.
+__device__ __forceinline__ bool has_high(const MfmaArgs &a, const PixelAt &at, int half, const KPos &k)
+{
+    const int ih = at.oh * a.sh + a.crop_h + k.fh;
+    if (!a.lay.tiles) return a.flags[((size_t)at.n * a.lay.Hp + ih) * a.lay.fy + k.cb / a.lay.cbf] != 0;
+    const int iw = at.ow * a.sw + a.crop_w + (a.lay.cp == 16 ? k.fg * 2 + half : k.fg) - a.lay.tpw;
+    const int h = ih - a.lay.tph;
+    if ((unsigned)h >= (unsigned)a.lay.th || (unsigned)iw >= (unsigned)a.lay.tw) return false;
+    const uint32_t p = (at.n * a.lay.th + h) * a.lay.tw + iw;
+    const int ch16 = a.lay.cp == 16 ? k.cb : k.cb * 2 + half;
+    return ch16 < a.lay.c16 && a.flags[(size_t)(p >> 5) * a.lay.c16 + ch16] != 0;
+}
+
+// Whether any input row of a tile has them: p0 and p1 are its first and last pixel.
+__device__ __forceinline__ bool any_high(const MfmaArgs &a, uint32_t p0, uint32_t p1, int lane)
+{
+    const PixelAt u = pixel_at(a, p0), v = pixel_at(a, p1);
+    int h0 = u.oh * a.sh + a.crop_h, h1 = v.oh * a.sh + a.crop_h + a.FH - 1;
+    size_t from, to;
+    if (!a.lay.tiles) {
+        from = ((size_t)u.n * a.lay.Hp + h0) * a.lay.fy;
+        to = ((size_t)v.n * a.lay.Hp + h1 + 1) * a.lay.fy;
+    } else {
+        h0 = h0 > a.lay.tph ? h0 - a.lay.tph : 0;
+        h1 = h1 - a.lay.tph;
+        if (h0 > a.lay.th - 1) h0 = a.lay.th - 1;
+        if (h1 > a.lay.th - 1) h1 = a.lay.th - 1;
+        if (h1 < 0) h1 = 0;
+        from = (((size_t)u.n * a.lay.th + h0) * a.lay.tw >> 5) * a.lay.c16;
+        to = (((((size_t)v.n * a.lay.th + h1 + 1) * a.lay.tw - 1) >> 5) + 1) * a.lay.c16;
+    }
+    int any = 0;
+    for (size_t i = from + lane; i < to; i += 64) any |= a.flags[i];
+    return __any(any);
+}
+
+// Digits d3 and d4 of the rows that have any: what they add to the sums, modulo 2^32.  One pass over the reduction with
+// an accumulator per power of two; a digit that was not written is masked after its load, not branched around.
+template <int MODE, int MT, int NT>
+__device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[64], int lane, const int8_t *w, int wtile,
+                                            int kb0, int kb1, const uint32_t (&px)[NT], const uint32_t (&pix)[NT])
+{
+    constexpr int G = mode_groups(MODE), Q = MODE == kI32S15 ? 3 : 1;
+    v16i acc[4][MT][NT] = {};   // 2^(7 i + 1)
+    PixelAt at[NT];
+#pragma unroll
+    for (int p = 0; p < NT; ++p) at[p] = pixel_at(a, pix[p] < a.pixels ? pix[p] : a.pixels - 1);
+    KPos k;
+    k_start(a, k, kb0);
+#pragma unroll 1
+    for (int kb = kb0; kb < kb1; ++kb, k_next(a, k)) {
+        v4i b[2][NT], sel[MT][G], wv[MT];
+#pragma unroll
+        for (int p = 0; p < NT; ++p) {
+#pragma unroll
+            for (int d = 0; d < 2; ++d) b[d][p] = *(const v4i *)(a.x + k.off + (3 + d) * a.lay.dstride + px[p]);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int g = 0; g < G; ++g) sel[m][g] = *(const v4i *)(w + (size_t)m * wtile + (kb * G + g) * 1024);
+#pragma unroll
+        for (int p = 0; p < NT; ++p) {
+            const uint32_t on = has_high(a, at[p], lane >> 5, k) ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int d = 0; d < 2; ++d) b[d][p] = and4(b[d][p], on);
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                if constexpr (G == 4) {
+                    wv[m] = q == 2 ? perm4(kNeg14, kPos14, sel[m][3])
+                                   : or4(perm4(kNegLo, kPosLo, sel[m][q == 0 ? 0 : 2]),
+                                         perm4(kNegHi, kPosHi, sel[m][q == 0 ? 1 : 3]));
+                } else {
+                    wv[m] = perm4(kNegLo, kPosLo, sel[m][0]);
+                    if constexpr (G == 2) wv[m] = or4(wv[m], perm4(kNegHi, kPosHi, sel[m][1]));
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < 2; ++d) product<MT, NT>(acc[3 + d - q - 1], wv, b[d]);
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int p = 0; p < NT; ++p)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                uint32_t v = 0;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v += (uint32_t)acc[c][m][p][i] << (7 * c + 1);
+                slot[(m * NT + p) * 16 + i][lane] = (int32_t)v;
+            }
 }
 
 // What follows the sums of R x 4 channels (R groups of four, 8 apart) at one pixel: the per-channel constants, then the
@@ -543,6 +598,7 @@ __device__ __forceinline__ void load_tail(const MfmaArgs &a, ChannelTail<R> &t, 
 struct OutAt {
     size_t i;         // of channel 0 in y / out / residual
     size_t j;         // of channel 0 in q
+    uint32_t p;
     bool in;
 };
 __device__ __forceinline__ OutAt out_at(const MfmaArgs &a, const PixelAt &at, uint32_t p)
@@ -550,41 +606,159 @@ __device__ __forceinline__ OutAt out_at(const MfmaArgs &a, const PixelAt &at, ui
     OutAt o;
     o.in = p < a.pixels;
     o.i = a.matrix ? (size_t)p * a.N : (size_t)at.n * a.ostride_n + (at.oh * a.OW + at.ow);
-    o.j = ((size_t)at.n * a.N * a.qHp + at.oh + a.qph) * a.qWp + at.ow + a.qpw;
+    o.p = p;
+    o.j = a.qflags ? (size_t)(at.n * a.qHp + at.oh + a.qph) * a.qlay.rstride + (at.ow + a.qpw) * a.qlay.cp
+                   : ((size_t)at.n * a.N * a.qHp + at.oh + a.qph) * a.qWp + at.ow + a.qpw;
     return o;
 }
+// R x 4 values per lane (channels ch0 + 8 g + 0..3, ch0 = 16 u + 4 (lane >> 5)) into the next layer's operand layout:
+// the halves of a wave swap words, so that a lane holds 4 R channels side by side and the 32 pixels of a digit are
+// stored in a row.  Digits d3 and d4 only, with a flag, where the 32 pixels x 16 channels have any.
 template <int R>
-__device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail<R> &t, const int32_t (&sum)[R * 4], int ch0,
-                                           const OutAt &o)
+__device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t (&qv)[R * 4], int ch0, const OutAt &o)
 {
-    const int qplane = a.qHp * a.qWp;
-    float res[R * 4];
-    if (a.residual) {
+    const int half = (ch0 >> 2) & 1, u16 = ch0 >> 4;   // half = lane >> 5: ch0 is a multiple of 16 plus 0 or 4
+    const MfmaX &L = a.qlay;
+    if (L.digits == 1) {
+        uint32_t b[R];
+#pragma unroll
+        for (int g = 0; g < R; ++g) {
+            const uint32_t lo = __builtin_amdgcn_perm((uint32_t)qv[g * 4 + 1], (uint32_t)qv[g * 4], 0x0c0c0400u);
+            const uint32_t hi = __builtin_amdgcn_perm((uint32_t)qv[g * 4 + 3], (uint32_t)qv[g * 4 + 2], 0x04000c0cu);
+            b[g] = lo | hi;
+        }
+        const int c = u16 * 16 + (R == 4 ? half * 16 : half * 8), cb = L.cp == 16 ? c >> 4 : c >> 5;
+        int8_t *q = (int8_t *)a.q + o.j + (size_t)cb * L.cbstride + (c & (L.cp - 1));
+        if constexpr (R == 4) {
+            const auto x = __builtin_amdgcn_permlane32_swap(b[0], b[2], false, false);
+            const auto y = __builtin_amdgcn_permlane32_swap(b[1], b[3], false, false);
+            if (o.in && cb < L.cb) *(v4i *)q = v4i{(int)x[0], (int)x[1], (int)y[0], (int)y[1]};
+        } else {
+            const auto x = __builtin_amdgcn_permlane32_swap(b[0], b[1], false, false);
+            if (o.in && cb < L.cb) *(uint2 *)q = uint2{x[0], x[1]};
+        }
+        return;
+    }
+    uint32_t w[kDigits][R];
+    uint32_t high[2] = {0, 0};
+#pragma unroll
+    for (int g = 0; g < R; ++g) {
+#pragma unroll
+        for (int d = 0; d < kDigits; ++d) w[d][g] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            int32_t dg[kDigits];
+            digits_of(qv[g * 4 + i], dg);
+#pragma unroll
+            for (int d = 0; d < kDigits; ++d) w[d][g] |= ((uint32_t)dg[d] & 255u) << (8 * i);
+        }
+        high[g >> 1] |= w[3][g] | w[4][g];
+    }
+    int to = 3;
+#pragma unroll
+    for (int f = 0; f < R / 2; ++f) {
+        const bool any = __any(o.in && high[f] != 0);
+        if (any) to = kDigits;
+        if (u16 + f < L.c16 && (threadIdx.x & 63) == 0 && o.in) a.qflags[(size_t)(o.p >> 5) * L.c16 + u16 + f] = any;
+    }
+    const int c = u16 * 16 + (R == 4 ? half * 16 : half * 8);   // first of the lane's 4 R channels after the swap
+    const int cb = L.cp == 16 ? c >> 4 : c >> 5;
+    int8_t *q = (int8_t *)a.q + o.j + (size_t)cb * L.cbstride + (c & (L.cp - 1));
+#pragma unroll
+    for (int d = 0; d < kDigits; ++d) {
+        if (d >= to) break;
+        if constexpr (R == 4) {
+            const auto x = __builtin_amdgcn_permlane32_swap(w[d][0], w[d][2], false, false);
+            const auto y = __builtin_amdgcn_permlane32_swap(w[d][1], w[d][3], false, false);
+            if (o.in && cb < L.cb) *(v4i *)(q + d * L.dstride) = v4i{(int)x[0], (int)x[1], (int)y[0], (int)y[1]};
+        } else {
+            const auto x = __builtin_amdgcn_permlane32_swap(w[d][0], w[d][1], false, false);
+            if (o.in && cb < L.cb) *(uint2 *)(q + d * L.dstride) = uint2{x[0], x[1]};
+        }
+    }
+}
+
+template <int R>
+__device__ __forceinline__ void load_residual(const MfmaArgs &a, float (&res)[R * 4], int ch0, const OutAt &o)
+{
+#pragma unroll
+    for (int i = 0; i < R * 4; ++i) {
+        // past the end: some value that is there (it is not used), so that no load waits behind a branch
+        const int ch = ch0 + 8 * (i >> 2) + (i & 3), c = ch < a.N ? ch : a.N - 1;
+        res[i] = a.residual[(o.in ? o.i : 0) + (size_t)c * a.ostride_c];
+    }
+}
+
+// Stores of R x 4 values; the uniform test spares full tiles the per-channel ones.
+template <int R, typename T>
+__device__ __forceinline__ void store_channels(T *dst, const T (&v)[R * 4], int ch0, int stride, int N, bool in)
+{
+    if ((ch0 & ~15) + R * 8 <= N) {
+        if (in)
+#pragma unroll
+            for (int i = 0; i < R * 4; ++i) dst[(size_t)(ch0 + 8 * (i >> 2) + (i & 3)) * stride] = v[i];
+    } else {
 #pragma unroll
         for (int i = 0; i < R * 4; ++i) {
             const int ch = ch0 + 8 * (i >> 2) + (i & 3);
-            res[i] = o.in && ch < a.N ? a.residual[o.i + (size_t)ch * a.ostride_c] : 0.0f;
+            if (in && ch < N) dst[(size_t)ch * stride] = v[i];
         }
     }
+}
+template <int R>
+__device__ __forceinline__ void quantize_all(const float (&f)[R * 4], int32_t (&q)[R * 4], const QuantSpec &spec)
+{
+    QuantSpec s = spec;
+    s.mode = DS_Q_ROUND_TO_FIXED;
+    if (spec.I == 1) {
+        s.I = 1;
 #pragma unroll
-    for (int i = 0; i < R * 4; ++i) {
-        const int ch = ch0 + 8 * (i >> 2) + (i & 3);
-        if (!o.in || ch >= a.N) continue;
-        const int32_t v = sum[i] + t.add[i];
-        const size_t at = o.i + (size_t)ch * a.ostride_c;
-        if (a.y) {
-            a.y[at] = v;
-            continue;
-        }
-        const float f = affine_one(v, a.inv, t.scale[i], t.shift[i], a.residual ? &res[i] : nullptr, a.relu);
-        if (a.out) a.out[at] = f;
-        if (a.q) {
-            const int32_t qv = quantize_one(f, a.qspec);
-            if (a.q_bytes == 1)
-                ((int8_t *)a.q)[o.j + (size_t)ch * qplane] = (int8_t)qv;
-            else
-                ((int32_t *)a.q)[o.j + (size_t)ch * qplane] = qv;
-        }
+        for (int i = 0; i < R * 4; ++i) q[i] = quantize_one(f[i], s);
+    } else {
+        s.I = 2;   // the bounds are in lo and hi
+#pragma unroll
+        for (int i = 0; i < R * 4; ++i) q[i] = quantize_one(f[i], s);
+    }
+}
+template <int R>
+__device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail<R> &t, const int32_t (&sum)[R * 4],
+                                           const float (&res)[R * 4], int ch0, const OutAt &o)
+{
+    int32_t v[R * 4];
+#pragma unroll
+    for (int i = 0; i < R * 4; ++i) v[i] = sum[i] + t.add[i];
+    if (a.y) {
+        store_channels<R>(a.y + o.i, v, ch0, a.ostride_c, a.N, o.in);
+        return;
+    }
+    float f[R * 4];
+    if (a.residual) {
+#pragma unroll
+        for (int i = 0; i < R * 4; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], &res[i], 0);
+    } else {
+#pragma unroll
+        for (int i = 0; i < R * 4; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], nullptr, 0);
+    }
+    if (a.relu)
+#pragma unroll
+        for (int i = 0; i < R * 4; ++i) f[i] = f[i] > 0.0f ? f[i] : 0.0f;
+    if (a.out) store_channels<R>(a.out + o.i, f, ch0, a.ostride_c, a.N, o.in);
+    if (!a.q) return;
+    int32_t qv[R * 4];
+    quantize_all<R>(f, qv, a.qspec);
+    if (a.qflags) {
+        if ((ch0 & ~15) + R * 8 > a.N)
+#pragma unroll
+            for (int i = 0; i < R * 4; ++i)
+                if (ch0 + 8 * (i >> 2) + (i & 3) >= a.N) qv[i] = 0;
+        store_operands<R>(a, qv, ch0, o);
+    } else if (a.q_bytes == 1) {
+        int8_t b[R * 4];
+#pragma unroll
+        for (int i = 0; i < R * 4; ++i) b[i] = (int8_t)qv[i];
+        store_channels<R>((int8_t *)a.q + o.j, b, ch0, a.qHp * a.qWp, a.N, o.in);
+    } else {
+        store_channels<R>((int32_t *)a.q + o.j, qv, ch0, a.qHp * a.qWp, a.N, o.in);
     }
 }
 
@@ -592,7 +766,7 @@ __device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail<
 // parts of a tile lie in one workgroup and meet in LDS).  No operand passes through LDS: activations and selectors are
 // fragments in memory already, each a contiguous KiB.
 template <int MODE, int MT, int NT>
-__global__ __launch_bounds__(256, 2) void mfma_kernel(MfmaArgs a)
+__global__ __launch_bounds__(256, mode_i8(MODE) ? 3 : 2) void mfma_kernel(MfmaArgs a)
 {
     __shared__ int32_t part[4][MT * NT * 16][64];
     const int lane = threadIdx.x & 63;
@@ -612,26 +786,22 @@ __global__ __launch_bounds__(256, 2) void mfma_kernel(MfmaArgs a)
     constexpr int G = mode_groups(MODE);
     const int wtile = a.KB * G * 1024;
     const bool live = c0 < a.N && p0 < a.pixels;
-    uint32_t pix[NT], px[NT], row[NT];
+    uint32_t pix[NT], px[NT];
 #pragma unroll
     for (int p = 0; p < NT; ++p) {
         pix[p] = p0 + p * 32 + (lane & 31);
         const uint32_t clamped = pix[p] < a.pixels ? pix[p] : a.pixels - 1;
         const PixelAt at = pixel_at(a, clamped);
-        row[p] = at.n * a.lay.Hp + at.oh * a.sh + a.crop_h;
-        px[p] = row[p] * a.lay.rstride + (at.ow * a.sw + a.crop_w) * a.lay.cp + (lane >> 5) * 16;
+        px[p] = (at.n * a.lay.Hp + at.oh * a.sh + a.crop_h) * a.lay.rstride + (at.ow * a.sw + a.crop_w) * a.lay.cp + (lane >> 5) * 16;
     }
     v16i total[MT][NT] = {};
     if (live && kb0 < kb1) {
         const int8_t *wl = a.blob + (size_t)(c0 >> 5) * wtile + lane * 16;
         bool high = false;
         if constexpr (!mode_i8(MODE)) {
-            const uint32_t r0 = __builtin_amdgcn_readfirstlane(row[0]);
-            const uint32_t r1 = __builtin_amdgcn_readlane(row[NT - 1], 31) + a.FH;
-            int any = 0;
-            for (uint32_t i = r0 * a.lay.fy + lane; i < r1 * a.lay.fy; i += 64) any |= a.flags[i];
-            high = __any(any);
-            if (high) high_digits<MODE, MT, NT>(a, part[wave], lane, wl, wtile, kb0, kb1, px, row);
+            const uint32_t last = p0 + NT * 32 - 1;
+            high = any_high(a, p0, last < a.pixels ? last : a.pixels - 1, lane);
+            if (high) high_digits<MODE, MT, NT>(a, part[wave], lane, wl, wtile, kb0, kb1, px, pix);
         }
         v16i acc[MT][NT] = {};
         Operands<MODE, MT, NT> o0;
@@ -713,16 +883,25 @@ __global__ __launch_bounds__(256, 2) void mfma_kernel(MfmaArgs a)
     const int chl = c0 + 4 * (lane >> 5);
     if (a.ks == 1) {
         if (!live) return;
+        // units of 16 channels x 32 pixels; every residual is on its way before the first value is stored
+        OutAt o[NT];
+        float res[MT * NT * 2][8];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            ChannelTail<4> t;
-            load_tail<4>(a, t, chl + m * 32);
+        for (int p = 0; p < NT; ++p) o[p] = out_at(a, pixel_at(a, pix[p]), pix[p]);
+        if (a.residual)
+#pragma unroll
+            for (int u = 0; u < MT * NT * 2; ++u)
+                load_residual<2>(a, res[u], chl + u / (NT * 2) * 32 + (u / NT & 1) * 16, o[u % NT]);
+#pragma unroll
+        for (int c = 0; c < MT * 2; ++c) {
+            ChannelTail<2> tl;
+            load_tail<2>(a, tl, chl + c * 16);
 #pragma unroll
             for (int p = 0; p < NT; ++p) {
-                int32_t v[16];
+                int32_t v[8];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[i] = total[m][p][i];
-                store_tail<4>(a, t, v, chl + m * 32, out_at(a, pixel_at(a, pix[p]), pix[p]));
+                for (int i = 0; i < 8; ++i) v[i] = total[c >> 1][p][(c & 1) * 8 + i];
+                store_tail<2>(a, tl, v, res[c * NT + p], chl + c * 16, o[p]);
             }
         }
         return;
@@ -740,16 +919,19 @@ __global__ __launch_bounds__(256, 2) void mfma_kernel(MfmaArgs a)
     for (int u = kpart * units; u < (kpart + 1) * units; ++u) {
         const int m = u / (NT * 2), p = (u >> 1) % NT;
         const int ch = chl + m * 32 + (u & 1) * 16;
+        const uint32_t pp = p0 + p * 32 + (lane & 31);
+        const OutAt o = out_at(a, pixel_at(a, pp), pp);
         ChannelTail<2> tl;
+        float res[8];
         load_tail<2>(a, tl, ch);
+        if (a.residual) load_residual<2>(a, res, ch, o);
         int32_t v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             v[i] = 0;
             for (int s = 0; s < a.ks; ++s) v[i] += part[t * a.ks + s][u * 8 + i][lane];
         }
-        const uint32_t pp = p0 + p * 32 + (lane & 31);
-        store_tail<2>(a, tl, v, ch, out_at(a, pixel_at(a, pp), pp));
+        store_tail<2>(a, tl, v, res, ch, o);
     }
 }
 
@@ -780,7 +962,7 @@ __global__ __launch_bounds__(256) void mfma_border_kernel(Q *__restrict__ q, int
 template <int MODE, int MT, int NT>
 static int launch_mfma(MfmaArgs &a, hipStream_t st)
 {
-    const int waves = device_cus() * 8;
+    const int waves = device_cus() * (mode_i8(MODE) ? 12 : 8);
     const int ctiles32 = ceil_div(a.N, MT * 32);
     const long tiles = (long)ctiles32 * ceil_div((int)a.pixels, NT * 32);
     // fewer tiles than three for every wave slot: the waves of a workgroup share tiles along the reduction
@@ -861,7 +1043,8 @@ DS_EXPORT size_t ds_mfma_input_bytes(int Nb, int C, int Hp, int Wp, int FH, int 
     const double bytes = (double)Nb * Hp * Wp * g.cb * g.cp * (x_bytes == 1 ? 1 : kDigits);
     if (bytes > 2.0e9 || (double)Nb * C * Hp * Wp > 2.0e9) return 0;
     const MfmaX x = mfma_x(Nb, C, Hp, Wp, g, x_bytes == 1);
-    return x.planes + align_up((size_t)x.rows * x.fy, 256);
+    const size_t by_row = (size_t)x.rows * x.fy, by_tile = ((size_t)x.rows * Wp / 32 + 1) * x.c16;
+    return x.planes + align_up(by_row > by_tile ? by_row : by_tile, 256);
 }
 
 DS_EXPORT int ds_mfma_prepare(const void *x, int source, void *dst, int Nb, int C, int H, int W, int ph, int pw, int FH,
@@ -899,9 +1082,11 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
                              const float *scale, const float *shift, const float *residual, int Nb, int C, int Hp, int Wp,
                              int O, int FH, int FW, int sh, int sw, int crop_h, int crop_w, int prep_FH, int prep_FW,
                              int matrix_rows, int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw,
-                             int q_bytes, ds_stream_t stream)
+                             int q_bytes, int q_FH, int q_FW, int prep_tiles, int prep_ph, int prep_pw,
+                             ds_stream_t stream)
 {
     const int border_kept = q_bytes & DS_Q_BORDER_KEPT;
+    const bool operands = (q_bytes & DS_Q_OPERANDS) != 0;
     q_bytes &= 0xff;
     if (!prepared || !blob || (!y && !out && !q) || (y && (out || q))) return DS_EINVAL;
     if (sh <= 0 || sw <= 0 || crop_h < 0 || crop_w < 0 || ph < 0 || pw < 0) return DS_EINVAL;
@@ -917,6 +1102,14 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     a.lay = mfma_x(Nb, C, Hp, Wp, g, x_bytes == 1);
     a.x = (const int8_t *)prepared;
     a.flags = (const uint8_t *)prepared + a.lay.planes;
+    if (prep_tiles) {
+        if (prep_ph < 0 || prep_pw < 0 || Hp <= 2 * prep_ph || Wp <= 2 * prep_pw || g.cp < 16) return DS_EINVAL;
+        a.lay.tiles = 1;
+        a.lay.th = Hp - 2 * prep_ph;
+        a.lay.tw = Wp - 2 * prep_pw;
+        a.lay.tph = prep_ph;
+        a.lay.tpw = prep_pw;
+    }
     a.blob = (const int8_t *)blob;
     a.corr = mode_i8(mode) ? (const int32_t *)((const char *)blob + mfma_blob_corr(g, mode)) : nullptr;
     a.bias = bias;
@@ -955,7 +1148,15 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     a.by_image = fast_div((uint32_t)(a.OH * a.OW));
     a.by_row = fast_div((uint32_t)a.OW);
     hipStream_t st = (hipStream_t)stream;
-    if (q && !border_kept && (ph || pw)) {
+    if (operands) {
+        // the caller keeps the padding of the operand layout zero
+        if (!q || !border_kept || a.matrix || ds_mfma_input_bytes(Nb, O, a.qHp, a.qWp, q_FH, q_FW, q_bytes) == 0)
+            return DS_EINVAL;
+        const MfmaGeom qg = mfma_geom(1, O, q_FH, q_FW);
+        if (qg.cp < 16) return DS_EINVAL;
+        a.qlay = mfma_x(Nb, O, a.qHp, a.qWp, qg, q_bytes == 1);
+        a.qflags = (uint8_t *)q + a.qlay.planes;
+    } else if (q && !border_kept && (ph || pw)) {
         const long cells = (long)Nb * O * (2L * ph * a.qWp + 2L * pw * a.OH);
         const unsigned blocks = (unsigned)((cells + 255) / 256 < 4096 ? (cells + 255) / 256 : 4096);
         if (q_bytes == 1)
@@ -969,8 +1170,8 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     case kI32S15: return launch_mfma<kI32S15, 1, 2>(a, st);
     case kI32S7: return launch_mfma<kI32S7, 1, 2>(a, st);
     case kI32S4: return launch_mfma<kI32S4, 1, 2>(a, st);
-    case kI8S8: return launch_mfma<kI8S8, 2, 2>(a, st);
-    case kI8S4: return launch_mfma<kI8S4, 2, 2>(a, st);
-    default: return launch_mfma<kI8S3, 2, 2>(a, st);
+    case kI8S8: return launch_mfma<kI8S8, 1, 2>(a, st);
+    case kI8S4: return launch_mfma<kI8S4, 1, 2>(a, st);
+    default: return launch_mfma<kI8S3, 1, 2>(a, st);
     }
 }

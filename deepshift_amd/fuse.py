@@ -118,6 +118,7 @@ class FusedConv2dShift(nn.Module):
         self.prequantized = False  # the input is this layer's int32 padded input, made by its producer
         self.input_nonneg = False  # ... and that producer ends in a ReLU
         self.emit = None           # (padding, I, F, want_float, dtype) of the consumers' input to produce
+        self.emit_filter = None    # the consumers' filter size, if they take the operand layout (kernels.Prepared)
         self.pool = None           # (kernel, stride, padding) of a max pooling that follows the ReLU
         if bn is not None:
             if bn.training or not bn.track_running_stats:
@@ -150,7 +151,7 @@ class FusedConv2dShift(nn.Module):
         self._check_handoff_dtype(input, conc_weight)
         return modules.conv_kernel_forward(conv, input, conc_weight, self.scale, self.shift,
                                            residual, self.relu, self.prequantized, self.emit, self.pool,
-                                           self.input_nonneg)
+                                           self.input_nonneg, self.emit_filter)
 
 
 class FusedShortcutPair(nn.Module):
@@ -185,7 +186,8 @@ class FusedShortcutPair(nn.Module):
         """Both convolutions from one preparation of the input, or ``None`` where the matrix-core kernels have no
         form for them (they group the taps of layers with few channels by the filter's size)."""
         a, b = self.first, self.shortcut
-        if xq.shape[1] <= 16 or xq.numel() == 0:
+        handed = isinstance(xq, kernels.Prepared)
+        if (xq.dims[1] if handed else xq.shape[1]) <= 16 or (not handed and xq.numel() == 0):
             return None
         blobs = []
         for fused, cw in ((a, cwa), (b, cwb)):
@@ -196,7 +198,7 @@ class FusedShortcutPair(nn.Module):
             if blob is None:
                 return None
             blobs.append((top, blob))
-        prepared = kernels.mfma_prepare(xq, 0, a.conv.kernel_size, 4)
+        prepared = xq if handed else kernels.mfma_prepare(xq, 0, a.conv.kernel_size, 4)
         if prepared is None:
             return None
         results = []
@@ -206,7 +208,7 @@ class FusedShortcutPair(nn.Module):
             want_float, spec = True, None
             if fused.emit is not None:
                 want_float = fused.emit[3]
-                spec = tuple(fused.emit[:3]) + (fused.emit[4] if len(fused.emit) == 5 else torch.int32,)
+                spec = tuple(fused.emit[:3]) + (fused.emit[4] if len(fused.emit) == 5 else torch.int32, fused.emit_filter)
             bias = conv._fixed_bias.get(conv.bias, conv.act_integer_bits, conv.act_fraction_bits, round_to_fixed=True)
             out, q = kernels.mfma_conv2d(prepared, blob, bias, conv.out_channels, conv.kernel_size, conv.stride, top, crop,
                                          a.conv.act_fraction_bits, fused.scale, fused.shift, residual, fused.relu, spec,
@@ -229,6 +231,9 @@ class FusedShortcutPair(nn.Module):
         both = self._on_matrix_cores(xq, cwa, cwb, residual_first, residual_shortcut)
         if both is not None:
             return both
+        if isinstance(xq, kernels.Prepared):
+            raise RuntimeError("the weights of a paired shortcut changed in a way that moves it off the matrix-core kernels; "
+                               "fuse the model again")
         (oa, qa), (ob, qb) = kernels.conv2d_tiled_fused_pair(
             xq, a.conv.stride, a.conv.act_fraction_bits,
             self._spec(a, cwa, (0, 0), residual_first), self._spec(b, cwb, tuple(a.conv.padding), residual_shortcut))
@@ -433,6 +438,18 @@ def _input_key(conv):
             torch.int8 if paired else torch.int32)
 
 
+def _operand_filter(convs, dtype):
+    """The filter size to write the operand layout of these consumers for, or ``None`` if one of them cannot take it
+    or they group taps differently."""
+    x_bytes = 1 if dtype == torch.int8 else 4
+    for conv in convs:
+        if not kernels.mfma_takes_prepared(conv.conc_weight, conv.out_channels, conv.in_channels, conv.kernel_size, x_bytes):
+            return None
+    if convs[0].in_channels <= 16 and any(tuple(c.kernel_size) != tuple(convs[0].kernel_size) for c in convs):
+        return None
+    return tuple(convs[0].kernel_size)
+
+
 def _hand_off_fixed_point(gm):
     """Second pass: a fused convolution whose result feeds fused convolutions also writes their
     fixed-point padded input, and they read that instead of converting the float tensor again."""
@@ -461,6 +478,7 @@ def _hand_off_fixed_point(gm):
         # the float result is still needed by any other use, including a taker's residual operand
         want_float = any(u not in takers or node in u.args[1:] for u in node.users)
         producer.emit = key[:3] + (want_float, key[3])
+        producer.emit_filter = _operand_filter([fused(t).conv for t in takers], key[3])
         if want_float:
             with gm.graph.inserting_after(node):
                 q = gm.graph.call_function(operator.getitem, (node, 1))
@@ -528,6 +546,9 @@ def _pair_shortcuts(gm):
                 name = "pair_%d" % count
                 count += 1
                 gm.add_module(name, FusedShortcutPair(A, B))
+                P = fused(producer)
+                if P is not None and (ca.in_channels <= 16 or _operand_filter([ca, cb], torch.int32) is None):
+                    P.emit_filter = None
                 res_a = node.args[1] if len(node.args) > 1 else None
                 res_b = user.args[1] if len(user.args) > 1 else None
                 with gm.graph.inserting_before(earlier):

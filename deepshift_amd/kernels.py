@@ -932,6 +932,11 @@ def _mfma_of(conc_weight, max_shift, x_bytes, N, C, FH=1, FW=1):
 def mfma_route(x, padding, conc_weight, O, kernel_size, x_bytes, integer_bits=16, fraction_bits=16,
                round_to_fixed=True):
     """``(prepared activations, blob, max_shift)`` of a layer that the matrix-core kernels serve, else ``None``."""
+    if isinstance(x, Prepared):
+        max_shift = mfma_shift(conc_weight, x.x_bytes)
+        blob = None if max_shift is None else _mfma_of(conc_weight, max_shift, x.x_bytes, O, x.dims[1],
+                                                       *_pair(kernel_size))
+        return None if blob is None else (x, blob, max_shift)
     if x.numel() == 0 or x.data_ptr() % 4:
         return None
     max_shift = mfma_shift(conc_weight, x_bytes)
@@ -964,15 +969,75 @@ def _mfma_linear(x, conc_weight, bias, N):
     return None if route is None else mfma_conv2d(route[0], route[1], bias, N, (1, 1), 1, route[2])
 
 
-class Prepared:
-    """Activations in the operand layout of the matrix-core kernels (:func:`mfma_prepare`)."""
+def mfma_takes_prepared(conc_weight, O, C, kernel_size, x_bytes):
+    """Whether a convolution can be handed its input in the operand layout by the one before it: the matrix-core
+    kernels have a form for it, and its pixels are whole 16-byte pieces there."""
+    FH, FW = _pair(kernel_size)
+    max_shift = mfma_shift(conc_weight, x_bytes)
+    if max_shift is None or (x_bytes == 4 and O <= 16 and C <= 16) or (C <= 8 and FH * FW > 1):
+        return False
+    return _lib.lib().ds_mfma_weight_bytes(O, C, FH, FW, max_shift, x_bytes) != 0
 
-    def __init__(self, data, dims, filt, rows, x_bytes):
+
+class Prepared:
+    """Activations in the operand layout of the matrix-core kernels, from :func:`mfma_prepare` or, with
+    ``written_by_conv = (ph, pw)``, from the epilogue of the convolution before."""
+
+    def __init__(self, data, dims, filt, rows, x_bytes, written_by_conv=None):
+        self.written_by_conv = written_by_conv
         self.data = data        # uint8, the digits and the row flags
         self.dims = dims        # (Nb, C, Hp, Wp)
         self.filter = filt      # the filter size it was grouped for
         self.rows = rows        # rows of a matrix, 0 for images
         self.x_bytes = x_bytes
+
+    @property
+    def dtype(self):
+        return torch.int8 if self.x_bytes == 1 else torch.int32
+
+    def padded(self):
+        """The padded NCHW int32 / int8 tensor that the layout holds (for inspection: a copy, in torch operations)."""
+        if self.written_by_conv is None:
+            raise ValueError("only the layout that a convolution wrote can be read back")
+        Nb, C, Hp, Wp = self.dims
+        cp = 16 if C <= 16 and self.filter != (1, 1) else 32
+        cb, digits = (C + cp - 1) // cp, 1 if self.x_bytes == 1 else 5
+        size = Nb * Hp * cb * digits * Wp * cp
+        d = self.data[:size].view(torch.int8).view(Nb, Hp, cb, digits, Wp, cp).permute(3, 0, 2, 5, 1, 4)
+        d = d.reshape(digits, Nb, cb * cp, Hp, Wp)[:, :, :C]
+        if self.x_bytes == 1:
+            return d[0].contiguous()
+        # digits 3 and 4 count only where the 32 pixels x 16 channels that were written together have a flag
+        ph, pw = self.written_by_conv
+        H, W, c16 = Hp - 2 * ph, Wp - 2 * pw, (C + 15) // 16
+        tiles = (Nb * H * W + 31) // 32
+        at = (size + 64 + 255) // 256 * 256
+        flags = self.data[at:at + tiles * c16].view(tiles, c16) != 0
+        flags = flags.repeat_interleave(32, 0)[:Nb * H * W].repeat_interleave(16, 1)[:, :C].view(Nb, H, W, C).permute(0, 3, 1, 2)
+        high = torch.zeros(Nb, C, Hp, Wp, dtype=torch.bool, device=self.data.device)
+        high[:, :, ph:Hp - ph, pw:Wp - pw] = flags
+        v = sum(d[i].int() << (7 * i) for i in range(3))
+        return v + torch.where(high, (d[3].int() << 21) + (d[4].int() << 28), torch.zeros_like(v))
+
+    def __getitem__(self, item):
+        return self.padded()[item]
+
+
+def _kept_operands(cache, dims, kernel_size, padding, x_bytes, device):
+    """:func:`_kept_padded_buffer` for the operand layout: ``None`` where the layout does not serve the size."""
+    nbytes = _lib.lib().ds_mfma_input_bytes(*dims, *_pair(kernel_size), x_bytes)
+    if not nbytes:
+        return None
+    key = ("operands", tuple(dims), tuple(kernel_size), tuple(padding), x_bytes, device)
+    q = cache.get(key) if cache is not None else None
+    if q is not None and sys.getrefcount(q) > 3:   # the cache, the local name, getrefcount's argument
+        q = None
+    if q is None:
+        q = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        if cache is not None:
+            cache.clear()
+            cache[key] = q
+    return q
 
 
 def mfma_prepare(x, padding, kernel_size, x_bytes, integer_bits=16, fraction_bits=16, round_to_fixed=True):
@@ -1000,7 +1065,9 @@ def mfma_prepare(x, padding, kernel_size, x_bytes, integer_bits=16, fraction_bit
 def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0, fraction_bits_in=None, scale=None,
                 shift=None, residual=None, relu=False, emit=None, want_float=True, q_cache=None):
     """The layer from prepared activations.  ``fraction_bits_in`` None: int32 sums (with ``bias``).  Otherwise what
-    :func:`conv2d_tiled_fused` returns for the same arguments.  A prepared matrix gives ``[M, O]``."""
+    :func:`conv2d_tiled_fused` returns for the same arguments.  A prepared matrix gives ``[M, O]``.  With a fifth
+    element in ``emit``, the filter size of the layer that will read it, ``q`` is :class:`Prepared` for that layer
+    (kept in ``q_cache`` like the padded buffer), or the padded tensor where the size does not allow it."""
     Nb, C, Hp, Wp = prepared.dims
     FH, FW = _pair(kernel_size)
     sh, sw = _pair(stride)
@@ -1017,7 +1084,8 @@ def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0,
         if tuple(residual.shape) != shape or residual.dtype != torch.float32:
             raise ValueError("residual must be float32 with the shape of the output")
         residual = residual.contiguous()
-    y = out = q = None
+    y = out = q = handed = None
+    qfilter = (1, 1)
     ph, pw, I, Fq, qb = 0, 0, 16, 16, 4
     if fraction_bits_in is None:
         y = torch.empty(shape, dtype=torch.int32, device=dev)
@@ -1027,11 +1095,19 @@ def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0,
         if want_float:
             out = torch.empty(shape, dtype=torch.float32, device=dev)
         if emit is not None:
-            padding, I, Fq, dtype = emit
+            padding, I, Fq, dtype = emit[:4]
             ph, pw = _pair(padding)
             qb = 1 if dtype == torch.int8 else 4
             qshape = (Nb, O, OH + 2 * ph, OW + 2 * pw)
-            if q_cache is not None and (ph or pw):
+            if len(emit) == 5 and emit[4] is not None:
+                qfilter = _pair(emit[4])
+                q = _kept_operands(q_cache, qshape, qfilter, (ph, pw), qb, dev)
+                if q is not None:
+                    handed = Prepared(q, qshape, qfilter, 0, qb, (ph, pw))
+                    qb |= _lib.DS_Q_BORDER_KEPT | _lib.DS_Q_OPERANDS
+            if handed is not None:
+                pass
+            elif q_cache is not None and (ph or pw):
                 q = _kept_padded_buffer(q_cache, qshape, dtype, dev)
                 qb |= _lib.DS_Q_BORDER_KEPT
             else:
@@ -1042,14 +1118,16 @@ def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0,
     def launch():
         _lib.call("ds_mfma_conv2d", *[_lib.ptr(t) for t in keep], Nb, C, Hp, Wp, O, FH, FW, sh, sw, ch, cw,
                   prepared.filter[0], prepared.filter[1], prepared.rows, max_shift, prepared.x_bytes,
-                  int(fraction_bits_in or 0), int(bool(relu)), int(I), int(Fq), ph, pw, qb, _lib.current_stream(dev))
+                  int(fraction_bits_in or 0), int(bool(relu)), int(I), int(Fq), ph, pw, qb, *qfilter,
+                  int(prepared.written_by_conv is not None), *(prepared.written_by_conv or (0, 0)),
+                  _lib.current_stream(dev))
 
     kind = "linear" if prepared.rows else "conv"
     with _Timed(kind, M, C * FH * FW, O, dev):
         launch()
     if _REPLAY_SINK is not None and fraction_bits_in is not None:
         _REPLAY_SINK.append((kind, M, C * FH * FW, O, launch))
-    return y if fraction_bits_in is None else (out, q)
+    return y if fraction_bits_in is None else (out, q if handed is None else handed)
 
 
 def conv2d(input, shift, sign, bias=None, conc_weight=None, stride=1, padding=0, dilation=1,

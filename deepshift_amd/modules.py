@@ -319,11 +319,14 @@ def _small_for_int8(module, input_shape, field_bits):
     return tiles * groups < 8192
 
 
-def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, prequantized, emit, pool):
+def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, prequantized, emit, pool, emit_filter):
     """:func:`conv_kernel_forward` on the matrix cores, or ``None`` where they have no form for the layer."""
     I, Fb = module.act_integer_bits, module.act_fraction_bits
     padding = (0, 0) if prequantized else module.padding
-    if prequantized:
+    handed = isinstance(input, kernels.Prepared)
+    if handed:
+        x_bytes = input.x_bytes
+    elif prequantized:
         x_bytes = input.element_size()
     else:
         x_bytes = 1 if I >= 2 and I + Fb <= 8 else 4
@@ -331,8 +334,10 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
         if module.padding_mode == 'circular':
             input = _circular_pad(input, padding)
             padding = (0, 0)
-    Nb, C, H, W = input.shape
-    if not input.is_cuda or not kernels._mfma_conv_serves(Nb, C, H + 2 * padding[0], W + 2 * padding[1], module.out_channels,
+    Nb, C, H, W = input.dims if handed else input.shape
+    if not handed and not input.is_cuda:
+        return None
+    if not kernels._mfma_conv_serves(Nb, C, H + 2 * padding[0], W + 2 * padding[1], module.out_channels,
                                                          module.kernel_size, module.stride, x_bytes):
         return None
     route = kernels.mfma_route(input, padding, conc_weight, module.out_channels, module.kernel_size, x_bytes, I, Fb)
@@ -348,7 +353,7 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
     want_float, spec = True, None
     if emit is not None:
         want_float = emit[3]
-        spec = tuple(emit[:3]) + (emit[4] if len(emit) == 5 else torch.int32,)
+        spec = tuple(emit[:3]) + (emit[4] if len(emit) == 5 else torch.int32, emit_filter)
     # the consumers' padded input lives in a buffer of this layer whose border is zeroed once
     cache = module.__dict__.setdefault("_handoff_buffers", {})
     fused = kernels.conv2d_paired_fused if int8_entry else kernels.mfma_conv2d
@@ -373,7 +378,7 @@ def _pooled(out, Fb, scale, shift, residual, relu, pool, emit):
 
 
 def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, residual=None, relu=False,
-                        prequantized=False, emit=None, pool=None, input_nonneg=False):
+                        prequantized=False, emit=None, pool=None, input_nonneg=False, emit_filter=None):
     """Fixed-point shift convolution of a float NCHW input (modules.py:152-162,317-337).
 
     ``scale``/``shift`` (per output channel), ``residual`` and ``relu`` describe what follows the
@@ -387,16 +392,22 @@ def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, resi
     ``want_float`` is false.  ``pool = (kernel, stride, padding)``:
     a max pooling follows the ReLU (no residual) and runs in the same pass.  ``input_nonneg``: the
     producer of a prequantized input vouches that it is the output of a ReLU (the int8 kernel then
-    knows a tighter bound on the activations and widens its 16-bit sums less often)."""
+    knows a tighter bound on the activations and widens its 16-bit sums less often).  ``emit_filter``: the filter
+    size of the consumers, which then take the operand layout of the matrix-core kernels (``kernels.Prepared``) where
+    this layer runs there too."""
     if not module.use_cuda:
         raise ValueError("conv_kernel_forward is the GPU path; use_cuda=False layers run conv_cpu_forward")
     if module.dilation != (1, 1) or module.groups != 1:
         raise NotImplementedError("the shift kernel supports dilation=1 and groups=1 only")
     I, Fb = module.act_integer_bits, module.act_fraction_bits
     # formats of at most 8 bits on narrow shift fields: int8 activations, two pixels per register
-    result = _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, prequantized, emit, pool)
+    result = _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, prequantized, emit, pool,
+                           emit_filter)
     if result is not None:
         return result
+    if isinstance(input, kernels.Prepared):
+        raise RuntimeError("the weights of a fused shift convolution changed in a way that moves it off the matrix-core "
+                           "kernels; fuse the model again")
     fields = kernels.paired_fields(conc_weight, module.out_channels, I, Fb)
     if prequantized:
         xq = input

@@ -363,6 +363,7 @@ int ds_cpu_conv2d_i32(const int32_t *x_padded, const int8_t *shift, const int32_
  * waves; elsewhere the launch form loses more than the separate pass costs).
  * No counterpart in the reference. */
 #define DS_Q_BORDER_KEPT 0x100
+#define DS_Q_OPERANDS 0x200   /* ds_mfma_conv2d only: q in the operand layout */
 int ds_conv2d_tiled_fusable(int Nb, int C, int Hp, int Wp, int O, int FH, int FW, int sh, int sw,
                             int bits, int base);
 int ds_conv2d_tiled_fused_i32(const int32_t *x_padded, const void *tiled, const int32_t *bias, float *out,
@@ -406,7 +407,9 @@ int ds_conv2d_tiled_fused_pair_i32(const int32_t *x_padded, int Nb, int C, int H
  * ds_mfma_conv2d: the layer, from prepared activations: either y (int32 sums + bias) or out / q as
  * ds_conv2d_tiled_fused_i32 writes them (q_bytes | DS_Q_BORDER_KEPT: the padding of q is zero already).  crop_h,
  * crop_w: rows / columns of the prepared tensor outside the convolution's window.  prep_FH, prep_FW: the filter given to
- * ds_mfma_prepare. */
+ * ds_mfma_prepare.  q_bytes | DS_Q_BORDER_KEPT | DS_Q_OPERANDS: q is the operand layout for a q_FH x q_FW filter instead
+ * (ds_mfma_input_bytes of the padded output; more than 16 channels, or more than 8 read by a larger filter; zeroed
+ * before its first use), to be read with prep_tiles = 1 and the padding it was made with as prep_ph, prep_pw. */
 size_t ds_mfma_weight_bytes(int N, int C, int FH, int FW, int max_shift, int x_bytes);
 int ds_mfma_tile_weights_i32(const int32_t *w_ref, void *blob, int N, int C, int FH, int FW, int bits, int max_shift,
                              int x_bytes, ds_stream_t stream);
@@ -416,8 +419,8 @@ int ds_mfma_prepare(const void *x, int source, void *dst, int Nb, int C, int H, 
 int ds_mfma_conv2d(const void *prepared, const void *blob, const int32_t *bias, int32_t *y, float *out, void *q,
                    const float *scale, const float *shift, const float *residual, int Nb, int C, int Hp, int Wp, int O,
                    int FH, int FW, int sh, int sw, int crop_h, int crop_w, int prep_FH, int prep_FW, int matrix_rows,
-                   int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw, int q_bytes,
-                   ds_stream_t stream);
+                   int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw, int q_bytes, int q_FH,
+                   int q_FW, int prep_tiles, int prep_ph, int prep_pw, ds_stream_t stream);
 
 /* ---- fixed-point conversion ------------------------------------------------------------ */
 

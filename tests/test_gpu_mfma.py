@@ -140,3 +140,47 @@ def test_modules_match_the_float_path(I, F):
     with torch.no_grad():
         want = torch.nn.functional.conv2d(x, layer.sign * 2.0 ** layer.shift, padding=1)
         assert torch.equal(layer(x), want)
+
+
+@pytest.mark.parametrize("I,F", [(16, 16), (3, 5)])
+@pytest.mark.parametrize("C,O,k,scale_up", [(32, 40, 3, 1.0), (32, 40, 3, 4000.0), (24, 16, 3, 1.0), (20, 130, 1, 4000.0)])
+def test_operands_from_the_epilogue_equal_the_padded_tensor(rng, I, F, C, O, k, scale_up):
+    """The hand-off in the operand layout: what it holds, and what the next layer makes of it, twice into the same buffer
+    (flags of the first pass must not survive), over values with and without digits 3 and 4."""
+    x_bytes, dtype = (4, torch.int32) if I + F > 8 else (1, torch.int8)
+    pad = k // 2
+    s, sign, cw = _weights(rng, (O, C, k, k), 14, ternary=False)
+    _, _, cw2 = _weights(rng, (48, O, 3, 3), 14, ternary=False)
+    assert kernels.mfma_takes_prepared(cw2, 48, O, (3, 3), x_bytes)
+    blob2 = kernels._mfma_of(cw2, 14, x_bytes, 48, O, 3, 3)
+    cache = {}
+    for H, amp in ((14, scale_up), (14, 1.0), (9, scale_up)):
+        x = _dev(_activations(rng, (3, C, H, H), x_bytes, 1 << 17))
+        prepared, blob, top = kernels.mfma_route(x, (pad, pad), cw, O, (k, k), x_bytes)
+        scale = (torch.rand(O, device=DEV) + 0.5) * amp
+        shift = torch.randn(O, device=DEV)
+        args = (prepared, blob, None, O, (k, k), (1, 1), top, 0, F, scale, shift, None, False)
+        _, want = kernels.mfma_conv2d(*args, ((1, 1), I, F, dtype), False)
+        out, got = kernels.mfma_conv2d(*args, ((1, 1), I, F, dtype, (3, 3)), True, cache)
+        assert isinstance(got, kernels.Prepared) and torch.equal(got.padded(), want)
+        if x_bytes == 4 and amp > 1:
+            assert bool((want.abs() >= 1 << 21).any())
+        y2 = kernels.mfma_conv2d(got, blob2, None, 48, (3, 3), (2, 2), 14)
+        again = kernels.mfma_conv2d(kernels.mfma_prepare(want, 0, (3, 3), x_bytes), blob2, None, 48, (3, 3), (2, 2), 14)
+        assert torch.equal(y2, again)
+        assert len(cache) == 1
+        del got
+
+
+def test_operand_buffers_are_not_reused_while_held(rng):
+    s, sign, cw = _weights(rng, (32, 32, 1, 1), 3, ternary=False)
+    prepared, blob, top = kernels.mfma_route(_dev(_activations(rng, (2, 32, 6, 6), 4, 1 << 17)), 0, cw, 32, (1, 1), 4)
+    cache = {}
+    args = (prepared, blob, None, 32, (1, 1), (1, 1), top, 0, 16, None, None, None, False, ((1, 1), 16, 16, torch.int32, (3, 3)),
+            False, cache)
+    first = kernels.mfma_conv2d(*args)[1]
+    second = kernels.mfma_conv2d(*args)[1]
+    assert first.data.data_ptr() != second.data.data_ptr()
+    held = second.data.data_ptr()
+    del second
+    assert kernels.mfma_conv2d(*args)[1].data.data_ptr() == held
