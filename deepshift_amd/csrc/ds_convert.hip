@@ -42,29 +42,61 @@ __global__ void convert_stats_init_kernel(int32_t *stats)
     }
 }
 
+// The code of a weight falls with |w| (logarithm, division and rounding are all monotone: neighbouring floats' logarithms
+// are 10^7 double ulps apart), so the range of the codes is that of the smallest and the largest |w|: no logarithm per
+// weight, one pair per workgroup.  Bound by the atomics before (16384 waves on the same three words across eight XCDs:
+// 390 us for 512 x 512 x 3 x 3 weights); now one workgroup in a thousand waves' work reaches them, and only with a value
+// that changes what is there (a stale read of a word that only grows costs a needless atomic, never a wrong result).
 __global__ __launch_bounds__(256) void convert_stats_kernel(const float *__restrict__ w, long n, int shift_min,
                                                             int shift_max, int32_t *stats)
 {
-    int hi = -2147483647 - 1, lo = 2147483647, zeros = 0;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const WeightCode c = weight_code(w[i], shift_min, shift_max);
-        if (c.zero) ++zeros;
-        else {
-            hi = c.s > hi ? c.s : hi;
-            lo = c.s < lo ? c.s : lo;
+    __shared__ uint32_t part[3][4];
+    // bits of |w|: ordered like the values; NaN above infinity, and counted with the zeros
+    uint32_t lo = 0x7f800001u, hi = 0, zeros = 0;
+    const auto take = [&](float v) {
+        const uint32_t a = __float_as_uint(v) & 0x7fffffffu;
+        if (a == 0 || a > 0x7f800000u) {
+            ++zeros;
+        } else {
+            lo = a < lo ? a : lo;
+            hi = a > hi ? a : hi;
         }
+    };
+    const long stride = (long)gridDim.x * blockDim.x, first = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long n4 = ((uintptr_t)w & 15) == 0 ? n >> 2 : 0;
+    for (long i = first; i < n4; i += stride) {
+        const float4 v = ((const float4 *)w)[i];
+        take(v.x);
+        take(v.y);
+        take(v.z);
+        take(v.w);
     }
+    for (long i = (n4 << 2) + first; i < n; i += stride) take(w[i]);
     for (int off = kWave / 2; off > 0; off >>= 1) {
-        const int h = __shfl_down(hi, off, kWave), l = __shfl_down(lo, off, kWave);
-        hi = h > hi ? h : hi;
+        const uint32_t l = __shfl_down(lo, off, kWave), h = __shfl_down(hi, off, kWave);
         lo = l < lo ? l : lo;
+        hi = h > hi ? h : hi;
         zeros += __shfl_down(zeros, off, kWave);
     }
     if ((threadIdx.x & (kWave - 1)) == 0) {
-        atomicMax(&stats[0], hi);
-        atomicMin(&stats[1], lo);
-        if (zeros) atomicAdd(&stats[2], zeros);
+        part[0][threadIdx.x / kWave] = lo;
+        part[1][threadIdx.x / kWave] = hi;
+        part[2][threadIdx.x / kWave] = zeros;
     }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int i = 1; i < 4; ++i) {
+        lo = part[0][i] < lo ? part[0][i] : lo;
+        hi = part[1][i] > hi ? part[1][i] : hi;
+        zeros += part[2][i];
+    }
+    if (hi != 0) {
+        const int top = weight_code(__uint_as_float(lo), shift_min, shift_max).s;
+        const int low = weight_code(__uint_as_float(hi), shift_min, shift_max).s;
+        if (__hip_atomic_load(&stats[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < top) atomicMax(&stats[0], top);
+        if (__hip_atomic_load(&stats[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > low) atomicMin(&stats[1], low);
+    }
+    if (zeros) atomicAdd(&stats[2], (int)zeros);
 }
 
 // One thread per output word of the reference format (shift.cu:27-38), straight from the float
@@ -181,8 +213,8 @@ DS_EXPORT int ds_convert_stats_f32(const float *w, int64_t n, int shift_min, int
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(convert_stats_init_kernel, dim3(1), dim3(64), 0, st, stats);
     if (n > 0)
-        hipLaunchKernelGGL(convert_stats_kernel, dim3(grid_for(n)), dim3(256), 0, st, w, (long)n, shift_min,
-                           shift_max, stats);
+        hipLaunchKernelGGL(convert_stats_kernel, dim3(grid_for(n) < 1024 ? grid_for(n) : 1024), dim3(256), 0, st, w, (long)n,
+                           shift_min, shift_max, stats);
     return launch_status();
 }
 

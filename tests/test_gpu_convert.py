@@ -205,3 +205,25 @@ def test_export_load_takes_field_range_from_the_words(tmp_path):
     export.load_packed(again, bare)
     with torch.no_grad():
         assert torch.equal(again(x), model(x))
+
+
+@pytest.mark.parametrize("n", [1, 3, 255, 1025, 300001])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_stats_equal_the_codes_of_every_weight(n, offset):
+    """The reduction over |w| against the element-wise codes: odd sizes and misaligned starts, all magnitudes (denormals,
+    infinities), zeros and NaN, the extremes at either end."""
+    g = torch.Generator().manual_seed(n)
+    w = torch.randn(n + offset, generator=g) * torch.exp2(torch.randint(-140, 120, (n + offset,), generator=g).float())
+    w[torch.randint(0, n + offset, (n // 7,), generator=g)] = 0.0
+    if n > 8:
+        w[offset + 1], w[-1], w[n // 2], w[n // 2 + 1] = float("nan"), 1e-45, float("inf"), -0.0
+    w = w.to("cuda:0")[offset:]
+    for lo, hi in ((-14, 0), (-31, 31), (-1, 5)):
+        stats = torch.empty(4, dtype=torch.int32, device=w.device)
+        s, sign = torch.empty(n, dtype=torch.int32, device=w.device), torch.empty(n, dtype=torch.int32, device=w.device)
+        st = _lib.current_stream(w.device)
+        _lib.call("ds_convert_stats_f32", _lib.ptr(w), n, lo, hi, _lib.ptr(stats), st)
+        _lib.call("ds_convert_codes_f32", _lib.ptr(w), _lib.ptr(s), _lib.ptr(sign), n, lo, hi, st)
+        real = s[sign != 0].tolist()
+        want = [max(real), min(real)] if real else [-2 ** 31, 2 ** 31 - 1]
+        assert stats[:3].tolist() == want + [int((sign == 0).sum())]
