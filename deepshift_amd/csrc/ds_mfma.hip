@@ -762,13 +762,13 @@ __device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail<
     }
 }
 
-// Four waves per workgroup; a wave owns MT * 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
+// Four or eight waves per workgroup; a wave owns MT * 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
 // parts of a tile lie in one workgroup and meet in LDS).  No operand passes through LDS: activations and selectors are
 // fragments in memory already, each a contiguous KiB.
-template <int MODE, int MT, int NT>
-__global__ __launch_bounds__(256, mode_i8(MODE) ? 3 : 2) void mfma_kernel(MfmaArgs a)
+template <int MODE, int MT, int NT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) void mfma_kernel(MfmaArgs a)
 {
-    __shared__ int32_t part[4][MT * NT * 16][64];
+    __shared__ int32_t part[WAVES][MT * NT * 16][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroups are dealt to the eight XCDs in turn: give each XCD neighbouring tiles
@@ -778,7 +778,7 @@ __global__ __launch_bounds__(256, mode_i8(MODE) ? 3 : 2) void mfma_kernel(MfmaAr
     const uint32_t pt = div_by_uniform(wg, a.by_ctiles);
     const int ct = (int)(wg - pt * a.ctiles);
     const int kpart = wave % a.ks, t = wave / a.ks;
-    const int pw = 4 / a.ks / a.tc;   // pixel tiles per workgroup
+    const int pw = WAVES / a.ks / a.tc;   // pixel tiles per workgroup
     const int c0 = (ct * a.tc + t % a.tc) * MT * 32;
     const uint32_t p0 = ((uint32_t)pt * pw + t / a.tc) * (NT * 32);
     const int kb0 = (int)((long)a.KB * kpart / a.ks), kb1 = (int)((long)a.KB * (kpart + 1) / a.ks);
@@ -915,8 +915,8 @@ __global__ __launch_bounds__(256, mode_i8(MODE) ? 3 : 2) void mfma_kernel(MfmaAr
     __syncthreads();
     if (!live) return;
     // the ks waves of a tile share its epilogue, in halves of 32 x 32 values
-    const int units = MT * NT * 2 / a.ks;
-    for (int u = kpart * units; u < (kpart + 1) * units; ++u) {
+    const int units = MT * NT * 2 > a.ks ? MT * NT * 2 / a.ks : 1;
+    for (int u = kpart * units; u < (kpart + 1) * units && u < MT * NT * 2; ++u) {
         const int m = u / (NT * 2), p = (u >> 1) % NT;
         const int ch = chl + m * 32 + (u & 1) * 16;
         const uint32_t pp = p0 + p * 32 + (lane & 31);
@@ -959,21 +959,32 @@ __global__ __launch_bounds__(256) void mfma_border_kernel(Q *__restrict__ q, int
     }
 }
 
-template <int MODE, int MT, int NT>
+template <int MODE, int MT, int NT, int WAVES>
+static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
+{
+    const int ctiles32 = ceil_div(a.N, MT * 32);
+    a.ks = ks;
+    while (a.ks > 1 && a.KB < 2 * a.ks) a.ks >>= 1;
+    a.tc = (WAVES / a.ks >= 2 && ctiles32 > 1) ? 2 : 1;
+    a.ctiles = ceil_div(ctiles32, a.tc);
+    a.ptiles = ceil_div((int)a.pixels, NT * 32 * (WAVES / a.ks / a.tc));
+    a.by_ctiles = fast_div((uint32_t)a.ctiles);
+    hipLaunchKernelGGL((mfma_kernel<MODE, MT, NT, WAVES>), dim3((unsigned)(a.ctiles * a.ptiles)), dim3(WAVES * 64), 0, st, a);
+    return launch_status();
+}
+
+template <int MODE>
 static int launch_mfma(MfmaArgs &a, hipStream_t st)
 {
-    const int waves = device_cus() * (mode_i8(MODE) ? 12 : 8);
-    const int ctiles32 = ceil_div(a.N, MT * 32);
-    const long tiles = (long)ctiles32 * ceil_div((int)a.pixels, NT * 32);
+    const long waves = (long)device_cus() * (mode_i8(MODE) ? 12 : 8);   // wave slots
+    const long tiles = (long)ceil_div(a.N, 32) * ceil_div((int)a.pixels, 64);
+    // Few tiles and a long reduction leave the chip idle behind one wave's serial chain: half the tile, and the
+    // reduction in eight parts (one image, 512 channels of 7 x 7, 16 tiles: 34 -> 22 us; 256 of 14 x 14, 32 tiles:
+    // 21 -> 16; 112 tiles: 38 -> 26).  Past a sixteenth of the slots the extra epilogues cost more than the shorter
+    // chain gives (200 tiles: 23.6 -> 25.1; 392 tiles: 18.6 -> 23), as they do on short reductions (18 blocks: even).
+    if (tiles <= waves / 16 && a.KB >= 32) return launch_tiles<MODE, 1, 1, 8>(a, 8, st);
     // fewer tiles than three for every wave slot: the waves of a workgroup share tiles along the reduction
-    a.ks = tiles >= 3L * waves ? 1 : tiles >= 3L * waves / 2 ? 2 : 4;
-    while (a.ks > 1 && a.KB < 2 * a.ks) a.ks >>= 1;
-    a.tc = (a.ks <= 2 && ctiles32 > 1) ? 2 : 1;
-    a.ctiles = ceil_div(ctiles32, a.tc);
-    a.ptiles = ceil_div((int)a.pixels, NT * 32 * (4 / a.ks / a.tc));
-    a.by_ctiles = fast_div((uint32_t)a.ctiles);
-    hipLaunchKernelGGL((mfma_kernel<MODE, MT, NT>), dim3((unsigned)(a.ctiles * a.ptiles)), dim3(256), 0, st, a);
-    return launch_status();
+    return launch_tiles<MODE, 1, 2, 4>(a, tiles >= 3 * waves ? 1 : tiles >= 3 * waves / 2 ? 2 : 4, st);
 }
 
 template <int SRC, bool I8>
@@ -1167,11 +1178,11 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
                                a.qWp, ph, pw);
     }
     switch (mode) {
-    case kI32S15: return launch_mfma<kI32S15, 1, 2>(a, st);
-    case kI32S7: return launch_mfma<kI32S7, 1, 2>(a, st);
-    case kI32S4: return launch_mfma<kI32S4, 1, 2>(a, st);
-    case kI8S8: return launch_mfma<kI8S8, 1, 2>(a, st);
-    case kI8S4: return launch_mfma<kI8S4, 1, 2>(a, st);
-    default: return launch_mfma<kI8S3, 1, 2>(a, st);
+    case kI32S15: return launch_mfma<kI32S15>(a, st);
+    case kI32S7: return launch_mfma<kI32S7>(a, st);
+    case kI32S4: return launch_mfma<kI32S4>(a, st);
+    case kI8S8: return launch_mfma<kI8S8>(a, st);
+    case kI8S4: return launch_mfma<kI8S4>(a, st);
+    default: return launch_mfma<kI8S3>(a, st);
     }
 }
