@@ -30,9 +30,14 @@ CLOCK_HZ = 2.4e9
 LANE_OPS = CU_COUNT * LANES_PER_CU * CLOCK_HZ  # 39.3e12 int32 lane-operations per second
 # The bound: a shift-add pair needs at least ONE vector instruction per lane (the accumulate; the shifted
 # operand can be shared between output channels, which is what the shift-plane kernels do), so no int32
-# kernel can exceed 39.3 Tpair/s; the int8 kernels hold two pixels per lane register: 0.5 per pair.
+# vector kernel can exceed 39.3 Tpair/s.
 PEAK_PAIRS = LANE_OPS / 1.0
-PEAK_PAIRS_INT8 = LANE_OPS / 0.5
+# The matrix-core kernels spend a fixed number of int8 products per pair (1024 per clock and SIMD): 18 for shifts up
+# to 14 on int32 activations, one per distinct shift (8 or 3 here) on 8-bit activations.
+MFMA_PRODUCTS = CU_COUNT * 4 * 1024 * CLOCK_HZ
+PEAK_PAIRS_MFMA = MFMA_PRODUCTS / 18
+PEAK_PAIRS_MFMA_ACT8 = MFMA_PRODUCTS / 8
+PEAK_PAIRS_MFMA_ACT8_2BIT = MFMA_PRODUCTS / 3
 # secondary figure: a kernel that shifts and accumulates every pair separately (v_ashrrev_i32 + v_xad_u32)
 PEAK_PAIRS_TWO_INSTR = LANE_OPS / 2.0
 HBM_PEAK = 8.0e12
@@ -41,11 +46,7 @@ BATCH = 64
 CHW = (3, 224, 224)
 
 # the kernel behind the 3x3 convolutions of the headline network, as rocprofv3 names it
-DOMINANT_KERNEL = "ds::shift_planes_wide_coop_kernel<4, 2, true, false>"
-# HBM bytes of one launch of that kernel on the layer1 shape: 77.0 MB read + 69.5 MB written (FETCH_SIZE /
-# WRITE_SIZE counters scaled by a 64 MiB copy kernel's readings); 106.6 MB are algorithmic, the rest are
-# the partial tiles that workgroups exchange through the workspace and what is left of the re-read halo rows
-TRAFFIC_LAYER1_BYTES = 146.5e6
+DOMINANT_KERNEL = "ds::mfma_kernel<0, 1, 2, 4>"
 
 
 def log(*a):
@@ -315,7 +316,7 @@ def config2(device, reps=10):
 
 
 def fused_model_timing(device, cls, batch, weight_bits, integer_bits, fraction_bits, workload, steps=5,
-                       chw=CHW, peak=PEAK_PAIRS, graph_replay=False):
+                       chw=CHW, peak=PEAK_PAIRS_MFMA, graph_replay=False):
     """Steps/s and shift-kernel rate of a converted, fused network on synthetic input."""
     from deepshift_amd import convert, fuse
     g = torch.Generator().manual_seed(0)
@@ -341,7 +342,7 @@ def fused_model_timing(device, cls, batch, weight_bits, integer_bits, fraction_b
     out = dict(workload=workload, ms_per_step=sec * 1e3, images_per_s=batch / sec, shift_layers=len(layers),
                pairs_per_step=pairs, shift_kernel_ms_per_step=kernel_s * 1e3,
                shift_tpairs_per_s=pairs / kernel_s / 1e12,
-               valu_bound_tpairs_per_s=peak / 1e12, valu_frac=pairs / kernel_s / peak,
+               bound_tpairs_per_s=peak / 1e12, bound_frac=pairs / kernel_s / peak,
                frac_of_two_instruction_peak=pairs / kernel_s / PEAK_PAIRS_TWO_INSTR)
     if graph_replay:
         out.update(graph_replay_timing(fused, x, steps))
@@ -384,22 +385,20 @@ def graph_replay_timing(fused, x, steps):
 
 def config5(device, steps=5):
     """Benchmark configuration 5: ResNet-50, batch 128, weight_bits 3 (2-bit shift fields), activations
-    3.5 (8 bits).  Every convolution has a multiple of 64 channels, so the fused pipeline runs them on
-    the int8 kernel (two pixels per register); the FC stays on the int32 kernel."""
+    3.5 (8 bits): the convolutions on the matrix-core kernels, three int8 products per pair."""
     from deepshift_amd import workloads
     return fused_model_timing(device, workloads.ResNet50, 128, 3, 3, 5,
                               "ResNet-50, batch 128 x 3x224x224, weight_bits 3, activations 3.5", steps,
-                              peak=PEAK_PAIRS_INT8)
+                              peak=PEAK_PAIRS_MFMA_ACT8_2BIT)
 
 
 def config4_act8(device, steps=5):
     """The headline network with the reference's 8-bit activation format (`-ab 3 5`, weight_bits 5):
-    the 3x3 layers and the stem run on the int8 kernel, the three 1x1 shortcuts and the FC on the
-    int32 kernels."""
+    the convolutions on the matrix-core kernels, eight int8 products per pair."""
     from deepshift_amd import workloads
     return fused_model_timing(device, workloads.ResNet18, BATCH, 5, 3, 5,
                               "ResNet-18, batch 64 x 3x224x224, weight_bits 5, activations 3.5", steps,
-                              peak=PEAK_PAIRS_INT8)
+                              peak=PEAK_PAIRS_MFMA_ACT8)
 
 
 def config3(device, steps=10):
@@ -837,9 +836,9 @@ def main():
     if args.layers:
         for L in layers:
             p = L["M"] * L["K"] * L["N"]
-            log("%-32s M=%-7d K=%-5d N=%-5d %8.1f us  %6.2f Tpair/s  %5.1f%% valu  %5.1f%% hbm" % (
+            log("%-32s M=%-7d K=%-5d N=%-5d %8.1f us  %6.2f Tpair/s  %5.1f%% mfma  %5.1f%% hbm" % (
                 L["name"], L["M"], L["K"], L["N"], L["seconds"] * 1e6, p / L["seconds"] / 1e12,
-                100 * p / L["seconds"] / PEAK_PAIRS, 100 * L["bytes"] / L["seconds"] / HBM_PEAK))
+                100 * p / L["seconds"] / PEAK_PAIRS_MFMA, 100 * L["bytes"] / L["seconds"] / HBM_PEAK))
 
     # The dominant kernel: the launches of the 3x3 convolutions (16 of the 21, 92 % of the pairs) all run
     # the same kernel; its roofline figures come from their HIP-event durations.
@@ -886,29 +885,24 @@ def main():
         "shift_gops": 2 * pairs / kernel_s / 1e9,
         "shift_layers_images_per_s": BATCH / kernel_s,
         "roofline": {
-            # Bound: vector ALU.  peak = 256 CUs x 64 lanes x 2.4 GHz / 1 vector instruction per pair (the
-            # accumulate; no int32 kernel can need fewer) = 39.3 Tpair/s.  achieved = the pairs of the
-            # dominant kernel's launches / their duration in this run, timed with HIP events around runs of
-            # those launches (replay_timing); avg_launch_us_in_step: an event pair around each one.
-            "bound": "valu",
+            # Bound: matrix cores.  peak = 256 CUs x 4 SIMDs x 1024 int8 products per clock x 2.4 GHz / 18 products
+            # per pair = 139.8 Tpair/s.  achieved = the pairs of the dominant kernel's launches / their duration in
+            # this run, timed with HIP events around runs of those launches (replay_timing);
+            # avg_launch_us_in_step: an event pair around each one.
+            "bound": "mfma",
             "kernel": DOMINANT_KERNEL,
             "launches_per_step": len(dominant),
             "achieved": dom_pairs / dom_s / 1e12,
-            "peak": PEAK_PAIRS / 1e12,
+            "peak": PEAK_PAIRS_MFMA / 1e12,
             "unit": "Tpair/s",
-            "frac": dom_pairs / dom_s / PEAK_PAIRS,
+            "frac": dom_pairs / dom_s / PEAK_PAIRS_MFMA,
             "avg_launch_us": dom_s / len(dominant) * 1e6,
             "avg_launch_us_in_step": dom_s_bracketed / len(dominant) * 1e6,
-            "frac_in_step": dom_pairs / dom_s_bracketed / PEAK_PAIRS,
+            "frac_in_step": dom_pairs / dom_s_bracketed / PEAK_PAIRS_MFMA,
             "pairs_per_launch": dom_pairs / len(dominant),
-            # HBM bytes of one launch of the dominant kernel on the layer1 shape (M = 200704, K = 576,
-            # N = 64; 106.6 MB algorithmic), a constant copied from the FETCH_SIZE / WRITE_SIZE runs in
-            # profiles/shift_kernel_layer1_conv_counters.md -- not measured in this run
-            "traffic": TRAFFIC_LAYER1_BYTES,
-            "traffic_source": "profiles/shift_kernel_layer1_conv_counters.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE)",
             # the whole step (all 21 launches, pre-fill passes included) against the same bound
             "step_achieved": pairs / kernel_s / 1e12,
-            "step_frac": pairs / kernel_s / PEAK_PAIRS,
+            "step_frac": pairs / kernel_s / PEAK_PAIRS_MFMA,
             # secondary: against a kernel that spends two vector instructions on every pair
             "peak_two_instruction": PEAK_PAIRS_TWO_INSTR / 1e12,
             "frac_of_two_instruction_peak": dom_pairs / dom_s / PEAK_PAIRS_TWO_INSTR,
