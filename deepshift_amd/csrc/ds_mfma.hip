@@ -265,13 +265,14 @@ __global__ __launch_bounds__(256) void mfma_prepare_kernel(PrepArgs a)
                     for (int q = 0; q < CH / 4; ++q) ((uint32_t *)(o + (size_t)d * L.dstride))[q] = words[d][q];
                 if (d >= 3)
 #pragma unroll
-                    for (int q = 0; q < CH / 4; ++q) high |= words[d][q] != 0;
+                    for (int q = 0; q < CH / 4; ++q) high |= words[d][q] != 0 ? (d == 3 ? 1 : 2) : 0;
             }
         }
         if (I8) return;
         if (pass == 0) {
+            const int high4 = __syncthreads_or(high & 2);
             high = __syncthreads_or(high);
-            if (threadIdx.x == 0) a.flags[(size_t)row * L.fy + part] = high ? 1 : 0;
+            if (threadIdx.x == 0) a.flags[(size_t)row * L.fy + part] = high4 ? 3 : high ? 1 : 0;
             if (!high) return;
         }
     }
@@ -493,8 +494,8 @@ __device__ __forceinline__ bool has_high(const MfmaArgs &a, const PixelAt &at, i
     return ch16 < a.lay.c16 && a.flags[(size_t)(p >> 5) * a.lay.c16 + ch16] != 0;
 }
 
-// Whether any input row of a tile has them: p0 and p1 are its first and last pixel.
-__device__ __forceinline__ bool any_high(const MfmaArgs &a, uint32_t p0, uint32_t p1, int lane)
+// Whether any input row of a tile has them (1), and digit d4 at that (2): p0 and p1 are its first and last pixel.
+__device__ __forceinline__ int any_high(const MfmaArgs &a, uint32_t p0, uint32_t p1, int lane)
 {
     const PixelAt u = pixel_at(a, p0), v = pixel_at(a, p1);
     int h0 = u.oh * a.sh + a.crop_h, h1 = v.oh * a.sh + a.crop_h + a.FH - 1;
@@ -513,14 +514,14 @@ __device__ __forceinline__ bool any_high(const MfmaArgs &a, uint32_t p0, uint32_
     }
     int any = 0;
     for (size_t i = from + lane; i < to; i += 64) any |= a.flags[i];
-    return __any(any);
+    return (__any(any) ? 1 : 0) | (__any(any & 2) ? 2 : 0);
 }
 
 // Digits d3 and d4 of the rows that have any: what they add to the sums, modulo 2^32.  One pass over the reduction with
 // an accumulator per power of two; a digit that was not written is masked after its load, not branched around.
 template <int MODE, int MT, int NT>
-__device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[64], int lane, const int8_t *w, int wtile,
-                                            int kb0, int kb1, const uint32_t (&px)[NT], const uint32_t (&pix)[NT])
+__device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[64], int lane, bool d4, const int8_t *w,
+                                            int wtile, int kb0, int kb1, const uint32_t (&px)[NT], const uint32_t (&pix)[NT])
 {
     constexpr int G = mode_groups(MODE), Q = MODE == kI32S15 ? 3 : 1;
     v16i acc[4][MT][NT] = {};   // 2^(7 i + 1)
@@ -535,7 +536,8 @@ __device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[6
 #pragma unroll
         for (int p = 0; p < NT; ++p) {
 #pragma unroll
-            for (int d = 0; d < 2; ++d) b[d][p] = *(const v4i *)(a.x + k.off + (3 + d) * a.lay.dstride + px[p]);
+            for (int d = 0; d < 2; ++d)
+                if (d == 0 || d4) b[d][p] = *(const v4i *)(a.x + k.off + (3 + d) * a.lay.dstride + px[p]);
         }
 #pragma unroll
         for (int m = 0; m < MT; ++m)
@@ -545,7 +547,8 @@ __device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[6
         for (int p = 0; p < NT; ++p) {
             const uint32_t on = has_high(a, at[p], lane >> 5, k) ? 0xffffffffu : 0u;
 #pragma unroll
-            for (int d = 0; d < 2; ++d) b[d][p] = and4(b[d][p], on);
+            for (int d = 0; d < 2; ++d)
+                if (d == 0 || d4) b[d][p] = and4(b[d][p], on);
         }
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
@@ -561,7 +564,8 @@ __device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[6
                 }
             }
 #pragma unroll
-            for (int d = 0; d < 2; ++d) product<MT, NT>(acc[3 + d - q - 1], wv, b[d]);
+            for (int d = 0; d < 2; ++d)
+                if (d == 0 || d4) product<MT, NT>(acc[3 + d - q - 1], wv, b[d]);
         }
     }
 #pragma unroll
@@ -640,7 +644,7 @@ __device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t 
         return;
     }
     uint32_t w[kDigits][R];
-    uint32_t high[2] = {0, 0};
+    uint32_t high[2] = {0, 0}, high4[2] = {0, 0};
 #pragma unroll
     for (int g = 0; g < R; ++g) {
 #pragma unroll
@@ -653,13 +657,16 @@ __device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t 
             for (int d = 0; d < kDigits; ++d) w[d][g] |= ((uint32_t)dg[d] & 255u) << (8 * i);
         }
         high[g >> 1] |= w[3][g] | w[4][g];
+        high4[g >> 1] |= w[4][g];
     }
     int to = 3;
 #pragma unroll
     for (int f = 0; f < R / 2; ++f) {
         const bool any = __any(o.in && high[f] != 0);
+        const bool any4 = __any(o.in && high4[f] != 0);
         if (any) to = kDigits;
-        if (u16 + f < L.c16 && (threadIdx.x & 63) == 0 && o.in) a.qflags[(size_t)(o.p >> 5) * L.c16 + u16 + f] = any;
+        if (u16 + f < L.c16 && (threadIdx.x & 63) == 0 && o.in)
+            a.qflags[(size_t)(o.p >> 5) * L.c16 + u16 + f] = any4 ? 3 : any ? 1 : 0;
     }
     const int c = u16 * 16 + (R == 4 ? half * 16 : half * 8);   // first of the lane's 4 R channels after the swap
     const int cb = L.cp == 16 ? c >> 4 : c >> 5;
@@ -797,11 +804,11 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
     v16i total[MT][NT] = {};
     if (live && kb0 < kb1) {
         const int8_t *wl = a.blob + (size_t)(c0 >> 5) * wtile + lane * 16;
-        bool high = false;
+        int high = 0;
         if constexpr (!mode_i8(MODE)) {
             const uint32_t last = p0 + NT * 32 - 1;
             high = any_high(a, p0, last < a.pixels ? last : a.pixels - 1, lane);
-            if (high) high_digits<MODE, MT, NT>(a, part[wave], lane, wl, wtile, kb0, kb1, px, pix);
+            if (high) high_digits<MODE, MT, NT>(a, part[wave], lane, (high & 2) != 0, wl, wtile, kb0, kb1, px, pix);
         }
         v16i acc[MT][NT] = {};
         Operands<MODE, MT, NT> o0;
