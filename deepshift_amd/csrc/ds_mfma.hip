@@ -966,6 +966,25 @@ __global__ __launch_bounds__(256) void mfma_border_kernel(Q *__restrict__ q, int
     }
 }
 
+// ... and of its operands, in pieces of 16 bytes: whole rows above and below, both ends of the columns of the others.
+// For buffers that no caller zeroed once (first use, and captured graphs, which own theirs).
+__global__ __launch_bounds__(256) void mfma_operand_border_kernel(int8_t *__restrict__ q, MfmaX lay, int ph, int pw)
+{
+    const int pixel = lay.cp >> 4, side = pw * pixel, segments = lay.cb * lay.digits;
+    for (long row = blockIdx.x; row < lay.rows; row += gridDim.x) {
+        v4i *r = (v4i *)(q + (size_t)row * lay.rstride);
+        const int h = (int)(row % lay.Hp);
+        if (h < ph || h >= lay.Hp - ph) {
+            for (int i = threadIdx.x; i < lay.rstride >> 4; i += 256) r[i] = v4i{};
+        } else {
+            for (int i = threadIdx.x; i < segments * 2 * side; i += 256) {
+                const int segment = i / (2 * side), j = i - segment * 2 * side;
+                r[segment * (lay.dstride >> 4) + (j < side ? j : (lay.Wp - 2 * pw) * pixel + j)] = v4i{};
+            }
+        }
+    }
+}
+
 template <int MODE, int MT, int NT, int WAVES>
 static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
 {
@@ -1167,13 +1186,16 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     a.by_row = fast_div((uint32_t)a.OW);
     hipStream_t st = (hipStream_t)stream;
     if (operands) {
-        // the caller keeps the padding of the operand layout zero
-        if (!q || !border_kept || a.matrix || ds_mfma_input_bytes(Nb, O, a.qHp, a.qWp, q_FH, q_FW, q_bytes) == 0)
+        if (!q || a.matrix || ds_mfma_input_bytes(Nb, O, a.qHp, a.qWp, q_FH, q_FW, q_bytes) == 0)
             return DS_EINVAL;
         const MfmaGeom qg = mfma_geom(1, O, q_FH, q_FW);
         if (qg.cp < 16) return DS_EINVAL;
         a.qlay = mfma_x(Nb, O, a.qHp, a.qWp, qg, q_bytes == 1);
         a.qflags = (uint8_t *)q + a.qlay.planes;
+        if (!border_kept && (ph || pw)) {
+            const unsigned blocks = (unsigned)(a.qlay.rows < 4096 ? a.qlay.rows : 4096);
+            hipLaunchKernelGGL(mfma_operand_border_kernel, dim3(blocks), dim3(256), 0, st, (int8_t *)q, a.qlay, ph, pw);
+        }
     } else if (q && !border_kept && (ph || pw)) {
         const long cells = (long)Nb * O * (2L * ph * a.qWp + 2L * pw * a.OH);
         const unsigned blocks = (unsigned)((cells + 255) / 256 < 4096 ? (cells + 255) / 256 : 4096);

@@ -50,20 +50,58 @@ def _workspace(nbytes, device):
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
 
-def _kept_padded_buffer(cache, shape, dtype, device):
+# Hand-off buffers that one layer keeps: one per stream that runs it, the oldest given back past this many.
+KEPT_STREAMS = 8
+
+
+def _stream_key(device):
+    """``(device, stream)`` that work issued now goes to; ``None`` while that stream is being captured."""
+    if device.type == "cpu":
+        return device, 0
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    return device, _lib.stream_handle(device)
+
+
+def _kept_padded_buffer(cache, shape, dtype, device, layout=None):
     """The zero padded hand-off buffer of a fused convolution, kept in ``cache`` between calls so that its
-    border is zeroed once and the kernel writes the interior only.  The buffer is reused only while nobody
-    else holds the tensor returned last time (or a view of it): a layer that is called again while an
-    earlier result is still alive -- a weight-shared branch whose consumer has not run yet -- gets a fresh
-    zeroed buffer instead of overwriting what that consumer is about to read."""
-    key = (tuple(shape), dtype, device)
+    border is zeroed once and the kernel writes the interior only.  The buffer is reused only
+
+    * by the stream it was made for: a result counts as dropped when its reader has been issued, not when it has
+      run, so only work on the same stream is ordered behind that reader;
+    * while nobody else holds the tensor returned last time (or a view of it): a layer that is called again while
+      an earlier result is still alive -- a weight-shared branch whose consumer has not run yet -- gets a fresh
+      zeroed buffer instead of overwriting what that consumer is about to read.
+
+    ``None`` while the stream is being captured: replays write the buffer on any stream and at any time, so it must
+    belong to the graph alone; the caller allocates one and has the launch write its border.  ``layout``: what else
+    a buffer has to agree in (the geometry behind a flat one)."""
+    at = _stream_key(device)
+    if at is None:
+        return None
+    key = (at, tuple(shape), dtype, layout)
     q = cache.get(key)
     if q is not None and sys.getrefcount(q) > 3:   # the cache, the local name, getrefcount's argument
         q = None
     if q is None:
-        cache.clear()            # one geometry at a time: a new batch size replaces the buffer
-        q = cache[key] = torch.zeros(shape, dtype=dtype, device=device)
+        q = torch.zeros(shape, dtype=dtype, device=device)
+        # one geometry at a time: a new batch size replaces this stream's buffer; another stream's, given back, is
+        # its allocator's again, which hands it to later work of that stream only
+        for old in [k for k in list(cache) if k[0] == at]:
+            cache.pop(old, None)
+        cache[key] = q
+        for old in list(cache)[:-KEPT_STREAMS]:
+            cache.pop(old, None)
     return q
+
+
+def _padded_output(cache, shape, padding, dtype, device):
+    """The tensor for a launch to write the next layer's zero padded input to, and what to add to ``q_bytes``."""
+    if cache is not None and any(padding):
+        q = _kept_padded_buffer(cache, shape, dtype, device)
+        if q is not None:
+            return q, _lib.DS_Q_BORDER_KEPT
+    return torch.empty(shape, dtype=dtype, device=device), 0
 
 
 _TIMING_SINK = None
@@ -701,12 +739,8 @@ def conv2d_tiled_fused(x_padded, tiled, bias, O, kernel_size, stride, bits, frac
         padding, I, Fq, dtype = emit
         ph, pw = _pair(padding)
         qb = 1 if dtype == torch.int8 else 4
-        shape = (Nb, O, OH + 2 * ph, OW + 2 * pw)
-        if q_cache is not None and (ph or pw):
-            q = _kept_padded_buffer(q_cache, shape, dtype, dev)
-            qb |= _lib.DS_Q_BORDER_KEPT
-        else:
-            q = torch.empty(shape, dtype=dtype, device=dev)
+        q, kept = _padded_output(q_cache, (Nb, O, OH + 2 * ph, OW + 2 * pw), (ph, pw), dtype, dev)
+        qb |= kept
     L = _lib.lib()
     ws_bytes = L.ds_conv2d_tiled_workspace_bytes(Nb, C, Hp, Wp, O, FH, FW, sh, sw, int(bits))
     ws = _workspace(ws_bytes, dev)
@@ -746,13 +780,8 @@ def _fused_conv_struct(x_shape, stride, spec, keep):
         padding, I, Fq, dtype = emit
         ph, pw = _pair(padding)
         qb = 1 if dtype == torch.int8 else 4
-        shape = (Nb, O, OH + 2 * ph, OW + 2 * pw)
-        cache = spec.get("q_cache")
-        if cache is not None and (ph or pw):
-            q = _kept_padded_buffer(cache, shape, dtype, dev)
-            qb |= _lib.DS_Q_BORDER_KEPT
-        else:
-            q = torch.empty(shape, dtype=dtype, device=dev)
+        q, kept = _padded_output(spec.get("q_cache"), (Nb, O, OH + 2 * ph, OW + 2 * pw), (ph, pw), dtype, dev)
+        qb |= kept
     residual = spec.get("residual")
     if residual is not None:
         if tuple(residual.shape) != (Nb, O, OH, OW) or residual.dtype != torch.float32:
@@ -863,12 +892,8 @@ def conv2d_paired_fused(x_padded, paired, bias, O, kernel_size, stride, field_bi
         padding, I, Fq, dtype = emit
         ph, pw = _pair(padding)
         qb = 1 if dtype == torch.int8 else 4
-        shape = (Nb, O, OH + 2 * ph, OW + 2 * pw)
-        if q_cache is not None and (ph or pw):
-            q = _kept_padded_buffer(q_cache, shape, dtype, dev)
-            qb |= _lib.DS_Q_BORDER_KEPT
-        else:
-            q = torch.empty(shape, dtype=dtype, device=dev)
+        q, kept = _padded_output(q_cache, (Nb, O, OH + 2 * ph, OW + 2 * pw), (ph, pw), dtype, dev)
+        qb |= kept
     L = _lib.lib()
     ws_bytes = L.ds_conv2d_paired_fused_workspace_bytes(Nb, C, Hp, Wp, O, FH, FW, sh, sw, int(field_bits),
                                                         int(x_bound))
@@ -1023,21 +1048,16 @@ class Prepared:
         return self.padded()[item]
 
 
-def _kept_operands(cache, dims, kernel_size, padding, x_bytes, device):
-    """:func:`_kept_padded_buffer` for the operand layout: ``None`` where the layout does not serve the size."""
-    nbytes = _lib.lib().ds_mfma_input_bytes(*dims, *_pair(kernel_size), x_bytes)
+def _operand_output(cache, dims, kernel_size, padding, x_bytes, device):
+    """:func:`_padded_output` for the operand layout: ``None`` where the layout does not serve the size."""
+    nbytes = _lib.lib().ds_mfma_input_bytes(*dims, *kernel_size, x_bytes)
     if not nbytes:
         return None
-    key = ("operands", tuple(dims), tuple(kernel_size), tuple(padding), x_bytes, device)
-    q = cache.get(key) if cache is not None else None
-    if q is not None and sys.getrefcount(q) > 3:   # the cache, the local name, getrefcount's argument
-        q = None
-    if q is None:
-        q = torch.zeros(nbytes, dtype=torch.uint8, device=device)
-        if cache is not None:
-            cache.clear()
-            cache[key] = q
-    return q
+    if cache is not None and any(padding):
+        q = _kept_padded_buffer(cache, (nbytes,), torch.uint8, device, (dims, kernel_size, padding, x_bytes))
+        if q is not None:
+            return q, _lib.DS_Q_OPERANDS | _lib.DS_Q_BORDER_KEPT
+    return torch.empty(nbytes, dtype=torch.uint8, device=device), _lib.DS_Q_OPERANDS
 
 
 def mfma_prepare(x, padding, kernel_size, x_bytes, integer_bits=16, fraction_bits=16, round_to_fixed=True):
@@ -1099,19 +1119,17 @@ def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0,
             ph, pw = _pair(padding)
             qb = 1 if dtype == torch.int8 else 4
             qshape = (Nb, O, OH + 2 * ph, OW + 2 * pw)
+            made = None
             if len(emit) == 5 and emit[4] is not None:
                 qfilter = _pair(emit[4])
-                q = _kept_operands(q_cache, qshape, qfilter, (ph, pw), qb, dev)
-                if q is not None:
-                    handed = Prepared(q, qshape, qfilter, 0, qb, (ph, pw))
-                    qb |= _lib.DS_Q_BORDER_KEPT | _lib.DS_Q_OPERANDS
-            if handed is not None:
-                pass
-            elif q_cache is not None and (ph or pw):
-                q = _kept_padded_buffer(q_cache, qshape, dtype, dev)
-                qb |= _lib.DS_Q_BORDER_KEPT
+                made = _operand_output(q_cache, qshape, qfilter, (ph, pw), qb, dev)
+            if made is not None:
+                handed = Prepared(made[0], qshape, qfilter, 0, qb, (ph, pw))
             else:
-                q = torch.empty(qshape, dtype=dtype, device=dev)
+                made = _padded_output(q_cache, qshape, (ph, pw), dtype, dev)
+            q, kept = made
+            del made
+            qb |= kept
     M = prepared.rows or Nb * OH * OW
     keep = (prepared.data, blob, bias, y, out, q, scale, shift, residual)
 

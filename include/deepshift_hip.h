@@ -407,9 +407,9 @@ int ds_conv2d_tiled_fused_pair_i32(const int32_t *x_padded, int Nb, int C, int H
  * ds_mfma_conv2d: the layer, from prepared activations: either y (int32 sums + bias) or out / q as
  * ds_conv2d_tiled_fused_i32 writes them (q_bytes | DS_Q_BORDER_KEPT: the padding of q is zero already).  crop_h,
  * crop_w: rows / columns of the prepared tensor outside the convolution's window.  prep_FH, prep_FW: the filter given to
- * ds_mfma_prepare.  q_bytes | DS_Q_BORDER_KEPT | DS_Q_OPERANDS: q is the operand layout for a q_FH x q_FW filter instead
- * (ds_mfma_input_bytes of the padded output; more than 16 channels, or more than 8 read by a larger filter; zeroed
- * before its first use), to be read with prep_tiles = 1 and the padding it was made with as prep_ph, prep_pw. */
+ * ds_mfma_prepare.  q_bytes | DS_Q_OPERANDS: q is the operand layout for a q_FH x q_FW filter instead
+ * (ds_mfma_input_bytes of the padded output; more than 16 channels, or more than 8 read by a larger filter), to be read
+ * with prep_tiles = 1 and the padding it was made with as prep_ph, prep_pw. */
 size_t ds_mfma_weight_bytes(int N, int C, int FH, int FW, int max_shift, int x_bytes);
 int ds_mfma_tile_weights_i32(const int32_t *w_ref, void *blob, int N, int C, int FH, int FW, int bits, int max_shift,
                              int x_bytes, ds_stream_t stream);

@@ -1,0 +1,96 @@
+"""GPU: the buffers that fused layers hand to each other, where a model runs on several streams, is captured into a graph,
+or is called with other sizes in between."""
+import pytest
+import torch
+import torch.nn as nn
+
+from deepshift_amd import convert, fuse, kernels
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+FORMATS = [(16, 16), (3, 5)]
+
+
+def _model(I, F, seed=0, widths=((32, 64, 3), (64, 64, 1), (64, 64, 3), (64, 32, 1))):
+    """Fused convolutions with padded and unpadded hand-offs."""
+    torch.manual_seed(seed)
+    layers = []
+    for C, O, k in widths:
+        layers += [nn.Conv2d(C, O, k, padding=k // 2, bias=False), nn.BatchNorm2d(O), nn.ReLU()]
+    model, n = convert.convert_to_shift(nn.Sequential(*layers).eval(), 1000, "PS", convert_weights=True, use_kernel=True,
+                                        weight_bits=5, act_integer_bits=I, act_fraction_bits=F)
+    assert n == len(widths)
+    return fuse.fuse_conv_epilogues(model.to(DEV))
+
+
+def _inputs(n, Nb=16, C=32, H=56):
+    g = torch.Generator(device=DEV).manual_seed(Nb)
+    return [torch.rand(Nb, C, H, H, generator=g, device=DEV) * 2 for _ in range(n)]
+
+
+@pytest.mark.parametrize("I,F", FORMATS)
+def test_two_streams_share_a_model(I, F):
+    """Passes of two streams alternate with nothing between them but the host."""
+    with torch.no_grad():
+        model = _model(I, F)
+        xs = _inputs(12)
+        want = [model(x) for x in xs]
+        torch.cuda.synchronize()
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        got = []
+        for i, x in enumerate(xs):
+            with torch.cuda.stream(streams[i % 2]):
+                got.append(model(x))
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("I,F", FORMATS)
+def test_a_captured_pass_owns_its_buffers(I, F):
+    """Eager passes right after a capture (which executes nothing), replays, and eager passes of another size between
+    the replays: each result is that of a pass by itself."""
+    with torch.no_grad():
+        model = _model(I, F)
+        small, large = _inputs(4, 2, H=15), _inputs(4, 5, H=15)
+        want_small, want_large = [model(x) for x in small], [model(x) for x in large]
+        model(_inputs(1, 3, H=9)[0])       # what is kept now fits neither
+        static = small[0].clone()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = model(static)
+        assert torch.equal(model(small[1]), want_small[1])
+        for i in range(4):
+            static.copy_(small[i])
+            graph.replay()
+            assert torch.equal(model(large[i]), want_large[i])
+            assert torch.equal(y, want_small[i])
+            graph.replay()
+            assert torch.equal(model(small[3 - i]), want_small[3 - i])
+            assert torch.equal(y, want_small[i])
+
+
+@pytest.mark.parametrize("x_bytes,O", [(4, 40), (4, 12), (1, 33), (1, 64)])
+@pytest.mark.parametrize("pad", [(1, 1), (2, 0), (0, 3), (0, 0)])
+def test_a_buffer_that_nobody_zeroed_gets_its_border(x_bytes, O, pad):
+    """The operand layout written into memory full of other values: border and unused channels included, it holds what
+    the padded tensor does."""
+    from tests.test_gpu_mfma import _activations, _weights
+    import numpy as np
+    rng = np.random.default_rng(O)
+    dtype, I, F = (torch.int32, 16, 16) if x_bytes == 4 else (torch.int8, 3, 5)
+    s, sign, cw = _weights(rng, (O, 24, 3, 3), 14, ternary=False)
+    x = torch.from_numpy(_activations(rng, (3, 24, 11, 9), x_bytes, 1 << 20)).to(DEV)
+    prepared, blob, top = kernels.mfma_route(x, (1, 1), cw, O, (3, 3), x_bytes)
+    args = (prepared, blob, None, O, (3, 3), (1, 1), top, 0, F, None, None, None, False)
+    _, want = kernels.mfma_conv2d(*args, (pad, I, F, dtype), False)
+    junk = torch.full((1 << 22,), 0x55, dtype=torch.uint8, device=DEV)
+    del junk                                # the allocator's next blocks hold 0x55
+    _, got = kernels.mfma_conv2d(*args, (pad, I, F, dtype, (3, 3)), False)
+    assert torch.equal(got.padded(), want)
+    _, _, cw2 = _weights(rng, (48, O, 3, 3), 14, ternary=False)
+    blob2 = kernels._mfma_of(cw2, 14, x_bytes, 48, O, 3, 3)
+    y = kernels.mfma_conv2d(got, blob2, None, 48, (3, 3), (1, 1), 14)
+    again = kernels.mfma_conv2d(kernels.mfma_prepare(want, 0, (3, 3), x_bytes), blob2, None, 48, (3, 3), (1, 1), 14)
+    assert torch.equal(y, again)

@@ -279,6 +279,33 @@ def test_kept_hand_off_buffer_is_not_reused_while_its_last_result_is_alive():
     assert e.shape[0] == 2 and len(cache) == 1, "a new geometry replaces the buffer"
 
 
+def test_kept_hand_off_buffers_belong_to_one_stream_and_to_no_graph(monkeypatch):
+    """A dropped result has been issued, not run: only the stream it was issued on may have the buffer again.  A
+    captured graph writes its buffers whenever it is replayed: none of them is kept, and no kept one is given to it."""
+    from types import SimpleNamespace
+    now = SimpleNamespace(stream=1, capturing=False)
+    monkeypatch.setattr(kernels._lib, "stream_handle", lambda device: now.stream, raising=False)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: now.capturing)
+    cache = {}
+
+    def kept(stream, Nb=1):
+        now.stream = stream
+        return kernels._kept_padded_buffer(cache, (Nb, 2, 4, 4), torch.int32, torch.device("meta"))
+
+    first = id(kept(1))
+    second = id(kept(2))
+    assert second != first and id(kept(1)) == first and id(kept(2)) == second
+    kept(2, Nb=3)
+    assert id(kept(1)) == first, "another stream's new geometry leaves this stream's buffer"
+    now.capturing = True
+    assert kept(1) is None and kept(3) is None
+    now.capturing = False
+    assert id(kept(1)) == first
+    for stream in range(100):
+        kept(stream)
+    assert len(cache) <= 16
+
+
 def test_hand_off_buffers_do_not_travel_with_copies_of_a_module():
     import copy
     import pickle
