@@ -573,9 +573,9 @@ def linear_chain(x2d, layers, integer_bits, fraction_bits, round_to_fixed, ws_ca
     grid with barriers between the layers), wider ones as a launch per layer issued inside the call;
     ``how`` = ``"one"`` / ``"each"`` forces either.  ``layers``: a list of
     ``(tiled, bias, K, N, bits, base, relu)``; ``ws_cache``: a dict that keeps the workspace (control block
-    zeroed once + hidden activations) between calls.  Returns float32 ``[M, N_last]``, or ``None`` when the
-    chain has no such form (mixed field widths, a K that is not a multiple of 4, ...): the caller then
-    runs the layers one by one.  The barriers of the one-launch form wait at most 2 s for the whole grid to
+    zeroed once + hidden activations) between calls, one per stream; a captured call has its own.  Returns
+    float32 ``[M, N_last]``, or ``None`` when the chain has no such form (mixed field widths, a K that is not a
+    multiple of 4, ...): the caller then runs the layers one by one.  The barriers of the one-launch form wait at most 2 s for the whole grid to
     be resident; :func:`linear_chain_status` tells whether one gave up."""
     x2d = x2d.contiguous()
     if x2d.dtype != torch.float32 or not x2d.is_cuda or x2d.dim() != 2:
@@ -592,11 +592,10 @@ def linear_chain(x2d, layers, integer_bits, fraction_bits, round_to_fixed, ws_ca
     ws_bytes = L.ds_linear_chain_workspace_bytes(M, arr, len(layers))
     if ws_bytes == 0 or x2d.data_ptr() % 16:
         return None
-    key = (ws_bytes, dev)
-    ws = ws_cache.get(key)
-    if ws is None:
-        ws_cache.clear()
-        ws = ws_cache[key] = torch.zeros(ws_bytes, dtype=torch.uint8, device=dev)   # control block zeroed once
+    ws = _kept_padded_buffer(ws_cache, (ws_bytes,), torch.uint8, dev)
+    if ws is None:   # being captured: kept for its status only
+        ws = ws_cache["captured"] = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        ws[:_lib.DS_CHAIN_CONTROL_BYTES].zero_()
     out = torch.empty([M, layers[-1][3]], dtype=torch.float32, device=dev)
     pairs = sum(M * K * N for (_, _, K, N, _, _, _) in layers)
     mode = _lib.DS_Q_ROUND_TO_FIXED if round_to_fixed else _lib.DS_Q_CAST
@@ -608,11 +607,13 @@ def linear_chain(x2d, layers, integer_bits, fraction_bits, round_to_fixed, ws_ca
 
 
 def linear_chain_status(ws_cache):
-    """0, or the number of the barrier at which a launch of :func:`linear_chain` on this workspace gave up
+    """0, or the number of the barrier at which a launch of :func:`linear_chain` on these workspaces gave up
     (its output was undefined).  Synchronises with the device."""
-    for ws in ws_cache.values():
-        at = _lib.DS_CHAIN_STATUS_AT
-        return int(ws[at:at + 4].view(torch.int32).item())
+    at = _lib.DS_CHAIN_STATUS_AT
+    for ws in list(ws_cache.values()):
+        status = int(ws[at:at + 4].view(torch.int32).item())
+        if status:
+            return status
     return 0
 
 

@@ -71,6 +71,45 @@ def test_a_captured_pass_owns_its_buffers(I, F):
             assert torch.equal(y, want_small[i])
 
 
+def _chain(widths):
+    torch.manual_seed(1)
+    layers = []
+    for K, N in zip(widths[:-1], widths[1:]):
+        layers += [nn.Linear(K, N), nn.ReLU()]
+    model, _ = convert.convert_to_shift(nn.Sequential(*layers[:-1]).eval(), 0, "PS", convert_weights=True, use_kernel=True)
+    fused = fuse.fuse_conv_epilogues(model.to(DEV))
+    assert any(isinstance(m, fuse.FusedLinearChain) for m in fused.modules())
+    return fused
+
+
+@pytest.mark.parametrize("widths", [(64, 64, 32, 8), (784, 512, 512, 10)], ids=["one launch", "launch per layer"])
+def test_streams_and_graphs_have_their_own_chain_workspace(widths):
+    with torch.no_grad():
+        model = _chain(widths)
+        chain = next(m for m in model.modules() if isinstance(m, fuse.FusedLinearChain))
+        g = torch.Generator(device=DEV).manual_seed(2)
+        xs = [torch.rand(64, widths[0], generator=g, device=DEV) for _ in range(16)]
+        want = [model(x) for x in xs]
+        torch.cuda.synchronize()
+        streams, got = [torch.cuda.Stream(), torch.cuda.Stream()], []
+        for i, x in enumerate(xs):
+            with torch.cuda.stream(streams[i % 2]):
+                got.append(model(x))
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        static = xs[0].clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = model(static)
+        assert torch.equal(model(xs[1]), want[1])
+        for i in range(4):
+            static.copy_(xs[i])
+            graph.replay()
+            assert torch.equal(model(xs[i + 4][:30]), want[i + 4][:30])
+            assert torch.equal(y, want[i])
+        assert chain.status() == 0
+
+
 @pytest.mark.parametrize("x_bytes,O", [(4, 40), (4, 12), (1, 33), (1, 64)])
 @pytest.mark.parametrize("pad", [(1, 1), (2, 0), (0, 3), (0, 0)])
 def test_a_buffer_that_nobody_zeroed_gets_its_border(x_bytes, O, pad):
