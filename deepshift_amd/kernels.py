@@ -290,6 +290,12 @@ def kernel_bits(conc_weight):
     return conc_weight.bits
 
 
+def _may_keep():
+    """Whether what a launch made just now can be kept for later calls: during a capture it has only been recorded,
+    and nobody but the graph's replays may rely on it."""
+    return not torch.cuda.is_current_stream_capturing()
+
+
 def _tiled_of(conc_weight, N, C, FH=1, FW=1):
     """The tiled blob of a ConcWeight, built once and cached on the object."""
     data = conc_weight.data
@@ -302,7 +308,8 @@ def _tiled_of(conc_weight, N, C, FH=1, FW=1):
         else:
             blob = tile_weights(data, N, C, FH, FW, conc_weight.bits, conc_weight.base)
         cached = (key, blob)
-        conc_weight._tiled = cached
+        if _may_keep():
+            conc_weight._tiled = cached
     return cached[1]
 
 
@@ -360,7 +367,8 @@ def _paired_of(conc_weight, fields, N, C, FH=1, FW=1):
     cached = getattr(conc_weight, "_paired", None)
     if cached is None or cached[0] != key:
         cached = (key, tile_weights_paired(data, N, C, FH, FW, fields[0], fields[1]))
-        conc_weight._paired = cached
+        if _may_keep():
+            conc_weight._paired = cached
     return cached[1]
 
 
@@ -951,7 +959,9 @@ def _mfma_of(conc_weight, max_shift, x_bytes, N, C, FH=1, FW=1):
             blob = torch.empty(nbytes, dtype=torch.uint8, device=data.device)
             _lib.call("ds_mfma_tile_weights_i32", _lib.ptr(packed), _lib.ptr(blob), N, C, FH, FW,
                       int(conc_weight.bits), max_shift, x_bytes, _lib.current_stream(data.device))
-        cached = cache[x_bytes] = (key, blob)
+        cached = (key, blob)
+        if _may_keep():
+            cache[x_bytes] = cached
     return cached[1]
 
 

@@ -108,9 +108,10 @@ class _FixedBias:
             return None
         key = (bias.data_ptr(), bias._version, integer_bits, fraction_bits, round_to_fixed)
         if key != self.key:
-            self.value = kernels.quantize(bias.detach().float(), integer_bits, fraction_bits,
-                                          round_to_fixed)
-            self.key = key
+            value = kernels.quantize(bias.detach().float(), integer_bits, fraction_bits, round_to_fixed)
+            if not kernels._may_keep():
+                return value
+            self.value, self.key = value, key
         return self.value
 
 

@@ -4,7 +4,7 @@ import pytest
 import torch
 import torch.nn as nn
 
-from deepshift_amd import convert, fuse, kernels
+from deepshift_amd import convert, fuse, kernels, modules
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -108,6 +108,40 @@ def test_streams_and_graphs_have_their_own_chain_workspace(widths):
             assert torch.equal(model(xs[i + 4][:30]), want[i + 4][:30])
             assert torch.equal(y, want[i])
         assert chain.status() == 0
+
+
+@pytest.mark.parametrize("M", [1024, 64])
+def test_what_a_capture_builds_is_not_kept(M):
+    """A capture records the layout passes of weights and bias and runs none of them: an eager call between capture and
+    first replay builds its own.  1024 rows take another kernel than the rows that warmed the layer up."""
+    torch.manual_seed(3)
+    layer = modules.LinearShift(512, 512, use_kernel=True).to(DEV)
+    layer.sign.data.copy_(torch.randint(0, 2, layer.sign.shape).float() * 2 - 1)
+    x = torch.randn(M, 512, device=DEV)
+    junk = torch.full((64 << 20,), 0x55, dtype=torch.uint8, device=DEV)
+    del junk                              # what is allocated next holds something
+    with torch.no_grad():
+        if M > 64:
+            want = torch.cat([layer(x[i:i + 64]) for i in range(0, M, 64)])
+        else:
+            layer.packed_weights()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = layer(x)
+        got = layer(x)
+        if M == 64:
+            graph_reads = layer.conc_weight
+            layer.conc_weight = None      # start over
+            layer._fixed_bias = modules._FixedBias()
+            want = layer(x)
+        assert torch.equal(got, want)
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            assert torch.equal(layer(x), want)
+            assert torch.equal(y, want)
+        assert M > 64 or graph_reads.data is not layer.conc_weight.data
 
 
 @pytest.mark.parametrize("x_bytes,O", [(4, 40), (4, 12), (1, 33), (1, 64)])
