@@ -232,8 +232,7 @@ class FusedShortcutPair(nn.Module):
         if both is not None:
             return both
         if isinstance(xq, kernels.Prepared):
-            raise RuntimeError("the weights of a paired shortcut changed in a way that moves it off the matrix-core kernels; "
-                               "fuse the model again")
+            xq = xq.padded()
         (oa, qa), (ob, qb) = kernels.conv2d_tiled_fused_pair(
             xq, a.conv.stride, a.conv.act_fraction_bits,
             self._spec(a, cwa, (0, 0), residual_first), self._spec(b, cwb, tuple(a.conv.padding), residual_shortcut))

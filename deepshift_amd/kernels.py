@@ -1032,7 +1032,8 @@ class Prepared:
         return torch.int8 if self.x_bytes == 1 else torch.int32
 
     def padded(self):
-        """The padded NCHW int32 / int8 tensor that the layout holds (for inspection: a copy, in torch operations)."""
+        """The padded NCHW int32 / int8 tensor that the layout holds: a copy, in torch operations, for the kernels that
+        read such a tensor and for inspection."""
         if self.written_by_conv is None:
             raise ValueError("only the layout that a convolution wrote can be read back")
         Nb, C, Hp, Wp = self.dims

@@ -407,8 +407,8 @@ def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, resi
     if result is not None:
         return result
     if isinstance(input, kernels.Prepared):
-        raise RuntimeError("the weights of a fused shift convolution changed in a way that moves it off the matrix-core "
-                           "kernels; fuse the model again")
+        # weights that the matrix cores have no form for, loaded after the model was fused
+        input = input.padded()
     fields = kernels.paired_fields(conc_weight, module.out_channels, I, Fb)
     if prequantized:
         xq = input

@@ -11,14 +11,16 @@ DEV = "cuda:0"
 FORMATS = [(16, 16), (3, 5)]
 
 
-def _model(I, F, seed=0, widths=((32, 64, 3), (64, 64, 1), (64, 64, 3), (64, 32, 1))):
+def _model(I, F, seed=0, widths=((32, 64, 3), (64, 64, 1), (64, 64, 3), (64, 32, 1)), weight_bits=5, scale=None):
     """Fused convolutions with padded and unpadded hand-offs."""
     torch.manual_seed(seed)
     layers = []
     for C, O, k in widths:
         layers += [nn.Conv2d(C, O, k, padding=k // 2, bias=False), nn.BatchNorm2d(O), nn.ReLU()]
+        if scale:                                      # no weight below 2^-14
+            nn.init.uniform_(layers[-3].weight, scale / 100, scale)
     model, n = convert.convert_to_shift(nn.Sequential(*layers).eval(), 1000, "PS", convert_weights=True, use_kernel=True,
-                                        weight_bits=5, act_integer_bits=I, act_fraction_bits=F)
+                                        weight_bits=weight_bits, act_integer_bits=I, act_fraction_bits=F)
     assert n == len(widths)
     return fuse.fuse_conv_epilogues(model.to(DEV))
 
@@ -142,6 +144,51 @@ def test_what_a_capture_builds_is_not_kept(M):
             assert torch.equal(layer(x), want)
             assert torch.equal(y, want)
         assert M > 64 or graph_reads.data is not layer.conc_weight.data
+
+
+@pytest.mark.parametrize("changed", [[1], [2], [1, 2, 3]], ids=str)
+def test_weights_loaded_after_fusing_may_need_the_older_kernels(changed):
+    """Shifts past 14 in layers that were fused for the operand layout: the layer before hands it over, the layer reads
+    it back."""
+    with torch.no_grad():
+        model = _model(16, 16, weight_bits=6, scale=0.3)
+        convs = [m for m in model.modules() if isinstance(m, modules.Conv2dShift)]
+        x = _inputs(1, 3, H=11)[0]
+        assert all(int(c.packed_weights().max_field) <= 14 for c in convs)
+        model(x)
+        for i in changed:
+            convs[i].shift.view(-1)[::7] = -15.0 - (i % 2) * 5
+        got = model(x)
+        assert all((int(c.packed_weights().max_field) > 14) == (i in changed) for i, c in enumerate(convs))
+        bns = [m for m in model.modules() if isinstance(m, fuse.FusedConv2dShift)]
+        want = x
+        for fused in bns:
+            y = kernels.conv2d(kernels.quantize(want), fused.conv.shift, fused.conv.sign, None, fused.conv.packed_weights(),
+                               1, fused.conv.padding)
+            want = kernels.dequantize_affine(y, 16, fused.scale, fused.shift, None, True)
+        assert torch.equal(got, want)
+
+
+def test_a_pair_whose_weights_reach_shift_15(rng):
+    """Both convolutions of a down-sampling block: the one-launch pair on the padded tensor serves them."""
+    from deepshift_amd import workloads
+    g = torch.Generator().manual_seed(7)
+    model = workloads.randomize_batchnorm(workloads.ResNet18(), g).eval()
+    model, _ = convert.convert_to_shift(model, 1000, "PS", convert_weights=True, use_kernel=True, weight_bits=6)
+    model = model.to(DEV)
+    x = torch.randn(2, 3, 64, 64, generator=g).to(DEV)
+    with torch.no_grad():
+        for m in model.modules():
+            if isinstance(m, modules.Conv2dShift):
+                m.shift.clamp_(-14, 0)
+        fused = fuse.fuse_conv_epilogues(model)
+        pair = next(m for m in fused.modules() if isinstance(m, fuse.FusedShortcutPair))
+        fused(x)
+        for conv in (pair.first.conv, pair.shortcut.conv):
+            conv.shift.view(-1)[:100] = -15.0
+        got = fused(x)
+        assert all(f.conv.packed_weights().max_field == 15 for f in (pair.first, pair.shortcut))
+        assert torch.equal(got, fuse.fuse_conv_epilogues(model, handoff=False)(x))
 
 
 @pytest.mark.parametrize("x_bytes,O", [(4, 40), (4, 12), (1, 33), (1, 64)])
