@@ -29,6 +29,8 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kDigits = 5;          // 7-bit digits of an int32 activation
 constexpr int kMfmaMaxK = 1 << 17;  // 64 * 127 * K stays within int32
+constexpr int kMaxRows = 1 << 24;   // ds_mfma_prepare launches 256 threads per row, and a launch has less than 2^32
+constexpr int kMaxPad = 1 << 28;
 
 // Which products a launch forms (MfmaMode): the widest shift that occurs, and the activations' width.
 enum { kI32S15 = 0, kI32S7 = 1, kI32S4 = 2, kI8S8 = 3, kI8S4 = 4, kI8S3 = 5 };
@@ -944,10 +946,10 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
 
 // The padding of the next layer's input.
 template <typename Q>
-__global__ __launch_bounds__(256) void mfma_border_kernel(Q *__restrict__ q, int planes, int Hp, int Wp, int ph, int pw)
+__global__ __launch_bounds__(256) void mfma_border_kernel(Q *__restrict__ q, long planes, int Hp, int Wp, int ph, int pw)
 {
     const int rows = 2 * ph * Wp, side = 2 * pw * (Hp - 2 * ph), per = rows + side;
-    const long total = (long)planes * per;
+    const long total = planes * per;
     for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long)gridDim.x * 256) {
         const long plane = i / per;
         int r = (int)(i - plane * per), h, w;
@@ -1075,7 +1077,7 @@ DS_EXPORT int ds_mfma_tile_weights_i32(const int32_t *w_ref, void *blob, int N, 
 DS_EXPORT size_t ds_mfma_input_bytes(int Nb, int C, int Hp, int Wp, int FH, int FW, int x_bytes)
 {
     if (Nb <= 0 || C <= 0 || Hp <= 0 || Wp <= 0 || FH <= 0 || FW <= 0 || (x_bytes != 1 && x_bytes != 4)) return 0;
-    if (Hp < FH || Wp < FW || (double)Nb * Hp > 2147483647.0) return 0;
+    if (Hp < FH || Wp < FW || (double)Nb * Hp >= kMaxRows) return 0;
     const MfmaGeom g = mfma_geom(1, C, FH, FW);
     const double bytes = (double)Nb * Hp * Wp * g.cb * g.cp * (x_bytes == 1 ? 1 : kDigits);
     if (bytes > 2.0e9 || (double)Nb * C * Hp * Wp > 2.0e9) return 0;
@@ -1087,7 +1089,8 @@ DS_EXPORT size_t ds_mfma_input_bytes(int Nb, int C, int Hp, int Wp, int FH, int 
 DS_EXPORT int ds_mfma_prepare(const void *x, int source, void *dst, int Nb, int C, int H, int W, int ph, int pw, int FH,
                               int FW, int matrix_rows, int x_bytes, int mode, int I, int F, ds_stream_t stream)
 {
-    if (!x || !dst || ph < 0 || pw < 0) return DS_EINVAL;
+    if (!x || !dst || ph < 0 || pw < 0 || ph > kMaxPad || pw > kMaxPad) return DS_EINVAL;
+    if (H <= 0 || W <= 0 || H > (1 << 30) || W > (1 << 30)) return DS_EINVAL;
     const bool matrix = matrix_rows > 0;
     if (matrix && (H != 1 || W != 64 || ph || pw || Nb != ceil_div(matrix_rows, 64))) return DS_EINVAL;
     if (source < kSrcF32 || source > kSrcI8 || (source == kSrcI32 && x_bytes != 4) || (source == kSrcI8 && x_bytes != 1))
@@ -1127,6 +1130,7 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     q_bytes &= 0xff;
     if (!prepared || !blob || (!y && !out && !q) || (y && (out || q))) return DS_EINVAL;
     if (sh <= 0 || sw <= 0 || crop_h < 0 || crop_w < 0 || ph < 0 || pw < 0) return DS_EINVAL;
+    if (crop_h > kMaxPad || crop_w > kMaxPad || ph > kMaxPad || pw > kMaxPad) return DS_EINVAL;
     if (q && q_bytes != 1 && q_bytes != 4) return DS_EINVAL;
     const int mode = mode_of(max_shift, x_bytes);
     if (mode < 0 || ds_mfma_weight_bytes(O, C, FH, FW, max_shift, x_bytes) == 0) return DS_EINVAL;
@@ -1180,6 +1184,7 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     a.qpw = pw;
     a.qHp = a.OH + 2 * ph;
     a.qWp = a.OW + 2 * pw;
+    if (q && (double)a.qHp * a.qWp > 2147483647.0) return DS_EINVAL;
     a.inv = ldexpf(1.0f, -F_in);
     a.qspec = make_spec(I, F, DS_Q_ROUND_TO_FIXED);
     a.by_image = fast_div((uint32_t)(a.OH * a.OW));
@@ -1200,10 +1205,10 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
         const long cells = (long)Nb * O * (2L * ph * a.qWp + 2L * pw * a.OH);
         const unsigned blocks = (unsigned)((cells + 255) / 256 < 4096 ? (cells + 255) / 256 : 4096);
         if (q_bytes == 1)
-            hipLaunchKernelGGL((mfma_border_kernel<int8_t>), dim3(blocks), dim3(256), 0, st, (int8_t *)q, Nb * O, a.qHp,
+            hipLaunchKernelGGL((mfma_border_kernel<int8_t>), dim3(blocks), dim3(256), 0, st, (int8_t *)q, (long)Nb * O, a.qHp,
                                a.qWp, ph, pw);
         else
-            hipLaunchKernelGGL((mfma_border_kernel<int32_t>), dim3(blocks), dim3(256), 0, st, (int32_t *)q, Nb * O, a.qHp,
+            hipLaunchKernelGGL((mfma_border_kernel<int32_t>), dim3(blocks), dim3(256), 0, st, (int32_t *)q, (long)Nb * O, a.qHp,
                                a.qWp, ph, pw);
     }
     switch (mode) {

@@ -92,6 +92,29 @@ def test_invalid_sizes_and_workspace():
     assert L.ds_quantize_f32_i32(None, None, 0, 16, 16, 0, None) == 0
 
 
+def test_matrix_core_entry_points_refuse_sizes_past_a_launch():
+    """Rows times 256 threads stay below the 2^32 of a launch (larger inputs keep the kernels they had); an image without
+    rows or columns is refused whatever its padding (an unsigned test against a negative height lets every row in)."""
+    L = _lib.lib()
+    one = ctypes.c_void_p(256)
+    assert L.ds_mfma_input_bytes(1, 1, (1 << 24) - 1, 1, 3, 1, 4) > 0
+    assert L.ds_mfma_input_bytes(1, 1, 1 << 24, 1, 3, 1, 4) == 0
+    assert L.ds_mfma_input_bytes(1 << 20, 1, 32, 1, 1, 1, 1) == 0
+
+    def prepare(H, W, ph, pw):
+        return L.ds_mfma_prepare(one, 1, one, 1, 64, H, W, ph, pw, 1, 1, 0, 4, 0, 16, 16, None)
+
+    for sizes in [(-1, 8, 4, 0), (0, 8, 4, 0), (8, -3, 0, 4), (8, 0, 0, 4), (8, 8, 1 << 29, 0), (8, 8, 0, 1 << 30)]:
+        assert prepare(*sizes) == -1, sizes
+
+    def conv(ph, pw, crop=0):
+        return L.ds_mfma_conv2d(one, one, None, None, one, one, None, None, None, 1, 64, 8, 8, 64, 1, 1, 1, 1, crop, 0, 1, 1,
+                                0, 14, 4, 16, 0, 16, 16, ph, pw, 4, 1, 1, 0, 0, 0, None)
+
+    assert conv(1 << 17, 1 << 17) == -1     # a plane of more than 2^31 values
+    assert conv(1 << 29, 0) == -1 and conv(0, 1 << 30) == -1 and conv(0, 0, 1 << 30) == -1
+
+
 def test_error_is_raised_as_exception():
     with pytest.raises(_lib.DeepShiftError) as err:
         _lib.call("ds_quantize_f32_i32", None, None, 10, 0, 16, 0, None)
