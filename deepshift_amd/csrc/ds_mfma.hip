@@ -1039,6 +1039,12 @@ static int mode_of(int max_shift, int x_bytes)
     return max_shift <= 3 ? kI32S4 : max_shift <= 6 ? kI32S7 : max_shift <= 14 ? kI32S15 : -1;
 }
 
+// The formats that the conversions take (ds_quantize_f32_i32, ds_quantize_pad_f32_i8).
+static bool format_ok(int I, int F, int bytes)
+{
+    return F >= 0 && (bytes == 1 ? I >= 2 && I + F <= 8 : I >= 1 && I + F <= 32);
+}
+
 }  // namespace ds
 
 using namespace ds;
@@ -1095,6 +1101,8 @@ DS_EXPORT int ds_mfma_prepare(const void *x, int source, void *dst, int Nb, int 
     if (matrix && (H != 1 || W != 64 || ph || pw || Nb != ceil_div(matrix_rows, 64))) return DS_EINVAL;
     if (source < kSrcF32 || source > kSrcI8 || (source == kSrcI32 && x_bytes != 4) || (source == kSrcI8 && x_bytes != 1))
         return DS_EINVAL;
+    if (source == kSrcF32 && (!format_ok(I, F, x_bytes) || (mode != DS_Q_ROUND_TO_FIXED && (mode != DS_Q_CAST || x_bytes == 1))))
+        return DS_EINVAL;
     const int Hp = H + 2 * ph, Wp = W + 2 * pw;
     if (ds_mfma_input_bytes(Nb, C, Hp, Wp, FH, FW, x_bytes) == 0) return DS_EINVAL;
     PrepArgs a{};
@@ -1131,7 +1139,8 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     if (!prepared || !blob || (!y && !out && !q) || (y && (out || q))) return DS_EINVAL;
     if (sh <= 0 || sw <= 0 || crop_h < 0 || crop_w < 0 || ph < 0 || pw < 0) return DS_EINVAL;
     if (crop_h > kMaxPad || crop_w > kMaxPad || ph > kMaxPad || pw > kMaxPad) return DS_EINVAL;
-    if (q && q_bytes != 1 && q_bytes != 4) return DS_EINVAL;
+    if (q && ((q_bytes != 1 && q_bytes != 4) || !format_ok(I, F, q_bytes))) return DS_EINVAL;
+    if (!y && (F_in < 0 || F_in > 31)) return DS_EINVAL;
     const int mode = mode_of(max_shift, x_bytes);
     if (mode < 0 || ds_mfma_weight_bytes(O, C, FH, FW, max_shift, x_bytes) == 0) return DS_EINVAL;
     if (ds_mfma_input_bytes(Nb, C, Hp, Wp, prep_FH, prep_FW, x_bytes) == 0) return DS_EINVAL;

@@ -1075,6 +1075,8 @@ def _operand_output(cache, dims, kernel_size, padding, x_bytes, device):
 def mfma_prepare(x, padding, kernel_size, x_bytes, integer_bits=16, fraction_bits=16, round_to_fixed=True):
     """float32 / int32 / int8 NCHW images, or a float32 / int32 matrix [M, K], -> :class:`Prepared`, or ``None``
     where the matrix-core kernels do not serve the size."""
+    if not x.is_cuda or x.dtype not in _MFMA_SRC or x.dim() not in (2, 4):
+        raise TypeError("mfma_prepare expects a matrix or NCHW images of float32, int32 or int8 on the GPU")
     x = x.contiguous()
     ph, pw = _pair(padding)
     FH, FW = _pair(kernel_size)

@@ -325,6 +325,8 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
     I, Fb = module.act_integer_bits, module.act_fraction_bits
     padding = (0, 0) if prequantized else module.padding
     handed = isinstance(input, kernels.Prepared)
+    if not handed and (input.dim() != 4 or not input.is_cuda):
+        return None
     if handed:
         x_bytes = input.x_bytes
     elif prequantized:
@@ -336,8 +338,6 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
             input = _circular_pad(input, padding)
             padding = (0, 0)
     Nb, C, H, W = input.dims if handed else input.shape
-    if not handed and not input.is_cuda:
-        return None
     if not kernels._mfma_conv_serves(Nb, C, H + 2 * padding[0], W + 2 * padding[1], module.out_channels,
                                                          module.kernel_size, module.stride, x_bytes):
         return None

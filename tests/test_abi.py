@@ -115,6 +115,28 @@ def test_matrix_core_entry_points_refuse_sizes_past_a_launch():
     assert conv(1 << 29, 0) == -1 and conv(0, 1 << 30) == -1 and conv(0, 0, 1 << 30) == -1
 
 
+def test_matrix_core_entry_points_refuse_the_formats_that_conversions_refuse():
+    L = _lib.lib()
+    one = ctypes.c_void_p(256)
+
+    def prepare(I, F, mode, x_bytes):
+        return L.ds_mfma_prepare(one, 0, one, 1, 64, 8, 8, 1, 1, 3, 3, 0, x_bytes, mode, I, F, None)
+
+    def conv(I, F, q_bytes, F_in=16):
+        return L.ds_mfma_conv2d(one, one, None, None, one, one, None, None, None, 1, 64, 8, 8, 64, 1, 1, 1, 1, 0, 0, 1, 1, 0,
+                                14, 4, F_in, 0, I, F, 0, 0, q_bytes, 1, 1, 0, 0, 0, None)
+
+    for I, F, mode in [(0, 16, 0), (20, 20, 0), (16, -1, 0), (40, -16, 1), (16, 16, 2), (16, 16, -1)]:
+        assert L.ds_quantize_f32_i32(one, one, 10, I, F, mode, None) == -1
+        assert prepare(I, F, mode, 4) == -1, (I, F, mode)
+    for I, F in [(1, 5), (5, 4), (12, -4)]:
+        assert L.ds_quantize_pad_f32_i8(one, one, 1, 1, 4, 4, 0, 0, I, F, None) == -1
+        assert prepare(I, F, 0, 1) == -1 and conv(I, F, 1) == -1, (I, F)
+    assert prepare(3, 5, 1, 1) == -1                     # 8-bit activations are rounded, never cast
+    assert conv(0, 16, 4) == -1 and conv(20, 20, 4) == -1 and conv(16, -1, 4) == -1
+    assert conv(16, 16, 4, -1) == -1 and conv(16, 16, 4, 32) == -1
+
+
 def test_error_is_raised_as_exception():
     with pytest.raises(_lib.DeepShiftError) as err:
         _lib.call("ds_quantize_f32_i32", None, None, 10, 0, 16, 0, None)

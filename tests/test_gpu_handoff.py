@@ -4,7 +4,7 @@ import pytest
 import torch
 import torch.nn as nn
 
-from deepshift_amd import convert, fuse, kernels, modules
+from deepshift_amd import _lib, convert, fuse, kernels, modules
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -214,3 +214,24 @@ def test_a_buffer_that_nobody_zeroed_gets_its_border(x_bytes, O, pad):
     y = kernels.mfma_conv2d(got, blob2, None, 48, (3, 3), (1, 1), 14)
     again = kernels.mfma_conv2d(kernels.mfma_prepare(want, 0, (3, 3), x_bytes), blob2, None, 48, (3, 3), (1, 1), 14)
     assert torch.equal(y, again)
+
+
+@pytest.mark.parametrize("fmt", [(0, 16), (20, 20), (12, -4), (1, 5)], ids=str)
+def test_modules_refuse_what_their_conversion_refuses(fmt):
+    """Formats past 32 bits or without an integer bit (1.5 is the reference's one-bit format: served), inputs on the host or
+    without a batch."""
+    I, F = fmt
+    conv = modules.Conv2dShift(64, 64, 3, padding=1, bias=False, use_kernel=True, act_integer_bits=I, act_fraction_bits=F).to(DEV)
+    linear = modules.LinearShift(2112, 64, bias=False, use_kernel=True, act_integer_bits=I, act_fraction_bits=F).to(DEV)
+    with torch.no_grad():
+        for layer, x in ((conv, torch.zeros(1, 64, 8, 8, device=DEV)), (linear, torch.zeros(3, 2112, device=DEV))):
+            if I == 1:
+                assert layer(x).device.type == "cuda"
+                with pytest.raises(TypeError):
+                    layer(x.cpu())
+            else:
+                with pytest.raises(_lib.DeepShiftError):
+                    layer(x)
+        if I == 1:
+            with pytest.raises(TypeError):
+                conv(torch.zeros(64, 8, 8, device=DEV))
