@@ -83,6 +83,14 @@ class ConcWeight():
         # the kernels then run the layer from a narrower private blob (0: not applicable).
         self.zero_top_bits = zero_top_bits
 
+    def __getstate__(self):
+        # the kernels' blobs (up to four bytes a weight) belong to the memory that ``data`` lies in: copies and files
+        # hold the words, and a copy lays its own out
+        state = self.__dict__.copy()
+        for blob in ("_tiled", "_paired", "_mfma"):
+            state.pop(blob, None)
+        return state
+
 
 def shift_field_bits(min_shift):
     """utils.py:72: ``ceil(log(1 - min(shift)) / ln 2)`` with the log taken in float32 like

@@ -319,3 +319,18 @@ def test_hand_off_buffers_do_not_travel_with_copies_of_a_module():
     convq = modules_q.Conv2dShiftQ(4, 8, 3, padding=1)
     convq.__dict__["_handoff_buffers"] = {"k": torch.zeros(3)}
     assert "_handoff_buffers" not in copy.deepcopy(convq).__dict__
+
+
+def test_kernel_blobs_do_not_travel_with_packed_weights():
+    import copy
+    import pickle
+    cw = utils.ConcWeight(torch.arange(6, dtype=torch.int32), 0, 4, 0, 14)
+    size = len(pickle.dumps(cw))
+    cw._tiled = ((1,), torch.zeros(1000))
+    cw._paired = ((1,), torch.zeros(1000))
+    cw._mfma = {4: ((1,), torch.zeros(1000))}
+    assert len(pickle.dumps(cw)) == size
+    for copied in (copy.deepcopy(cw), pickle.loads(pickle.dumps(cw))):
+        assert torch.equal(copied.data, cw.data) and (copied.base, copied.bits, copied.max_field) == (0, 4, 14)
+        assert not {"_tiled", "_paired", "_mfma"} & set(copied.__dict__)
+    assert len(cw._mfma) == 1
