@@ -632,10 +632,12 @@ def linear_forward(x2d, conc_weight, bias, N, integer_bits, fraction_bits, round
     M, K = x2d.shape
     # the one-launch kernel's time grows with K whatever M is (1 x 4096 x 4096: 128 us against 51 here), and with the
     # pairs (512 x 512 x 512: 21 against 25 us, 128 x 2048 x 1000: 42 against 30)
-    if not (small_linear_serves(M, K, N) and K <= 2048 and M * K * N <= 1 << 27):
-        route = mfma_route(x2d, 0, conc_weight, N, (1, 1), 4, integer_bits, fraction_bits, round_to_fixed)
-        if route is not None:
-            return mfma_conv2d(route[0], route[1], bias, N, (1, 1), 1, route[2], 0, fraction_bits, relu=relu)[0]
+    if K <= 2048 and M * K * N <= 1 << 27 and small_linear_serves(M, K, N):
+        return linear_small(x2d, _tiled_of(conc_weight, N, K), bias, N, kernel_bits(conc_weight), conc_weight.base,
+                            integer_bits, fraction_bits, round_to_fixed, relu)
+    route = mfma_route(x2d, 0, conc_weight, N, (1, 1), 4, integer_bits, fraction_bits, round_to_fixed)
+    if route is not None:
+        return mfma_conv2d(route[0], route[1], bias, N, (1, 1), 1, route[2], 0, fraction_bits, relu=relu)[0]
     return linear_layer(x2d, _tiled_of(conc_weight, N, K), bias, N, kernel_bits(conc_weight), conc_weight.base,
                         integer_bits, fraction_bits, round_to_fixed, relu)
 

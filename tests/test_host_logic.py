@@ -334,3 +334,15 @@ def test_kernel_blobs_do_not_travel_with_packed_weights():
         assert torch.equal(copied.data, cw.data) and (copied.base, copied.bits, copied.max_field) == (0, 4, 14)
         assert not {"_tiled", "_paired", "_mfma"} & set(copied.__dict__)
     assert len(cw._mfma) == 1
+
+
+def test_small_linear_layers_are_routed_once(monkeypatch):
+    """The one-launch kernel's layers are bound by the host: one look at the sizes, one call."""
+    asked, launched = [], []
+    real = kernels.small_linear_serves
+    monkeypatch.setattr(kernels, "small_linear_serves", lambda *a: asked.append(a) or real(*a))
+    monkeypatch.setattr(kernels, "_tiled_of", lambda *a: "tiled")
+    monkeypatch.setattr(kernels, "linear_small", lambda *a: launched.append(a[1]) or "out")
+    cw = utils.ConcWeight(None, 0, 4, 0, 14)
+    assert kernels.linear_forward(torch.zeros(8, 329), cw, None, 10, 16, 16, False) == "out"
+    assert asked == [(8, 329, 10)] and launched == ["tiled"]
