@@ -327,20 +327,24 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
     handed = isinstance(input, kernels.Prepared)
     if not handed and (input.dim() != 4 or not input.is_cuda):
         return None
+    circular = not prequantized and module.padding_mode == 'circular'
     if handed:
         x_bytes = input.x_bytes
     elif prequantized:
         x_bytes = input.element_size()
     else:
         x_bytes = 1 if I >= 2 and I + Fb <= 8 else 4
-        input = input.float()
-        if module.padding_mode == 'circular':
-            input = _circular_pad(input, padding)
-            padding = (0, 0)
     Nb, C, H, W = input.dims if handed else input.shape
-    if not kernels._mfma_conv_serves(Nb, C, H + 2 * padding[0], W + 2 * padding[1], module.out_channels,
-                                                         module.kernel_size, module.stride, x_bytes):
+    around = 1 if circular else 2            # circular padding adds its size once (_circular_pad)
+    if not kernels._mfma_conv_serves(Nb, C, H + around * padding[0], W + around * padding[1], module.out_channels,
+                                     module.kernel_size, module.stride, x_bytes):
         return None
+    if not prequantized:
+        if circular:
+            if kernels.mfma_shift(conc_weight, x_bytes) is None:
+                return None
+            input, padding = _circular_pad(input.float(), padding), (0, 0)
+        input = input.float()
     route = kernels.mfma_route(input, padding, conc_weight, module.out_channels, module.kernel_size, x_bytes, I, Fb)
     if route is None:
         return None

@@ -235,3 +235,23 @@ def test_modules_refuse_what_their_conversion_refuses(fmt):
         if I == 1:
             with pytest.raises(TypeError):
                 conv(torch.zeros(64, 8, 8, device=DEV))
+
+
+@pytest.mark.parametrize("C,O,top", [(24, 40, 14), (8, 8, 14), (24, 40, 20)])
+@pytest.mark.parametrize("pad", [(1, 1), (2, 1), (3, 2)])
+def test_circular_padding_is_made_once(monkeypatch, C, O, top, pad):
+    """... on whichever kernel the layer runs: matrix cores, few channels, shifts past 14."""
+    torch.manual_seed(4)
+    layer = modules.Conv2dShift(C, O, 3, padding=pad, padding_mode="circular", use_kernel=True, weight_bits=6, bias=False).to(DEV)
+    layer.shift.data.copy_(torch.randint(-top, 1, layer.shift.shape).float())
+    layer.shift.data.view(-1)[0] = -top
+    layer.sign.data.copy_(torch.randint(0, 2, layer.sign.shape).float() * 2 - 1)
+    x = torch.randn(2, C, 9, 7, device=DEV)
+    made = []
+    real = modules._circular_pad
+    monkeypatch.setattr(modules, "_circular_pad", lambda *a: made.append(1) or real(*a))
+    with torch.no_grad():
+        got = layer(x)
+        assert len(made) == 1
+        y = kernels.conv2d(kernels.quantize(real(x, pad)), layer.shift, layer.sign, None, layer.packed_weights())
+        assert torch.equal(got, kernels.dequantize(y))
