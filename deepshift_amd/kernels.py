@@ -844,10 +844,7 @@ def conv2d_paired(x_padded, paired, bias, O, kernel_size, stride, field_bits, x_
     """Shift convolution on an already padded int8 NCHW input and the blob of
     :func:`tile_weights_paired`; the int32 result of :func:`conv2d_tiled` on the same values.
     ``x_bound``: a bound on ``|x|`` that the caller vouches for (128 always holds); a smaller one lets
-    the kernel widen its 16-bit sums less often.  Activations that :func:`mfma_prepare` laid out go to the matrix
-    cores, with the blob and the ``max_shift`` of :func:`mfma_route` as ``paired`` and ``field_bits``."""
-    if isinstance(x_padded, Prepared):
-        return mfma_conv2d(x_padded, paired, bias, O, kernel_size, stride, field_bits)
+    the kernel widen its 16-bit sums less often."""
     if x_padded.dtype != torch.int8 or not x_padded.is_cuda or x_padded.dim() != 4:
         raise TypeError("x_padded must be a 4-D int8 GPU tensor")
     x_padded = x_padded.contiguous()
@@ -873,11 +870,7 @@ def conv2d_paired_fused(x_padded, paired, bias, O, kernel_size, stride, field_bi
     result ``act(y / 2**F * scale[c] + shift[c] + residual)`` (``None`` unless ``want_float``) and, with
     ``emit = (padding, integer_bits, fraction_bits, dtype)``, the next shift convolution's round-to-fixed,
     zero padded input.  Bit-identical to :func:`conv2d_paired` followed by :func:`requantize_affine_pad`
-    / :func:`dequantize_affine`; no pre-fill, no atomics, the int32 sums are never stored.  Prepared
-    activations as for :func:`conv2d_paired`."""
-    if isinstance(x_padded, Prepared):
-        return mfma_conv2d(x_padded, paired, bias, O, kernel_size, stride, field_bits, 0, fraction_bits_in, scale, shift,
-                           residual, relu, emit, want_float, q_cache)
+    / :func:`dequantize_affine`; no pre-fill, no atomics, the int32 sums are never stored."""
     if x_padded.dtype != torch.int8 or not x_padded.is_cuda or x_padded.dim() != 4:
         raise TypeError("x_padded must be a 4-D int8 GPU tensor")
     x_padded = x_padded.contiguous()

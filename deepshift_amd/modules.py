@@ -298,10 +298,10 @@ def conv_cpu_forward(module, input, shift, sign):
     return (out.float() / 2.0 ** Fb).to(input.device)
 
 
-# Switch for the fused convolution epilogue (kernels.conv2d_tiled_fused); off = always the separate
-# conversion pass, which the tests compare it with.
+# Switch for the fused convolution epilogues (kernels.mfma_conv2d, kernels.conv2d_tiled_fused); off = always the
+# separate conversion pass, which the tests compare them with.
 _FUSE_EPILOGUE = True
-_FUSE_INT8 = True   # ... and the int8 kernel's (kernels.conv2d_paired_fused)
+_FUSE_INT8 = True   # ... and those of launches on int8 activations (kernels.mfma_conv2d, kernels.conv2d_paired_fused)
 
 
 def _small_for_int8(module, input_shape, field_bits):
@@ -350,36 +350,43 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
         return None
     prepared, blob, max_shift = route
     bias = module._fixed_bias.get(module.bias, I, Fb, round_to_fixed=True)
-    int8_entry = x_bytes == 1 and kernels.paired_fields(conc_weight, module.out_channels, I, Fb)
-    if pool is not None:
-        sums = kernels.conv2d_paired if int8_entry else kernels.mfma_conv2d
-        out = sums(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift)
-        return _pooled(out, Fb, scale, shift, residual, relu, pool, emit)
+    if pool is not None or not _FUSE_EPILOGUE or (x_bytes == 1 and not _FUSE_INT8):
+        out = kernels.mfma_conv2d(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift)
+        return _separate_pass(out, Fb, scale, shift, residual, relu, pool, emit)
     want_float, spec = True, None
     if emit is not None:
         want_float = emit[3]
         spec = tuple(emit[:3]) + (emit[4] if len(emit) == 5 else torch.int32, emit_filter)
     # the consumers' padded input lives in a buffer of this layer whose border is zeroed once
     cache = module.__dict__.setdefault("_handoff_buffers", {})
-    fused = kernels.conv2d_paired_fused if int8_entry else kernels.mfma_conv2d
-    f, q = fused(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift, 0, Fb, scale,
-                 shift, residual, relu, spec, want_float, cache)
+    f, q = kernels.mfma_conv2d(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift, 0, Fb,
+                               scale, shift, residual, relu, spec, want_float, cache)
     if emit is None:
         return f
     return (f, q) if want_float else q
 
 
-def _pooled(out, Fb, scale, shift, residual, relu, pool, emit):
-    """The pass behind a convolution whose ReLU is followed by a max pooling."""
-    if residual is not None:
-        raise ValueError("a fused max pooling cannot follow a residual add")
-    if emit is None:
-        return kernels.requantize_affine_maxpool(out, Fb, scale, shift, relu, pool)[0]
-    next_padding, next_I, next_F, want_float = emit[:4]
-    dtype = emit[4] if len(emit) == 5 else torch.int32
-    f, q = kernels.requantize_affine_maxpool(out, Fb, scale, shift, relu, pool, next_padding, next_I, next_F, want_float,
+def _separate_pass(out, Fb, scale, shift, residual, relu, pool, emit):
+    """What follows a convolution's int32 sums in a pass of its own: a max pooling behind the ReLU always, the rest where
+    no launch with a fused epilogue serves the layer."""
+    if emit is not None:
+        next_padding, next_I, next_F, want_float = emit[:4]
+        dtype = emit[4] if len(emit) == 5 else torch.int32
+    if pool is not None:
+        if residual is not None:
+            raise ValueError("a fused max pooling cannot follow a residual add")
+        if emit is None:
+            return kernels.requantize_affine_maxpool(out, Fb, scale, shift, relu, pool)[0]
+        f, q = kernels.requantize_affine_maxpool(out, Fb, scale, shift, relu, pool, next_padding, next_I, next_F, want_float,
+                                                 dtype)
+        return (f, q) if want_float else q
+    if emit is not None:
+        f, q = kernels.requantize_affine_pad(out, Fb, scale, shift, residual, relu, next_padding, next_I, next_F, want_float,
                                              dtype)
-    return (f, q) if want_float else q
+        return (f, q) if want_float else q
+    if scale is None and shift is None and residual is None and not relu:
+        return kernels.dequantize(out, Fb)
+    return kernels.dequantize_affine(out, Fb, scale, shift, residual, relu)
 
 
 def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, residual=None, relu=False,
@@ -405,7 +412,6 @@ def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, resi
     if module.dilation != (1, 1) or module.groups != 1:
         raise NotImplementedError("the shift kernel supports dilation=1 and groups=1 only")
     I, Fb = module.act_integer_bits, module.act_fraction_bits
-    # formats of at most 8 bits on narrow shift fields: int8 activations, two pixels per register
     result = _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, prequantized, emit, pool,
                            emit_filter)
     if result is not None:
@@ -413,6 +419,7 @@ def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, resi
     if isinstance(input, kernels.Prepared):
         # weights that the matrix cores have no form for, loaded after the model was fused
         input = input.padded()
+    # formats of at most 8 bits on narrow shift fields: int8 activations, two pixels per register
     fields = kernels.paired_fields(conc_weight, module.out_channels, I, Fb)
     if prequantized:
         xq = input
@@ -475,19 +482,7 @@ def conv_kernel_forward(module, input, conc_weight, scale=None, shift=None, resi
             return (f, q) if want_float else q
         out = kernels.conv2d_tiled(xq, tiled, bias, module.out_channels, module.kernel_size,
                                    module.stride, kbits, conc_weight.base)
-    if pool is not None:
-        return _pooled(out, Fb, scale, shift, residual, relu, pool, emit)
-    emit_dtype = torch.int32
-    if emit is not None and len(emit) == 5:
-        emit, emit_dtype = emit[:4], emit[4]
-    if emit is not None:
-        next_padding, next_I, next_F, want_float = emit
-        f, q = kernels.requantize_affine_pad(out, Fb, scale, shift, residual, relu, next_padding,
-                                             next_I, next_F, want_float, emit_dtype)
-        return (f, q) if want_float else q
-    if scale is None and shift is None and residual is None and not relu:
-        return kernels.dequantize(out, Fb)
-    return kernels.dequantize_affine(out, Fb, scale, shift, residual, relu)
+    return _separate_pass(out, Fb, scale, shift, residual, relu, pool, emit)
 
 
 class Conv2dShift(_ConvNdShift):

@@ -227,42 +227,58 @@ def test_int8_conversions_refuse_wider_formats():
 # ----------------------------------------------------------------------------- through the modules
 
 def test_models_with_8_bit_activations_take_the_int8_kernel_and_keep_their_output(monkeypatch):
-    """ResNet-50 with weight_bits 3 and 3.5 activations: the fused model runs its 64-channel layers on
-    the int8 kernel; switching that off (int32 kernels on the same values) must not change a bit."""
-    from deepshift_amd import convert, fuse, kernels, workloads
+    """ResNet-50 with weight_bits 3 and 3.5 activations: every convolution runs on 8-bit activations on the matrix cores,
+    fused or not; without those the 64-channel layers of the fused model run on the int8 vector kernel; without that
+    (int32 kernels on the same values) and without fused launches no bit changes either."""
+    from deepshift_amd import convert, fuse, kernels, modules, workloads
     g = torch.Generator().manual_seed(3)
     model = workloads.randomize_batchnorm(workloads.ResNet50(), g).eval()
     model, n = convert.convert_to_shift(model, 1000, 'PS', convert_weights=True, use_kernel=True,
                                         weight_bits=3, act_integer_bits=3, act_fraction_bits=5)
     model = model.to(DEV)
     x = torch.randn(2, 3, 64, 64, generator=g).to(DEV)
-    calls = []
-    real, real_fused = kernels.conv2d_paired, kernels.conv2d_paired_fused
-    monkeypatch.setattr(kernels, "conv2d_paired", lambda *a, **k: calls.append(1) or real(*a, **k))
-    monkeypatch.setattr(kernels, "conv2d_paired_fused", lambda *a, **k: calls.append(1) or real_fused(*a, **k))
-    with torch.no_grad():
-        fused = fuse.fuse_conv_epilogues(model)
-        got = fused(x)
-        unfused = model(x)
+    matrix, vector, fused_launches = [], [], []
+    real_mfma, real, real_fused = kernels.mfma_conv2d, kernels.conv2d_paired, kernels.conv2d_paired_fused
+
+    def mfma(prepared, *a, **k):
+        if not prepared.rows:
+            matrix.append(prepared.x_bytes)
+        return real_mfma(prepared, *a, **k)
+
+    monkeypatch.setattr(kernels, "mfma_conv2d", mfma)
+    monkeypatch.setattr(kernels, "conv2d_paired", lambda *a, **k: vector.append(1) or real(*a, **k))
+    monkeypatch.setattr(kernels, "conv2d_paired_fused",
+                        lambda *a, **k: vector.append(1) or fused_launches.append(1) or real_fused(*a, **k))
+
+    def both():
+        with torch.no_grad():
+            return fuse.fuse_conv_epilogues(model)(x), model(x)
+
+    got, unfused = both()
+    assert matrix == [1] * (2 * 53) and not vector
+    monkeypatch.setattr(modules, "_FUSE_INT8", False)
+    want, want_unfused = both()
+    assert torch.equal(got, want) and torch.equal(unfused, want_unfused)
+    monkeypatch.setattr(modules, "_FUSE_INT8", True)
     # every convolution of ResNet-50 has a multiple of 64 channels; at this image size the layers that
     # convert their own input are small enough to stay on the int32 kernels, the ones that are handed
     # int8 activations by their producer are not asked
-    taken = len(calls)
-    assert 30 <= taken <= 2 * 53
-    monkeypatch.setattr(kernels, "paired_fields", lambda *a, **k: None)
-    with torch.no_grad():
-        want = fuse.fuse_conv_epilogues(model)(x)
-        want_unfused = model(x)
-    assert len(calls) == taken
-    assert torch.equal(got, want)
-    assert torch.equal(unfused, want_unfused)
+    monkeypatch.setattr(kernels, "mfma_shift", lambda *a: None)
+    taken = len(matrix)
+    want, want_unfused = both()
+    assert len(matrix) == taken and 30 <= len(vector) <= 2 * 53 and len(fused_launches) >= 30
+    assert torch.equal(got, want) and torch.equal(unfused, want_unfused)
     # ... and neither does switching the int8 kernel's fused launch off (int8 kernel + conversion pass)
-    monkeypatch.undo()
-    from deepshift_amd import modules
     monkeypatch.setattr(modules, "_FUSE_INT8", False)
-    with torch.no_grad():
-        assert torch.equal(fuse.fuse_conv_epilogues(model)(x), got)
-        assert torch.equal(model(x), unfused)
+    launched = len(fused_launches)
+    want, want_unfused = both()
+    assert len(fused_launches) == launched and len(vector) >= 60
+    assert torch.equal(got, want) and torch.equal(unfused, want_unfused)
+    monkeypatch.setattr(kernels, "paired_fields", lambda *a, **k: None)
+    taken = len(vector)
+    want, want_unfused = both()
+    assert len(vector) == taken
+    assert torch.equal(got, want) and torch.equal(unfused, want_unfused)
 
 
 @pytest.mark.parametrize("seed", range(24))
