@@ -1051,8 +1051,28 @@ class Prepared:
         v = sum(d[i].int() << (7 * i) for i in range(3))
         return v + torch.where(high, (d[3].int() << 21) + (d[4].int() << 28), torch.zeros_like(v))
 
+    # Hooks and other readers of a hand-off find what a padded int32 / int8 tensor answers; each such look is a copy.
+    @property
+    def shape(self):
+        return torch.Size(self.dims)
+
+    @property
+    def device(self):
+        return self.data.device
+
     def __getitem__(self, item):
         return self.padded()[item]
+
+    def __getattr__(self, name):
+        if name.startswith("_") or name in ("written_by_conv", "data", "dims", "filter", "rows", "x_bytes") or self.written_by_conv is None:
+            raise AttributeError(name)
+        return getattr(self.padded(), name)
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        args, kwargs = torch.utils._pytree.tree_map(lambda v: v.padded() if isinstance(v, Prepared) else v,
+                                                    (args, kwargs or {}))
+        return func(*args, **kwargs)
 
 
 def _operand_output(cache, dims, kernel_size, padding, x_bytes, device):

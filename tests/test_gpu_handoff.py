@@ -255,3 +255,28 @@ def test_circular_padding_is_made_once(monkeypatch, C, O, top, pad):
         assert len(made) == 1
         y = kernels.conv2d(kernels.quantize(real(x, pad)), layer.shift, layer.sign, None, layer.packed_weights())
         assert torch.equal(got, kernels.dequantize(y))
+
+
+def test_forward_hooks_read_a_hand_off_as_a_tensor():
+    import copy
+    with torch.no_grad():
+        model = _model(16, 16)
+        x = _inputs(1, 2, H=9)[0]
+        seen = []
+
+        def hook(module, args, out):
+            if isinstance(out, kernels.Prepared):
+                seen.append((tuple(out.shape), out.dtype, out.device, out.dim(), out.size(1), out.float().mean().item(),
+                             int(torch.count_nonzero(out)), torch.equal(out, out.padded()), tuple(out[0, :2].shape)))
+
+        for m in model.modules():
+            if isinstance(m, fuse.FusedConv2dShift):
+                m.register_forward_hook(hook)
+        want = model(x)
+        assert len(seen) == 3
+        for shape, dtype, device, dim, channels, mean, count, same, first in seen:
+            assert len(shape) == dim == 4 and channels == shape[1] == 64 and dtype == torch.int32 and device == x.device
+            assert mean > 0 and count > 0 and same and first == (2,) + shape[2:]
+        q = model.get_submodule("fused_0")(x)
+        assert not hasattr(q, "no_such_name") and copy.copy(q).dims == q.dims
+        assert torch.equal(model(x), want)
