@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from deepshift_amd import kernels, modules, utils
+from deepshift_amd import kernels, modules, modules_q, utils
 from tests.conftest import random_codes
 
 pytestmark = pytest.mark.gpu
@@ -184,3 +184,79 @@ def test_operand_buffers_are_not_reused_while_held(rng):
     held = second.data.data_ptr()
     del second
     assert kernels.mfma_conv2d(*args)[1].data.data_ptr() == held
+
+
+@pytest.mark.parametrize("K", [2050, 2112])
+@pytest.mark.parametrize("rounded", [False, True], ids=["cast", "round"])
+def test_float_matrices_match_the_oracle(oracle, rng, K, rounded):
+    """The route of large LinearShift / LinearShiftQ layers: float rows converted on the way in, from an odd address, a
+    row count past a block of 64, an odd row length (no four-wide loads) and one of fours, ReLU, values past the format,
+    infinities and NaN."""
+    M, N, I, F = 70, 45, 16, 16
+    cls = modules_q.LinearShiftQ if rounded else modules.LinearShift
+    layer = cls(K, N, use_kernel=True).to(DEV)
+    s, sign = random_codes(rng, (N, K), max_s=14)
+    with torch.no_grad():
+        if rounded:
+            layer.weight.copy_(_dev((sign * 2.0 ** -s).astype(np.float32)))
+        else:
+            layer.shift.copy_(_dev(-s.astype(np.float32)))
+            layer.sign.copy_(_dev(sign.astype(np.float32)))
+        layer.bias.copy_(torch.randn(N))
+    x = (rng.standard_normal((M, K)) * 2.0 ** rng.integers(-18, 18, size=(M, K))).astype(np.float32)
+    x.flat[::97] = np.float32("nan")
+    x.flat[5::89] = np.float32("inf")
+    x.flat[7::83] = -np.float32("inf")
+    x.flat[11::79] = -0.0
+    x.flat[13::71] = 1e-40
+    x[3] = 0.25                         # a row without any of these
+    base = torch.empty(M * K + 1, device=DEV)
+    base[1:] = _dev(x).reshape(-1)
+    convert = (lambda v: oracle.quantize(v, I, F)) if rounded else (lambda v: oracle.cast(v, F))
+    bias = convert(layer.bias.detach().cpu().numpy())
+    want = oracle.linear(convert(x), -s.astype(np.int32), sign.astype(np.int32), bias).astype(np.float32) / np.float32(2.0 ** F)
+    with torch.no_grad():
+        for xd in (_dev(x), base[1:].view(M, K)):
+            np.testing.assert_array_equal(layer(xd).cpu().numpy(), want)
+        np.testing.assert_array_equal(layer._kernel_forward(_dev(x), relu=True).cpu().numpy(), np.maximum(want, 0))
+
+
+# Tiles of 32 x 64: enough for a part of the reduction per wave (ks 1) and for two waves a tile (ks 2), whatever the
+# number of compute units up to 256: more than 3 and 1.5 times the 12 or 8 waves each holds.  Pixel counts end inside a
+# tile, channels inside a tile of 32 and, where two are odd, inside a pair of them.
+LARGE = [("ks1", 4, 70, (29, 7, 667)), ("ks1", 4, 20, (9, 1, 43781)), ("ks1", 1, 70, (31, 9, 709)),
+         ("ks2", 4, 70, (13, 7, 733)), ("ks2", 1, 33, (19, 9, 877))]
+
+
+@pytest.mark.parametrize("form,x_bytes,O,pixels", LARGE, ids=lambda v: str(v).replace(" ", ""))
+@pytest.mark.parametrize("top", [14, 6, 2])
+def test_epilogues_of_large_launches(oracle, rng, form, x_bytes, O, pixels, top):
+    """The register epilogue of launches with many tiles, and the one that two waves share: sums against the oracle; float,
+    padded and operand-layout results, with and without residual, against the separate passes."""
+    Nb, H, W = pixels
+    C, k = 20, 3
+    P = Nb * H * W
+    waves = 256 * (12 if x_bytes == 1 else 8)
+    tiles = -(-O // 32) * -(-P // 64)
+    assert P % 64 and (tiles >= 3 * waves if form == "ks1" else 3 * waves / 2 <= tiles < 3 * waves)
+    s, sign, cw = _weights(rng, (O, C, k, k), top, ternary=True)
+    x = _activations(rng, (Nb, C, H, W), x_bytes, 1 << 18)
+    if x_bytes == 4:
+        x[-1, ..., -1] = -2 ** 31           # high digits in the last tile
+    bias = rng.integers(-2 ** 20, 2 ** 20, size=O).astype(np.int32)
+    prepared, blob, shift_top = kernels.mfma_route(_dev(x), 1, cw, O, (k, k), x_bytes)
+    y = kernels.mfma_conv2d(prepared, blob, _dev(bias), O, (k, k), 1, shift_top)
+    xp = np.pad(x.astype(np.int32), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    want = oracle.conv2d(xp, -s.astype(np.int32), sign.astype(np.int32), bias, (1, 1), nthreads=16)
+    np.testing.assert_array_equal(y.cpu().numpy(), want)
+    F_in, I, F, dtype = (16, 16, 16, torch.int32) if x_bytes == 4 else (5, 3, 5, torch.int8)
+    scale, shift = (torch.rand(O, device=DEV) + 0.5), torch.randn(O, device=DEV)
+    for residual in (None, torch.randn(y.shape, device=DEV)):
+        f, q = kernels.requantize_affine_pad(y, F_in, scale, shift, residual, True, (1, 1), I, F, True, dtype)
+        args = (prepared, blob, _dev(bias), O, (k, k), 1, shift_top, 0, F_in, scale, shift, residual, True)
+        out, padded = kernels.mfma_conv2d(*args, ((1, 1), I, F, dtype), True)
+        assert torch.equal(out, f) and torch.equal(padded, q)
+        out, handed = kernels.mfma_conv2d(*args, ((1, 1), I, F, dtype, (3, 3)), True)
+        assert torch.equal(out, f) and torch.equal(handed.padded(), q)
+        only, handed = kernels.mfma_conv2d(*args, ((1, 1), I, F, dtype, (3, 3)), False)
+        assert only is None and torch.equal(handed.padded(), q)
