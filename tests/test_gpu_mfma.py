@@ -221,24 +221,25 @@ def test_float_matrices_match_the_oracle(oracle, rng, K, rounded):
         np.testing.assert_array_equal(layer._kernel_forward(_dev(x), relu=True).cpu().numpy(), np.maximum(want, 0))
 
 
-# Tiles of 32 x 64: enough for a part of the reduction per wave (ks 1) and for two waves a tile (ks 2), whatever the
-# number of compute units up to 256: more than 3 and 1.5 times the 12 or 8 waves each holds.  Pixel counts end inside a
-# tile, channels inside a tile of 32 and, where two are odd, inside a pair of them.
-LARGE = [("ks1", 4, 70, (29, 7, 667)), ("ks1", 4, 20, (9, 1, 43781)), ("ks1", 1, 70, (31, 9, 709)),
-         ("ks2", 4, 70, (13, 7, 733)), ("ks2", 1, 33, (19, 9, 877))]
+# (parts of the reduction, x_bytes, C, O, pixels): tiles of 32 x 64 past the fill of the chip's wave slots at which the
+# reduction is one wave's (9 blocks: a quarter), and between one and one and a quarter tiles a slot, where two waves share
+# a long one (36 blocks).  Pixel counts end inside a tile, channels inside a tile of 32 and, where the tiles of 32 are odd
+# in number, inside a pair of them.
+LARGE = [(1, 4, 20, 70, (29, 7, 667)), (1, 4, 20, 20, (9, 1, 4789)), (1, 1, 20, 70, (31, 9, 709)), (1, 4, 120, 40, (19, 9, 733)),
+         (2, 4, 120, 40, (13, 9, 667)), (2, 1, 120, 33, (13, 9, 877))]
 
 
-@pytest.mark.parametrize("form,x_bytes,O,pixels", LARGE, ids=lambda v: str(v).replace(" ", ""))
+@pytest.mark.parametrize("parts,x_bytes,C,O,pixels", LARGE, ids=lambda v: str(v).replace(" ", ""))
 @pytest.mark.parametrize("top", [14, 6, 2])
-def test_epilogues_of_large_launches(oracle, rng, form, x_bytes, O, pixels, top):
+def test_epilogues_of_large_launches(oracle, rng, parts, x_bytes, C, O, pixels, top):
     """The register epilogue of launches with many tiles, and the one that two waves share: sums against the oracle; float,
     padded and operand-layout results, with and without residual, against the separate passes."""
     Nb, H, W = pixels
-    C, k = 20, 3
-    P = Nb * H * W
+    k, P = 3, Nb * H * W
     waves = 256 * (12 if x_bytes == 1 else 8)
     tiles = -(-O // 32) * -(-P // 64)
-    assert P % 64 and (tiles >= 3 * waves if form == "ks1" else 3 * waves / 2 <= tiles < 3 * waves)
+    fill, long = tiles / waves, C > 64
+    assert P % 64 and (1 < fill <= 1.25 and long if parts == 2 else fill > (1.25 if long else 0.25))
     s, sign, cw = _weights(rng, (O, C, k, k), top, ternary=True)
     x = _activations(rng, (Nb, C, H, W), x_bytes, 1 << 18)
     if x_bytes == 4:
