@@ -993,6 +993,18 @@ def _mfma_conv_serves(Nb, C, Hp, Wp, O, kernel_size, stride, x_bytes=4):
     return 0 < pixels <= 10 ** 9 and pixels * O <= 8 * 10 ** 9
 
 
+def _layout_pass_pays(Nb, H, W, K, O, stride, one_tap):
+    """Whether the matrix cores win by more than their layout pass against kernels that read an unpadded int32 input as it
+    is, in one launch.  Us there and here, 128 x 56 x 56 images, 1 x 1: 4 -> 64 channels 24, 68; 24 -> 128: 84, 103;
+    32 -> 64: 63, 66; 32 -> 128: 117, 103; 64 -> 16: 46, 69; 3 x 3: 4 -> 64: 60, 67.  Small images, where two launches
+    cost the host 23: K = 24: 15, K = 32 and 36: 17 to 22, K = 64: 25."""
+    sh, sw = _pair(stride)
+    pixels = Nb * (H // sh) * (W // sw)
+    if K <= 40:
+        return one_tap and K >= 32 and O >= 128 and pixels >= 1 << 15
+    return O > 16 or pixels < 1 << 18
+
+
 def _mfma_linear(x, conc_weight, bias, N):
     if x.shape[0] * N == 0:
         return None
@@ -1200,7 +1212,8 @@ def conv2d(input, shift, sign, bias=None, conc_weight=None, stride=1, padding=0,
         raise ValueError("filter has %d input channels, input has %d" % (Cw, C))
     if bias is not None:
         bias = _require_device_i32("bias", bias)
-    if _mfma_conv_serves(Nb, C, H + 2 * ph, W + 2 * pw, O, (FH, FW), stride):
+    if _mfma_conv_serves(Nb, C, H + 2 * ph, W + 2 * pw, O, (FH, FW), stride) and \
+            (ph or pw or _layout_pass_pays(Nb, H, W, C * FH * FW, O, stride, FH * FW == 1)):
         route = mfma_route(input, (ph, pw), conc_weight, O, (FH, FW), 4)
         if route is not None:
             return mfma_conv2d(route[0], route[1], bias, O, (FH, FW), stride, route[2])

@@ -280,3 +280,27 @@ def test_forward_hooks_read_a_hand_off_as_a_tensor():
         q = model.get_submodule("fused_0")(x)
         assert not hasattr(q, "no_such_name") and copy.copy(q).dims == q.dims
         assert torch.equal(model(x), want)
+
+
+@pytest.mark.parametrize("C,O,k,Nb,H,matrix", [(4, 64, 1, 2, 9, False), (31, 128, 1, 40, 30, False), (32, 127, 1, 40, 30, False),
+                                               (32, 128, 1, 2, 9, False), (32, 128, 1, 40, 30, True), (40, 17, 1, 2, 9, False), (41, 17, 1, 2, 9, True),
+                                               (64, 16, 1, 270, 32, False), (64, 17, 1, 270, 32, True), (64, 16, 1, 2, 9, True),
+                                               (4, 140, 3, 40, 30, False), (5, 40, 3, 2, 11, True)])
+def test_unpadded_integer_convolutions_take_the_kernel_that_pays(oracle, monkeypatch, C, O, k, Nb, H, matrix):
+    """kernels.conv2d on both sides of every line of its rule, against the oracle; padded inputs are not asked."""
+    from tests.test_gpu_mfma import _activations, _weights
+    import numpy as np
+    rng = np.random.default_rng(C * O)
+    s, sign, cw = _weights(rng, (O, C, k, k), 14, ternary=False)
+    x = _activations(rng, (Nb, C, H, H), 4, 1 << 24)
+    launches = []
+    real = kernels.mfma_conv2d
+    monkeypatch.setattr(kernels, "mfma_conv2d", lambda *a, **kw: launches.append(1) or real(*a, **kw))
+    args = [torch.from_numpy(np.ascontiguousarray(a)).to(DEV) for a in (x, -s.astype(np.int32), sign.astype(np.int32))]
+    got = kernels.conv2d(*args, None, cw)
+    assert len(launches) == matrix
+    want = oracle.conv2d(x, -s.astype(np.int32), sign.astype(np.int32), None, (1, 1), nthreads=16)
+    np.testing.assert_array_equal(got.cpu().numpy(), want)
+    padded = kernels.conv2d(*args, None, cw, 1, 1)
+    assert len(launches) == matrix + 1
+    assert k > 1 or torch.equal(padded[:, :, 1:-1, 1:-1], got)
