@@ -52,8 +52,8 @@ class FusedLinearChain(nn.Module):
     grid is small enough for its barriers to cost less than the launches they save), else a launch per
     layer issued inside the call (the 512-wide MNIST MLP at batch 64 takes 50 us as one launch, 39 us as
     three).  Bit-identical to the layers run one by one from Python, which is what happens where the
-    library has no such form: layers of different field widths or activation formats, a layer too large
-    for the one-launch kernel, host execution."""
+    library has no such form or a layer is large enough for the matrix cores: layers of different field widths
+    or activation formats, a layer too large for the one-launch kernel, host execution."""
 
     def __init__(self, linears, relus):
         super().__init__()
@@ -80,7 +80,8 @@ class FusedLinearChain(nn.Module):
         lead = input.shape[:-1]
         x2d = input.reshape(-1, first.in_features).float()
         M = x2d.shape[0]
-        if not x2d.is_cuda or not all(kernels.small_linear_serves(M, m.in_features, m.out_features)
+        if not x2d.is_cuda or not all(kernels.small_linear_serves(M, m.in_features, m.out_features) if self.force else
+                                      kernels.one_launch_linear(M, m.in_features, m.out_features, True)
                                       for m in self.linears):
             return self._one_by_one(input)
         round_to_fixed = isinstance(first, modules_q.LinearShiftQ)   # modules_q.py:115-125 / modules.py:24-31

@@ -625,14 +625,21 @@ def linear_chain_status(ws_cache):
     return 0
 
 
+def one_launch_linear(M, K, N, in_chain=False):
+    """Whether a LinearShift layer runs on the one-launch kernel, not on the matrix cores: its time grows with the pairs
+    (512 x 512 x 512: 21 us against 25, 128 x 2048 x 1000: 42 and 30; a chain of 784, 1024, 1024, 10 at batch 512: 121 and
+    78) and with K whatever M is (1 x 3072 x 512: 37 and 30, 1 x 2049 x 512: 28 and 26).  In a chain, one call of the
+    library, a long K stays: layer by layer the host needs more than the kernel saves (3072, 512, 10 at batch 1: 46 us
+    and 51)."""
+    return (in_chain or K <= 2048) and M * K * N <= 1 << 27 and small_linear_serves(M, K, N)
+
+
 def linear_forward(x2d, conc_weight, bias, N, integer_bits, fraction_bits, round_to_fixed, relu=False):
     """float32 ``[M, K]`` -> float32 ``[M, N]`` of a LinearShift layer from its packed weights, on whichever kernel
     serves the size best: one launch for small problems, the matrix cores for others they have a form for, else
     :func:`linear_layer` (same results)."""
     M, K = x2d.shape
-    # the one-launch kernel's time grows with K whatever M is (1 x 4096 x 4096: 128 us against 51 here), and with the
-    # pairs (512 x 512 x 512: 21 against 25 us, 128 x 2048 x 1000: 42 against 30)
-    if K <= 2048 and M * K * N <= 1 << 27 and small_linear_serves(M, K, N):
+    if one_launch_linear(M, K, N):
         return linear_small(x2d, _tiled_of(conc_weight, N, K), bias, N, kernel_bits(conc_weight), conc_weight.base,
                             integer_bits, fraction_bits, round_to_fixed, relu)
     route = mfma_route(x2d, 0, conc_weight, N, (1, 1), 4, integer_bits, fraction_bits, round_to_fixed)

@@ -304,3 +304,23 @@ def test_unpadded_integer_convolutions_take_the_kernel_that_pays(oracle, monkeyp
     padded = kernels.conv2d(*args, None, cw, 1, 1)
     assert len(launches) == matrix + 1
     assert k > 1 or torch.equal(padded[:, :, 1:-1, 1:-1], got)
+
+
+@pytest.mark.parametrize("M,widths,alone", [(64, (784, 512, 512, 10), False), (512, (784, 1024, 1024, 10), True),
+                                            (4, (3072, 64, 8), False)])
+def test_chains_and_single_layers_follow_one_rule(monkeypatch, M, widths, alone):
+    """A chain is one call of the library while its layers are small; large ones take the matrix cores there as they do
+    alone."""
+    calls = []
+    real = kernels.linear_chain
+    monkeypatch.setattr(kernels, "linear_chain", lambda *a: calls.append(1) or real(*a))
+    with torch.no_grad():
+        model = _chain(widths)
+        x = torch.rand(M, widths[0], device=DEV)
+        got = model(x)
+        assert bool(calls) != alone
+        chain = next(m for m in model.modules() if isinstance(m, fuse.FusedLinearChain))
+        want = x
+        for layer, relu in zip(chain.linears, chain.relus):
+            want = torch.relu(layer(want)) if relu else layer(want)
+        assert torch.equal(got, want)
