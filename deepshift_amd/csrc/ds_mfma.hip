@@ -337,70 +337,63 @@ constexpr uint32_t kPosHi = 0x00010204u, kNegHi = 0x00fffefcu;   // r = 4..6: 4,
 constexpr uint32_t kPos14 = 0x40000000u, kNeg14 = 0xc0000000u;   // s = 14, the last of its group: 64
 __host__ __device__ constexpr uint32_t low_bytes(uint32_t v, int n) { return n >= 4 ? v : v & ((1u << (8 * n)) - 1u); }
 
-template <int MODE, int MT, int NT>
+template <int MODE, int NT>
 struct Operands {
     static constexpr int G = mode_groups(MODE), D = mode_i8(MODE) ? 1 : 3;
-    v4i sel[MT][G];
+    v4i sel[G];
     v4i dig[NT][D];
 };
 
-template <int MT, int NT>
-__device__ __forceinline__ void product(v16i (&acc)[MT][NT], const v4i (&w)[MT], const v4i (&b)[NT])
+template <int NT>
+__device__ __forceinline__ void product(v16i (&acc)[NT], const v4i &w, const v4i (&b)[NT])
 {
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int p = 0; p < NT; ++p) acc[m][p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[m], b[p], acc[m][p], 0, 0, 0);
+    for (int p = 0; p < NT; ++p) acc[p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, b[p], acc[p], 0, 0, 0);
 }
 
 // The seven bit products of digit q: adds to an, leaves the full weight plane 2^(6-r) in w.
-template <int MODE, int MT, int NT>
-__device__ __forceinline__ void bit_products(const Operands<MODE, MT, NT> &o, int q, v16i (&an)[MT][NT], v4i (&w)[MT])
+template <int MODE, int NT>
+__device__ __forceinline__ void bit_products(const Operands<MODE, NT> &o, int q, v16i (&an)[NT], v4i &w)
 {
-    v4i b[NT], w3[MT];
+    v4i b[NT], w3;
 #pragma unroll
     for (int j = 0; j < 7; ++j) {
         // shifts of at most 3: bits 3 to 6 meet the same weights
         if (MODE == kI32S4 && j > 3) break;
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            if (j <= 3) {
-                w[m] = perm4(low_bytes(kNegLo, j + 1), low_bytes(kPosLo, j + 1), o.sel[m][2 * q]);
-                w3[m] = w[m];
-            } else if constexpr (Operands<MODE, MT, NT>::G > 1) {
-                w[m] = or4(w3[m], perm4(low_bytes(kNegHi, j - 3), low_bytes(kPosHi, j - 3), o.sel[m][2 * q + 1]));
-            }
+        if (j <= 3) {
+            w = perm4(low_bytes(kNegLo, j + 1), low_bytes(kPosLo, j + 1), o.sel[2 * q]);
+            w3 = w;
+        } else if constexpr (Operands<MODE, NT>::G > 1) {
+            w = or4(w3, perm4(low_bytes(kNegHi, j - 3), low_bytes(kPosHi, j - 3), o.sel[2 * q + 1]));
         }
         const uint32_t mask = MODE == kI32S4 && j == 3 ? 0x78787878u : 0x01010101u << j;
 #pragma unroll
         for (int p = 0; p < NT; ++p) b[p] = and4(o.dig[p][q], mask);
-        product<MT, NT>(an, w, b);
+        product<NT>(an, w, b);
     }
 }
 
-template <int MODE, int MT, int NT>
-__device__ __forceinline__ void digit_product(const Operands<MODE, MT, NT> &o, int d, v16i (&acc)[MT][NT], const v4i (&w)[MT])
+template <int MODE, int NT>
+__device__ __forceinline__ void digit_product(const Operands<MODE, NT> &o, int d, v16i (&acc)[NT], const v4i &w)
 {
     v4i b[NT];
 #pragma unroll
     for (int p = 0; p < NT; ++p) b[p] = o.dig[p][d];
-    product<MT, NT>(acc, w, b);
+    product<NT>(acc, w, b);
 }
 
-template <int MODE, int MT, int NT>
-__device__ __forceinline__ void block_i8(const Operands<MODE, MT, NT> &o, v16i (&acc)[MT][NT])
+template <int MODE, int NT>
+__device__ __forceinline__ void block_i8(const Operands<MODE, NT> &o, v16i (&acc)[NT])
 {
     constexpr int S = MODE == kI8S8 ? 8 : MODE == kI8S4 ? 4 : 3;
-    v4i b[NT], u[NT], w[MT];
+    v4i b[NT], u[NT], w;
 #pragma unroll
     for (int p = 0; p < NT; ++p)
 #pragma unroll
         for (int i = 0; i < 4; ++i) u[p][i] = o.dig[p][0][i] ^ (int)0x80808080;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-            w[m] = perm4(0xffu << (8 * (s & 3)), 0x01u << (8 * (s & 3)), o.sel[m][s >> 2]);
+            w = perm4(0xffu << (8 * (s & 3)), 0x01u << (8 * (s & 3)), o.sel[s >> 2]);
 #pragma unroll
         for (int p = 0; p < NT; ++p) {
             if (s == 0)
@@ -409,7 +402,7 @@ __device__ __forceinline__ void block_i8(const Operands<MODE, MT, NT> &o, v16i (
 #pragma unroll
                 for (int i = 0; i < 4; ++i) b[p][i] = (int)(((uint32_t)u[p][i] >> s) & ((0xffu >> s) * 0x01010101u));
         }
-        product<MT, NT>(acc, w, b);
+        product<NT>(acc, w, b);
     }
 }
 
@@ -418,33 +411,32 @@ struct KPos {
     int cb, fh, fg, off;
 };
 
-template <int MODE, int MT, int NT>
-__device__ __forceinline__ void load_digits(const MfmaArgs &a, Operands<MODE, MT, NT> &o, int from, int to, const KPos &k,
+template <int MODE, int NT>
+__device__ __forceinline__ void load_digits(const MfmaArgs &a, Operands<MODE, NT> &o, int from, int to, const KPos &k,
                                             const uint32_t (&px)[NT])
 {
     const int8_t *xb = a.x + k.off;
 #pragma unroll
-    for (int d = 0; d < Operands<MODE, MT, NT>::D; ++d)
+    for (int d = 0; d < Operands<MODE, NT>::D; ++d)
         if (d >= from && d < to)
 #pragma unroll
             for (int p = 0; p < NT; ++p) o.dig[p][d] = *(const v4i *)(xb + d * a.lay.dstride + px[p]);
 }
-template <int MODE, int MT, int NT>
-__device__ __forceinline__ void load_selectors(Operands<MODE, MT, NT> &o, int from, int to, const int8_t *w, int wtile, int kb)
+template <int MODE, int NT>
+__device__ __forceinline__ void load_selectors(Operands<MODE, NT> &o, int from, int to, const int8_t *w, int kb)
 {
-    constexpr int G = Operands<MODE, MT, NT>::G;
+    constexpr int G = Operands<MODE, NT>::G;
 #pragma unroll
     for (int g = 0; g < G; ++g)
         if (g >= from && g < to)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) o.sel[m][g] = *(const v4i *)(w + (size_t)m * wtile + (kb * G + g) * 1024);
+            o.sel[g] = *(const v4i *)(w + (kb * G + g) * 1024);
 }
-template <int MODE, int MT, int NT>
-__device__ __forceinline__ void load_block(const MfmaArgs &a, Operands<MODE, MT, NT> &o, const int8_t *w, int wtile, int kb,
+template <int MODE, int NT>
+__device__ __forceinline__ void load_block(const MfmaArgs &a, Operands<MODE, NT> &o, const int8_t *w, int kb,
                                            const KPos &k, const uint32_t (&px)[NT])
 {
-    load_selectors<MODE, MT, NT>(o, 0, 4, w, wtile, kb);
-    load_digits<MODE, MT, NT>(a, o, 0, 3, k, px);
+    load_selectors<MODE, NT>(o, 0, 4, w, kb);
+    load_digits<MODE, NT>(a, o, 0, 3, k, px);
 }
 
 __device__ __forceinline__ void k_start(const MfmaArgs &a, KPos &k, int kb)
@@ -521,12 +513,12 @@ __device__ __forceinline__ int any_high(const MfmaArgs &a, uint32_t p0, uint32_t
 
 // Digits d3 and d4 of the rows that have any: what they add to the sums, modulo 2^32.  One pass over the reduction with
 // an accumulator per power of two; a digit that was not written is masked after its load, not branched around.
-template <int MODE, int MT, int NT>
+template <int MODE, int NT>
 __device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[64], int lane, bool d4, const int8_t *w,
-                                            int wtile, int kb0, int kb1, const uint32_t (&px)[NT], const uint32_t (&pix)[NT])
+                                            int kb0, int kb1, const uint32_t (&px)[NT], const uint32_t (&pix)[NT])
 {
     constexpr int G = mode_groups(MODE), Q = MODE == kI32S15 ? 3 : 1;
-    v16i acc[4][MT][NT] = {};   // 2^(7 i + 1)
+    v16i acc[4][NT] = {};   // 2^(7 i + 1)
     PixelAt at[NT];
 #pragma unroll
     for (int p = 0; p < NT; ++p) at[p] = pixel_at(a, pix[p] < a.pixels ? pix[p] : a.pixels - 1);
@@ -534,7 +526,7 @@ __device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[6
     k_start(a, k, kb0);
 #pragma unroll 1
     for (int kb = kb0; kb < kb1; ++kb, k_next(a, k)) {
-        v4i b[2][NT], sel[MT][G], wv[MT];
+        v4i b[2][NT], sel[G], wv;
 #pragma unroll
         for (int p = 0; p < NT; ++p) {
 #pragma unroll
@@ -542,9 +534,7 @@ __device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[6
                 if (d == 0 || d4) b[d][p] = *(const v4i *)(a.x + k.off + (3 + d) * a.lay.dstride + px[p]);
         }
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int g = 0; g < G; ++g) sel[m][g] = *(const v4i *)(w + (size_t)m * wtile + (kb * G + g) * 1024);
+            for (int g = 0; g < G; ++g) sel[g] = *(const v4i *)(w + (kb * G + g) * 1024);
 #pragma unroll
         for (int p = 0; p < NT; ++p) {
             const uint32_t on = has_high(a, at[p], lane >> 5, k) ? 0xffffffffu : 0u;
@@ -554,47 +544,40 @@ __device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[6
         }
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                if constexpr (G == 4) {
-                    wv[m] = q == 2 ? perm4(kNeg14, kPos14, sel[m][3])
-                                   : or4(perm4(kNegLo, kPosLo, sel[m][q == 0 ? 0 : 2]),
-                                         perm4(kNegHi, kPosHi, sel[m][q == 0 ? 1 : 3]));
-                } else {
-                    wv[m] = perm4(kNegLo, kPosLo, sel[m][0]);
-                    if constexpr (G == 2) wv[m] = or4(wv[m], perm4(kNegHi, kPosHi, sel[m][1]));
-                }
+            if constexpr (G == 4) {
+                wv = q == 2 ? perm4(kNeg14, kPos14, sel[3])
+                            : or4(perm4(kNegLo, kPosLo, sel[q == 0 ? 0 : 2]), perm4(kNegHi, kPosHi, sel[q == 0 ? 1 : 3]));
+            } else {
+                wv = perm4(kNegLo, kPosLo, sel[0]);
+                if constexpr (G == 2) wv = or4(wv, perm4(kNegHi, kPosHi, sel[1]));
             }
 #pragma unroll
             for (int d = 0; d < 2; ++d)
-                if (d == 0 || d4) product<MT, NT>(acc[3 + d - q - 1], wv, b[d]);
+                if (d == 0 || d4) product<NT>(acc[3 + d - q - 1], wv, b[d]);
         }
     }
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int p = 0; p < NT; ++p)
 #pragma unroll
-        for (int p = 0; p < NT; ++p)
+        for (int i = 0; i < 16; ++i) {
+            uint32_t v = 0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                uint32_t v = 0;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) v += (uint32_t)acc[c][m][p][i] << (7 * c + 1);
-                slot[(m * NT + p) * 16 + i][lane] = (int32_t)v;
-            }
+            for (int c = 0; c < 4; ++c) v += (uint32_t)acc[c][p][i] << (7 * c + 1);
+            slot[p * 16 + i][lane] = (int32_t)v;
+        }
 }
 
-// What follows the sums of R x 4 channels (R groups of four, 8 apart) at one pixel: the per-channel constants, then the
+// What follows the sums of eight channels (two groups of four, 8 apart) at one pixel: the per-channel constants, then the
 // residuals, are all asked for before the first value is stored (one wait each, not one per value).
-template <int R>
+constexpr int kUnit = 8;
 struct ChannelTail {
-    int32_t add[R * 4];
-    float scale[R * 4], shift[R * 4];
+    int32_t add[kUnit];
+    float scale[kUnit], shift[kUnit];
 };
-template <int R>
-__device__ __forceinline__ void load_tail(const MfmaArgs &a, ChannelTail<R> &t, int ch0)
+__device__ __forceinline__ void load_tail(const MfmaArgs &a, ChannelTail &t, int ch0)
 {
 #pragma unroll
-    for (int i = 0; i < R * 4; ++i) {
+    for (int i = 0; i < kUnit; ++i) {
         const int ch = ch0 + 8 * (i >> 2) + (i & 3), c = ch < a.N ? ch : a.N - 1;
         t.add[i] = (a.bias ? a.bias[c] : 0) - (a.corr ? a.corr[c] : 0);
         t.scale[i] = a.scale ? a.scale[c] : 1.0f;
@@ -617,40 +600,30 @@ __device__ __forceinline__ OutAt out_at(const MfmaArgs &a, const PixelAt &at, ui
                    : ((size_t)at.n * a.N * a.qHp + at.oh + a.qph) * a.qWp + at.ow + a.qpw;
     return o;
 }
-// R x 4 values per lane (channels ch0 + 8 g + 0..3, ch0 = 16 u + 4 (lane >> 5)) into the next layer's operand layout:
-// the halves of a wave swap words, so that a lane holds 4 R channels side by side and the 32 pixels of a digit are
-// stored in a row.  Digits d3 and d4 only, with a flag, where the 32 pixels x 16 channels have any.
-template <int R>
-__device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t (&qv)[R * 4], int ch0, const OutAt &o)
+// Eight values per lane (channels ch0 + 8 g + 0..3, ch0 = 16 u + 4 (lane >> 5)) into the next layer's operand layout: the
+// halves of a wave swap words, so that a lane holds eight channels side by side and the 32 pixels of a digit are stored
+// in a row.  Digits d3 and d4 only, with a flag, where the 32 pixels x 16 channels have any.
+__device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t (&qv)[kUnit], int ch0, const OutAt &o)
 {
     const int half = (ch0 >> 2) & 1, u16 = ch0 >> 4;   // half = lane >> 5: ch0 is a multiple of 16 plus 0 or 4
     const MfmaX &L = a.qlay;
+    const int c = u16 * 16 + half * 8, cb = L.cp == 16 ? c >> 4 : c >> 5;   // the lane's channels after the swap
+    int8_t *q = (int8_t *)a.q + o.j + (size_t)cb * L.cbstride + (c & (L.cp - 1));
     if (L.digits == 1) {
-        uint32_t b[R];
+        uint32_t b[2];
 #pragma unroll
-        for (int g = 0; g < R; ++g) {
+        for (int g = 0; g < 2; ++g) {
             const uint32_t lo = __builtin_amdgcn_perm((uint32_t)qv[g * 4 + 1], (uint32_t)qv[g * 4], 0x0c0c0400u);
             const uint32_t hi = __builtin_amdgcn_perm((uint32_t)qv[g * 4 + 3], (uint32_t)qv[g * 4 + 2], 0x04000c0cu);
             b[g] = lo | hi;
         }
-        const int c = u16 * 16 + (R == 4 ? half * 16 : half * 8), cb = L.cp == 16 ? c >> 4 : c >> 5;
-        int8_t *q = (int8_t *)a.q + o.j + (size_t)cb * L.cbstride + (c & (L.cp - 1));
-        if constexpr (R == 4) {
-            const auto x = __builtin_amdgcn_permlane32_swap(b[0], b[2], false, false);
-            const auto y = __builtin_amdgcn_permlane32_swap(b[1], b[3], false, false);
-            if (o.in && cb < L.cb) *(v4i *)q = v4i{(int)x[0], (int)x[1], (int)y[0], (int)y[1]};
-        } else {
-            const auto x = __builtin_amdgcn_permlane32_swap(b[0], b[1], false, false);
-            if (o.in && cb < L.cb) *(uint2 *)q = uint2{x[0], x[1]};
-        }
+        const auto x = __builtin_amdgcn_permlane32_swap(b[0], b[1], false, false);
+        if (o.in && cb < L.cb) *(uint2 *)q = uint2{x[0], x[1]};
         return;
     }
-    uint32_t w[kDigits][R];
-    uint32_t high[2] = {0, 0}, high4[2] = {0, 0};
+    uint32_t w[kDigits][2] = {};
 #pragma unroll
-    for (int g = 0; g < R; ++g) {
-#pragma unroll
-        for (int d = 0; d < kDigits; ++d) w[d][g] = 0;
+    for (int g = 0; g < 2; ++g) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             int32_t dg[kDigits];
@@ -658,126 +631,108 @@ __device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t 
 #pragma unroll
             for (int d = 0; d < kDigits; ++d) w[d][g] |= ((uint32_t)dg[d] & 255u) << (8 * i);
         }
-        high[g >> 1] |= w[3][g] | w[4][g];
-        high4[g >> 1] |= w[4][g];
     }
-    int to = 3;
-#pragma unroll
-    for (int f = 0; f < R / 2; ++f) {
-        const bool any = __any(o.in && high[f] != 0);
-        const bool any4 = __any(o.in && high4[f] != 0);
-        if (any) to = kDigits;
-        if (u16 + f < L.c16 && (threadIdx.x & 63) == 0 && o.in)
-            a.qflags[(size_t)(o.p >> 5) * L.c16 + u16 + f] = any4 ? 3 : any ? 1 : 0;
-    }
-    const int c = u16 * 16 + (R == 4 ? half * 16 : half * 8);   // first of the lane's 4 R channels after the swap
-    const int cb = L.cp == 16 ? c >> 4 : c >> 5;
-    int8_t *q = (int8_t *)a.q + o.j + (size_t)cb * L.cbstride + (c & (L.cp - 1));
+    const uint32_t high4 = w[4][0] | w[4][1], high = w[3][0] | w[3][1] | high4;
+    const bool any = __any(o.in && high != 0);
+    const bool any4 = __any(o.in && high4 != 0);
+    if (u16 < L.c16 && (threadIdx.x & 63) == 0 && o.in)
+        a.qflags[(size_t)(o.p >> 5) * L.c16 + u16] = any4 ? 3 : any ? 1 : 0;
 #pragma unroll
     for (int d = 0; d < kDigits; ++d) {
-        if (d >= to) break;
-        if constexpr (R == 4) {
-            const auto x = __builtin_amdgcn_permlane32_swap(w[d][0], w[d][2], false, false);
-            const auto y = __builtin_amdgcn_permlane32_swap(w[d][1], w[d][3], false, false);
-            if (o.in && cb < L.cb) *(v4i *)(q + d * L.dstride) = v4i{(int)x[0], (int)x[1], (int)y[0], (int)y[1]};
-        } else {
-            const auto x = __builtin_amdgcn_permlane32_swap(w[d][0], w[d][1], false, false);
-            if (o.in && cb < L.cb) *(uint2 *)(q + d * L.dstride) = uint2{x[0], x[1]};
-        }
+        if (d >= 3 && !any) break;
+        const auto x = __builtin_amdgcn_permlane32_swap(w[d][0], w[d][1], false, false);
+        if (o.in && cb < L.cb) *(uint2 *)(q + d * L.dstride) = uint2{x[0], x[1]};
     }
 }
 
-template <int R>
-__device__ __forceinline__ void load_residual(const MfmaArgs &a, float (&res)[R * 4], int ch0, const OutAt &o)
+__device__ __forceinline__ void load_residual(const MfmaArgs &a, float (&res)[kUnit], int ch0, const OutAt &o)
 {
 #pragma unroll
-    for (int i = 0; i < R * 4; ++i) {
+    for (int i = 0; i < kUnit; ++i) {
         // past the end: some value that is there (it is not used), so that no load waits behind a branch
         const int ch = ch0 + 8 * (i >> 2) + (i & 3), c = ch < a.N ? ch : a.N - 1;
         res[i] = a.residual[(o.in ? o.i : 0) + (size_t)c * a.ostride_c];
     }
 }
 
-// Stores of R x 4 values; the uniform test spares full tiles the per-channel ones.
-template <int R, typename T>
-__device__ __forceinline__ void store_channels(T *dst, const T (&v)[R * 4], int ch0, int stride, int N, bool in)
+// Stores of eight values; the uniform test spares full tiles the per-channel ones.
+template <typename T>
+__device__ __forceinline__ void store_channels(T *dst, const T (&v)[kUnit], int ch0, int stride, int N, bool in)
 {
-    if ((ch0 & ~15) + R * 8 <= N) {
+    if ((ch0 & ~15) + 2 * kUnit <= N) {
         if (in)
 #pragma unroll
-            for (int i = 0; i < R * 4; ++i) dst[(size_t)(ch0 + 8 * (i >> 2) + (i & 3)) * stride] = v[i];
+            for (int i = 0; i < kUnit; ++i) dst[(size_t)(ch0 + 8 * (i >> 2) + (i & 3)) * stride] = v[i];
     } else {
 #pragma unroll
-        for (int i = 0; i < R * 4; ++i) {
+        for (int i = 0; i < kUnit; ++i) {
             const int ch = ch0 + 8 * (i >> 2) + (i & 3);
             if (in && ch < N) dst[(size_t)ch * stride] = v[i];
         }
     }
 }
-template <int R>
-__device__ __forceinline__ void quantize_all(const float (&f)[R * 4], int32_t (&q)[R * 4], const QuantSpec &spec)
+__device__ __forceinline__ void quantize_all(const float (&f)[kUnit], int32_t (&q)[kUnit], const QuantSpec &spec)
 {
     QuantSpec s = spec;
     s.mode = DS_Q_ROUND_TO_FIXED;
     if (spec.I == 1) {
         s.I = 1;
 #pragma unroll
-        for (int i = 0; i < R * 4; ++i) q[i] = quantize_one(f[i], s);
+        for (int i = 0; i < kUnit; ++i) q[i] = quantize_one(f[i], s);
     } else {
         s.I = 2;   // the bounds are in lo and hi
 #pragma unroll
-        for (int i = 0; i < R * 4; ++i) q[i] = quantize_one(f[i], s);
+        for (int i = 0; i < kUnit; ++i) q[i] = quantize_one(f[i], s);
     }
 }
-template <int R>
-__device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail<R> &t, const int32_t (&sum)[R * 4],
-                                           const float (&res)[R * 4], int ch0, const OutAt &o)
+__device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail &t, const int32_t (&sum)[kUnit],
+                                           const float (&res)[kUnit], int ch0, const OutAt &o)
 {
-    int32_t v[R * 4];
+    int32_t v[kUnit];
 #pragma unroll
-    for (int i = 0; i < R * 4; ++i) v[i] = sum[i] + t.add[i];
+    for (int i = 0; i < kUnit; ++i) v[i] = sum[i] + t.add[i];
     if (a.y) {
-        store_channels<R>(a.y + o.i, v, ch0, a.ostride_c, a.N, o.in);
+        store_channels(a.y + o.i, v, ch0, a.ostride_c, a.N, o.in);
         return;
     }
-    float f[R * 4];
+    float f[kUnit];
     if (a.residual) {
 #pragma unroll
-        for (int i = 0; i < R * 4; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], &res[i], 0);
+        for (int i = 0; i < kUnit; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], &res[i], 0);
     } else {
 #pragma unroll
-        for (int i = 0; i < R * 4; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], nullptr, 0);
+        for (int i = 0; i < kUnit; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], nullptr, 0);
     }
     if (a.relu)
 #pragma unroll
-        for (int i = 0; i < R * 4; ++i) f[i] = f[i] > 0.0f ? f[i] : 0.0f;
-    if (a.out) store_channels<R>(a.out + o.i, f, ch0, a.ostride_c, a.N, o.in);
+        for (int i = 0; i < kUnit; ++i) f[i] = f[i] > 0.0f ? f[i] : 0.0f;
+    if (a.out) store_channels(a.out + o.i, f, ch0, a.ostride_c, a.N, o.in);
     if (!a.q) return;
-    int32_t qv[R * 4];
-    quantize_all<R>(f, qv, a.qspec);
+    int32_t qv[kUnit];
+    quantize_all(f, qv, a.qspec);
     if (a.qflags) {
-        if ((ch0 & ~15) + R * 8 > a.N)
+        if ((ch0 & ~15) + 2 * kUnit > a.N)
 #pragma unroll
-            for (int i = 0; i < R * 4; ++i)
+            for (int i = 0; i < kUnit; ++i)
                 if (ch0 + 8 * (i >> 2) + (i & 3) >= a.N) qv[i] = 0;
-        store_operands<R>(a, qv, ch0, o);
+        store_operands(a, qv, ch0, o);
     } else if (a.q_bytes == 1) {
-        int8_t b[R * 4];
+        int8_t b[kUnit];
 #pragma unroll
-        for (int i = 0; i < R * 4; ++i) b[i] = (int8_t)qv[i];
-        store_channels<R>((int8_t *)a.q + o.j, b, ch0, a.qHp * a.qWp, a.N, o.in);
+        for (int i = 0; i < kUnit; ++i) b[i] = (int8_t)qv[i];
+        store_channels((int8_t *)a.q + o.j, b, ch0, a.qHp * a.qWp, a.N, o.in);
     } else {
-        store_channels<R>((int32_t *)a.q + o.j, qv, ch0, a.qHp * a.qWp, a.N, o.in);
+        store_channels((int32_t *)a.q + o.j, qv, ch0, a.qHp * a.qWp, a.N, o.in);
     }
 }
 
-// Four or eight waves per workgroup; a wave owns MT * 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
+// Four or eight waves per workgroup; a wave owns 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
 // parts of a tile lie in one workgroup and meet in LDS).  No operand passes through LDS: activations and selectors are
 // fragments in memory already, each a contiguous KiB.
-template <int MODE, int MT, int NT, int WAVES>
+template <int MODE, int NT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) void mfma_kernel(MfmaArgs a)
 {
-    __shared__ int32_t part[WAVES][MT * NT * 16][64];
+    __shared__ int32_t part[WAVES][NT * 16][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroups are dealt to the eight XCDs in turn: give each XCD neighbouring tiles
@@ -788,7 +743,7 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
     const int ct = (int)(wg - pt * a.ctiles);
     const int kpart = wave % a.ks, t = wave / a.ks;
     const int pw = WAVES / a.ks / a.tc;   // pixel tiles per workgroup
-    const int c0 = (ct * a.tc + t % a.tc) * MT * 32;
+    const int c0 = (ct * a.tc + t % a.tc) * 32;
     const uint32_t p0 = ((uint32_t)pt * pw + t / a.tc) * (NT * 32);
     const int kb0 = (int)((long)a.KB * kpart / a.ks), kb1 = (int)((long)a.KB * (kpart + 1) / a.ks);
 
@@ -803,90 +758,82 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
         const PixelAt at = pixel_at(a, clamped);
         px[p] = (at.n * a.lay.Hp + at.oh * a.sh + a.crop_h) * a.lay.rstride + (at.ow * a.sw + a.crop_w) * a.lay.cp + (lane >> 5) * 16;
     }
-    v16i total[MT][NT] = {};
+    v16i total[NT] = {};
     if (live && kb0 < kb1) {
         const int8_t *wl = a.blob + (size_t)(c0 >> 5) * wtile + lane * 16;
         int high = 0;
         if constexpr (!mode_i8(MODE)) {
             const uint32_t last = p0 + NT * 32 - 1;
             high = any_high(a, p0, last < a.pixels ? last : a.pixels - 1, lane);
-            if (high) high_digits<MODE, MT, NT>(a, part[wave], lane, (high & 2) != 0, wl, wtile, kb0, kb1, px, pix);
+            if (high) high_digits<MODE, NT>(a, part[wave], lane, (high & 2) != 0, wl, kb0, kb1, px, pix);
         }
-        v16i acc[MT][NT] = {};
-        Operands<MODE, MT, NT> o0;
+        v16i acc[NT] = {};
+        Operands<MODE, NT> o0;
         KPos k;
         k_start(a, k, kb0);
         int kb = kb0;
-        load_block<MODE, MT, NT>(a, o0, wl, wtile, kb, k, px);
+        load_block<MODE, NT>(a, o0, wl, kb, k, px);
         if constexpr (mode_i8(MODE)) {
-            Operands<MODE, MT, NT> o1;
+            Operands<MODE, NT> o1;
             while (true) {
                 if (kb + 1 < kb1) {
                     k_next(a, k);
-                    load_block<MODE, MT, NT>(a, o1, wl, wtile, kb + 1, k, px);
+                    load_block<MODE, NT>(a, o1, wl, kb + 1, k, px);
                 }
-                block_i8<MODE, MT, NT>(o0, acc);
+                block_i8<MODE, NT>(o0, acc);
                 if (++kb >= kb1) break;
                 if (kb + 1 < kb1) {
                     k_next(a, k);
-                    load_block<MODE, MT, NT>(a, o0, wl, wtile, kb + 1, k, px);
+                    load_block<MODE, NT>(a, o0, wl, kb + 1, k, px);
                 }
-                block_i8<MODE, MT, NT>(o1, acc);
+                block_i8<MODE, NT>(o1, acc);
                 if (++kb >= kb1) break;
             }
 #pragma unroll
-            for (int m = 0; m < MT; ++m)
-#pragma unroll
-                for (int p = 0; p < NT; ++p) total[m][p] = acc[m][p];
+            for (int p = 0; p < NT; ++p) total[p] = acc[p];
         } else {
             // every operand is loaded again as soon as its last product is issued: the loads of the next block are
             // in flight during this one's remaining products, with one set of registers
-            v16i a0[MT][NT] = {}, a1[MT][NT] = {};
+            v16i a0[NT] = {}, a1[NT] = {};
             while (true) {
-                v4i w[MT];
+                v4i w;
                 const bool more = kb + 1 < kb1;
                 if (more) k_next(a, k);
                 const int kn = more ? kb + 1 : kb;
-                bit_products<MODE, MT, NT>(o0, 0, acc, w);
+                bit_products<MODE, NT>(o0, 0, acc, w);
                 if constexpr (MODE == kI32S15) {
-                    load_selectors<MODE, MT, NT>(o0, 0, 2, wl, wtile, kn);
-                    load_digits<MODE, MT, NT>(a, o0, 0, 1, k, px);
+                    load_selectors<MODE, NT>(o0, 0, 2, wl, kn);
+                    load_digits<MODE, NT>(a, o0, 0, 1, k, px);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                digit_product<MODE, MT, NT>(o0, 1, a0, w);
-                digit_product<MODE, MT, NT>(o0, 2, a1, w);
+                digit_product<MODE, NT>(o0, 1, a0, w);
+                digit_product<MODE, NT>(o0, 2, a1, w);
                 if constexpr (MODE == kI32S15) {
-                    bit_products<MODE, MT, NT>(o0, 1, acc, w);
-                    load_selectors<MODE, MT, NT>(o0, 2, 3, wl, wtile, kn);
-                    load_digits<MODE, MT, NT>(a, o0, 1, 2, k, px);
+                    bit_products<MODE, NT>(o0, 1, acc, w);
+                    load_selectors<MODE, NT>(o0, 2, 3, wl, kn);
+                    load_digits<MODE, NT>(a, o0, 1, 2, k, px);
                     __builtin_amdgcn_sched_barrier(0);
-                    digit_product<MODE, MT, NT>(o0, 2, a0, w);
-#pragma unroll
-                    for (int m = 0; m < MT; ++m) w[m] = perm4(kNeg14, kPos14, o0.sel[m][3]);
-                    digit_product<MODE, MT, NT>(o0, 2, acc, w);
-                    load_selectors<MODE, MT, NT>(o0, 3, 4, wl, wtile, kn);
-                    load_digits<MODE, MT, NT>(a, o0, 2, 3, k, px);
+                    digit_product<MODE, NT>(o0, 2, a0, w);
+                    w = perm4(kNeg14, kPos14, o0.sel[3]);
+                    digit_product<MODE, NT>(o0, 2, acc, w);
+                    load_selectors<MODE, NT>(o0, 3, 4, wl, kn);
+                    load_digits<MODE, NT>(a, o0, 2, 3, k, px);
                 } else {
-                    load_block<MODE, MT, NT>(a, o0, wl, wtile, kn, k, px);
+                    load_block<MODE, NT>(a, o0, wl, kn, k, px);
                 }
                 if (!more) break;
                 ++kb;
             }
 #pragma unroll
-            for (int m = 0; m < MT; ++m)
+            for (int p = 0; p < NT; ++p)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    total[p][i] = (acc[p][i] >> 6) + (int)((uint32_t)a0[p][i] << 1) + (int)((uint32_t)a1[p][i] << 8);
+            if (high)
 #pragma unroll
                 for (int p = 0; p < NT; ++p)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        total[m][p][i] = (acc[m][p][i] >> 6) + (int)((uint32_t)a0[m][p][i] << 1) +
-                                         (int)((uint32_t)a1[m][p][i] << 8);
-            if (high)
-#pragma unroll
-                for (int m = 0; m < MT; ++m)
-#pragma unroll
-                    for (int p = 0; p < NT; ++p)
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) total[m][p][i] += part[wave][(m * NT + p) * 16 + i][lane];
+                    for (int i = 0; i < 16; ++i) total[p][i] += part[wave][p * 16 + i][lane];
         }
     }
     const int chl = c0 + 4 * (lane >> 5);
@@ -894,53 +841,50 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
         if (!live) return;
         // units of 16 channels x 32 pixels; every residual is on its way before the first value is stored
         OutAt o[NT];
-        float res[MT * NT * 2][8];
+        float res[NT * 2][8];
 #pragma unroll
         for (int p = 0; p < NT; ++p) o[p] = out_at(a, pixel_at(a, pix[p]), pix[p]);
         if (a.residual)
 #pragma unroll
-            for (int u = 0; u < MT * NT * 2; ++u)
-                load_residual<2>(a, res[u], chl + u / (NT * 2) * 32 + (u / NT & 1) * 16, o[u % NT]);
+            for (int u = 0; u < NT * 2; ++u)
+                load_residual(a, res[u], chl + u / NT * 16, o[u % NT]);
 #pragma unroll
-        for (int c = 0; c < MT * 2; ++c) {
-            ChannelTail<2> tl;
-            load_tail<2>(a, tl, chl + c * 16);
+        for (int c = 0; c < 2; ++c) {
+            ChannelTail tl;
+            load_tail(a, tl, chl + c * 16);
 #pragma unroll
             for (int p = 0; p < NT; ++p) {
                 int32_t v[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = total[c >> 1][p][(c & 1) * 8 + i];
-                store_tail<2>(a, tl, v, res[c * NT + p], chl + c * 16, o[p]);
+                for (int i = 0; i < 8; ++i) v[i] = total[p][c * 8 + i];
+                store_tail(a, tl, v, res[c * NT + p], chl + c * 16, o[p]);
             }
         }
         return;
     }
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int p = 0; p < NT; ++p)
 #pragma unroll
-        for (int p = 0; p < NT; ++p)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) part[wave][(m * NT + p) * 16 + i][lane] = total[m][p][i];
+        for (int i = 0; i < 16; ++i) part[wave][p * 16 + i][lane] = total[p][i];
     __syncthreads();
     if (!live) return;
     // the ks waves of a tile share its epilogue, in halves of 32 x 32 values
-    const int units = MT * NT * 2 > a.ks ? MT * NT * 2 / a.ks : 1;
-    for (int u = kpart * units; u < (kpart + 1) * units && u < MT * NT * 2; ++u) {
-        const int m = u / (NT * 2), p = (u >> 1) % NT;
-        const int ch = chl + m * 32 + (u & 1) * 16;
-        const uint32_t pp = p0 + p * 32 + (lane & 31);
+    const int units = NT * 2 > a.ks ? NT * 2 / a.ks : 1;
+    for (int u = kpart * units; u < (kpart + 1) * units && u < NT * 2; ++u) {
+        const int ch = chl + (u & 1) * 16;
+        const uint32_t pp = p0 + (u >> 1) * 32 + (lane & 31);
         const OutAt o = out_at(a, pixel_at(a, pp), pp);
-        ChannelTail<2> tl;
+        ChannelTail tl;
         float res[8];
-        load_tail<2>(a, tl, ch);
-        if (a.residual) load_residual<2>(a, res, ch, o);
+        load_tail(a, tl, ch);
+        if (a.residual) load_residual(a, res, ch, o);
         int32_t v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             v[i] = 0;
             for (int s = 0; s < a.ks; ++s) v[i] += part[t * a.ks + s][u * 8 + i][lane];
         }
-        store_tail<2>(a, tl, v, res, ch, o);
+        store_tail(a, tl, v, res, ch, o);
     }
 }
 
@@ -987,16 +931,16 @@ __global__ __launch_bounds__(256) void mfma_operand_border_kernel(int8_t *__rest
     }
 }
 
-template <int MODE, int MT, int NT, int WAVES>
+template <int MODE, int NT, int WAVES>
 static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
 {
-    const int ctiles32 = ceil_div(a.N, MT * 32);
+    const int ctiles32 = ceil_div(a.N, 32);
     a.ks = ks;
     a.tc = (WAVES / a.ks >= 2 && ctiles32 > 1) ? 2 : 1;
     a.ctiles = ceil_div(ctiles32, a.tc);
     a.ptiles = ceil_div((int)a.pixels, NT * 32 * (WAVES / a.ks / a.tc));
     a.by_ctiles = fast_div((uint32_t)a.ctiles);
-    hipLaunchKernelGGL((mfma_kernel<MODE, MT, NT, WAVES>), dim3((unsigned)(a.ctiles * a.ptiles)), dim3(WAVES * 64), 0, st, a);
+    hipLaunchKernelGGL((mfma_kernel<MODE, NT, WAVES>), dim3((unsigned)(a.ctiles * a.ptiles)), dim3(WAVES * 64), 0, st, a);
     return launch_status();
 }
 
@@ -1028,8 +972,8 @@ static int launch_mfma(MfmaArgs &a, hipStream_t st)
     // reduction in eight parts (one image, 512 channels of 7 x 7, 16 tiles: 34 -> 22 us; 256 of 14 x 14, 32 tiles:
     // 21 -> 16; 112 tiles: 38 -> 26).  Past a sixteenth of the slots the extra epilogues cost more than the shorter
     // chain gives (200 tiles: 23.6 -> 25.1; 392 tiles: 18.6 -> 23), as they do on short reductions (18 blocks: even).
-    if (tiles <= waves / 16 && a.KB >= 32) return launch_tiles<MODE, 1, 1, 8>(a, 8, st);
-    return launch_tiles<MODE, 1, 2, 4>(a, reduction_parts(tiles, waves, a.KB), st);
+    if (tiles <= waves / 16 && a.KB >= 32) return launch_tiles<MODE, 1, 8>(a, 8, st);
+    return launch_tiles<MODE, 2, 4>(a, reduction_parts(tiles, waves, a.KB), st);
 }
 
 template <int SRC, bool I8>
