@@ -946,7 +946,7 @@ static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
 
 // Waves that share a tile's reduction, of `blocks` blocks.  A part pays for the start of its loads, its share of an
 // epilogue and the meeting in LDS, so short reductions are cut only where most wave slots would stay empty, longer ones
-// as long as the parts fill slots that whole tiles leave empty, and in two where a few tiles would need another round.
+// as long as the parts fill slots that whole tiles leave empty, and in two where a few tiles would need a second round.
 // Measured with 1, 2 and 4 parts, int32 activations, shifts to 14 (us; 2048 wave slots):
 //   blocks    512 tiles         1024              1536              2048              2560              4096
 //     4       10.6 10.2  9.6    12.1 13.6 17.1    16.0 20.4 23.8    17.2 24.1 31.2                      29.0 43.1 56.3
@@ -954,13 +954,15 @@ static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
 //    18       21.8 16.7 14.9    23.6 23.4 25.5    34.8 33.4 34.6    37.4 41.1 45.4    51.1 50.7 54.4    68.2 73.0 83.6
 //    36       34.3 23.2 20.7    37.8 35.8 36.4    56.8 50.9 52.4    60.0 63.9 67.5    83.3 77.5 82.9   118.7  123  132
 //   144        114 65.6 64.0     116  112  114     194  164  168     211  216  222     304  266  279
-// 8-bit activations (3072 slots) turn at about the same fill.  Cutting up to three tiles a slot, whatever the length,
-// left layers of few channels behind the vector kernels: 17 -> 64 channels, 3 x 3, 64 images of 32 x 32, with the layout
-// pass: 55 us against 45 there and 42 with this rule; 9 -> 128: 62 against 52 and 47.
-static int reduction_parts(long tiles, long waves, int blocks)
+// The second walk for digits 3 and 4 lengthens some tiles only, which two parts even out: 3584 tiles of 72 blocks 317,
+// 295, 300.  8-bit activations (3072 slots) have none, and turn at about the same fill otherwise.
+// Cutting up to three tiles a slot, whatever the length, left layers of few channels behind the vector kernels: 17 -> 64
+// channels, 3 x 3, 64 images of 32 x 32, with the layout pass: 55 us against 45 there and 42 with this rule; 9 -> 128: 62
+// against 52 and 47.
+static int reduction_parts(long tiles, long waves, int blocks, bool i8)
 {
     if (tiles * 8 <= waves * (blocks < 16 ? 2 : blocks < 32 ? 6 : 7)) return blocks >= 4 ? 4 : 1;
-    return blocks >= 32 && tiles > waves && tiles * 4 <= waves * 5 ? 2 : 1;
+    return !i8 && blocks >= 32 && tiles > waves && tiles < 2 * waves ? 2 : 1;
 }
 
 template <int MODE>
@@ -973,7 +975,7 @@ static int launch_mfma(MfmaArgs &a, hipStream_t st)
     // 21 -> 16; 112 tiles: 38 -> 26).  Past a sixteenth of the slots the extra epilogues cost more than the shorter
     // chain gives (200 tiles: 23.6 -> 25.1; 392 tiles: 18.6 -> 23), as they do on short reductions (18 blocks: even).
     if (tiles <= waves / 16 && a.KB >= 32) return launch_tiles<MODE, 1, 8>(a, 8, st);
-    return launch_tiles<MODE, 2, 4>(a, reduction_parts(tiles, waves, a.KB), st);
+    return launch_tiles<MODE, 2, 4>(a, reduction_parts(tiles, waves, a.KB, mode_i8(MODE)), st);
 }
 
 template <int SRC, bool I8>
