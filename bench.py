@@ -265,7 +265,8 @@ def calibrate_valu(device):
 
 
 def config2(device, reps=10):
-    """Benchmark configuration 2: the 3x3 conv (32x64x56x56, 64 -> 64) and the 4096^3 shift GEMM."""
+    """Benchmark configuration 2: the 3x3 conv (32x64x56x56, 64 -> 64) and the 4096^3 shift GEMM.  Shifts 0..15: one
+    more than the matrix cores take with int32 activations, so these are the vector kernels, called directly."""
     from deepshift_amd import kernels, utils
     g = torch.Generator().manual_seed(0)
     out = {}
@@ -900,7 +901,8 @@ def main():
             "avg_launch_us_in_step": dom_s_bracketed / len(dominant) * 1e6,
             "frac_in_step": dom_pairs / dom_s_bracketed / PEAK_PAIRS_MFMA,
             "pairs_per_launch": dom_pairs / len(dominant),
-            # the whole step (all 21 launches, pre-fill passes included) against the same bound
+            # the whole step (all 21 shift launches; the layout passes in front of the stem and behind the pooling,
+            # and the pooling pass, are not among them) against the same bound
             "step_achieved": pairs / kernel_s / 1e12,
             "step_frac": pairs / kernel_s / PEAK_PAIRS_MFMA,
             # secondary: against a kernel that spends two vector instructions on every pair

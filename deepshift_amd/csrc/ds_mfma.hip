@@ -11,14 +11,15 @@
 // any plane; 12 selects the constant 0.  Fields of up to 14 take 18 products of int8 per term, of up to 6 nine, of up
 // to 3 six; activations of 8 bits take one product per distinct shift (x >> s, selected by +-1).  The matrix cores do
 // 1024 such products per clock and SIMD, so 18 per term end at 139 Tpair/s, where the vector kernels' one instruction
-// per term ends at 39.3.  Measured, 64 -> 64 channels, 3 x 3, 64 images of 56 x 56, shifts to 14: 115 us (65 Tpair/s)
-// and 21 us for the layout pass, against 300 us; shifts to 2 on 8-bit activations, 512 -> 512 channels, 128 images of
-// 7 x 7: 66 us (223 Tpair/s).  A pure loop of v_mfma_i32_32x32x32_i8 reaches 0.7 of the nominal rate (47 clocks of
-// 2.4 GHz for 32): what is left between the two is the vector work that makes the planes, in part under the MFMAs.
+// per term ends at 39.3.  Measured, 64 -> 64 channels, 3 x 3, 64 images of 56 x 56, shifts to 14: 111 us (66 Tpair/s)
+// and 24 us for the layout pass, against 300 us; shifts to 2 on 8-bit activations, 512 -> 512 channels, 128 images of
+// 7 x 7: 62 us (238 Tpair/s).  A pure loop of v_mfma_i32_32x32x32_i8 reaches 0.7 of the nominal rate (45 to 48 clocks
+// of 2.4 GHz for 32): what is left between the two is the vector work that makes the planes, in part under the MFMAs.
 //
 // Activations are laid out first (ds_mfma_prepare): [image][row][32-channel block][digit][column][32 channels], so that
-// the 32 pixels x 32 channels of one operand are 1 KiB in a row; d3 and d4 are written, and read, only for rows in
-// which one of them is not zero (|x| >= 16 in 16.16).
+// the 32 pixels x 32 channels of one operand are 1 KiB in a row; d3 and d4 are written, and read, only where one of them
+// is not zero (|x| >= 16 in 16.16): flags tell it per row and share of its channels or, where the convolution before wrote
+// the layout from its epilogue, per 32 of its pixels x 16 channels.
 #include "ds_common.h"
 #include "ds_epilogue.h"
 

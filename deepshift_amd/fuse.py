@@ -157,9 +157,10 @@ class FusedConv2dShift(nn.Module):
 
 class FusedShortcutPair(nn.Module):
     """A residual block's first convolution and its 1 x 1 shortcut, both fused convolutions over the same
-    tensor with the same stride, run as ONE launch (``kernels.conv2d_tiled_fused_pair``): the shortcut
-    reads the centre taps of the padded fixed-point input that was made for the first convolution, so
-    it needs neither a conversion pass of its own nor the float form of the block's input.  Returns
+    tensor with the same stride, from one fixed-point input: the shortcut reads the centre taps of the padded
+    input that was made for the first convolution, so it needs neither a conversion pass of its own nor the
+    float form of the block's input.  Two launches on the matrix cores, from one layout of the input; where
+    those have no form for the weights, ONE launch (``kernels.conv2d_tiled_fused_pair``).  Returns
     ``(result of the first, result of the shortcut)``, each what the module by itself would return."""
 
     def __init__(self, first, shortcut):
