@@ -496,7 +496,7 @@ def _hand_off_fixed_point(gm):
 def _pair_shortcuts(gm):
     """Third pass: where a fused k x k convolution A reads the fixed-point tensor its producer P made for
     it, and a fused 1 x 1 convolution B with the same stride and no padding reads P's float result -- the
-    two branches of a down-sampling residual block -- run A and B as one launch on P's fixed-point tensor
+    two branches of a down-sampling residual block -- run A and B together on P's fixed-point tensor
     (B reads the centre taps: the padded tensor cropped by A's padding).  If nothing else reads P's
     float result it is no longer written."""
     mods = dict(gm.named_modules())
