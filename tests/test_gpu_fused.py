@@ -359,10 +359,17 @@ def test_fused_entry_point_refuses_what_it_cannot_do(rng):
     assert L.ds_conv2d_tiled_fusable(64, 64, 58, 58, 48, 3, 3, 1, 1, 4, -2) == 0
 
 
-def test_fused_module_path_equals_the_separate_passes():
+@pytest.mark.parametrize("route", ["matrix cores", "vector"])
+def test_fused_module_path_equals_the_separate_passes(route, monkeypatch):
     """conv_kernel_forward with the fused epilogue against the same call with it switched off (int32 sums,
-    then the conversion pass): every output bit-identical."""
+    then the conversion pass): every output bit-identical, on the matrix cores and on the shift-plane kernel."""
     from deepshift_amd import modules
+    if route == "vector":
+        monkeypatch.setattr(kernels, "mfma_shift", lambda *a: None)
+    fused_launches = []
+    for name in ("mfma_conv2d", "conv2d_tiled_fused"):
+        real = getattr(kernels, name)
+        monkeypatch.setattr(kernels, name, lambda *a, real=real, **k: (fused_launches.append(len(a) > 7), real(*a, **k))[1])
     torch.manual_seed(3)
     conv = modules.Conv2dShift(64, 128, 3, stride=1, padding=1, use_kernel=True).to(DEV)
     conv.sign.data = torch.where(conv.sign.data >= 0, torch.ones_like(conv.sign), -torch.ones_like(conv.sign))
@@ -396,6 +403,7 @@ def test_fused_module_path_equals_the_separate_passes():
                 ]
         finally:
             modules._FUSE_EPILOGUE = True
+        assert sum(fused_launches) == len(results[True]), "the switch takes the fused launches away"
     for a, b in zip(results[True], results[False]):
         a = a if isinstance(a, tuple) else (a,)
         b = b if isinstance(b, tuple) else (b,)
@@ -458,11 +466,18 @@ def test_pair_launch_matches_oracle_chain(oracle, rng, geom):
         kernels.conv2d_tiled_fused_pair(_dev(xp), (st, st), 16, first, dict(second, crop=(0, 0)))
 
 
-def test_fused_resnet18_pairs_its_shortcuts():
+@pytest.mark.parametrize("route", ["matrix cores", "vector"])
+def test_fused_resnet18_pairs_its_shortcuts(route, monkeypatch):
     """fuse_conv_epilogues on a ResNet-18: the three down-sampling blocks run their first convolution and
-    their shortcut as one launch, and the network output equals the pipeline without the in-kernel
-    epilogue (int32 sums + separate conversion passes, separate shortcut launches) bit for bit."""
+    their shortcut from one fixed-point input -- on the vector kernels as one launch -- and the network output
+    equals the pipeline without the in-kernel epilogue (int32 sums + separate conversion passes, separate
+    shortcut launches) bit for bit."""
     from deepshift_amd import convert, fuse, modules, workloads
+    if route == "vector":
+        monkeypatch.setattr(kernels, "mfma_shift", lambda *a: None)
+    launches = []
+    real = kernels.conv2d_tiled_fused_pair
+    monkeypatch.setattr(kernels, "conv2d_tiled_fused_pair", lambda *a: launches.append(1) or real(*a))
     g = torch.Generator().manual_seed(7)
     model = workloads.randomize_batchnorm(workloads.ResNet18(), g).eval()
     model, _ = convert.convert_to_shift(model, 1000, 'PS', convert_weights=True, use_kernel=True)
@@ -474,6 +489,7 @@ def test_fused_resnet18_pairs_its_shortcuts():
         pairs = [m for m in fused.modules() if isinstance(m, fuse.FusedShortcutPair)]
         assert len(pairs) == 3
         got = fused(x).clone()
+        assert len(launches) == (3 if route == "vector" else 0)
         modules._FUSE_EPILOGUE = False
         try:
             plain = fuse.fuse_conv_epilogues(model, handoff=False)
