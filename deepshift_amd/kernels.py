@@ -87,11 +87,12 @@ def _kept_padded_buffer(cache, shape, dtype, device, layout=None):
         q = torch.zeros(shape, dtype=dtype, device=device)
         # one geometry at a time: a new batch size replaces this stream's buffer; another stream's, given back, is
         # its allocator's again, which hands it to later work of that stream only
-        for old in [k for k in list(cache) if k[0] == at]:
+        kept = [k for k in list(cache) if isinstance(k, tuple)]
+        mine = [k for k in kept if k[0] == at]
+        others = [k for k in kept if k[0] != at]
+        for old in mine + others[:max(0, len(others) + 1 - KEPT_STREAMS)]:
             cache.pop(old, None)
         cache[key] = q
-        for old in list(cache)[:-KEPT_STREAMS]:
-            cache.pop(old, None)
     return q
 
 
@@ -583,8 +584,8 @@ def linear_chain(x2d, layers, integer_bits, fraction_bits, round_to_fixed, ws_ca
     ``(tiled, bias, K, N, bits, base, relu)``; ``ws_cache``: a dict that keeps the workspace (control block
     zeroed once + hidden activations) between calls, one per stream; a captured call has its own.  Returns
     float32 ``[M, N_last]``, or ``None`` when the chain has no such form (mixed field widths, a K that is not a
-    multiple of 4, ...): the caller then runs the layers one by one.  The barriers of the one-launch form wait at most 2 s for the whole grid to
-    be resident; :func:`linear_chain_status` tells whether one gave up."""
+    multiple of 4, ...): the caller then runs the layers one by one.  The barriers of the one-launch form wait
+    at most 2 s for the whole grid to be resident; :func:`linear_chain_status` tells whether one gave up."""
     x2d = x2d.contiguous()
     if x2d.dtype != torch.float32 or not x2d.is_cuda or x2d.dim() != 2:
         raise TypeError("linear_chain expects a 2-D float32 GPU tensor")
@@ -601,9 +602,15 @@ def linear_chain(x2d, layers, integer_bits, fraction_bits, round_to_fixed, ws_ca
     if ws_bytes == 0 or x2d.data_ptr() % 16:
         return None
     ws = _kept_padded_buffer(ws_cache, (ws_bytes,), torch.uint8, dev)
-    if ws is None:   # being captured: kept for its status only
-        ws = ws_cache["captured"] = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        ws[:_lib.DS_CHAIN_CONTROL_BYTES].zero_()
+    captured = ws is None
+    if captured:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        if how is None:   # the library's own choice, which decides whether there are barriers
+            how = "one" if all((N + 1) // 2 * ((M + 63) // 64) <= 64 for (_, _, _, N, _, _, _) in layers) else "each"
+        if how == "one":
+            ws[:_lib.DS_CHAIN_CONTROL_BYTES].zero_()
+    elif dev not in ws_cache:
+        ws_cache[dev] = torch.zeros(1, dtype=torch.int32, device=dev)   # the highest status of captured calls
     out = torch.empty([M, layers[-1][3]], dtype=torch.float32, device=dev)
     pairs = sum(M * K * N for (_, _, K, N, _, _, _) in layers)
     mode = _lib.DS_Q_ROUND_TO_FIXED if round_to_fixed else _lib.DS_Q_CAST
@@ -611,15 +618,24 @@ def linear_chain(x2d, layers, integer_bits, fraction_bits, round_to_fixed, ws_ca
     with _Timed("linear", M, pairs // (M * layers[-1][3]) if M else 0, layers[-1][3], dev):
         _lib.call("ds_linear_chain_f32", _lib.ptr(x2d), arr, len(layers), _lib.ptr(out), M, mode, int(integer_bits),
                   int(fraction_bits), _lib.ptr(ws), ws_bytes, _lib.current_stream(dev))
+    if captured and how == "one" and dev in ws_cache:
+        # in memory that the graph does not own
+        status = ws_cache[dev]
+        torch.maximum(status, _chain_status_word(ws), out=status)
     return out
+
+
+def _chain_status_word(ws):
+    return ws[_lib.DS_CHAIN_STATUS_AT:_lib.DS_CHAIN_STATUS_AT + 4].view(torch.int32)
 
 
 def linear_chain_status(ws_cache):
     """0, or the number of the barrier at which a launch of :func:`linear_chain` on these workspaces gave up
-    (its output was undefined).  Synchronises with the device."""
-    at = _lib.DS_CHAIN_STATUS_AT
-    for ws in list(ws_cache.values()):
-        status = int(ws[at:at + 4].view(torch.int32).item())
+    (its output was undefined), replays of captured calls included where a call came before the capture.
+    Synchronises with the device."""
+    for key, kept in list(ws_cache.items()):
+        torch.cuda.synchronize(kept.device)
+        status = int((kept if isinstance(key, torch.device) else _chain_status_word(kept)).item())
         if status:
             return status
     return 0

@@ -5,6 +5,7 @@ import torch
 import torch.nn as nn
 
 from deepshift_amd import _lib, convert, fuse, kernels, modules
+from tests.conftest import Tune
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -103,13 +104,36 @@ def test_streams_and_graphs_have_their_own_chain_workspace(widths):
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             y = model(static)
-        assert torch.equal(model(xs[1]), want[1])
+        assert chain.status() == 0 and torch.equal(model(xs[1]), want[1])
         for i in range(4):
             static.copy_(xs[i])
             graph.replay()
             assert torch.equal(model(xs[i + 4][:30]), want[i + 4][:30])
             assert torch.equal(y, want[i])
         assert chain.status() == 0
+
+
+def test_replays_report_a_barrier_that_gave_up():
+    """The test hook makes the barriers of a captured launch wait, 200 us at most, for one arrival more than the grid has."""
+    with torch.no_grad():
+        model = _chain((64, 64, 32, 8))
+        chain = next(m for m in model.modules() if isinstance(m, fuse.FusedLinearChain))
+        x = torch.rand(64, 64, device=DEV)
+        want = model(x)
+        torch.cuda.synchronize()
+        graphs = []
+        for knobs in (dict(), dict(chain_spin_us=200, chain_extra=1)):
+            graphs.append(torch.cuda.CUDAGraph())
+            with Tune(**knobs), torch.cuda.graph(graphs[-1]):
+                y = model(x)
+            if not knobs:
+                first = y
+        graphs[0].replay()
+        assert chain.status() == 0 and torch.equal(first, want)
+        graphs[1].replay()
+        assert chain.status() == 1
+        graphs[0].replay()
+        assert chain.status() == 1 and torch.equal(first, want) and torch.equal(model(x), want)
 
 
 @pytest.mark.parametrize("M", [1024, 64])
