@@ -1,4 +1,4 @@
-// Shift convolutions and shift GEMMs on the matrix cores (int8 MFMA, int32 accumulation), exact modulo 2^32.
+// Shift convolutions and shift GEMMs on the matrix cores (int8 sparse MFMA, int32 accumulation), exact modulo 2^32.
 //
 // A term sgn * (x >> s) is not linear in x, but it is a short sum of products of 8-bit numbers.  With x written in
 // 7-bit digits, x = d0 + 2^7 d1 + 2^14 d2 + 2^21 d3 + 2^28 d4 (d0, d1 in 0..127, the others balanced), and
@@ -6,20 +6,27 @@
 //     x >> s = (d_q >> r) + sum_{i > q} d_i * 2^(6-r) * 2^(7(i-q-1)+1)
 //     64 * (d_q >> r) = sum_j (bit j of d_q, in place) * [r <= j] 2^(6-r)
 // i.e. bit masks of a digit (one AND per four activations) times weight planes that hold 0 or a signed power of two
-// up to 64 -- all of them int8 -- plus products of whole digits with the full weight plane of their q.  A weight is
-// stored as up to four selector bytes, one per group of four shifts, from which one v_perm_b32 per four weights makes
-// any plane; 12 selects the constant 0.  Fields of up to 14 take 18 products of int8 per term, of up to 6 nine, of up
-// to 3 six; activations of 8 bits take one product per distinct shift (x >> s, selected by +-1).  The matrix cores do
-// 1024 such products per clock and SIMD, so 18 per term end at 139 Tpair/s, where the vector kernels' one instruction
-// per term ends at 39.3.  Measured, 64 -> 64 channels, 3 x 3, 64 images of 56 x 56, shifts to 14: 111 us (66 Tpair/s)
-// and 24 us for the layout pass, against 300 us; shifts to 2 on 8-bit activations, 512 -> 512 channels, 128 images of
-// 7 x 7: 62 us (238 Tpair/s).  A pure loop of v_mfma_i32_32x32x32_i8 reaches 0.7 of the nominal rate (45 to 48 clocks
-// of 2.4 GHz for 32): what is left between the two is the vector work that makes the planes, in part under the MFMAs.
+// up to 64 -- all of them int8 -- plus products of whole digits with the full weight plane of their q.  A weight has one
+// q: of the digits d0 and d1 it meets one, of d1 and d2 (next power) one, and so on.  That is the matrix cores' 2:4
+// sparsity: with digits (d0, d1) of each activation side by side, a weight is one of the two places, the index of
+// v_smfmac_i32_32x32x64_i8 says which, and one instruction does for both q what took two.  A weight is stored as its
+// index and one or two selector bytes (r <= 3 and r >= 4), from which one v_perm_b32 per four weights makes any plane;
+// 12 selects the constant 0.  Shifts to 14 take 10 products per term (7 for the bits, one each for the two powers above
+// them, one for s = 14; 2 more where a digit d3 is not zero), to 6 six, to 3 four: there the pair is one digit twice,
+// masked differently for small and large r.  8-bit activations: x >> s selected from the pair (x, x >> 4), four products,
+// or (x, x >> 2), two.
 //
-// Activations are laid out first (ds_mfma_prepare): [image][row][32-channel block][digit][column][32 channels], so that
-// the 32 pixels x 32 channels of one operand are 1 KiB in a row; d3 and d4 are written, and read, only where one of them
-// is not zero (|x| >= 16 in 16.16): flags tell it per row and share of its channels or, where the convolution before wrote
-// the layout from its epilogue, per 32 of its pixels x 16 channels.
+// Measured (us, dense products of one digit each -> this; 64 images, 3 x 3 layers, with their hand-off): shifts to 14, 64
+// channels of 56 x 56: 107 -> 91, 512 of 7 x 7: 105 -> 78, with digit d3 164 -> 119 and 175 -> 107; 8-bit activations 63 ->
+// 48 and 62 -> 39.  4096^3: 772 -> 551 us, 125 Tpair/s.  What bounds it is power: a loop of one product and seven vector
+// instructions takes 28 ns (68 clocks of 2.4 GHz, of which the matrix core needs 32) on random bytes, 21 on bit planes and
+// 26 on whole digits, whatever the number of waves; 4096^3 takes 27.  Sparse and dense products cost the same (22 ns alone
+// on random bytes), so the number of products is what counts.
+//
+// Activations are laid out first (ds_mfma_prepare): [image][row][32-channel block][digits 0 and 1 in pairs, 2, 3, 4][column]
+// [channels], so that the 32 pixels x 32 channels of one operand are a KiB in a row, two for the pairs; d3 and d4 are
+// written, and read, only where one of them is not zero (|x| >= 16 in 16.16): flags tell it per row and share of its
+// channels or, where the convolution before wrote the layout from its epilogue, per 32 of its pixels x 16 channels.
 #include "ds_common.h"
 #include "ds_epilogue.h"
 
@@ -34,11 +41,11 @@ constexpr int kMaxRows = 1 << 24;   // ds_mfma_prepare launches 256 threads per 
 constexpr int kMaxPad = 1 << 28;
 
 // Which products a launch forms (MfmaMode): the widest shift that occurs, and the activations' width.
-enum { kI32S15 = 0, kI32S7 = 1, kI32S4 = 2, kI8S8 = 3, kI8S4 = 4, kI8S3 = 5 };
-__host__ __device__ constexpr int mode_groups(int mode)
-{
-    return mode == kI32S15 ? 4 : (mode == kI32S7 || mode == kI8S8) ? 2 : 1;
-}
+enum { kI32S15 = 0, kI32S7 = 1, kI32S4 = 2, kI8S8 = 3, kI8S4 = 4 };
+// Selector bytes per weight, and bytes of a 32-channel tile's share of one block: the selectors, then 4 bytes of indices
+// per lane (which of two activation bytes each weight meets).
+__host__ __device__ constexpr int mode_sels(int mode) { return mode == kI32S15 || mode == kI32S7 ? 2 : 1; }
+__host__ __device__ constexpr int mode_block(int mode) { return mode_sels(mode) * 1024 + 256; }
 __host__ __device__ constexpr bool mode_i8(int mode) { return mode >= kI8S8; }
 
 // The reduction in blocks of 32 activation bytes that lie side by side: 32 channels of one tap, or, where a pixel has
@@ -58,10 +65,12 @@ inline MfmaGeom mfma_geom(int N, int C, int FH, int FW)
     g.ntiles = ceil_div(N, 64) * 2;
     return g;
 }
-inline size_t mfma_blob_corr(const MfmaGeom &g, int mode) { return (size_t)g.ntiles * g.kb * mode_groups(mode) * 1024; }
+inline size_t mfma_blob_corr(const MfmaGeom &g, int mode) { return (size_t)g.ntiles * g.kb * mode_block(mode); }
 
-// One thread per (channel tile, block, lane): the 16 selector bytes per group of its fragment.
-__global__ __launch_bounds__(256) void mfma_tile_kernel(const int32_t *__restrict__ w_ref, v4i *__restrict__ blob, int N,
+// One thread per (channel tile, block, lane): the selector bytes of its 16 weights, and which byte of a pair each meets.
+// Weight i of lane l is reduction index 16 (i / 8) + 8 (l / 32) + i % 8 of the block: the half i / 8 of the wave holds the
+// activations that it meets, 16 indices in a row.
+__global__ __launch_bounds__(256) void mfma_tile_kernel(const int32_t *__restrict__ w_ref, int8_t *__restrict__ blob, int N,
                                                         int C, int FH, int FW, int bits, int mode, int cp, int cb,
                                                         int taps, int fwg, int kb, long total)
 {
@@ -73,12 +82,12 @@ __global__ __launch_bounds__(256) void mfma_tile_kernel(const int32_t *__restric
     const int fg = b % fwg, fh = b / fwg % FH, c0 = b / fwg / FH * cp;
     const int n = tile * 32 + (lane & 31);
     const int K = C * FH * FW, num = codes_per_word(bits), comm = ceil_div(K, num);
-    const int groups = mode_groups(mode);
-    uint32_t sel[4][4];
-    for (int g = 0; g < 4; ++g)
+    uint32_t sel[2][4], index = 0;
+    for (int g = 0; g < 2; ++g)
         for (int w = 0; w < 4; ++w) sel[g][w] = 0x0c0c0c0cu;
     for (int i = 0; i < 16; ++i) {
-        const int kk = (lane >> 5) * 16 + i;
+        index |= (uint32_t)(2 * (i & 1)) << (2 * i);
+        const int kk = (i >> 3) * 16 + (lane >> 5) * 8 + (i & 7);
         const int c = c0 + kk % cp, fw = fg * taps + kk / cp;
         if (n >= N || c >= C || fw >= FW) continue;
         const int k = (c * FH + fh) * FW + fw;
@@ -86,39 +95,52 @@ __global__ __launch_bounds__(256) void mfma_tile_kernel(const int32_t *__restric
         uint32_t s = code & ((1u << bits) - 1u);
         const uint32_t neg = ((code >> bits) & 1u) ? 0u : 4u;
         if (s >= 32) continue;  // a zero weight
-        uint32_t g, l;
-        if (mode_i8(mode)) {
+        uint32_t g = 0, l, second;   // selector, its value, the second byte of the pair
+        if (mode == kI8S8) {
             s = s < 7 ? s : 7;
-            g = s >> 2;
             l = s & 3;
+            second = s >> 2;
+        } else if (mode == kI8S4) {
+            l = s & 1;
+            second = s >> 1;
+        } else if (mode == kI32S4) {
+            l = s;
+            second = s >> 1;
         } else {
-            g = s < 4 ? 0 : s < 7 ? 1 : s < 11 ? 2 : 3;
-            l = s - (g == 0 ? 0 : g == 1 ? 4 : g == 2 ? 7 : 11);
+            const uint32_t q = s / 7, r = s - 7 * q;
+            g = q == 2 || r >= 4 ? 1 : 0;
+            l = q == 2 ? 3 : r & 3;
+            second = mode == kI32S7 ? g : q & 1;
         }
-        if (g >= (uint32_t)groups || l > 3) continue;  // the caller vouches that it does not occur
+        if (l > 3 || second > 1) continue;  // the caller vouches that it does not occur
+        index |= second << (2 * i);
         const int at = (i & 3) * 8;
         sel[g][i >> 2] = (sel[g][i >> 2] & ~(255u << at)) | ((l | neg) << at);
     }
-    for (int g = 0; g < groups; ++g) {
+    int8_t *o = blob + tile_kb * mode_block(mode);
+    for (int g = 0; g < mode_sels(mode); ++g) {
         v4i v;
         for (int w = 0; w < 4; ++w) v[w] = (int)sel[g][w];
-        blob[(tile_kb * groups + g) * 64 + lane] = v;
+        *(v4i *)(o + g * 1024 + lane * 16) = v;
     }
+    *(uint32_t *)(o + mode_sels(mode) * 1024 + lane * 4) = index;
 }
 
-// Per channel, what the +128 on the shifted 8-bit activations adds: sum_k sgn * 2^(7-s) over s >= 1.
+// Per channel, what the offset of the second byte of 8-bit activations adds (offset 8 for x >> 4, 32 for x >> 2):
+// sum_k sgn * (offset >> (s - 4 or 2)) over the shifts that take it.
 __global__ __launch_bounds__(64) void mfma_corr_kernel(const int32_t *__restrict__ w_ref, int32_t *__restrict__ corr, int N,
-                                                       int K, int bits)
+                                                       int K, int bits, int mode)
 {
     const int n = blockIdx.x, num = codes_per_word(bits), comm = ceil_div(K, num);
+    const uint32_t from = mode == kI8S8 ? 4 : 2, offset = mode == kI8S8 ? 8 : 32;
     int sum = 0;
     if (n < N)
         for (int k = threadIdx.x; k < K; k += 64) {
             const uint32_t code = (uint32_t)w_ref[(long)n * comm + k / num] >> ((k % num) * (bits + 1));
             uint32_t s = code & ((1u << bits) - 1u);
-            if (s == 0 || s >= 32) continue;
+            if (s < from || s >= 32) continue;
             s = s < 7 ? s : 7;
-            const int v = 1 << (7 - s);
+            const int v = (int)(offset >> (s - from));
             sum += ((code >> bits) & 1u) ? v : -v;
         }
     for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o);
@@ -133,6 +155,7 @@ __global__ __launch_bounds__(64) void mfma_corr_kernel(const int32_t *__restrict
 struct MfmaX {
     int Hp, Wp, cp, cb, digits;
     int dstride, cbstride, rstride;  // bytes between digits, 32-channel blocks, rows
+    int px01, half01, piece01;       // digits 0 and 1, side by side: bytes between pixels, halves of a wave, pieces of a block
     int fy, cbf;                     // flag bytes per row, channel blocks that each of them covers
     int tiles, th, tw, tph, tpw;     // written by a convolution: one flag per 32 of its th x tw pixels and 16 channels
     int c16;
@@ -150,6 +173,9 @@ inline MfmaX mfma_x(int Nb, int C, int Hp, int Wp, const MfmaGeom &g, bool i8)
     x.dstride = Wp * g.cp;
     x.cbstride = x.dstride * x.digits;
     x.rstride = x.cbstride * g.cb;
+    x.px01 = g.cp == 32 ? 32 : 2 * g.cp;
+    x.half01 = g.cp == 32 ? 16 : 32;
+    x.piece01 = g.cp == 32 ? x.dstride : 16;
     x.rows = (long)Nb * Hp;
     // enough workgroups to fill the chip: a row's channel blocks are shared out over up to eight of them
     int fy = 1;
@@ -194,6 +220,9 @@ __device__ __forceinline__ void digits_of(int32_t v, int32_t d[kDigits])
     d[3] = (int32_t)((uint32_t)c << 25) >> 25;
     d[4] = (c - d[3]) >> 7;
 }
+
+// Digits 0 and 1 of a value in two bytes.
+__device__ __forceinline__ uint32_t pair01(int32_t v) { return ((uint32_t)v & 127u) | (((uint32_t)v << 1) & 0x7f00u); }
 
 // Workgroup (row, part): CH channels of one pixel per thread and step, two threads side by side for the halves of a
 // 32-channel block, so that loads run along the row and stores are contiguous.  Bound by memory: 4 bytes read and 3
@@ -243,8 +272,9 @@ __global__ __launch_bounds__(256) void mfma_prepare_kernel(PrepArgs a)
                     v[i] = (in && c0 + i < a.C) ? prep_value<SRC>(a.x, base + i * plane, a.spec) : 0;
             }
             int8_t *o = dst + (size_t)cb * L.cbstride + wp * L.cp + half * CH;
+            int8_t *o01 = dst + (size_t)cb * L.cbstride + wp * L.px01 + half * L.half01;
             constexpr int D = I8 ? 1 : kDigits;
-            uint32_t words[D][CH / 4];
+            uint32_t words[D][CH / 4], pairs[I8 ? 1 : CH / 2];
 #pragma unroll
             for (int q = 0; q < CH / 4; ++q) {
 #pragma unroll
@@ -257,10 +287,20 @@ __global__ __launch_bounds__(256) void mfma_prepare_kernel(PrepArgs a)
                     else
                         digits_of(v[q * 4 + i], dg);
 #pragma unroll
-                    for (int d = 0; d < D; ++d) words[d][q] |= ((uint32_t)dg[d] & 255u) << (8 * i);
+                    for (int d = 0; d < D; ++d)
+                        if (I8 || d >= 2) words[d][q] |= ((uint32_t)dg[d] & 255u) << (8 * i);
+                }
+                if (!I8) {
+                    pairs[q * 2] = pair01(v[q * 4]) | pair01(v[q * 4 + 1]) << 16;
+                    pairs[q * 2 + 1] = pair01(v[q * 4 + 2]) | pair01(v[q * 4 + 3]) << 16;
                 }
             }
-            const int lo = pass == 0 ? 0 : 3, hi = I8 ? 1 : pass == 0 ? 3 : 5;
+            if (!I8 && pass == 0) {
+                // eight channels a piece
+#pragma unroll
+                for (int q = 0; q < CH / 2; ++q) ((uint32_t *)(o01 + (q >> 2) * L.piece01))[q & 3] = pairs[q];
+            }
+            const int lo = I8 ? 0 : pass == 0 ? 2 : 3, hi = I8 ? 1 : pass == 0 ? 3 : 5;
 #pragma unroll
             for (int d = 0; d < D; ++d) {
                 if (d >= lo && d < hi)
@@ -295,7 +335,7 @@ struct MfmaArgs {
     void *q;                    // the next layer's input
     const float *scale, *shift, *residual;
     MfmaX lay;
-    int N, KB, FH, fwg, tapstep;
+    int N, KB, FH, fwg, tapstep, tapstep01;
     int OH, OW, sh, sw, crop_h, crop_w;
     uint32_t pixels;
     int ks, tc, ctiles, ptiles;   // K parts, channel tiles per workgroup, workgroups along channels and pixels
@@ -338,107 +378,248 @@ constexpr uint32_t kPosHi = 0x00010204u, kNegHi = 0x00fffefcu;   // r = 4..6: 4,
 constexpr uint32_t kPos14 = 0x40000000u, kNeg14 = 0xc0000000u;   // s = 14, the last of its group: 64
 __host__ __device__ constexpr uint32_t low_bytes(uint32_t v, int n) { return n >= 4 ? v : v & ((1u << (8 * n)) - 1u); }
 
-template <int MODE, int NT>
+typedef int v8i __attribute__((ext_vector_type(8)));
+
+// What a wave holds of one block: CT x 32 channels, NT x 32 pixels.  lo: digits 0 and 1 in pairs, or the 8-bit values.
+template <int MODE, int CT, int NT, bool HIGH>
 struct Operands {
-    static constexpr int G = mode_groups(MODE), D = mode_i8(MODE) ? 1 : 3;
-    v4i sel[G];
-    v4i dig[NT][D];
+    static constexpr int S = mode_sels(MODE), L = mode_i8(MODE) ? 1 : 2;
+    v4i sel[CT][S];
+    int index[CT];
+    v4i lo[NT][L];
+    v4i d2[mode_i8(MODE) ? 1 : NT], d3[HIGH ? NT : 1];
+    uint32_t on[HIGH ? NT : 1];   // the flag of d3, and whether its place is inside the image
+    bool in[HIGH ? NT : 1];
 };
 
-template <int NT>
-__device__ __forceinline__ void product(v16i (&acc)[NT], const v4i &w, const v4i (&b)[NT])
+template <int CT, int NT>
+__device__ __forceinline__ void product(v16i (&acc)[CT][NT], const v4i (&w)[CT], const v8i (&b)[NT], const int (&index)[CT])
 {
 #pragma unroll
-    for (int p = 0; p < NT; ++p) acc[p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, b[p], acc[p], 0, 0, 0);
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int p = 0; p < NT; ++p)
+            acc[c][p] = __builtin_amdgcn_smfmac_i32_32x32x64_i8(w[c], b[p], acc[c][p], index[c], 0, 0);
+}
+template <int CT>
+__device__ __forceinline__ void weights(v4i (&w)[CT], uint32_t neg, uint32_t pos, const v4i (&sel)[CT])
+{
+#pragma unroll
+    for (int c = 0; c < CT; ++c) w[c] = perm4(neg, pos, sel[c]);
+}
+template <int CT>
+__device__ __forceinline__ void both(v4i (&w)[CT], const v4i (&a)[CT], const v4i (&b)[CT])
+{
+#pragma unroll
+    for (int c = 0; c < CT; ++c) w[c] = or4(a[c], b[c]);
+}
+__device__ __forceinline__ v8i and8(const v8i &v, uint32_t m)
+{
+    v8i r;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = v[i] & (int)m;
+    return r;
+}
+__device__ __forceinline__ v8i join8(const v4i &a, const v4i &b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+// Pairs of bytes: byte i of a beside byte i of b (16 activations).
+__device__ __forceinline__ v8i pairs_of(const v4i &a, const v4i &b)
+{
+    v8i r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        r[2 * i] = (int)__builtin_amdgcn_perm((uint32_t)b[i], (uint32_t)a[i], 0x05010400u);
+        r[2 * i + 1] = (int)__builtin_amdgcn_perm((uint32_t)b[i], (uint32_t)a[i], 0x07030602u);
+    }
+    return r;
+}
+__device__ __forceinline__ v8i pairs_with_zero(const v4i &a)
+{
+    v8i r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        r[2 * i] = (int)__builtin_amdgcn_perm(0u, (uint32_t)a[i], 0x0c010c00u);
+        r[2 * i + 1] = (int)__builtin_amdgcn_perm(0u, (uint32_t)a[i], 0x0c030c02u);
+    }
+    return r;
+}
+// Digit 1 of pairs (0, 1) beside digit 2.
+__device__ __forceinline__ v8i pairs12(const v8i &p01, const v4i &d2)
+{
+    v8i r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        r[2 * i] = (int)__builtin_amdgcn_perm((uint32_t)d2[i], (uint32_t)p01[2 * i], 0x05030401u);
+        r[2 * i + 1] = (int)__builtin_amdgcn_perm((uint32_t)d2[i], (uint32_t)p01[2 * i + 1], 0x07030601u);
+    }
+    return r;
 }
 
-// The seven bit products of digit q: adds to an, leaves the full weight plane 2^(6-r) in w.
-template <int MODE, int NT>
-__device__ __forceinline__ void bit_products(const Operands<MODE, NT> &o, int q, v16i (&an)[NT], v4i &w)
+// The sums of a tile: bits (times 64), and whole digits by power of two, 2^(7 i + 1).
+template <int CT, int NT, bool HIGH>
+struct Sums {
+    v16i bits[CT][NT], d[HIGH ? 3 : 2][CT][NT];
+};
+
+// Shifts to 14.  s = 7 q + r: the first byte of each pair is q's digit 0, the second digit 1, and so on up; q = 2 meets
+// first bytes only, in products of its own.
+template <int CT, int NT, bool HIGH, typename Reload>
+__device__ __forceinline__ void block_s15(const Operands<kI32S15, CT, NT, HIGH> &o, Sums<CT, NT, HIGH> &t, Reload reload)
 {
-    v4i b[NT], w3;
+    v8i x01[NT], b[NT];
+    v4i w[CT], wlo[CT], slo[CT], shi[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        slo[c] = o.sel[c][0];
+        shi[c] = o.sel[c][1];
+    }
+#pragma unroll
+    for (int p = 0; p < NT; ++p) x01[p] = join8(o.lo[p][0], o.lo[p][1]);
 #pragma unroll
     for (int j = 0; j < 7; ++j) {
-        // shifts of at most 3: bits 3 to 6 meet the same weights
-        if (MODE == kI32S4 && j > 3) break;
-        if (j <= 3) {
-            w = perm4(low_bytes(kNegLo, j + 1), low_bytes(kPosLo, j + 1), o.sel[2 * q]);
-            w3 = w;
-        } else if constexpr (Operands<MODE, NT>::G > 1) {
-            w = or4(w3, perm4(low_bytes(kNegHi, j - 3), low_bytes(kPosHi, j - 3), o.sel[2 * q + 1]));
-        }
-        const uint32_t mask = MODE == kI32S4 && j == 3 ? 0x78787878u : 0x01010101u << j;
+        // r <= 3: bits 3 to 6 meet the same weights; r >= 4: bits 4, 5, 6 one by one
+        if (j <= 3)
+            weights<CT>(w, low_bytes(kNegLo, j + 1), low_bytes(kPosLo, j + 1), slo);
+        else
+            weights<CT>(w, low_bytes(kNegHi, j - 3), low_bytes(kPosHi, j - 3), shi);
 #pragma unroll
-        for (int p = 0; p < NT; ++p) b[p] = and4(o.dig[p][q], mask);
-        product<NT>(an, w, b);
+        for (int p = 0; p < NT; ++p) b[p] = and8(x01[p], j == 3 ? 0x78787878u : 0x01010101u << j);
+        product<CT, NT>(t.bits, w, b, o.index);
+        if (j == 3) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) wlo[c] = w[c];
+        }
+    }
+    both<CT>(wlo, wlo, w);
+#pragma unroll
+    for (int p = 0; p < NT; ++p) b[p] = pairs12(x01[p], o.d2[p]);
+    product<CT, NT>(t.d[0], wlo, b, o.index);
+    weights<CT>(w, kNeg14, kPos14, shi);
+    if constexpr (HIGH) {
+        v8i b3[NT];
+        int index[CT];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) index[c] = o.index[c];
+#pragma unroll
+        for (int p = 0; p < NT; ++p) {
+            const v4i d3 = and4(o.d3[p], o.in[p] && o.on[p] ? 0xffffffffu : 0u);
+            b[p] = pairs_of(o.d2[p], d3);
+            b3[p] = pairs_with_zero(d3);
+        }
+        reload();
+        product<CT, NT>(t.d[1], wlo, b, index);
+        product<CT, NT>(t.bits, w, b, index);
+        product<CT, NT>(t.d[2], wlo, b3, index);
+        product<CT, NT>(t.d[0], w, b3, index);
+    } else {
+#pragma unroll
+        for (int p = 0; p < NT; ++p) b[p] = pairs_with_zero(o.d2[p]);
+        product<CT, NT>(t.d[1], wlo, b, o.index);
+        product<CT, NT>(t.bits, w, b, o.index);
     }
 }
 
-template <int MODE, int NT>
-__device__ __forceinline__ void digit_product(const Operands<MODE, NT> &o, int d, v16i (&acc)[NT], const v4i &w)
+// Shifts to 6 or to 3: every weight meets digit 0; the pair is that digit twice, masked differently for small and large
+// shifts.
+template <int MODE, int CT, int NT, bool HIGH, typename Reload>
+__device__ __forceinline__ void block_s7(const Operands<MODE, CT, NT, HIGH> &o, Sums<CT, NT, HIGH> &t, Reload reload)
 {
-    v4i b[NT];
+    v8i x01[NT], x0[NT], b[NT];
+    v4i w[CT], full[CT], slo[CT], shi[CT];
 #pragma unroll
-    for (int p = 0; p < NT; ++p) b[p] = o.dig[p][d];
-    product<NT>(acc, w, b);
+    for (int c = 0; c < CT; ++c) {
+        slo[c] = o.sel[c][0];
+        shi[c] = o.sel[c][mode_sels(MODE) - 1];
+    }
+#pragma unroll
+    for (int p = 0; p < NT; ++p) {
+        x01[p] = join8(o.lo[p][0], o.lo[p][1]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x0[p][i] = (int)__builtin_amdgcn_perm(0u, (uint32_t)x01[p][i], 0x02020000u);
+    }
+    if constexpr (MODE == kI32S4) {
+        // shifts 0, 1 beside 2, 3: bit 0 for a shift of 0 beside bit 2 for one of 2, then the rest of both
+#pragma unroll
+        for (int p = 0; p < NT; ++p) b[p] = and8(x0[p], 0x04010401u);
+        weights<CT>(w, kNegLo & 0x00ff00ffu, kPosLo & 0x00ff00ffu, slo);
+        product<CT, NT>(t.bits, w, b, o.index);
+#pragma unroll
+        for (int p = 0; p < NT; ++p) b[p] = and8(x0[p], 0x787e787eu);
+        weights<CT>(full, kNegLo, kPosLo, slo);
+        product<CT, NT>(t.bits, full, b, o.index);
+    } else {
+        // shifts 0 to 3 beside 4 to 6: bits j beside bits 4 + j, then bits 3 to 6 of the former
+        v4i hi[CT];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            weights<CT>(w, low_bytes(kNegLo, j + 1), low_bytes(kPosLo, j + 1), slo);
+            if (j < 3) {
+                weights<CT>(hi, low_bytes(kNegHi, j + 1), low_bytes(kPosHi, j + 1), shi);
+                v4i sum[CT];
+                both<CT>(sum, w, hi);
+#pragma unroll
+                for (int p = 0; p < NT; ++p) b[p] = and8(x0[p], 0x10011001u << j);
+                product<CT, NT>(t.bits, sum, b, o.index);
+            } else {
+#pragma unroll
+                for (int p = 0; p < NT; ++p) b[p] = and8(x0[p], 0x00780078u);
+                product<CT, NT>(t.bits, w, b, o.index);
+            }
+        }
+        both<CT>(full, w, hi);
+    }
+    // whole digits: first or second bytes of pairs (1, 2), (3, 0) for all weights
+    int first[CT], second[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        first[c] = (int)0x88888888u;
+        second[c] = (int)0xddddddddu;
+    }
+#pragma unroll
+    for (int p = 0; p < NT; ++p) b[p] = pairs12(x01[p], o.d2[p]);
+    if constexpr (HIGH) {
+        v8i b3[NT];
+#pragma unroll
+        for (int p = 0; p < NT; ++p) b3[p] = pairs_with_zero(and4(o.d3[p], o.in[p] && o.on[p] ? 0xffffffffu : 0u));
+        reload();
+        product<CT, NT>(t.d[2], full, b3, first);
+    }
+    product<CT, NT>(t.d[0], full, b, first);
+    product<CT, NT>(t.d[1], full, b, second);
 }
 
-template <int MODE, int NT>
-__device__ __forceinline__ void block_i8(const Operands<MODE, NT> &o, v16i (&acc)[NT])
+// 8-bit activations: x >> s = (y >> l), y the value itself for small shifts, x >> 4 (or >> 2) with an offset that makes it
+// positive for large ones: a pair of bytes, of which every shift l takes the upper 8 - l bits.
+template <int MODE, int CT, int NT>
+__device__ __forceinline__ void block_i8(const Operands<MODE, CT, NT, false> &o, v16i (&acc)[CT][NT])
 {
-    constexpr int S = MODE == kI8S8 ? 8 : MODE == kI8S4 ? 4 : 3;
-    v4i b[NT], u[NT], w;
+    constexpr int S = MODE == kI8S8 ? 4 : 2;
+    v8i x[NT], b[NT];
+    v4i w[CT], sel[CT];
 #pragma unroll
-    for (int p = 0; p < NT; ++p)
+    for (int c = 0; c < CT; ++c) sel[c] = o.sel[c][0];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) u[p][i] = o.dig[p][0][i] ^ (int)0x80808080;
+    for (int p = 0; p < NT; ++p) {
+        v4i y;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-            w = perm4(0xffu << (8 * (s & 3)), 0x01u << (8 * (s & 3)), o.sel[s >> 2]);
+        for (int i = 0; i < 4; ++i)
+            y[i] = MODE == kI8S8 ? (int)((((uint32_t)o.lo[p][0][i] >> 4) & 0x0f0f0f0fu) ^ 0x08080808u)
+                                 : (int)((((uint32_t)o.lo[p][0][i] >> 2) & 0x3f3f3f3fu) ^ 0x20202020u);
+        x[p] = pairs_of(o.lo[p][0], y);
+    }
 #pragma unroll
-        for (int p = 0; p < NT; ++p) {
-            if (s == 0)
-                b[p] = o.dig[p][0];
-            else
+    for (int l = 0; l < S; ++l) {
+        constexpr uint32_t pos = MODE == kI8S8 ? 0x01020408u : 0x0102u, neg = MODE == kI8S8 ? 0xfffefcf8u : 0xfffeu;
+        weights<CT>(w, neg & (0xffu << (8 * l)), pos & (0xffu << (8 * l)), sel);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) b[p][i] = (int)(((uint32_t)u[p][i] >> s) & ((0xffu >> s) * 0x01010101u));
-        }
-        product<NT>(acc, w, b);
+        for (int p = 0; p < NT; ++p) b[p] = l == 0 ? x[p] : and8(x[p], ((0xffu << l) & 0xffu) * 0x01010101u);
+        product<CT, NT>(acc, w, b, o.index);
     }
 }
 
 // Position in the reduction: blocks run over (32-channel block, filter row, group of taps), the last fastest.
 struct KPos {
-    int cb, fh, fg, off;
+    int cb, fh, fg, off, off01;
 };
-
-template <int MODE, int NT>
-__device__ __forceinline__ void load_digits(const MfmaArgs &a, Operands<MODE, NT> &o, int from, int to, const KPos &k,
-                                            const uint32_t (&px)[NT])
-{
-    const int8_t *xb = a.x + k.off;
-#pragma unroll
-    for (int d = 0; d < Operands<MODE, NT>::D; ++d)
-        if (d >= from && d < to)
-#pragma unroll
-            for (int p = 0; p < NT; ++p) o.dig[p][d] = *(const v4i *)(xb + d * a.lay.dstride + px[p]);
-}
-template <int MODE, int NT>
-__device__ __forceinline__ void load_selectors(Operands<MODE, NT> &o, int from, int to, const int8_t *w, int kb)
-{
-    constexpr int G = Operands<MODE, NT>::G;
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-        if (g >= from && g < to)
-            o.sel[g] = *(const v4i *)(w + (kb * G + g) * 1024);
-}
-template <int MODE, int NT>
-__device__ __forceinline__ void load_block(const MfmaArgs &a, Operands<MODE, NT> &o, const int8_t *w, int kb,
-                                           const KPos &k, const uint32_t (&px)[NT])
-{
-    load_selectors<MODE, NT>(o, 0, 4, w, kb);
-    load_digits<MODE, NT>(a, o, 0, 3, k, px);
-}
 
 __device__ __forceinline__ void k_start(const MfmaArgs &a, KPos &k, int kb)
 {
@@ -447,19 +628,24 @@ __device__ __forceinline__ void k_start(const MfmaArgs &a, KPos &k, int kb)
     const int rest = kb - k.cb * per;
     k.fh = rest / a.fwg;
     k.fg = rest - k.fh * a.fwg;
-    k.off = k.cb * a.lay.cbstride + k.fh * a.lay.rstride + k.fg * a.tapstep;
+    const int row = k.cb * a.lay.cbstride + k.fh * a.lay.rstride;
+    k.off = row + k.fg * a.tapstep;
+    k.off01 = row + k.fg * a.tapstep01;
 }
 __device__ __forceinline__ void k_next(const MfmaArgs &a, KPos &k)
 {
     k.off += a.tapstep;
+    k.off01 += a.tapstep01;
     if (++k.fg == a.fwg) {
         k.fg = 0;
-        k.off += a.lay.rstride - a.fwg * a.tapstep;
+        int step = a.lay.rstride;
         if (++k.fh == a.FH) {
             k.fh = 0;
             ++k.cb;
-            k.off += a.lay.cbstride - a.FH * a.lay.rstride;
+            step += a.lay.cbstride - a.FH * a.lay.rstride;
         }
+        k.off += step - a.fwg * a.tapstep;
+        k.off01 += step - a.fwg * a.tapstep01;
     }
 }
 
@@ -476,17 +662,48 @@ __device__ __forceinline__ PixelAt pixel_at(const MfmaArgs &a, uint32_t p)
     return r;
 }
 
-// Whether the 16 bytes that a lane reads at tap (fh, fg) of channel block cb have digits d3 and d4.
-__device__ __forceinline__ bool has_high(const MfmaArgs &a, const PixelAt &at, int half, const KPos &k)
+// The flag of digits d3 and d4 for the 16 bytes that a lane reads at a block: where it lies, and whether they are inside
+// the image (some flag that is there if they are not, so that no load waits behind a branch).
+__device__ __forceinline__ const uint8_t *high_flag(const MfmaArgs &a, const PixelAt &at, int half, const KPos &k, bool &in)
 {
     const int ih = at.oh * a.sh + a.crop_h + k.fh;
-    if (!a.lay.tiles) return a.flags[((size_t)at.n * a.lay.Hp + ih) * a.lay.fy + k.cb / a.lay.cbf] != 0;
+    in = true;
+    if (!a.lay.tiles) return a.flags + ((size_t)at.n * a.lay.Hp + ih) * a.lay.fy + k.cb / a.lay.cbf;
     const int iw = at.ow * a.sw + a.crop_w + (a.lay.cp == 16 ? k.fg * 2 + half : k.fg) - a.lay.tpw;
     const int h = ih - a.lay.tph;
-    if ((unsigned)h >= (unsigned)a.lay.th || (unsigned)iw >= (unsigned)a.lay.tw) return false;
-    const uint32_t p = (at.n * a.lay.th + h) * a.lay.tw + iw;
     const int ch16 = a.lay.cp == 16 ? k.cb : k.cb * 2 + half;
-    return ch16 < a.lay.c16 && a.flags[(size_t)(p >> 5) * a.lay.c16 + ch16] != 0;
+    in = (unsigned)h < (unsigned)a.lay.th && (unsigned)iw < (unsigned)a.lay.tw && ch16 < a.lay.c16;
+    const uint32_t p = (at.n * a.lay.th + h) * a.lay.tw + iw;
+    return a.flags + (in ? (size_t)(p >> 5) * a.lay.c16 + ch16 : 0);
+}
+
+template <int MODE, int CT, int NT, bool HIGH>
+__device__ __forceinline__ void load_block(const MfmaArgs &a, Operands<MODE, CT, NT, HIGH> &o, const int8_t *w, int kb,
+                                           const KPos &k, const uint32_t (&px)[NT], const uint32_t (&px01)[NT],
+                                           const PixelAt (&at)[NT], int lane)
+{
+    const int wtile = a.KB * mode_block(MODE);
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const int8_t *wb = w + c * wtile + kb * mode_block(MODE);
+#pragma unroll
+        for (int g = 0; g < mode_sels(MODE); ++g) o.sel[c][g] = *(const v4i *)(wb + g * 1024 + lane * 16);
+        o.index[c] = *(const int *)(wb + mode_sels(MODE) * 1024 + lane * 4);
+    }
+#pragma unroll
+    for (int p = 0; p < NT; ++p) {
+        if constexpr (mode_i8(MODE)) {
+            o.lo[p][0] = *(const v4i *)(a.x + k.off + px[p]);
+        } else {
+            o.lo[p][0] = *(const v4i *)(a.x + k.off01 + px01[p]);
+            o.lo[p][1] = *(const v4i *)(a.x + (k.off01 + a.lay.piece01) + px01[p]);
+            o.d2[p] = *(const v4i *)(a.x + (k.off + 2 * a.lay.dstride) + px[p]);
+        }
+        if constexpr (HIGH) {
+            o.d3[p] = *(const v4i *)(a.x + (k.off + 3 * a.lay.dstride) + px[p]);
+            o.on[p] = *high_flag(a, at[p], lane >> 5, k, o.in[p]);
+        }
+    }
 }
 
 // Whether any input row of a tile has them (1), and digit d4 at that (2): p0 and p1 are its first and last pixel.
@@ -512,60 +729,150 @@ __device__ __forceinline__ int any_high(const MfmaArgs &a, uint32_t p0, uint32_t
     return (__any(any) ? 1 : 0) | (__any(any & 2) ? 2 : 0);
 }
 
-// Digits d3 and d4 of the rows that have any: what they add to the sums, modulo 2^32.  One pass over the reduction with
-// an accumulator per power of two; a digit that was not written is masked after its load, not branched around.
-template <int MODE, int NT>
-__device__ __forceinline__ void high_digits(const MfmaArgs &a, int32_t (*slot)[64], int lane, bool d4, const int8_t *w,
-                                            int kb0, int kb1, const uint32_t (&px)[NT], const uint32_t (&pix)[NT])
+// Digit d4 of the rows that have any (|x| past 2^27, saturated values as a rule): what it adds to the sums, modulo 2^32.  A
+// walk of its own over the reduction; a digit that was not written is masked after its load, not branched around.
+template <int MODE, int CT, int NT>
+__device__ __forceinline__ void digit4(const MfmaArgs &a, int32_t (*slot)[64], int lane, const int8_t *w, int kb0, int kb1,
+                                       const uint32_t (&px)[NT], const PixelAt (&at)[NT])
 {
-    constexpr int G = mode_groups(MODE), Q = MODE == kI32S15 ? 3 : 1;
-    v16i acc[4][NT] = {};   // 2^(7 i + 1)
-    PixelAt at[NT];
+    constexpr bool S15 = MODE == kI32S15;
+    v16i acc[3][CT][NT] = {};   // 2^22, 2^15, 2^8
+    int first[CT], second[CT];
 #pragma unroll
-    for (int p = 0; p < NT; ++p) at[p] = pixel_at(a, pix[p] < a.pixels ? pix[p] : a.pixels - 1);
+    for (int c = 0; c < CT; ++c) {
+        first[c] = (int)0x88888888u;
+        second[c] = (int)0xddddddddu;
+    }
     KPos k;
     k_start(a, k, kb0);
 #pragma unroll 1
     for (int kb = kb0; kb < kb1; ++kb, k_next(a, k)) {
-        v4i b[2][NT], sel[G], wv;
+        v8i b[NT];
+        v4i full[CT], lo[CT], hi[CT];
+        int index[CT];
+        const int wtile = a.KB * mode_block(MODE);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            const int8_t *wb = w + c * wtile + kb * mode_block(MODE);
+            lo[c] = *(const v4i *)(wb + lane * 16);
+            hi[c] = *(const v4i *)(wb + (mode_sels(MODE) - 1) * 1024 + lane * 16);
+            index[c] = *(const int *)(wb + mode_sels(MODE) * 1024 + lane * 4);
+        }
+        v4i d4[NT];
 #pragma unroll
         for (int p = 0; p < NT; ++p) {
-#pragma unroll
-            for (int d = 0; d < 2; ++d)
-                if (d == 0 || d4) b[d][p] = *(const v4i *)(a.x + k.off + (3 + d) * a.lay.dstride + px[p]);
+            bool in;
+            const uint8_t *flag = high_flag(a, at[p], lane >> 5, k, in);
+            d4[p] = *(const v4i *)(a.x + (k.off + 4 * a.lay.dstride) + px[p]);
+            d4[p] = and4(d4[p], *flag && in ? 0xffffffffu : 0u);
+            b[p] = pairs_with_zero(d4[p]);
         }
-#pragma unroll
-            for (int g = 0; g < G; ++g) sel[g] = *(const v4i *)(w + (kb * G + g) * 1024);
-#pragma unroll
-        for (int p = 0; p < NT; ++p) {
-            const uint32_t on = has_high(a, at[p], lane >> 5, k) ? 0xffffffffu : 0u;
-#pragma unroll
-            for (int d = 0; d < 2; ++d)
-                if (d == 0 || d4) b[d][p] = and4(b[d][p], on);
+        weights<CT>(full, kNegLo, kPosLo, lo);
+        if constexpr (mode_sels(MODE) == 2) {
+            v4i top[CT];
+            weights<CT>(top, kNegHi, kPosHi, hi);
+            both<CT>(full, full, top);
         }
+        if constexpr (S15) {
+            // q = 0 meets d4 at 2^22, q = 1 (second bytes) at 2^15, q = 2 at 2^8
+            product<CT, NT>(acc[0], full, b, index);
+            weights<CT>(lo, kNeg14, kPos14, hi);
+            product<CT, NT>(acc[2], lo, b, first);
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            if constexpr (G == 4) {
-                wv = q == 2 ? perm4(kNeg14, kPos14, sel[3])
-                            : or4(perm4(kNegLo, kPosLo, sel[q == 0 ? 0 : 2]), perm4(kNegHi, kPosHi, sel[q == 0 ? 1 : 3]));
-            } else {
-                wv = perm4(kNegLo, kPosLo, sel[0]);
-                if constexpr (G == 2) wv = or4(wv, perm4(kNegHi, kPosHi, sel[1]));
-            }
+            for (int p = 0; p < NT; ++p)
 #pragma unroll
-            for (int d = 0; d < 2; ++d)
-                if (d == 0 || d4) product<NT>(acc[3 + d - q - 1], wv, b[d]);
+                for (int i = 0; i < 8; ++i) b[p][i] = (int)((uint32_t)b[p][i] << 8);
+            product<CT, NT>(acc[1], full, b, index);
+        } else {
+            product<CT, NT>(acc[0], full, b, first);
         }
     }
 #pragma unroll
-    for (int p = 0; p < NT; ++p)
+    for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            uint32_t v = 0;
+        for (int p = 0; p < NT; ++p)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) v += (uint32_t)acc[c][p][i] << (7 * c + 1);
-            slot[p * 16 + i][lane] = (int32_t)v;
+            for (int i = 0; i < 16; ++i) {
+                uint32_t v = (uint32_t)acc[0][c][p][i] << 22;
+                if (S15) v += ((uint32_t)acc[1][c][p][i] << 15) + ((uint32_t)acc[2][c][p][i] << 8);
+                slot[(c * NT + p) * 16 + i][lane] = (int32_t)v;
+            }
+}
+
+// The sums of one wave's tile over blocks kb0 .. kb1 - 1.  Two sets of operands, the loads of a block in flight during the
+// products of the one before; with digit d3, whose sums leave no room for them (14 VGPRs went to scratch and back in every
+// block), one set, loaded again once the last operands of a block are formed and behind its last products.
+template <int MODE, int CT, int NT, bool HIGH>
+__device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT], const int8_t *w, int kb0, int kb1,
+                                         const uint32_t (&px)[NT], const uint32_t (&px01)[NT], const PixelAt (&at)[NT], int lane)
+{
+    typedef Operands<MODE, CT, NT, HIGH> Ops;
+    Sums<CT, NT, HIGH> t = {};
+    Ops o0;
+    KPos k;
+    k_start(a, k, kb0);
+    int kb = kb0;
+    const auto load = [&](Ops &o) { load_block<MODE, CT, NT, HIGH>(a, o, w, kb, k, px, px01, at, lane); };
+    const auto multiply = [&](const Ops &o, const auto &reload) {
+        if constexpr (mode_i8(MODE))
+            block_i8<MODE, CT, NT>(o, t.bits);
+        else if constexpr (MODE == kI32S15)
+            block_s15<CT, NT, HIGH>(o, t, reload);
+        else
+            block_s7<MODE, CT, NT, HIGH>(o, t, reload);
+    };
+    load(o0);
+    if constexpr (HIGH) {
+#pragma unroll 1
+        for (bool more = true; more;) {
+            multiply(o0, [&] {
+                more = kb + 1 < kb1;
+                if (more) {
+                    ++kb;
+                    k_next(a, k);
+                }
+                load(o0);   // the last block once more at the end: nobody waits for it
+                __builtin_amdgcn_sched_barrier(0);
+            });
         }
+    } else {
+        Ops o1;
+        const auto none = [] {};
+#pragma unroll 1
+        while (kb + 2 < kb1) {
+            ++kb;
+            k_next(a, k);
+            load(o1);
+            multiply(o0, none);
+            ++kb;
+            k_next(a, k);
+            load(o0);
+            multiply(o1, none);
+        }
+        if (kb + 1 < kb1) {
+            ++kb;
+            k_next(a, k);
+            load(o1);
+            multiply(o0, none);
+            multiply(o1, none);
+        } else {
+            multiply(o0, none);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int p = 0; p < NT; ++p)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if constexpr (mode_i8(MODE)) {
+                    total[c][p][i] = t.bits[c][p][i] >> (MODE == kI8S8 ? 3 : 1);
+                } else {
+                    uint32_t v = (uint32_t)(t.bits[c][p][i] >> 6) + ((uint32_t)t.d[0][c][p][i] << 1) + ((uint32_t)t.d[1][c][p][i] << 8);
+                    if constexpr (HIGH) v += (uint32_t)t.d[2][c][p][i] << 15;
+                    total[c][p][i] = (int)v;
+                }
+            }
 }
 
 // What follows the sums of eight channels (two groups of four, 8 apart) at one pixel: the per-channel constants, then the
@@ -587,7 +894,7 @@ __device__ __forceinline__ void load_tail(const MfmaArgs &a, ChannelTail &t, int
 }
 struct OutAt {
     size_t i;         // of channel 0 in y / out / residual
-    size_t j;         // of channel 0 in q
+    size_t j, j01;    // of channel 0 in q; of its digits 0 and 1
     uint32_t p;
     bool in;
 };
@@ -599,6 +906,7 @@ __device__ __forceinline__ OutAt out_at(const MfmaArgs &a, const PixelAt &at, ui
     o.p = p;
     o.j = a.qflags ? (size_t)(at.n * a.qHp + at.oh + a.qph) * a.qlay.rstride + (at.ow + a.qpw) * a.qlay.cp
                    : ((size_t)at.n * a.N * a.qHp + at.oh + a.qph) * a.qWp + at.ow + a.qpw;
+    o.j01 = (size_t)(at.n * a.qHp + at.oh + a.qph) * a.qlay.rstride + (at.ow + a.qpw) * a.qlay.px01;
     return o;
 }
 // Eight values per lane (channels ch0 + 8 g + 0..3, ch0 = 16 u + 4 (lane >> 5)) into the next layer's operand layout: the
@@ -622,7 +930,7 @@ __device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t 
         if (o.in && cb < L.cb) *(uint2 *)q = uint2{x[0], x[1]};
         return;
     }
-    uint32_t w[kDigits][2] = {};
+    uint32_t w[kDigits][2] = {}, e[2][2];
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
 #pragma unroll
@@ -630,19 +938,29 @@ __device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t 
             int32_t dg[kDigits];
             digits_of(qv[g * 4 + i], dg);
 #pragma unroll
-            for (int d = 0; d < kDigits; ++d) w[d][g] |= ((uint32_t)dg[d] & 255u) << (8 * i);
+            for (int d = 2; d < kDigits; ++d) w[d][g] |= ((uint32_t)dg[d] & 255u) << (8 * i);
         }
+        e[g][0] = pair01(qv[g * 4]) | pair01(qv[g * 4 + 1]) << 16;
+        e[g][1] = pair01(qv[g * 4 + 2]) | pair01(qv[g * 4 + 3]) << 16;
     }
     const uint32_t high4 = w[4][0] | w[4][1], high = w[3][0] | w[3][1] | high4;
     const bool any = __any(o.in && high != 0);
     const bool any4 = __any(o.in && high4 != 0);
     if (u16 < L.c16 && (threadIdx.x & 63) == 0 && o.in)
         a.qflags[(size_t)(o.p >> 5) * L.c16 + u16] = any4 ? 3 : any ? 1 : 0;
+    const bool mine = o.in && cb < L.cb;
+    {
+        // eight channels of pairs: a 32-channel block keeps them by their place in its halves, others in a row
+        const auto x = __builtin_amdgcn_permlane32_swap(e[0][0], e[1][0], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(e[0][1], e[1][1], false, false);
+        int8_t *q01 = (int8_t *)a.q + o.j01 + (size_t)cb * L.cbstride + (L.cp == 32 ? (u16 & 1) * 16 : 0) + half * L.piece01;
+        if (mine) *(v4i *)q01 = v4i{(int)x[0], (int)y[0], (int)x[1], (int)y[1]};
+    }
 #pragma unroll
-    for (int d = 0; d < kDigits; ++d) {
+    for (int d = 2; d < kDigits; ++d) {
         if (d >= 3 && !any) break;
         const auto x = __builtin_amdgcn_permlane32_swap(w[d][0], w[d][1], false, false);
-        if (o.in && cb < L.cb) *(uint2 *)(q + d * L.dstride) = uint2{x[0], x[1]};
+        if (mine) *(uint2 *)(q + d * L.dstride) = uint2{x[0], x[1]};
     }
 }
 
@@ -727,13 +1045,13 @@ __device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail 
     }
 }
 
-// Four or eight waves per workgroup; a wave owns 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
+// Four or eight waves per workgroup; a wave owns CT * 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
 // parts of a tile lie in one workgroup and meet in LDS).  No operand passes through LDS: activations and selectors are
 // fragments in memory already, each a contiguous KiB.
-template <int MODE, int NT, int WAVES>
+template <int MODE, int CT, int NT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) void mfma_kernel(MfmaArgs a)
 {
-    __shared__ int32_t part[WAVES][NT * 16][64];
+    __shared__ int32_t part[WAVES][CT * NT * 16][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroups are dealt to the eight XCDs in turn: give each XCD neighbouring tiles
@@ -744,97 +1062,42 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
     const int ct = (int)(wg - pt * a.ctiles);
     const int kpart = wave % a.ks, t = wave / a.ks;
     const int pw = WAVES / a.ks / a.tc;   // pixel tiles per workgroup
-    const int c0 = (ct * a.tc + t % a.tc) * 32;
+    const int c0 = (ct * a.tc + t % a.tc) * (CT * 32);
     const uint32_t p0 = ((uint32_t)pt * pw + t / a.tc) * (NT * 32);
     const int kb0 = (int)((long)a.KB * kpart / a.ks), kb1 = (int)((long)a.KB * (kpart + 1) / a.ks);
 
-    constexpr int G = mode_groups(MODE);
-    const int wtile = a.KB * G * 1024;
     const bool live = c0 < a.N && p0 < a.pixels;
-    uint32_t pix[NT], px[NT];
+    uint32_t pix[NT], px[NT], px01[NT];
+    PixelAt at[NT];
 #pragma unroll
     for (int p = 0; p < NT; ++p) {
         pix[p] = p0 + p * 32 + (lane & 31);
-        const uint32_t clamped = pix[p] < a.pixels ? pix[p] : a.pixels - 1;
-        const PixelAt at = pixel_at(a, clamped);
-        px[p] = (at.n * a.lay.Hp + at.oh * a.sh + a.crop_h) * a.lay.rstride + (at.ow * a.sw + a.crop_w) * a.lay.cp + (lane >> 5) * 16;
+        at[p] = pixel_at(a, pix[p] < a.pixels ? pix[p] : a.pixels - 1);
+        const uint32_t row = (at[p].n * a.lay.Hp + at[p].oh * a.sh + a.crop_h) * a.lay.rstride, col = at[p].ow * a.sw + a.crop_w;
+        px[p] = row + col * a.lay.cp + (lane >> 5) * 16;
+        px01[p] = row + col * a.lay.px01 + (lane >> 5) * a.lay.half01;
     }
-    v16i total[NT] = {};
+    v16i total[CT][NT] = {};
     if (live && kb0 < kb1) {
-        const int8_t *wl = a.blob + (size_t)(c0 >> 5) * wtile + lane * 16;
-        int high = 0;
-        if constexpr (!mode_i8(MODE)) {
-            const uint32_t last = p0 + NT * 32 - 1;
-            high = any_high(a, p0, last < a.pixels ? last : a.pixels - 1, lane);
-            if (high) high_digits<MODE, NT>(a, part[wave], lane, (high & 2) != 0, wl, kb0, kb1, px, pix);
-        }
-        v16i acc[NT] = {};
-        Operands<MODE, NT> o0;
-        KPos k;
-        k_start(a, k, kb0);
-        int kb = kb0;
-        load_block<MODE, NT>(a, o0, wl, kb, k, px);
+        const int8_t *w = a.blob + (size_t)(c0 >> 5) * (a.KB * mode_block(MODE));
         if constexpr (mode_i8(MODE)) {
-            Operands<MODE, NT> o1;
-            while (true) {
-                if (kb + 1 < kb1) {
-                    k_next(a, k);
-                    load_block<MODE, NT>(a, o1, wl, kb + 1, k, px);
-                }
-                block_i8<MODE, NT>(o0, acc);
-                if (++kb >= kb1) break;
-                if (kb + 1 < kb1) {
-                    k_next(a, k);
-                    load_block<MODE, NT>(a, o0, wl, kb + 1, k, px);
-                }
-                block_i8<MODE, NT>(o1, acc);
-                if (++kb >= kb1) break;
-            }
-#pragma unroll
-            for (int p = 0; p < NT; ++p) total[p] = acc[p];
+            contract<MODE, CT, NT, false>(a, total, w, kb0, kb1, px, px01, at, lane);
         } else {
-            // every operand is loaded again as soon as its last product is issued: the loads of the next block are
-            // in flight during this one's remaining products, with one set of registers
-            v16i a0[NT] = {}, a1[NT] = {};
-            while (true) {
-                v4i w;
-                const bool more = kb + 1 < kb1;
-                if (more) k_next(a, k);
-                const int kn = more ? kb + 1 : kb;
-                bit_products<MODE, NT>(o0, 0, acc, w);
-                if constexpr (MODE == kI32S15) {
-                    load_selectors<MODE, NT>(o0, 0, 2, wl, kn);
-                    load_digits<MODE, NT>(a, o0, 0, 1, k, px);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                digit_product<MODE, NT>(o0, 1, a0, w);
-                digit_product<MODE, NT>(o0, 2, a1, w);
-                if constexpr (MODE == kI32S15) {
-                    bit_products<MODE, NT>(o0, 1, acc, w);
-                    load_selectors<MODE, NT>(o0, 2, 3, wl, kn);
-                    load_digits<MODE, NT>(a, o0, 1, 2, k, px);
-                    __builtin_amdgcn_sched_barrier(0);
-                    digit_product<MODE, NT>(o0, 2, a0, w);
-                    w = perm4(kNeg14, kPos14, o0.sel[3]);
-                    digit_product<MODE, NT>(o0, 2, acc, w);
-                    load_selectors<MODE, NT>(o0, 3, 4, wl, kn);
-                    load_digits<MODE, NT>(a, o0, 2, 3, k, px);
-                } else {
-                    load_block<MODE, NT>(a, o0, wl, kn, k, px);
-                }
-                if (!more) break;
-                ++kb;
+            const uint32_t last = p0 + NT * 32 - 1;
+            const int high = any_high(a, p0, last < a.pixels ? last : a.pixels - 1, lane);
+            if (high) {
+                if (high & 2) digit4<MODE, CT, NT>(a, part[wave], lane, w, kb0, kb1, px, at);
+                contract<MODE, CT, NT, true>(a, total, w, kb0, kb1, px, px01, at, lane);
+                if (high & 2)
+#pragma unroll
+                    for (int c = 0; c < CT; ++c)
+#pragma unroll
+                        for (int p = 0; p < NT; ++p)
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) total[c][p][i] += part[wave][(c * NT + p) * 16 + i][lane];
+            } else {
+                contract<MODE, CT, NT, false>(a, total, w, kb0, kb1, px, px01, at, lane);
             }
-#pragma unroll
-            for (int p = 0; p < NT; ++p)
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    total[p][i] = (acc[p][i] >> 6) + (int)((uint32_t)a0[p][i] << 1) + (int)((uint32_t)a1[p][i] << 8);
-            if (high)
-#pragma unroll
-                for (int p = 0; p < NT; ++p)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) total[p][i] += part[wave][p * 16 + i][lane];
         }
     }
     const int chl = c0 + 4 * (lane >> 5);
@@ -842,38 +1105,40 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
         if (!live) return;
         // units of 16 channels x 32 pixels; every residual is on its way before the first value is stored
         OutAt o[NT];
-        float res[NT * 2][8];
+        float res[CT * 2 * NT][8];
 #pragma unroll
-        for (int p = 0; p < NT; ++p) o[p] = out_at(a, pixel_at(a, pix[p]), pix[p]);
+        for (int p = 0; p < NT; ++p) o[p] = out_at(a, at[p], pix[p]);
         if (a.residual)
 #pragma unroll
-            for (int u = 0; u < NT * 2; ++u)
-                load_residual(a, res[u], chl + u / NT * 16, o[u % NT]);
+            for (int u = 0; u < CT * 2 * NT; ++u) load_residual(a, res[u], chl + u / NT * 16, o[u % NT]);
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
+        for (int c = 0; c < CT * 2; ++c) {
             ChannelTail tl;
             load_tail(a, tl, chl + c * 16);
 #pragma unroll
             for (int p = 0; p < NT; ++p) {
                 int32_t v[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = total[p][c * 8 + i];
+                for (int i = 0; i < 8; ++i) v[i] = total[c >> 1][p][(c & 1) * 8 + i];
                 store_tail(a, tl, v, res[c * NT + p], chl + c * 16, o[p]);
             }
         }
         return;
     }
 #pragma unroll
-    for (int p = 0; p < NT; ++p)
+    for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) part[wave][p * 16 + i][lane] = total[p][i];
+        for (int p = 0; p < NT; ++p)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) part[wave][(c * NT + p) * 16 + i][lane] = total[c][p][i];
     __syncthreads();
     if (!live) return;
     // the ks waves of a tile share its epilogue, in halves of 32 x 32 values
-    const int units = NT * 2 > a.ks ? NT * 2 / a.ks : 1;
-    for (int u = kpart * units; u < (kpart + 1) * units && u < NT * 2; ++u) {
-        const int ch = chl + (u & 1) * 16;
-        const uint32_t pp = p0 + (u >> 1) * 32 + (lane & 31);
+    constexpr int all = CT * NT * 2;
+    const int units = all > a.ks ? all / a.ks : 1;
+    for (int u = kpart * units; u < (kpart + 1) * units && u < all; ++u) {
+        const int ch = chl + (u >> 1) / NT * 32 + (u & 1) * 16;
+        const uint32_t pp = p0 + (u >> 1) % NT * 32 + (lane & 31);
         const OutAt o = out_at(a, pixel_at(a, pp), pp);
         ChannelTail tl;
         float res[8];
@@ -917,31 +1182,41 @@ __global__ __launch_bounds__(256) void mfma_border_kernel(Q *__restrict__ q, lon
 // For buffers that no caller zeroed once (first use, and captured graphs, which own theirs).
 __global__ __launch_bounds__(256) void mfma_operand_border_kernel(int8_t *__restrict__ q, MfmaX lay, int ph, int pw)
 {
-    const int pixel = lay.cp >> 4, side = pw * pixel, segments = lay.cb * lay.digits;
+    // digits 0 and 1 of 16-channel blocks lie side by side: one segment of two pieces a pixel in place of two of one
+    const bool joined = lay.digits > 1 && lay.cp == 16;
+    const int segments = lay.cb * lay.digits, pieces = lay.dstride >> 4, wide = lay.cp >> 4;
     for (long row = blockIdx.x; row < lay.rows; row += gridDim.x) {
         v4i *r = (v4i *)(q + (size_t)row * lay.rstride);
         const int h = (int)(row % lay.Hp);
         if (h < ph || h >= lay.Hp - ph) {
             for (int i = threadIdx.x; i < lay.rstride >> 4; i += 256) r[i] = v4i{};
         } else {
+            const int side = pw * wide;
             for (int i = threadIdx.x; i < segments * 2 * side; i += 256) {
                 const int segment = i / (2 * side), j = i - segment * 2 * side;
-                r[segment * (lay.dstride >> 4) + (j < side ? j : (lay.Wp - 2 * pw) * pixel + j)] = v4i{};
+                const int digit = segment % lay.digits;
+                if (joined && digit < 2) {
+                    // digit 0's share clears the left columns, digit 1's the right ones
+                    const int base = (segment - digit) * pieces;
+                    r[base + (digit == 0 ? j : 2 * (lay.Wp - pw) + j)] = v4i{};
+                } else {
+                    r[segment * pieces + (j < side ? j : (lay.Wp - 2 * pw) * wide + j)] = v4i{};
+                }
             }
         }
     }
 }
 
-template <int MODE, int NT, int WAVES>
+template <int MODE, int CT, int NT, int WAVES>
 static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
 {
-    const int ctiles32 = ceil_div(a.N, 32);
+    const int ctiles = ceil_div(a.N, CT * 32);
     a.ks = ks;
-    a.tc = (WAVES / a.ks >= 2 && ctiles32 > 1) ? 2 : 1;
-    a.ctiles = ceil_div(ctiles32, a.tc);
+    a.tc = CT == 1 && WAVES / a.ks >= 2 && ctiles > 1 ? 2 : 1;
+    a.ctiles = ceil_div(ctiles, a.tc);
     a.ptiles = ceil_div((int)a.pixels, NT * 32 * (WAVES / a.ks / a.tc));
     a.by_ctiles = fast_div((uint32_t)a.ctiles);
-    hipLaunchKernelGGL((mfma_kernel<MODE, NT, WAVES>), dim3((unsigned)(a.ctiles * a.ptiles)), dim3(WAVES * 64), 0, st, a);
+    hipLaunchKernelGGL((mfma_kernel<MODE, CT, NT, WAVES>), dim3((unsigned)(a.ctiles * a.ptiles)), dim3(WAVES * 64), 0, st, a);
     return launch_status();
 }
 
@@ -970,13 +1245,15 @@ template <int MODE>
 static int launch_mfma(MfmaArgs &a, hipStream_t st)
 {
     const long waves = (long)device_cus() * (mode_i8(MODE) ? 12 : 8);   // wave slots
-    const long tiles = (long)ceil_div(a.N, 32) * ceil_div((int)a.pixels, 64);
+    const bool pair = a.N > 32;
+    const long tiles = pair ? (long)ceil_div(a.N, 64) * ceil_div((int)a.pixels, 32) : (long)ceil_div((int)a.pixels, 64);
     // Few tiles and a long reduction leave the chip idle behind one wave's serial chain: half the tile, and the
     // reduction in eight parts (one image, 512 channels of 7 x 7, 16 tiles: 34 -> 22 us; 256 of 14 x 14, 32 tiles:
     // 21 -> 16; 112 tiles: 38 -> 26).  Past a sixteenth of the slots the extra epilogues cost more than the shorter
     // chain gives (200 tiles: 23.6 -> 25.1; 392 tiles: 18.6 -> 23), as they do on short reductions (18 blocks: even).
-    if (tiles <= waves / 16 && a.KB >= 32) return launch_tiles<MODE, 1, 8>(a, 8, st);
-    return launch_tiles<MODE, 2, 4>(a, reduction_parts(tiles, waves, a.KB, mode_i8(MODE)), st);
+    if (tiles <= waves / 16 && a.KB >= 32) return launch_tiles<MODE, 1, 1, 8>(a, 8, st);
+    const int ks = reduction_parts(tiles, waves, a.KB, mode_i8(MODE));
+    return pair ? launch_tiles<MODE, 2, 1, 4>(a, ks, st) : launch_tiles<MODE, 1, 2, 4>(a, ks, st);
 }
 
 template <int SRC, bool I8>
@@ -998,7 +1275,7 @@ static int launch_prepare(const PrepArgs &a, bool matrix, hipStream_t st)
 static int mode_of(int max_shift, int x_bytes)
 {
     if (max_shift < 0 || max_shift > 31) return -1;
-    if (x_bytes == 1) return max_shift <= 2 ? kI8S3 : max_shift <= 3 ? kI8S4 : kI8S8;
+    if (x_bytes == 1) return max_shift <= 3 ? kI8S4 : kI8S8;
     if (x_bytes != 4) return -1;
     return max_shift <= 3 ? kI32S4 : max_shift <= 6 ? kI32S7 : max_shift <= 14 ? kI32S15 : -1;
 }
@@ -1019,7 +1296,7 @@ DS_EXPORT size_t ds_mfma_weight_bytes(int N, int C, int FH, int FW, int max_shif
     if (mode < 0 || N <= 0 || C <= 0 || FH <= 0 || FW <= 0) return 0;
     if ((double)C * FH * FW > kMfmaMaxK) return 0;
     const MfmaGeom g = mfma_geom(N, C, FH, FW);
-    if ((double)g.kb * mode_groups(mode) * 1024 > (double)(1u << 30)) return 0;   // 32-bit offsets within a tile
+    if ((double)g.kb * mode_block(mode) > (double)(1u << 30)) return 0;   // 32-bit offsets within a tile
     return mfma_blob_corr(g, mode) + (size_t)g.ntiles * 32 * 4;
 }
 
@@ -1033,12 +1310,12 @@ DS_EXPORT int ds_mfma_tile_weights_i32(const int32_t *w_ref, void *blob, int N, 
     const MfmaGeom g = mfma_geom(N, C, FH, FW);
     hipStream_t st = (hipStream_t)stream;
     const long total = (long)g.ntiles * g.kb * 64;
-    hipLaunchKernelGGL(mfma_tile_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, w_ref, (v4i *)blob, N, C,
+    hipLaunchKernelGGL(mfma_tile_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, w_ref, (int8_t *)blob, N, C,
                        FH, FW, bits, mode, g.cp, g.cb, g.taps, g.fwg, g.kb, total);
     int rc = launch_status();
     if (rc != DS_OK || !mode_i8(mode)) return rc;
     hipLaunchKernelGGL(mfma_corr_kernel, dim3((unsigned)(g.ntiles * 32)), dim3(64), 0, st, w_ref,
-                       (int32_t *)((char *)blob + mfma_blob_corr(g, mode)), N, C * FH * FW, bits);
+                       (int32_t *)((char *)blob + mfma_blob_corr(g, mode)), N, C * FH * FW, bits, mode);
     return launch_status();
 }
 
@@ -1138,6 +1415,7 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     a.FH = FH;
     a.fwg = g.fwg;
     a.tapstep = g.taps * g.cp;
+    a.tapstep01 = g.taps * a.lay.px01;
     a.sh = sh;
     a.sw = sw;
     a.crop_h = crop_h;
@@ -1189,7 +1467,6 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     case kI32S7: return launch_mfma<kI32S7>(a, st);
     case kI32S4: return launch_mfma<kI32S4>(a, st);
     case kI8S8: return launch_mfma<kI8S8>(a, st);
-    case kI8S4: return launch_mfma<kI8S4>(a, st);
-    default: return launch_mfma<kI8S3>(a, st);
+    default: return launch_mfma<kI8S4>(a, st);
     }
 }

@@ -1070,10 +1070,16 @@ class Prepared:
         cp = 16 if C <= 16 and self.filter != (1, 1) else 32
         cb, digits = (C + cp - 1) // cp, 1 if self.x_bytes == 1 else 5
         size = Nb * Hp * cb * digits * Wp * cp
-        d = self.data[:size].view(torch.int8).view(Nb, Hp, cb, digits, Wp, cp).permute(3, 0, 2, 5, 1, 4)
-        d = d.reshape(digits, Nb, cb * cp, Hp, Wp)[:, :, :C]
+        d = self.data[:size].view(torch.int8).view(Nb, Hp, cb, digits, Wp, cp)
         if self.x_bytes == 1:
-            return d[0].contiguous()
+            return d[:, :, :, 0].permute(0, 2, 4, 1, 3).reshape(Nb, cb * cp, Hp, Wp)[:, :C].contiguous()
+        # digits 0 and 1 in pairs; 32-channel blocks keep the first and second eight channels of their halves apart
+        if cp == 32:
+            low = d[:, :, :, :2].reshape(Nb, Hp, cb, 2, Wp, 2, 8, 2).permute(7, 0, 2, 5, 3, 6, 1, 4)
+        else:
+            low = d[:, :, :, :2].reshape(Nb, Hp, cb, Wp, cp, 2).permute(5, 0, 2, 4, 1, 3)
+        low = low.reshape(2, Nb, cb * cp, Hp, Wp)
+        d = torch.cat([low, d[:, :, :, 2:].permute(3, 0, 2, 5, 1, 4).reshape(3, Nb, cb * cp, Hp, Wp)])[:, :, :C]
         # digits 3 and 4 count only where the 32 pixels x 16 channels that were written together have a flag
         ph, pw = self.written_by_conv
         H, W, c16 = Hp - 2 * ph, Wp - 2 * pw, (C + 15) // 16

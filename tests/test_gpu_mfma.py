@@ -261,3 +261,23 @@ def test_epilogues_of_large_launches(oracle, rng, parts, x_bytes, C, O, pixels, 
         assert torch.equal(out, f) and torch.equal(handed.padded(), q)
         only, handed = kernels.mfma_conv2d(*args, ((1, 1), I, F, dtype, (3, 3)), False)
         assert only is None and torch.equal(handed.padded(), q)
+
+
+@pytest.mark.parametrize("top,x_bytes", [(14, 4), (6, 4), (3, 4), (14, 1), (3, 1)], ids=lambda v: str(v))
+@pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5])
+def test_short_reductions_of_every_digit(oracle, rng, top, x_bytes, blocks):
+    """The two-set loop over odd and even numbers of blocks and the one-set loop of digit 3: channels at the edges of one
+    and two tiles of 32, activations with no digit past d2, with d3 alone, with d4, and with all of them by row."""
+    for N in (31, 32, 33, 64, 65):
+        C = blocks * 32 - (N & 1) * 5
+        s, sign, cw = _weights(rng, (N, C, 1, 1), top, ternary=N == 33)
+        bias = rng.integers(-2 ** 20, 2 ** 20, size=N).astype(np.int32)
+        for spread in (1 << 20, 1 << 26, 2 ** 31 - 1) if x_bytes == 4 else (128,):
+            x = rng.integers(-spread, spread, size=(2, C, 5, 9)).astype(np.int32 if x_bytes == 4 else np.int8)
+            if spread == 2 ** 31 - 1:
+                x[:, :, 1] >>= 5
+                x[:, :, 2:4] >>= 12
+            prepared, blob, at = kernels.mfma_route(_dev(x), 0, cw, N, (1, 1), x_bytes)
+            got = kernels.mfma_conv2d(prepared, blob, _dev(bias), N, (1, 1), 1, at)
+            want = oracle.conv2d(x.astype(np.int32), -s.astype(np.int32), sign.astype(np.int32), bias, (1, 1))
+            np.testing.assert_array_equal(got.cpu().numpy(), want)
