@@ -875,21 +875,38 @@ __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT
             }
 }
 
-// What follows the sums of eight channels (two groups of four, 8 apart) at one pixel: the per-channel constants, then the
-// residuals, are all asked for before the first value is stored (one wait each, not one per value).
+// What follows the sums of eight channels (two groups of four, 8 apart) at one pixel.  The per-channel constants of a
+// workgroup's channels lie in LDS: read from memory by every wave they were 96 loads of one word per 64 channels, which
+// bounded short reductions (8-bit activations, 64 -> 256 channels, 1 x 1, 128 images of 56 x 56: 146 -> 97 us, with
+// residual and float result 245 -> 195, the rate of a copy; 256 -> 64: 58 -> 45).
 constexpr int kUnit = 8;
+template <int CHANNELS>
+struct ChannelTails {
+    int32_t add[CHANNELS];
+    float scale[CHANNELS], shift[CHANNELS];
+};
+template <int CHANNELS>
+__device__ __forceinline__ void stage_tails(const MfmaArgs &a, ChannelTails<CHANNELS> &t, int first, int count)
+{
+    const int i = threadIdx.x, ch = first + i, c = ch < a.N ? ch : a.N - 1;
+    if (i >= count) return;
+    t.add[i] = (a.bias ? a.bias[c] : 0) - (a.corr ? a.corr[c] : 0);
+    t.scale[i] = a.scale ? a.scale[c] : 1.0f;
+    t.shift[i] = a.shift ? a.shift[c] : 0.0f;
+}
 struct ChannelTail {
     int32_t add[kUnit];
     float scale[kUnit], shift[kUnit];
 };
-__device__ __forceinline__ void load_tail(const MfmaArgs &a, ChannelTail &t, int ch0)
+template <int CHANNELS>
+__device__ __forceinline__ void load_tail(const ChannelTails<CHANNELS> &t, ChannelTail &tl, int at)
 {
 #pragma unroll
     for (int i = 0; i < kUnit; ++i) {
-        const int ch = ch0 + 8 * (i >> 2) + (i & 3), c = ch < a.N ? ch : a.N - 1;
-        t.add[i] = (a.bias ? a.bias[c] : 0) - (a.corr ? a.corr[c] : 0);
-        t.scale[i] = a.scale ? a.scale[c] : 1.0f;
-        t.shift[i] = a.shift ? a.shift[c] : 0.0f;
+        const int c = at + 8 * (i >> 2) + (i & 3);
+        tl.add[i] = t.add[c];
+        tl.scale[i] = t.scale[c];
+        tl.shift[i] = t.shift[c];
     }
 }
 struct OutAt {
@@ -1024,11 +1041,17 @@ __device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail 
     }
     if (a.relu)
 #pragma unroll
-        for (int i = 0; i < kUnit; ++i) f[i] = f[i] > 0.0f ? f[i] : 0.0f;
+        for (int i = 0; i < kUnit; ++i) f[i] = fmaxf(f[i], 0.0f);
     if (a.out) store_channels(a.out + o.i, f, ch0, a.ostride_c, a.N, o.in);
     if (!a.q) return;
     int32_t qv[kUnit];
-    quantize_all(f, qv, a.qspec);
+    if (a.relu && a.qspec.I != 1) {
+        // neither negative nor NaN: the conversion's truncation is the floor, the lower bound is met
+#pragma unroll
+        for (int i = 0; i < kUnit; ++i) qv[i] = f2i_sat(fminf(f[i] * a.qspec.scale, a.qspec.hi));
+    } else {
+        quantize_all(f, qv, a.qspec);
+    }
     if (a.qflags) {
         if ((ch0 & ~15) + 2 * kUnit > a.N)
 #pragma unroll
@@ -1052,6 +1075,7 @@ template <int MODE, int CT, int NT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) void mfma_kernel(MfmaArgs a)
 {
     __shared__ int32_t part[WAVES][CT * NT * 16][64];
+    __shared__ ChannelTails<CT * 64> tails;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroups are dealt to the eight XCDs in turn: give each XCD neighbouring tiles
@@ -1077,6 +1101,9 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
         px[p] = row + col * a.lay.cp + (lane >> 5) * 16;
         px01[p] = row + col * a.lay.px01 + (lane >> 5) * a.lay.half01;
     }
+    const int tail0 = t % a.tc * (CT * 32) + 4 * (lane >> 5);   // the lane's first channel there
+    stage_tails(a, tails, ct * a.tc * (CT * 32), a.tc * (CT * 32));
+    __syncthreads();
     v16i total[CT][NT] = {};
     if (live && kb0 < kb1) {
         const int8_t *w = a.blob + (size_t)(c0 >> 5) * (a.KB * mode_block(MODE));
@@ -1114,7 +1141,7 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
 #pragma unroll
         for (int c = 0; c < CT * 2; ++c) {
             ChannelTail tl;
-            load_tail(a, tl, chl + c * 16);
+            load_tail(tails, tl, tail0 + c * 16);
 #pragma unroll
             for (int p = 0; p < NT; ++p) {
                 int32_t v[8];
@@ -1142,7 +1169,7 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
         const OutAt o = out_at(a, pixel_at(a, pp), pp);
         ChannelTail tl;
         float res[8];
-        load_tail(a, tl, ch);
+        load_tail(tails, tl, tail0 + ch - chl);
         if (a.residual) load_residual(a, res, ch, o);
         int32_t v[8];
 #pragma unroll
