@@ -177,10 +177,9 @@ inline MfmaX mfma_x(int Nb, int C, int Hp, int Wp, const MfmaGeom &g, bool i8)
     x.half01 = g.cp == 32 ? 16 : 32;
     x.piece01 = g.cp == 32 ? x.dstride : 16;
     x.rows = (long)Nb * Hp;
-    // enough workgroups to fill the chip: a row's channel blocks are shared out over up to eight of them
-    int fy = 1;
-    while (fy < 8 && x.rows * fy < 1024 && g.cb >= 2 * fy) fy *= 2;
-    x.cbf = ceil_div(g.cb, fy);
+    // as many channel blocks of a row per workgroup as its threads take at a go (mfma_prepare_kernel)
+    const int per_block = Wp * (g.cp == 32 ? 2 : 1);
+    x.cbf = per_block >= 256 ? 1 : 256 / per_block < g.cb ? 256 / per_block : g.cb;
     x.fy = ceil_div(g.cb, x.cbf);
     // a block of several taps may read up to 32 bytes past the last pixel
     x.planes = align_up((size_t)x.rows * x.rstride + 64, 256);
@@ -199,15 +198,31 @@ struct PrepArgs {
     int C, H, W, ph, pw;
     int M, K;        // rows of a matrix: image n holds rows 64 n .. 64 n + 63, C = K
     int vec;         // a matrix whose rows can be read four values at a time
+    int per, rpw;    // items of a row's part, rows per workgroup
+    FastDiv by_per, by_wp, by_hp;
     QuantSpec spec;
 };
 
-template <int SRC>
-__device__ __forceinline__ int32_t prep_value(const void *x, size_t i, const QuantSpec &spec)
+template <int CH>
+__device__ __forceinline__ void quantize_many(const int32_t (&raw)[CH], int32_t (&v)[CH], const QuantSpec &spec)
 {
-    if (SRC == kSrcF32) return quantize_one(((const float *)x)[i], spec);
-    if (SRC == kSrcI32) return ((const int32_t *)x)[i];
-    return ((const int8_t *)x)[i];
+    // one look at the mode, not one per value
+    QuantSpec s = spec;
+    if (spec.mode == DS_Q_CAST) {
+        s.mode = DS_Q_CAST;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) v[i] = quantize_one(__int_as_float(raw[i]), s);
+    } else if (spec.I == 1) {
+        s.mode = DS_Q_ROUND_TO_FIXED;
+        s.I = 1;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) v[i] = quantize_one(__int_as_float(raw[i]), s);
+    } else {
+        s.mode = DS_Q_ROUND_TO_FIXED;
+        s.I = 2;   // the bounds are in lo and hi
+#pragma unroll
+        for (int i = 0; i < CH; ++i) v[i] = quantize_one(__int_as_float(raw[i]), s);
+    }
 }
 
 __device__ __forceinline__ void digits_of(int32_t v, int32_t d[kDigits])
@@ -224,99 +239,163 @@ __device__ __forceinline__ void digits_of(int32_t v, int32_t d[kDigits])
 // Digits 0 and 1 of a value in two bytes.
 __device__ __forceinline__ uint32_t pair01(int32_t v) { return ((uint32_t)v & 127u) | (((uint32_t)v << 1) & 0x7f00u); }
 
-// Workgroup (row, part): CH channels of one pixel per thread and step, two threads side by side for the halves of a
-// 32-channel block, so that loads run along the row and stores are contiguous.  Bound by memory: 4 bytes read and 3
-// written per element (5 where a digit d3 or d4 of the row is not zero: a second sweep writes those).
+// CH channels of one pixel: what a thread of mfma_prepare_kernel converts.  All values are asked for before the first is
+// converted; outside the image some value that is there, so that no load waits behind a branch.
+template <int SRC, bool MATRIX, int CH>
+__device__ __forceinline__ void prep_values(const PrepArgs &a, int n, int h, int wp, int c0, int32_t (&v)[CH])
+{
+    int32_t raw[CH];
+    bool in;
+    if (MATRIX) {
+        const int m = n * 64 + wp;
+        in = m < a.M;
+        const size_t base = (size_t)(in ? m : 0) * a.K;
+        if (a.vec) {
+            // rows and base aligned: four values per load
+#pragma unroll
+            for (int q = 0; q < CH / 4; ++q) {
+                const int c = c0 + 4 * q;
+                const v4i r = *(const v4i *)((const int32_t *)a.x + base + (c < a.K ? c : 0));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) raw[4 * q + i] = r[i];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < CH; ++i)
+                raw[i] = ((const int32_t *)a.x)[base + (c0 + i < a.K ? c0 + i : 0)];
+        }
+    } else {
+        const int w = wp - a.pw;
+        in = (unsigned)h < (unsigned)a.H && (unsigned)w < (unsigned)a.W;
+        const size_t plane = (size_t)a.H * a.W;
+        const size_t base = (size_t)n * a.C * plane + (in ? (size_t)h * a.W + w : 0);
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const size_t at = base + (c0 + i < a.C ? c0 + i : a.C - 1) * plane;
+            raw[i] = SRC == kSrcI8 ? ((const int8_t *)a.x)[at] : ((const int32_t *)a.x)[at];
+        }
+    }
+    if (SRC == kSrcF32)
+        quantize_many<CH>(raw, v, a.spec);
+    else
+#pragma unroll
+        for (int i = 0; i < CH; ++i) v[i] = raw[i];
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+        if (!in || c0 + i >= a.C) v[i] = 0;
+}
+
+// Words to an address of any four bytes, in one store.
+template <int N>
+__device__ __forceinline__ void store_words(int8_t *o, const uint32_t (&w)[N])
+{
+    typedef uint32_t words __attribute__((ext_vector_type(N), aligned(4)));
+    words v;
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = w[i];
+    *(words *)o = v;
+}
+
+// A thread converts CH channels of one pixel, two threads side by side for the halves of a 32-channel block, so that loads
+// run along the row and stores are contiguous; a workgroup takes the blocks of one part of a row, or of several rows where
+// they are short.  Bound by memory: 4 bytes read and 3 written per element (5 where a digit d3 or d4 of the row's part is not
+// zero: they wait in registers until the workgroup knows; rows of more than 256 items are read a second time for them).
+// Before, every value was loaded behind its own bounds check and waited for, and a workgroup had one row: us then and now,
+// with the ordinary range and, second, with d3 in every row: 64 images of 64 x 56 x 56, 3 x 3: 33 and 21 (4.4 TB/s), 55 and
+// 23; 256 of 16 x 32 x 32: 42 and 9, 61 and 10; 128 of 256 x 56 x 56, unpadded: 295 and 152 (4.7 TB/s).
 template <int SRC, bool I8, bool MATRIX, int CH>
 __global__ __launch_bounds__(256) void mfma_prepare_kernel(PrepArgs a)
 {
+    __shared__ int seen[256];   // of a row: 1, d3 or d4; 2, d4
     const MfmaX &L = a.lay;
-    const int row = blockIdx.x, part = blockIdx.y;
-    const int n = row / L.Hp, hp = row - n * L.Hp, h = hp - a.ph;
+    const int part = blockIdx.y;
     const int halves = CH == 16 && L.cp == 32 ? 2 : 1;
     const int cb0 = part * L.cbf, cb1 = cb0 + L.cbf < L.cb ? cb0 + L.cbf : L.cb;
-    const int items = (cb1 - cb0) * L.Wp * halves;
+    const int items = (cb1 - cb0) * L.Wp * halves;   // of a row
+    const int r = a.rpw == 1 ? 0 : (int)div_by(threadIdx.x, a.by_per);
+    const int first = (int)threadIdx.x - r * a.per;
+    const long at = (long)blockIdx.x * a.rpw + r;
+    const bool on = r < a.rpw && at < L.rows && first < items;
+    const uint32_t row = (uint32_t)(on ? at : 0);
+    const int n = (int)div_by(row, a.by_hp), h = (int)row - n * L.Hp - a.ph;
     int8_t *dst = a.dst + (size_t)row * L.rstride;
-    const bool row_in = MATRIX || (unsigned)h < (unsigned)a.H;
-    int high = 0;
-    for (int pass = 0; pass < 2; ++pass) {
-        for (int t = threadIdx.x; t < items; t += 256) {
-            const int half = halves == 2 ? t & 1 : 0;
-            const int tw = halves == 2 ? t >> 1 : t;
-            const int cbi = tw / L.Wp, wp = tw - cbi * L.Wp, cb = cb0 + cbi;
-            const int c0 = cb * L.cp + half * CH;
-            int32_t v[CH];
-            if (MATRIX) {
-                const int m = n * 64 + wp;
-                const size_t base = (size_t)m * a.K + c0;
-                if (a.vec && m < a.M && c0 + CH <= a.K) {
-                    // rows and base aligned: four values per load
+    constexpr int Q = CH / 4;
+
+    // Item t: its digits 0 to 2 (or its 8-bit values) stored if `low`; the others left in w3, w4, to be stored at `o`.
+    const auto convert = [&](int t, bool low, int8_t *&o, uint32_t (&w3)[Q], uint32_t (&w4)[Q]) {
+        const int half = halves == 2 ? t & 1 : 0;
+        const uint32_t tw = halves == 2 ? t >> 1 : t;
+        const int cbi = (int)div_by(tw, a.by_wp), wp = (int)tw - cbi * L.Wp, cb = cb0 + cbi;
+        int32_t v[CH];
+        prep_values<SRC, MATRIX, CH>(a, n, h, wp, cb * L.cp + half * CH, v);
+        o = dst + (size_t)cb * L.cbstride + wp * L.cp + half * CH;
+        uint32_t w2[Q];
 #pragma unroll
-                    for (int q = 0; q < CH / 4; ++q) {
-                        const v4i r = *(const v4i *)((const int32_t *)a.x + base + 4 * q);
+        for (int q = 0; q < Q; ++q) {
+            w2[q] = w3[q] = w4[q] = 0;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            v[4 * q + i] = SRC == kSrcF32 ? quantize_one(__int_as_float(r[i]), a.spec) : r[i];
-                    }
-                } else
-#pragma unroll
-                for (int i = 0; i < CH; ++i)
-                    v[i] = (m < a.M && c0 + i < a.K) ? prep_value<SRC>(a.x, base + i, a.spec) : 0;
-            } else {
-                const int w = wp - a.pw;
-                const bool in = row_in && (unsigned)w < (unsigned)a.W;
-                const size_t base = ((size_t)n * a.C + c0) * a.H * a.W + (size_t)h * a.W + w;
-                const size_t plane = (size_t)a.H * a.W;
-#pragma unroll
-                for (int i = 0; i < CH; ++i)
-                    v[i] = (in && c0 + i < a.C) ? prep_value<SRC>(a.x, base + i * plane, a.spec) : 0;
-            }
-            int8_t *o = dst + (size_t)cb * L.cbstride + wp * L.cp + half * CH;
-            int8_t *o01 = dst + (size_t)cb * L.cbstride + wp * L.px01 + half * L.half01;
-            constexpr int D = I8 ? 1 : kDigits;
-            uint32_t words[D][CH / 4], pairs[I8 ? 1 : CH / 2];
-#pragma unroll
-            for (int q = 0; q < CH / 4; ++q) {
-#pragma unroll
-                for (int d = 0; d < D; ++d) words[d][q] = 0;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    int32_t dg[kDigits];
-                    if (I8)
-                        dg[0] = v[q * 4 + i];
-                    else
-                        digits_of(v[q * 4 + i], dg);
-#pragma unroll
-                    for (int d = 0; d < D; ++d)
-                        if (I8 || d >= 2) words[d][q] |= ((uint32_t)dg[d] & 255u) << (8 * i);
+            for (int i = 0; i < 4; ++i) {
+                if (I8) {
+                    w2[q] |= ((uint32_t)v[q * 4 + i] & 255u) << (8 * i);
+                    continue;
                 }
-                if (!I8) {
-                    pairs[q * 2] = pair01(v[q * 4]) | pair01(v[q * 4 + 1]) << 16;
-                    pairs[q * 2 + 1] = pair01(v[q * 4 + 2]) | pair01(v[q * 4 + 3]) << 16;
-                }
-            }
-            if (!I8 && pass == 0) {
-                // eight channels a piece
-#pragma unroll
-                for (int q = 0; q < CH / 2; ++q) ((uint32_t *)(o01 + (q >> 2) * L.piece01))[q & 3] = pairs[q];
-            }
-            const int lo = I8 ? 0 : pass == 0 ? 2 : 3, hi = I8 ? 1 : pass == 0 ? 3 : 5;
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                if (d >= lo && d < hi)
-#pragma unroll
-                    for (int q = 0; q < CH / 4; ++q) ((uint32_t *)(o + (size_t)d * L.dstride))[q] = words[d][q];
-                if (d >= 3)
-#pragma unroll
-                    for (int q = 0; q < CH / 4; ++q) high |= words[d][q] != 0 ? (d == 3 ? 1 : 2) : 0;
+                int32_t dg[kDigits];
+                digits_of(v[q * 4 + i], dg);
+                w2[q] |= ((uint32_t)dg[2] & 255u) << (8 * i);
+                w3[q] |= ((uint32_t)dg[3] & 255u) << (8 * i);
+                w4[q] |= ((uint32_t)dg[4] & 255u) << (8 * i);
             }
         }
-        if (I8) return;
-        if (pass == 0) {
-            const int high4 = __syncthreads_or(high & 2);
-            high = __syncthreads_or(high);
-            if (threadIdx.x == 0) a.flags[(size_t)row * L.fy + part] = high4 ? 3 : high ? 1 : 0;
-            if (!high) return;
+        if (low) {
+            store_words<Q>(o + (I8 ? 0 : 2) * L.dstride, w2);
+            if (!I8) {
+                // digits 0 and 1 in pairs, eight channels a piece
+                int8_t *o01 = dst + (size_t)cb * L.cbstride + wp * L.px01 + half * L.half01;
+                constexpr int P = CH < 8 ? CH / 2 : 4;
+#pragma unroll
+                for (int p = 0; p < CH / 2 / P; ++p) {
+                    uint32_t pairs[P];
+#pragma unroll
+                    for (int i = 0; i < P; ++i) pairs[i] = pair01(v[(p * P + i) * 2]) | pair01(v[(p * P + i) * 2 + 1]) << 16;
+                    store_words<P>(o01 + p * L.piece01, pairs);
+                }
+            }
+        }
+        int high = 0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) high |= w4[q] ? 3 : w3[q] ? 1 : 0;
+        return high;
+    };
+    const auto store_high = [&](int8_t *o, const uint32_t (&w3)[Q], const uint32_t (&w4)[Q]) {
+        store_words<Q>(o + 3 * L.dstride, w3);
+        store_words<Q>(o + 4 * L.dstride, w4);
+    };
+
+    if (!I8) {
+        if ((int)threadIdx.x < a.rpw) seen[threadIdx.x] = 0;
+        __syncthreads();
+    }
+    int8_t *o = nullptr;
+    uint32_t w3[Q], w4[Q];
+    int high = 0;
+    if (a.per <= 256) {
+        if (on) high = convert(first, true, o, w3, w4);
+    } else {
+        for (int t = first; t < items; t += 256) high |= convert(t, true, o, w3, w4);
+    }
+    if (I8) return;
+    if (high) atomicOr(&seen[r], high);
+    __syncthreads();
+    if (!on) return;
+    const int any = seen[r];
+    if (first == 0) a.flags[(size_t)row * L.fy + part] = (uint8_t)any;
+    if (!any) return;
+    if (a.per <= 256) {
+        store_high(o, w3, w4);
+    } else {
+        for (int t = first; t < items; t += 256) {
+            convert(t, false, o, w3, w4);
+            store_high(o, w3, w4);
         }
     }
 }
@@ -1286,7 +1365,7 @@ static int launch_mfma(MfmaArgs &a, hipStream_t st)
 template <int SRC, bool I8>
 static int launch_prepare(const PrepArgs &a, bool matrix, hipStream_t st)
 {
-    const dim3 grid((unsigned)a.lay.rows, (unsigned)a.lay.fy);
+    const dim3 grid((unsigned)((a.lay.rows + a.rpw - 1) / a.rpw), (unsigned)a.lay.fy);
     if (matrix)
         hipLaunchKernelGGL((mfma_prepare_kernel<SRC, I8, true, 16>), grid, dim3(256), 0, st, a);
     else if (a.lay.cp >= 16)
@@ -1387,6 +1466,11 @@ DS_EXPORT int ds_mfma_prepare(const void *x, int source, void *dst, int Nb, int 
     a.M = matrix_rows;
     a.K = C;
     a.vec = matrix && source != kSrcI8 && C % 4 == 0 && (uintptr_t)x % 16 == 0;
+    a.per = a.lay.cbf * Wp * (a.lay.cp == 32 ? 2 : 1);
+    a.rpw = a.per >= 256 ? 1 : 256 / a.per;
+    a.by_per = fast_div((uint32_t)a.per);
+    a.by_wp = fast_div((uint32_t)Wp);
+    a.by_hp = fast_div((uint32_t)Hp);
     a.spec = make_spec(I, F, mode);
     hipStream_t st = (hipStream_t)stream;
     if (source == kSrcI8) return launch_prepare<kSrcI8, true>(a, matrix, st);

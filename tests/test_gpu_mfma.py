@@ -281,3 +281,37 @@ def test_short_reductions_of_every_digit(oracle, rng, top, x_bytes, blocks):
             got = kernels.mfma_conv2d(prepared, blob, _dev(bias), N, (1, 1), 1, at)
             want = oracle.conv2d(x.astype(np.int32), -s.astype(np.int32), sign.astype(np.int32), bias, (1, 1))
             np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+# (Nb, C, H, W, k): rows of one to several workgroup's shares -- many short rows in one workgroup, the last one not full,
+# parts of 32-channel blocks that fill 256 threads or just miss them, rows that take two goes
+LAYOUTS = [(3, 16, 7, 5, 3), (1, 3, 9, 83, 3), (2, 40, 3, 128, 1), (1, 33, 2, 129, 1), (1, 100, 3, 41, 1), (1, 8, 2, 255, 3), (1, 8, 2, 254, 3),
+           (1, 2, 2, 600, 3), (1, 70, 2, 300, 1)]
+
+
+@pytest.mark.parametrize("x_bytes", [4, 1])
+@pytest.mark.parametrize("Nb,C,H,W,k", LAYOUTS, ids=lambda v: str(v))
+def test_the_layout_pass_at_the_edges_of_its_workgroups(oracle, rng, x_bytes, Nb, C, H, W, k):
+    """Rows with digit d3 alone, with d4 and with neither side by side, from float, int32 or int8 images."""
+    s, sign, cw = _weights(rng, (33, C, k, k), 6, ternary=False)
+    x = _activations(rng, (Nb, C, H, W), x_bytes, 2 ** 31 - 1)
+    if x_bytes == 4:
+        x[:, :, 0] >>= 12
+        x[..., W // 3:, 1] >>= 5
+    pad = k // 2
+    xp = np.pad(x.astype(np.int32), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+    want = oracle.conv2d(xp, -s.astype(np.int32), sign.astype(np.int32), None, (1, 1))
+    F = 16 if x_bytes == 4 else 5
+    exact = np.float32(x) == x       # values that a float holds
+    for source in (x, np.where(exact, x, 0).astype(np.float32) / np.float32(2.0 ** F)):
+        if source.dtype == np.float32 and not exact.all():
+            xf = np.pad(np.where(exact, x, 0).astype(np.int32), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+            xf = np.clip(xf, -2 ** 31, (2 ** 15 - 1) * 2 ** 16)
+            want = oracle.conv2d(xf, -s.astype(np.int32), sign.astype(np.int32), None, (1, 1))
+        I, Fb = (16, 16) if x_bytes == 4 else (3, 5)
+        route = kernels.mfma_route(_dev(source), (pad, pad), cw, 33, (k, k), x_bytes, I, Fb)
+        got = kernels.mfma_conv2d(route[0], route[1], None, 33, (k, k), 1, route[2])
+        if source.dtype == np.float32 and x_bytes == 1:
+            xf = np.pad(np.clip(x.astype(np.int32), -128, 96), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+            want = oracle.conv2d(xf, -s.astype(np.int32), sign.astype(np.int32), None, (1, 1))
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
