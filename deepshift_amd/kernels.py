@@ -1004,13 +1004,19 @@ def mfma_route(x, padding, conc_weight, O, kernel_size, x_bytes, integer_bits=16
     return None if prepared is None else (prepared, blob, max_shift)
 
 
+def _too_few_terms(O, C, FH, FW, x_bytes):
+    """Layers of int32 activations that the two-instruction kernel keeps: at most 16 channels on both sides, of which half
+    of every 32-channel tile is padding, and fewer than 64 terms.  Us there and on the matrix cores, 256 images of 32 x 32 as
+    modules: 4 -> 16 channels, 3 x 3 (36 terms) 29, 27, as ``conv2d`` 26, 25, 32 images of 112 x 112 40, 39 and 35, 37; 1 -> 16, 5 x 5
+    (25) 27, 32; 8 -> 8, 3 x 3 (72) 37, 30; 16 -> 16, 3 x 3 (144) 57, 38, and one layer after another 52, 28."""
+    return x_bytes == 4 and O <= 16 and C <= 16 and C * FH * FW < 64
+
+
 def _mfma_conv_serves(Nb, C, Hp, Wp, O, kernel_size, stride, x_bytes=4):
-    """Whether the output has anything in it, its offsets fit, and the matrix cores are the faster place: with int32
-    activations and at most 16 channels on both sides, half of every 32-channel tile is padding (256 x 16 x 32 x 32 -> 16:
-    74 us against 54 on the two-instruction kernel, 17 -> 17 channels are even)."""
+    """Whether the output has anything in it, its offsets fit, and the matrix cores are the faster place."""
     FH, FW = _pair(kernel_size)
     sh, sw = _pair(stride)
-    if Hp < FH or Wp < FW or sh <= 0 or sw <= 0 or O == 0 or (x_bytes == 4 and O <= 16 and C <= 16):
+    if Hp < FH or Wp < FW or sh <= 0 or sw <= 0 or O == 0 or _too_few_terms(O, C, FH, FW, x_bytes):
         return False
     pixels = Nb * ((Hp - FH) // sh + 1) * ((Wp - FW) // sw + 1)
     return 0 < pixels <= 10 ** 9 and pixels * O <= 8 * 10 ** 9
@@ -1040,7 +1046,7 @@ def mfma_takes_prepared(conc_weight, O, C, kernel_size, x_bytes):
     kernels have a form for it, and its pixels are whole 16-byte pieces there."""
     FH, FW = _pair(kernel_size)
     max_shift = mfma_shift(conc_weight, x_bytes)
-    if max_shift is None or (x_bytes == 4 and O <= 16 and C <= 16) or (C <= 8 and FH * FW > 1):
+    if max_shift is None or _too_few_terms(O, C, FH, FW, x_bytes) or (C <= 8 and FH * FW > 1):
         return False
     return _lib.lib().ds_mfma_weight_bytes(O, C, FH, FW, max_shift, x_bytes) != 0
 

@@ -315,3 +315,31 @@ def test_the_layout_pass_at_the_edges_of_its_workgroups(oracle, rng, x_bytes, Nb
             xf = np.pad(np.clip(x.astype(np.int32), -128, 96), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
             want = oracle.conv2d(xf, -s.astype(np.int32), sign.astype(np.int32), None, (1, 1))
         np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("C,O,k", [(16, 16, 3), (16, 4, 2), (8, 16, 3), (7, 16, 3), (3, 16, 5), (16, 16, 1), (15, 16, 2)])
+def test_few_channels_agree_on_both_kernels(rng, C, O, k):
+    """Layers of at most 16 channels around the number of terms from which the matrix cores take them: as the public entry
+    points route them against the general kernels, and handed from layer to layer."""
+    s, sign, cw = _weights(rng, (O, C, k, k), 14, ternary=False)
+    x = _dev(_activations(rng, (5, C, 9, 11), 4, 2 ** 31 - 1))
+    got = kernels.conv2d(x, _dev(s), _dev(sign), None, cw, 1, k // 2)
+    xp = torch.nn.functional.pad(x, (k // 2,) * 4)
+    want = kernels.conv2d_tiled(xp, kernels._tiled_of(cw, O, C, k, k), None, O, (k, k), 1, kernels.kernel_bits(cw))
+    assert torch.equal(got, want)
+    serves = kernels._mfma_conv_serves(5, C, xp.shape[2], xp.shape[3], O, (k, k), 1)
+    assert serves == (C * k * k >= 64)
+    assert kernels.mfma_takes_prepared(cw, O, C, (k, k), 4) == (serves and C > 8)
+    if not serves or C <= 8:
+        return
+    _, _, before = _weights(rng, (C, 24, 3, 3), 14, ternary=False)
+    prepared, blob, top = kernels.mfma_route(_dev(_activations(rng, (5, 24, 9, 11), 4, 1 << 18)), 1, before, C, (3, 3), 4)
+    scale, shift = torch.full((C,), 40.0, device=DEV), torch.randn(C, device=DEV)
+    args = (prepared, blob, None, C, (3, 3), (1, 1), top, 0, 16, scale, shift, None, False)
+    pads = (k // 2, k // 2)
+    padded = kernels.mfma_conv2d(*args, (pads, 16, 16, torch.int32), False)[1]
+    handed = kernels.mfma_conv2d(*args, (pads, 16, 16, torch.int32, (k, k)), False)[1]
+    assert torch.equal(handed.padded(), padded)
+    blob = kernels._mfma_of(cw, 14, 4, O, C, k, k)
+    assert torch.equal(kernels.mfma_conv2d(handed, blob, None, O, (k, k), 1, 14),
+                       kernels.conv2d_tiled(padded, kernels._tiled_of(cw, O, C, k, k), None, O, (k, k), 1, kernels.kernel_bits(cw)))
