@@ -90,6 +90,8 @@ SIGNATURES = {
     "ds_mfma_input_bytes": (_size, [_c_int] * 7),
     "ds_mfma_prepare": (_c_int, [_ptr, _c_int, _ptr] + [_c_int] * 13 + [_ptr]),
     "ds_mfma_conv2d": (_c_int, [_ptr] * 9 + [_c_int] * 28 + [_ptr]),
+    "ds_mfma_pool_serves": (_c_int, [_c_int] * 5),
+    "ds_mfma_conv2d_pool": (_c_int, [_ptr] * 7 + [_c_int] * 28 + [_ptr]),
     "ds_quantize_f32_i32": (_c_int, [_ptr, _ptr, _c_i64, _c_int, _c_int, _c_int, _ptr]),
     "ds_quantize_pad_f32_i32": (_c_int, [_ptr, _ptr] + [_c_int] * 9 + [_ptr]),
     "ds_quantize_transpose_f32_i32": (_c_int, [_ptr, _ptr] + [_c_int] * 6 + [_ptr]),

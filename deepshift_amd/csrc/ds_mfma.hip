@@ -424,6 +424,7 @@ struct MfmaArgs {
     MfmaX qlay;                 // q in the operand layout of the next layer (qlay.planes != 0)
     uint8_t *qflags;
     int relu, q_bytes, qHp, qWp, qph, qpw;
+    int qscattered;             // a unit's pixels are not 32 in a row of the output: its flags are shared with other units
     float inv;
     QuantSpec qspec;
     FastDiv by_image, by_row, by_ctiles;
@@ -569,15 +570,15 @@ __device__ __forceinline__ void block_s15(const Operands<kI32S15, CT, NT, HIGH> 
         }
     }
     both<CT>(wlo, wlo, w);
+    int index[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) index[c] = o.index[c];
 #pragma unroll
     for (int p = 0; p < NT; ++p) b[p] = pairs12(x01[p], o.d2[p]);
     product<CT, NT>(t.d[0], wlo, b, o.index);
     weights<CT>(w, kNeg14, kPos14, shi);
     if constexpr (HIGH) {
         v8i b3[NT];
-        int index[CT];
-#pragma unroll
-        for (int c = 0; c < CT; ++c) index[c] = o.index[c];
 #pragma unroll
         for (int p = 0; p < NT; ++p) {
             const v4i d3 = and4(o.d3[p], o.in[p] && o.on[p] ? 0xffffffffu : 0u);
@@ -592,8 +593,9 @@ __device__ __forceinline__ void block_s15(const Operands<kI32S15, CT, NT, HIGH> 
     } else {
 #pragma unroll
         for (int p = 0; p < NT; ++p) b[p] = pairs_with_zero(o.d2[p]);
-        product<CT, NT>(t.d[1], wlo, b, o.index);
-        product<CT, NT>(t.bits, w, b, o.index);
+        reload();
+        product<CT, NT>(t.d[1], wlo, b, index);
+        product<CT, NT>(t.bits, w, b, index);
     }
 }
 
@@ -661,6 +663,8 @@ __device__ __forceinline__ void block_s7(const Operands<MODE, CT, NT, HIGH> &o, 
         for (int p = 0; p < NT; ++p) b3[p] = pairs_with_zero(and4(o.d3[p], o.in[p] && o.on[p] ? 0xffffffffu : 0u));
         reload();
         product<CT, NT>(t.d[2], full, b3, first);
+    } else {
+        reload();
     }
     product<CT, NT>(t.d[0], full, b, first);
     product<CT, NT>(t.d[1], full, b, second);
@@ -881,7 +885,7 @@ __device__ __forceinline__ void digit4(const MfmaArgs &a, int32_t (*slot)[64], i
 // The sums of one wave's tile over blocks kb0 .. kb1 - 1.  Two sets of operands, the loads of a block in flight during the
 // products of the one before; with digit d3, whose sums leave no room for them (14 VGPRs went to scratch and back in every
 // block), one set, loaded again once the last operands of a block are formed and behind its last products.
-template <int MODE, int CT, int NT, bool HIGH>
+template <int MODE, int CT, int NT, bool HIGH, bool ONE_SET = HIGH>
 __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT], const int8_t *w, int kb0, int kb1,
                                          const uint32_t (&px)[NT], const uint32_t (&px01)[NT], const PixelAt (&at)[NT], int lane)
 {
@@ -901,9 +905,10 @@ __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT
             block_s7<MODE, CT, NT, HIGH>(o, t, reload);
     };
     load(o0);
-    if constexpr (HIGH) {
+    if constexpr (ONE_SET) {
+        bool more;
 #pragma unroll 1
-        for (bool more = true; more;) {
+        do {
             multiply(o0, [&] {
                 more = kb + 1 < kb1;
                 if (more) {
@@ -913,7 +918,7 @@ __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT
                 load(o0);   // the last block once more at the end: nobody waits for it
                 __builtin_amdgcn_sched_barrier(0);
             });
-        }
+        } while (more);
     } else {
         Ops o1;
         const auto none = [] {};
@@ -1040,10 +1045,19 @@ __device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t 
         e[g][1] = pair01(qv[g * 4 + 2]) | pair01(qv[g * 4 + 3]) << 16;
     }
     const uint32_t high4 = w[4][0] | w[4][1], high = w[3][0] | w[3][1] | high4;
-    const bool any = __any(o.in && high != 0);
-    const bool any4 = __any(o.in && high4 != 0);
-    if (u16 < L.c16 && (threadIdx.x & 63) == 0 && o.in)
-        a.qflags[(size_t)(o.p >> 5) * L.c16 + u16] = any4 ? 3 : any ? 1 : 0;
+    bool any = true;
+    if (a.qscattered) {
+        // d3 and d4 are always there; flags, zero before the launch, gather what their 32 pixels have
+        if (u16 < L.c16 && o.in && high) {
+            const size_t at = (size_t)(o.p >> 5) * L.c16 + u16;
+            atomicOr((uint32_t *)a.qflags + (at >> 2), (high4 ? 3u : 1u) << (8 * (at & 3)));
+        }
+    } else {
+        any = __any(o.in && high != 0);
+        const bool any4 = __any(o.in && high4 != 0);
+        if (u16 < L.c16 && (threadIdx.x & 63) == 0 && o.in)
+            a.qflags[(size_t)(o.p >> 5) * L.c16 + u16] = any4 ? 3 : any ? 1 : 0;
+    }
     const bool mine = o.in && cb < L.cb;
     {
         // eight channels of pairs: a 32-channel block keeps them by their place in its halves, others in a row
@@ -1260,6 +1274,162 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
     }
 }
 
+// A convolution with a max pooling behind it (a ResNet's stem).
+struct MfmaPool {
+    int pk, ps, pp;             // window, stride, padding
+    int POH, POW;               // pooled rows and columns
+    int th, tw, PH, PW;         // of a workgroup: its pooled rows and columns, and the convolution's that they take
+    int tiles_h, tiles_w;
+    FastDiv by_pw, by_tw, by_tiles_w, by_tiles_h;
+};
+constexpr int kPoolPixels = 256, kPoolStride = 68;   // words per pixel: 64 channels, and 4 to spread rows over the banks
+
+// A workgroup forms the sums of 64 channels x a rectangle of pixels (32 at a time per wave, as mfma_kernel does), leaves them
+// in LDS and pools from there, so that the sums are neither written nor read: with a pass of its own they were, 4 bytes each,
+// and the padded result was laid out by a third.  Rectangles overlap by pk - ps rows and columns: 15 x 17 pixels give 7 x 8
+// windows of 3 x 3 with stride 2, an eighth of the products done twice.  The affine step is monotonic in the sum (every
+// rounding is), so a window's value is that of its largest sum, or smallest where the scale is negative, which are kept
+// inverted.  us, layer, pooling pass and layout pass before, and this: 64 images of 224 x 224, 3 -> 64 channels, 7 x 7, shifts to
+// 14: 162 + 68 + 23 and 170; 8-bit activations 87 + 61 + 17 and 88; 128 images, shifts to 2: 164 + 110 + 54 (two layers read it)
+// and 123.  What bounds it: vector instructions, about 700 for 32 pixels x 64 channels beside 56 or 140 products.
+template <int MODE, bool K3>
+__global__ __launch_bounds__(256, 2) void mfma_pool_kernel(MfmaArgs a, MfmaPool m)
+{
+    __shared__ int32_t sums[kPoolPixels * kPoolStride];
+    __shared__ ChannelTails<64> tails;
+    __shared__ int32_t flips[64];   // all ones where the smallest sum counts
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t wg = blockIdx.x;
+    const uint32_t per = gridDim.x >> 3;
+    if (wg < per * 8) wg = (wg & 7) * per + (wg >> 3);
+    uint32_t rest = div_by_uniform(wg, a.by_ctiles);
+    const int c0 = (int)(wg - rest * a.ctiles) * 64;
+    const uint32_t tiles = div_by_uniform(rest, m.by_tiles_w);
+    const int w0 = (int)(rest - tiles * m.tiles_w) * m.tw;
+    const uint32_t n = div_by_uniform(tiles, m.by_tiles_h);
+    const int h0 = (int)(tiles - n * m.tiles_h) * m.th;
+    const int r0 = h0 * m.ps - m.pp, q0 = w0 * m.ps - m.pp;   // the rectangle's first row and column
+    const int pixels = m.PH * m.PW;
+    stage_tails(a, tails, c0, 64);
+    if (threadIdx.x < 64) flips[threadIdx.x] = tails.scale[threadIdx.x] < 0.0f ? -1 : 0;
+    __syncthreads();
+    const int8_t *w = a.blob + (size_t)(c0 >> 5) * (a.KB * mode_block(MODE));
+    int high = 0;
+    if constexpr (!mode_i8(MODE)) {
+        const int first = r0 < 0 ? 0 : r0, last = r0 + m.PH < a.OH ? r0 + m.PH - 1 : a.OH - 1;
+        high = any_high(a, (n * a.OH + first) * a.OW, (n * a.OH + last) * a.OW + a.OW - 1, lane);
+    }
+    for (int t = wave; t * 32 < pixels; t += 4) {
+        const int pos = t * 32 + (lane & 31);
+        const uint32_t clamped = pos < pixels ? pos : pixels - 1, r = div_by(clamped, m.by_pw);
+        int oh = r0 + (int)r, ow = q0 + (int)(clamped - r * m.PW);
+        oh = oh < 0 ? 0 : oh < a.OH ? oh : a.OH - 1;
+        ow = ow < 0 ? 0 : ow < a.OW ? ow : a.OW - 1;
+        const PixelAt at[1] = {{n, (uint32_t)oh, (uint32_t)ow}};
+        const uint32_t row = (n * a.lay.Hp + oh * a.sh + a.crop_h) * a.lay.rstride, col = ow * a.sw + a.crop_w;
+        const uint32_t px[1] = {row + col * a.lay.cp + (lane >> 5) * 16};
+        const uint32_t px01[1] = {row + col * a.lay.px01 + (lane >> 5) * a.lay.half01};
+        v16i total[2][1];
+        int32_t (*slot)[64] = (int32_t (*)[64])(sums + t * 32 * kPoolStride);   // this tile's own place, before its sums
+        if constexpr (mode_i8(MODE)) {
+            contract<MODE, 2, 1, false>(a, total, w, 0, a.KB, px, px01, at, lane);
+        } else if (high) {
+            if (high & 2) digit4<MODE, 2, 1>(a, slot, lane, w, 0, a.KB, px, at);
+            contract<MODE, 2, 1, true>(a, total, w, 0, a.KB, px, px01, at, lane);
+            if (high & 2)
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) total[c][0][i] += slot[c * 16 + i][lane];
+        } else {
+            contract<MODE, 2, 1, false, true>(a, total, w, 0, a.KB, px, px01, at, lane);
+        }
+        asm volatile("" ::: "memory");   // the constants are read here, not kept in 96 registers through the loop
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int ch = u * 16 + 4 * (lane >> 5);
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                v4i v = *(const v4i *)(tails.add + ch + 8 * g);
+                const v4i flip = *(const v4i *)(flips + ch + 8 * g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = (total[u >> 1][0][(u & 1) * 8 + g * 4 + i] + v[i]) ^ flip[i];
+                *(v4i *)(sums + pos * kPoolStride + ch + 8 * g) = v;
+            }
+        }
+    }
+    __syncthreads();
+    // a wave pools 16 of the channels
+    const int ch = wave * 16 + 4 * (lane >> 5), windows = m.th * m.tw;
+    if (c0 + wave * 16 >= a.N) return;
+    ChannelTail tl;
+    load_tail(tails, tl, ch);
+    for (int g = 0; g < windows; g += 32) {
+        const int idx = g + (lane & 31), clamped = idx < windows ? idx : windows - 1;
+        const int i0 = (int)div_by((uint32_t)clamped, m.by_tw), j0 = clamped - i0 * m.tw;
+        const int oh = h0 + i0, ow = w0 + j0;
+        int32_t best[kUnit];
+#pragma unroll
+        for (int i = 0; i < kUnit; ++i) best[i] = INT32_MIN;
+        // rows and columns outside the image: the nearest one inside, which is in the window too
+        const auto row = [&](int i) {
+            const int r = oh * m.ps - m.pp + i;
+            return ((r < 0 ? 0 : r < a.OH ? r : a.OH - 1) - r0) * m.PW;
+        };
+        const auto column = [&](int j) {
+            const int c = ow * m.ps - m.pp + j;
+            return (c < 0 ? 0 : c < a.OW ? c : a.OW - 1) - q0;
+        };
+        const auto take = [&](int at) {
+            const v4i v0 = *(const v4i *)(sums + at * kPoolStride + ch), v1 = *(const v4i *)(sums + at * kPoolStride + ch + 8);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                best[k] = v0[k] > best[k] ? v0[k] : best[k];
+                best[4 + k] = v1[k] > best[4 + k] ? v1[k] : best[4 + k];
+            }
+        };
+        if constexpr (K3) {
+            int c[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) c[j] = column(j);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const int r = row(i);
+#pragma unroll
+                for (int j = 0; j < 3; ++j) take(r + c[j]);
+            }
+        } else {
+            for (int i = 0; i < m.pk; ++i) {
+                const int r = row(i);
+                for (int j = 0; j < m.pk; ++j) take(r + column(j));
+            }
+        }
+        OutAt o;
+        o.in = idx < windows && oh < m.POH && ow < m.POW;
+        o.p = o.in ? (n * m.POH + oh) * m.POW + ow : 0;
+        o.i = (size_t)n * a.ostride_n + (oh * m.POW + ow);
+        const size_t qrow = (size_t)(n * a.qHp + oh + a.qph);
+        o.j = a.qflags ? qrow * a.qlay.rstride + (ow + a.qpw) * a.qlay.cp
+                       : ((size_t)n * a.N * a.qHp + oh + a.qph) * a.qWp + ow + a.qpw;
+        o.j01 = qrow * a.qlay.rstride + (ow + a.qpw) * a.qlay.px01;
+        const float res[kUnit] = {};
+        ChannelTail plain = tl;
+#pragma unroll
+        for (int i = 0; i < kUnit; ++i) {
+            best[i] ^= flips[ch + 8 * (i >> 2) + (i & 3)];
+            plain.add[i] = 0;   // it is in the sums
+        }
+        store_tail(a, plain, best, res, c0 + ch, o);
+    }
+}
+
+// Zeros for flags that a launch gathers.
+__global__ __launch_bounds__(256) void mfma_clear_kernel(uint32_t *__restrict__ words, long count)
+{
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < count; i += (long)gridDim.x * 256) words[i] = 0;
+}
+
 // The padding of the next layer's input.
 template <typename Q>
 __global__ __launch_bounds__(256) void mfma_border_kernel(Q *__restrict__ q, long planes, int Hp, int Wp, int ph, int pw)
@@ -1360,6 +1530,40 @@ static int launch_mfma(MfmaArgs &a, hipStream_t st)
     if (tiles <= waves / 16 && a.KB >= 32) return launch_tiles<MODE, 1, 1, 8>(a, 8, st);
     const int ks = reduction_parts(tiles, waves, a.KB, mode_i8(MODE));
     return pair ? launch_tiles<MODE, 2, 1, 4>(a, ks, st) : launch_tiles<MODE, 1, 2, 4>(a, ks, st);
+}
+
+// The rectangle of pooled pixels of a workgroup, whose convolution takes at most `limit` pixels: the one with the fewest tiles
+// of 32 pixels over an image.
+static bool pool_tile(MfmaPool &m, int limit)
+{
+    long best = 0;
+    for (int th = 1; th <= m.POH; ++th) {
+        const long PH = (long)(th - 1) * m.ps + m.pk;
+        if (PH * m.pk > limit) break;
+        long tw = (limit / PH - m.pk) / m.ps + 1;   // the widest, then as wide as that many in a row need to be
+        if (tw > m.POW) tw = m.POW;
+        const int across = ceil_div(m.POW, (int)tw);
+        tw = ceil_div(m.POW, across);
+        const long PW = (tw - 1) * m.ps + m.pk;
+        const long spent = (long)ceil_div(m.POH, th) * across * ((PH * PW + 31) / 32);
+        if (best && spent >= best) continue;
+        best = spent;
+        m.th = th;
+        m.tw = (int)tw;
+        m.PH = (int)PH;
+        m.PW = (int)PW;
+    }
+    return best > 0;
+}
+
+template <int MODE>
+static int launch_pool(MfmaArgs &a, MfmaPool &m, unsigned grid, hipStream_t st)
+{
+    if (m.pk == 3)
+        hipLaunchKernelGGL((mfma_pool_kernel<MODE, true>), dim3(grid), dim3(256), 0, st, a, m);
+    else
+        hipLaunchKernelGGL((mfma_pool_kernel<MODE, false>), dim3(grid), dim3(256), 0, st, a, m);
+    return launch_status();
 }
 
 template <int SRC, bool I8>
@@ -1478,12 +1682,13 @@ DS_EXPORT int ds_mfma_prepare(const void *x, int source, void *dst, int Nb, int 
     return x_bytes == 1 ? launch_prepare<kSrcF32, true>(a, matrix, st) : launch_prepare<kSrcF32, false>(a, matrix, st);
 }
 
-DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32_t *bias, int32_t *y, float *out, void *q,
-                             const float *scale, const float *shift, const float *residual, int Nb, int C, int Hp, int Wp,
-                             int O, int FH, int FW, int sh, int sw, int crop_h, int crop_w, int prep_FH, int prep_FW,
-                             int matrix_rows, int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw,
-                             int q_bytes, int q_FH, int q_FW, int prep_tiles, int prep_ph, int prep_pw,
-                             ds_stream_t stream)
+// ds_mfma_conv2d and ds_mfma_conv2d_pool (pool_k > 0).
+static int mfma_conv2d_any(const void *prepared, const void *blob, const int32_t *bias, int32_t *y, float *out, void *q,
+                           const float *scale, const float *shift, const float *residual, int Nb, int C, int Hp, int Wp,
+                           int O, int FH, int FW, int sh, int sw, int crop_h, int crop_w, int prep_FH, int prep_FW,
+                           int matrix_rows, int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw,
+                           int q_bytes, int q_FH, int q_FW, int prep_tiles, int prep_ph, int prep_pw, int pool_k, int pool_s,
+                           int pool_p, ds_stream_t stream)
 {
     const int border_kept = q_bytes & DS_Q_BORDER_KEPT;
     const bool operands = (q_bytes & DS_Q_OPERANDS) != 0;
@@ -1538,14 +1743,25 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     a.matrix = matrix_rows > 0;
     a.pixels = a.matrix ? (uint32_t)matrix_rows : (uint32_t)pixels;
     if (a.matrix && ((double)matrix_rows > pixels || q)) return DS_EINVAL;
-    a.ostride_c = a.matrix ? 1 : a.OH * a.OW;
+    MfmaPool m{};
+    int rows = a.OH, columns = a.OW;   // of the result
+    if (pool_k) {
+        if (!ds_mfma_pool_serves(a.OH, a.OW, pool_k, pool_s, pool_p) || a.matrix || y || residual || pixels * O * 4 >= 2147483648.0)
+            return DS_EINVAL;
+        m.pk = pool_k;
+        m.ps = pool_s;
+        m.pp = pool_p;
+        m.POH = rows = (a.OH + 2 * pool_p - pool_k) / pool_s + 1;
+        m.POW = columns = (a.OW + 2 * pool_p - pool_k) / pool_s + 1;
+    }
+    a.ostride_c = a.matrix ? 1 : rows * columns;
     a.ostride_n = (long)a.ostride_c * O;
     a.relu = relu;
     a.q_bytes = q_bytes;
     a.qph = ph;
     a.qpw = pw;
-    a.qHp = a.OH + 2 * ph;
-    a.qWp = a.OW + 2 * pw;
+    a.qHp = rows + 2 * ph;
+    a.qWp = columns + 2 * pw;
     if (q && (double)a.qHp * a.qWp > 2147483647.0) return DS_EINVAL;
     a.inv = ldexpf(1.0f, -F_in);
     a.qspec = make_spec(I, F, DS_Q_ROUND_TO_FIXED);
@@ -1564,7 +1780,7 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
             hipLaunchKernelGGL(mfma_operand_border_kernel, dim3(blocks), dim3(256), 0, st, (int8_t *)q, a.qlay, ph, pw);
         }
     } else if (q && !border_kept && (ph || pw)) {
-        const long cells = (long)Nb * O * (2L * ph * a.qWp + 2L * pw * a.OH);
+        const long cells = (long)Nb * O * (2L * ph * a.qWp + 2L * pw * rows);
         const unsigned blocks = (unsigned)((cells + 255) / 256 < 4096 ? (cells + 255) / 256 : 4096);
         if (q_bytes == 1)
             hipLaunchKernelGGL((mfma_border_kernel<int8_t>), dim3(blocks), dim3(256), 0, st, (int8_t *)q, (long)Nb * O, a.qHp,
@@ -1573,6 +1789,36 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
             hipLaunchKernelGGL((mfma_border_kernel<int32_t>), dim3(blocks), dim3(256), 0, st, (int32_t *)q, (long)Nb * O, a.qHp,
                                a.qWp, ph, pw);
     }
+    if (pool_k) {
+        // rectangles of up to 256 pixels; half of that where they would leave half of the chip without one
+        a.ctiles = ceil_div(O, 64);
+        a.by_ctiles = fast_div((uint32_t)a.ctiles);
+        long grid = 0;
+        for (int limit = kPoolPixels; limit >= 128; limit /= 2) {
+            if (!pool_tile(m, limit)) break;
+            m.tiles_h = ceil_div(m.POH, m.th);
+            m.tiles_w = ceil_div(m.POW, m.tw);
+            grid = (long)Nb * m.tiles_h * m.tiles_w * a.ctiles;
+            if (grid >= device_cus()) break;
+        }
+        m.by_pw = fast_div((uint32_t)m.PW);
+        m.by_tw = fast_div((uint32_t)m.tw);
+        m.by_tiles_w = fast_div((uint32_t)m.tiles_w);
+        m.by_tiles_h = fast_div((uint32_t)m.tiles_h);
+        a.qscattered = 1;
+        if (operands && q_bytes == 4) {
+            const long words = (long)(align_up(((size_t)Nb * rows * columns / 32 + 1) * a.qlay.c16, 4) / 4);
+            hipLaunchKernelGGL(mfma_clear_kernel, dim3((unsigned)(words / 256 < 1024 ? words / 256 + 1 : 1024)), dim3(256), 0, st,
+                               (uint32_t *)a.qflags, words);
+        }
+        switch (mode) {
+        case kI32S15: return launch_pool<kI32S15>(a, m, (unsigned)grid, st);
+        case kI32S7: return launch_pool<kI32S7>(a, m, (unsigned)grid, st);
+        case kI32S4: return launch_pool<kI32S4>(a, m, (unsigned)grid, st);
+        case kI8S8: return launch_pool<kI8S8>(a, m, (unsigned)grid, st);
+        default: return launch_pool<kI8S4>(a, m, (unsigned)grid, st);
+        }
+    }
     switch (mode) {
     case kI32S15: return launch_mfma<kI32S15>(a, st);
     case kI32S7: return launch_mfma<kI32S7>(a, st);
@@ -1580,4 +1826,36 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
     case kI8S8: return launch_mfma<kI8S8>(a, st);
     default: return launch_mfma<kI8S4>(a, st);
     }
+}
+
+DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32_t *bias, int32_t *y, float *out, void *q,
+                             const float *scale, const float *shift, const float *residual, int Nb, int C, int Hp, int Wp,
+                             int O, int FH, int FW, int sh, int sw, int crop_h, int crop_w, int prep_FH, int prep_FW,
+                             int matrix_rows, int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw,
+                             int q_bytes, int q_FH, int q_FW, int prep_tiles, int prep_ph, int prep_pw,
+                             ds_stream_t stream)
+{
+    return mfma_conv2d_any(prepared, blob, bias, y, out, q, scale, shift, residual, Nb, C, Hp, Wp, O, FH, FW, sh, sw, crop_h,
+                           crop_w, prep_FH, prep_FW, matrix_rows, max_shift, x_bytes, F_in, relu, I, F, ph, pw, q_bytes, q_FH,
+                           q_FW, prep_tiles, prep_ph, prep_pw, 0, 0, 0, stream);
+}
+
+// The max pooling windows that the fused launch has a form for: at least one pixel of the image in each, and a convolution
+// rectangle that fits a workgroup.
+DS_EXPORT int ds_mfma_pool_serves(int OH, int OW, int pool_k, int pool_s, int pool_p)
+{
+    if (pool_k < 1 || pool_s < 1 || pool_p < 0 || 2 * (long)pool_p > pool_k || pool_k > 11) return 0;
+    return OH > 0 && OW > 0 && OH + 2 * (long)pool_p >= pool_k && OW + 2 * (long)pool_p >= pool_k;
+}
+
+DS_EXPORT int ds_mfma_conv2d_pool(const void *prepared, const void *blob, const int32_t *bias, float *out, void *q,
+                                  const float *scale, const float *shift, int Nb, int C, int Hp, int Wp, int O, int FH, int FW,
+                                  int sh, int sw, int prep_FH, int prep_FW, int max_shift, int x_bytes, int F_in, int relu,
+                                  int I, int F, int ph, int pw, int q_bytes, int q_FH, int q_FW, int prep_tiles, int prep_ph,
+                                  int prep_pw, int pool_k, int pool_s, int pool_p, ds_stream_t stream)
+{
+    if (pool_k < 1) return DS_EINVAL;
+    return mfma_conv2d_any(prepared, blob, bias, nullptr, out, q, scale, shift, nullptr, Nb, C, Hp, Wp, O, FH, FW, sh, sw, 0, 0,
+                           prep_FH, prep_FW, 0, max_shift, x_bytes, F_in, relu, I, F, ph, pw, q_bytes, q_FH, q_FW, prep_tiles,
+                           prep_ph, prep_pw, pool_k, pool_s, pool_p, stream);
 }

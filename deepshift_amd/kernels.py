@@ -1022,6 +1022,12 @@ def _mfma_conv_serves(Nb, C, Hp, Wp, O, kernel_size, stride, x_bytes=4):
     return 0 < pixels <= 10 ** 9 and pixels * O <= 8 * 10 ** 9
 
 
+def mfma_pool_serves(Nb, OH, OW, O, pool):
+    """Whether a convolution on the matrix cores takes the max pooling behind it into its launch: more than 32 channels (half
+    of its tiles of 64 would be padding), and the window and the size before the pooling have a form there."""
+    return O > 32 and Nb * O * OH * OW < 1 << 29 and bool(_lib.lib().ds_mfma_pool_serves(OH, OW, *pool))
+
+
 def _layout_pass_pays(Nb, H, W, K, O, stride, one_tap):
     """Whether the matrix cores win by more than their layout pass against kernels that read an unpadded int32 input as it
     is, in one launch.  Us there and here, 128 x 56 x 56 images, 1 x 1: 4 -> 64 channels 24, 68; 24 -> 128: 84, 103;
@@ -1159,17 +1165,25 @@ def mfma_prepare(x, padding, kernel_size, x_bytes, integer_bits=16, fraction_bit
 
 
 def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0, fraction_bits_in=None, scale=None,
-                shift=None, residual=None, relu=False, emit=None, want_float=True, q_cache=None):
+                shift=None, residual=None, relu=False, emit=None, want_float=True, q_cache=None, pool=None):
     """The layer from prepared activations.  ``fraction_bits_in`` None: int32 sums (with ``bias``).  Otherwise what
     :func:`conv2d_tiled_fused` returns for the same arguments.  A prepared matrix gives ``[M, O]``.  With a fifth
     element in ``emit``, the filter size of the layer that will read it, ``q`` is :class:`Prepared` for that layer
-    (kept in ``q_cache`` like the padded buffer), or the padded tensor where the size does not allow it."""
+    (kept in ``q_cache`` like the padded buffer), or the padded tensor where the size does not allow it.
+    ``pool = (kernel, stride, padding)``: a max pooling behind the ReLU, for what :func:`mfma_pool_serves` takes (images, no
+    residual, no crop); the results are those of :func:`requantize_affine_maxpool` on the sums."""
     Nb, C, Hp, Wp = prepared.dims
     FH, FW = _pair(kernel_size)
     sh, sw = _pair(stride)
     ch, cw = _pair(crop)
     OH, OW = (Hp - 2 * ch - FH) // sh + 1, (Wp - 2 * cw - FW) // sw + 1
     dev = prepared.data.device
+    pixels = Nb * OH * OW
+    if pool is not None:
+        if residual is not None or prepared.rows or ch or cw or fraction_bits_in is None:
+            raise ValueError("a pooled layer has images, a float result, and neither residual nor crop")
+        pk, ps, pp = pool
+        OH, OW = (OH + 2 * pp - pk) // ps + 1, (OW + 2 * pp - pk) // ps + 1
     if bias is not None:
         bias = _require_device_i32("bias", bias)
     shape = (prepared.rows, O) if prepared.rows else (Nb, O, OH, OW)
@@ -1206,10 +1220,16 @@ def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0,
             q, kept = made
             del made
             qb |= kept
-    M = prepared.rows or Nb * OH * OW
+    M = prepared.rows or pixels
     keep = (prepared.data, blob, bias, y, out, q, scale, shift, residual)
 
     def launch():
+        if pool is not None:
+            _lib.call("ds_mfma_conv2d_pool", *[_lib.ptr(t) for t in keep[:3] + keep[4:8]], Nb, C, Hp, Wp, O, FH, FW, sh, sw,
+                      *prepared.filter, max_shift, prepared.x_bytes, int(fraction_bits_in), int(bool(relu)), int(I), int(Fq),
+                      ph, pw, qb, *qfilter, int(prepared.written_by_conv is not None), *(prepared.written_by_conv or (0, 0)),
+                      *pool, _lib.current_stream(dev))
+            return
         _lib.call("ds_mfma_conv2d", *[_lib.ptr(t) for t in keep], Nb, C, Hp, Wp, O, FH, FW, sh, sw, ch, cw,
                   prepared.filter[0], prepared.filter[1], prepared.rows, max_shift, prepared.x_bytes,
                   int(fraction_bits_in or 0), int(bool(relu)), int(I), int(Fq), ph, pw, qb, *qfilter,

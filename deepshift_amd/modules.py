@@ -350,7 +350,11 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
         return None
     prepared, blob, max_shift = route
     bias = module._fixed_bias.get(module.bias, I, Fb, round_to_fixed=True)
-    if pool is not None or not _FUSE_EPILOGUE or (x_bytes == 1 and not _FUSE_INT8):
+    fused = _FUSE_EPILOGUE and (x_bytes == 4 or _FUSE_INT8)
+    if fused and pool is not None:
+        sums = [(prepared.dims[2 + i] - module.kernel_size[i]) // module.stride[i] + 1 for i in (0, 1)]
+        fused = residual is None and kernels.mfma_pool_serves(Nb, *sums, module.out_channels, pool)
+    if not fused:
         out = kernels.mfma_conv2d(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift)
         return _separate_pass(out, Fb, scale, shift, residual, relu, pool, emit)
     want_float, spec = True, None
@@ -360,14 +364,14 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
     # the consumers' padded input lives in a buffer of this layer whose border is zeroed once
     cache = module.__dict__.setdefault("_handoff_buffers", {})
     f, q = kernels.mfma_conv2d(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift, 0, Fb,
-                               scale, shift, residual, relu, spec, want_float, cache)
+                               scale, shift, residual, relu, spec, want_float, cache, pool)
     if emit is None:
         return f
     return (f, q) if want_float else q
 
 
 def _separate_pass(out, Fb, scale, shift, residual, relu, pool, emit):
-    """What follows a convolution's int32 sums in a pass of its own: a max pooling behind the ReLU always, the rest where
+    """What follows a convolution's int32 sums in a pass of its own, a max pooling behind the ReLU among it, where
     no launch with a fused epilogue serves the layer."""
     if emit is not None:
         next_padding, next_I, next_F, want_float = emit[:4]

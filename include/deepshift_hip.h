@@ -421,6 +421,17 @@ int ds_mfma_conv2d(const void *prepared, const void *blob, const int32_t *bias, 
                    int FH, int FW, int sh, int sw, int crop_h, int crop_w, int prep_FH, int prep_FW, int matrix_rows,
                    int max_shift, int x_bytes, int F_in, int relu, int I, int F, int ph, int pw, int q_bytes, int q_FH,
                    int q_FW, int prep_tiles, int prep_ph, int prep_pw, ds_stream_t stream);
+/* ds_mfma_conv2d with a max pooling (window pool_k x pool_k, stride pool_s, implicit -inf padding pool_p, floor mode, as
+ * nn.MaxPool2d) between the affine / ReLU and the conversion, in the same launch: out and q as
+ * ds_requantize_affine_maxpool_i32 / _i8 write them from the layer's sums, or q in the operand layout.  ds_mfma_pool_serves:
+ * whether there is a form for that window on an OH x OW result (2 pool_p <= pool_k <= 11; 0 or 1); DS_EINVAL also for
+ * results of 2 GB and more before the pooling. */
+int ds_mfma_pool_serves(int OH, int OW, int pool_k, int pool_s, int pool_p);
+int ds_mfma_conv2d_pool(const void *prepared, const void *blob, const int32_t *bias, float *out, void *q,
+                        const float *scale, const float *shift, int Nb, int C, int Hp, int Wp, int O, int FH, int FW,
+                        int sh, int sw, int prep_FH, int prep_FW, int max_shift, int x_bytes, int F_in, int relu, int I,
+                        int F, int ph, int pw, int q_bytes, int q_FH, int q_FW, int prep_tiles, int prep_ph, int prep_pw,
+                        int pool_k, int pool_s, int pool_p, ds_stream_t stream);
 
 /* ---- fixed-point conversion ------------------------------------------------------------ */
 

@@ -343,3 +343,49 @@ def test_few_channels_agree_on_both_kernels(rng, C, O, k):
     blob = kernels._mfma_of(cw, 14, 4, O, C, k, k)
     assert torch.equal(kernels.mfma_conv2d(handed, blob, None, O, (k, k), 1, 14),
                        kernels.conv2d_tiled(padded, kernels._tiled_of(cw, O, C, k, k), None, O, (k, k), 1, kernels.kernel_bits(cw)))
+
+
+# (Nb, C, H, W, O, k, stride, pad), (pool kernel, stride, padding)
+POOLED = [((2, 3, 45, 37, 64, 7, 2, 3), (3, 2, 1)), ((3, 20, 14, 9, 70, 3, 1, 1), (2, 2, 0)), ((1, 64, 9, 12, 33, 1, 1, 0), (3, 1, 1)),
+          ((2, 8, 23, 23, 129, 3, 1, 1), (11, 4, 5)), ((40, 3, 64, 64, 40, 3, 2, 1), (3, 2, 0)), ((1, 33, 5, 70, 34, 3, 1, 1), (5, 3, 2)),
+          ((130, 32, 8, 8, 64, 3, 1, 1), (8, 8, 0))]
+
+
+@pytest.mark.parametrize("top,x_bytes", [(14, 4), (6, 4), (3, 4), (14, 1), (3, 1)], ids=lambda v: str(v))
+@pytest.mark.parametrize("shape,pool", POOLED, ids=lambda v: str(v).replace(" ", ""))
+def test_pooling_in_the_launch_matches_the_separate_pass(rng, top, x_bytes, shape, pool):
+    """The fused max pooling against the sums and the pooling pass: windows that overlap and do not, rectangles past the
+    image's edges, scales of both signs, zero and NaN, activations with digits 3 and 4 and results with them."""
+    Nb, C, H, W, O, k, st, pad = shape
+    s, sign, cw = _weights(rng, (O, C, k, k), top, ternary=True)
+    x = _activations(rng, (Nb, C, H, W), x_bytes, 1 << 18)
+    if x_bytes == 4:
+        x[0, :, : H // 2] <<= 5            # d3
+        x[-1, :, H - 1, W - 1] = -2 ** 31  # d4
+    bias = _dev(rng.integers(-2 ** 20, 2 ** 20, size=O).astype(np.int32))
+    prepared, blob, at = kernels.mfma_route(_dev(x), pad, cw, O, (k, k), x_bytes)
+    F_in, I, F, dtype = (16, 16, 16, torch.int32) if x_bytes == 4 else (5, 3, 5, torch.int8)
+    y = kernels.mfma_conv2d(prepared, blob, bias, O, (k, k), st, at)
+    assert kernels.mfma_pool_serves(Nb, y.shape[2], y.shape[3], O, pool)
+    scale, shift = torch.randn(O, device=DEV), torch.randn(O, device=DEV)
+    scale[1], scale[2], shift[3] = 0.0, float("nan"), float("nan")
+    for relu in (True, False):
+        f, q = kernels.requantize_affine_maxpool(y, F_in, scale, shift, relu, pool, (1, 1), I, F, True, dtype)
+        args = (prepared, blob, bias, O, (k, k), st, at, 0, F_in, scale, shift, None, relu)
+        cache = {}
+        for filt in ((3, 3), (3, 3), None):
+            out, got = kernels.mfma_conv2d(*args, ((1, 1), I, F, dtype, filt), True, cache, pool)
+            assert torch.equal(torch.nan_to_num(out, nan=7.0), torch.nan_to_num(f, nan=7.0))
+            assert torch.equal(got.padded() if filt else got, q)
+            del got
+        out, _ = kernels.mfma_conv2d(*args, None, True, None, pool)
+        assert torch.equal(torch.nan_to_num(out, nan=7.0), torch.nan_to_num(f, nan=7.0))
+        _, got = kernels.mfma_conv2d(*args, ((0, 1), I, F, dtype, (1, 3)), False, None, pool)
+        assert torch.equal(got.padded(), q[:, :, 1:-1])
+
+
+def test_windows_without_a_form_keep_their_pass():
+    serves = kernels._lib.lib().ds_mfma_pool_serves
+    assert serves(8, 8, 3, 2, 1) == 1 and serves(1, 1, 1, 1, 0) == 1 and serves(11, 11, 11, 1, 0) == 1
+    assert serves(8, 8, 12, 1, 0) == 0 and serves(8, 8, 3, 2, 2) == 0 and serves(2, 8, 3, 1, 0) == 0 and serves(8, 8, 3, 0, 1) == 0
+    assert not kernels.mfma_pool_serves(1, 8, 8, 32, (3, 2, 1)) and not kernels.mfma_pool_serves(64, 1024, 1024, 64, (3, 2, 1))
