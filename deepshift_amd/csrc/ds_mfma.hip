@@ -1840,6 +1840,16 @@ DS_EXPORT int ds_mfma_conv2d(const void *prepared, const void *blob, const int32
                            q_FW, prep_tiles, prep_ph, prep_pw, 0, 0, 0, stream);
 }
 
+// ds_mfma_conv2d and ds_mfma_conv2d_pool with their arguments in two arrays.
+DS_EXPORT int ds_mfma_conv2d_packed(const void *const *p, const int32_t *d, ds_stream_t stream)
+{
+    if (!p || !d) return DS_EINVAL;
+    return mfma_conv2d_any(p[0], p[1], (const int32_t *)p[2], (int32_t *)p[3], (float *)p[4], (void *)p[5], (const float *)p[6],
+                           (const float *)p[7], (const float *)p[8], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7], d[8], d[9],
+                           d[10], d[11], d[12], d[13], d[14], d[15], d[16], d[17], d[18], d[19], d[20], d[21], d[22], d[23],
+                           d[24], d[25], d[26], d[27], d[28], d[29], d[30], stream);
+}
+
 // The max pooling windows that the fused launch has a form for: at least one pixel of the image in each, and a convolution
 // rectangle that fits a workgroup.
 DS_EXPORT int ds_mfma_pool_serves(int OH, int OW, int pool_k, int pool_s, int pool_p)

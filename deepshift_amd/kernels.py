@@ -19,6 +19,8 @@ Differences from the reference, all deliberate:
 """
 
 import ctypes
+import functools
+import struct
 import sys
 
 import torch
@@ -31,6 +33,8 @@ __all__ = ["linear", "conv2d", "compress_sign_and_shift", "quantize", "quantize_
 
 
 def _pair(v):
+    if type(v) is tuple and len(v) == 2 and type(v[0]) is int and type(v[1]) is int:
+        return v
     if isinstance(v, (tuple, list)):
         if len(v) == 1:
             return int(v[0]), int(v[0])
@@ -1012,6 +1016,16 @@ def _too_few_terms(O, C, FH, FW, x_bytes):
     return x_bytes == 4 and O <= 16 and C <= 16 and C * FH * FW < 64
 
 
+# What depends on sizes alone is worked out once per set of them: the host otherwise needs longer to issue the small layers of
+# one image than the GPU to run them (ResNet-18, batch 1: 22 us a launch, of which the launch itself is 4).
+_SIZES = 4096
+
+
+@functools.lru_cache(_SIZES)
+def _input_bytes(Nb, C, Hp, Wp, FH, FW, x_bytes):
+    return _lib.lib().ds_mfma_input_bytes(Nb, C, Hp, Wp, FH, FW, x_bytes)
+
+
 def _mfma_conv_serves(Nb, C, Hp, Wp, O, kernel_size, stride, x_bytes=4):
     """Whether the output has anything in it, its offsets fit, and the matrix cores are the faster place."""
     FH, FW = _pair(kernel_size)
@@ -1025,7 +1039,7 @@ def _mfma_conv_serves(Nb, C, Hp, Wp, O, kernel_size, stride, x_bytes=4):
 def mfma_pool_serves(Nb, OH, OW, O, pool):
     """Whether a convolution on the matrix cores takes the max pooling behind it into its launch: more than 32 channels (half
     of its tiles of 64 would be padding), and the window and the size before the pooling have a form there."""
-    return O > 32 and Nb * O * OH * OW < 1 << 29 and bool(_lib.lib().ds_mfma_pool_serves(OH, OW, *pool))
+    return O > 32 and Nb * O * OH * OW < 1 << 29 and bool(_lib.lib().ds_mfma_pool_serves(OH, OW, *(int(v) for v in pool)))
 
 
 def _layout_pass_pays(Nb, H, W, K, O, stride, one_tap):
@@ -1130,7 +1144,7 @@ class Prepared:
 
 def _operand_output(cache, dims, kernel_size, padding, x_bytes, device):
     """:func:`_padded_output` for the operand layout: ``None`` where the layout does not serve the size."""
-    nbytes = _lib.lib().ds_mfma_input_bytes(*dims, *kernel_size, x_bytes)
+    nbytes = _input_bytes(*dims, *kernel_size, x_bytes)
     if not nbytes:
         return None
     if cache is not None and any(padding):
@@ -1154,7 +1168,7 @@ def mfma_prepare(x, padding, kernel_size, x_bytes, integer_bits=16, fraction_bit
     else:
         rows = 0
         Nb, C, H, W = x.shape
-    nbytes = _lib.lib().ds_mfma_input_bytes(Nb, C, H + 2 * ph, W + 2 * pw, FH, FW, x_bytes)
+    nbytes = _input_bytes(Nb, C, H + 2 * ph, W + 2 * pw, FH, FW, x_bytes)
     if not nbytes:
         return None
     data = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
@@ -1172,76 +1186,106 @@ def mfma_conv2d(prepared, blob, bias, O, kernel_size, stride, max_shift, crop=0,
     (kept in ``q_cache`` like the padded buffer), or the padded tensor where the size does not allow it.
     ``pool = (kernel, stride, padding)``: a max pooling behind the ReLU, for what :func:`mfma_pool_serves` takes (images, no
     residual, no crop); the results are those of :func:`requantize_affine_maxpool` on the sums."""
-    Nb, C, Hp, Wp = prepared.dims
-    FH, FW = _pair(kernel_size)
-    sh, sw = _pair(stride)
-    ch, cw = _pair(crop)
-    OH, OW = (Hp - 2 * ch - FH) // sh + 1, (Wp - 2 * cw - FW) // sw + 1
     dev = prepared.data.device
-    pixels = Nb * OH * OW
-    if pool is not None:
-        if residual is not None or prepared.rows or ch or cw or fraction_bits_in is None:
-            raise ValueError("a pooled layer has images, a float result, and neither residual nor crop")
-        pk, ps, pp = pool
-        OH, OW = (OH + 2 * pp - pk) // ps + 1, (OW + 2 * pp - pk) // ps + 1
+    sums_only = fraction_bits_in is None
+    plan = _conv_plan(prepared.dims, prepared.filter, prepared.rows, prepared.x_bytes, prepared.written_by_conv, int(O),
+                      _pair(kernel_size), _pair(stride), _pair(crop), int(max_shift), None if sums_only else int(fraction_bits_in),
+                      bool(relu), None if emit is None else (_pair(emit[0]), int(emit[1]), int(emit[2]), emit[3] == torch.int8),
+                      None if emit is None or len(emit) < 5 or emit[4] is None else _pair(emit[4]),
+                      None if pool is None else tuple(int(v) for v in pool))
     if bias is not None:
         bias = _require_device_i32("bias", bias)
-    shape = (prepared.rows, O) if prepared.rows else (Nb, O, OH, OW)
     for name, t in (("scale", scale), ("shift", shift)):
         if t is not None and (t.dtype != torch.float32 or t.numel() != O or not t.is_contiguous()):
             raise ValueError("%s must be a contiguous float32 tensor of %d elements" % (name, O))
     if residual is not None:
-        if tuple(residual.shape) != shape or residual.dtype != torch.float32:
+        if pool is not None:
+            raise ValueError("a pooled layer takes no residual")
+        if tuple(residual.shape) != plan.shape or residual.dtype != torch.float32:
             raise ValueError("residual must be float32 with the shape of the output")
         residual = residual.contiguous()
     y = out = q = handed = None
-    qfilter = (1, 1)
-    ph, pw, I, Fq, qb = 0, 0, 16, 16, 4
-    if fraction_bits_in is None:
-        y = torch.empty(shape, dtype=torch.int32, device=dev)
+    ints = plan.ints
+    if sums_only:
+        y = torch.empty(plan.shape, dtype=torch.int32, device=dev)
     else:
         if emit is None and not want_float:
             raise ValueError("nothing to produce")
         if want_float:
-            out = torch.empty(shape, dtype=torch.float32, device=dev)
+            out = torch.empty(plan.shape, dtype=torch.float32, device=dev)
         if emit is not None:
-            padding, I, Fq, dtype = emit[:4]
-            ph, pw = _pair(padding)
-            qb = 1 if dtype == torch.int8 else 4
-            qshape = (Nb, O, OH + 2 * ph, OW + 2 * pw)
             made = None
-            if len(emit) == 5 and emit[4] is not None:
-                qfilter = _pair(emit[4])
-                made = _operand_output(q_cache, qshape, qfilter, (ph, pw), qb, dev)
+            if plan.qfilter is not None:
+                made = _operand_output(q_cache, plan.qshape, plan.qfilter, plan.qpad, plan.q_bytes, dev)
             if made is not None:
-                handed = Prepared(made[0], qshape, qfilter, 0, qb, (ph, pw))
+                handed = Prepared(made[0], plan.qshape, plan.qfilter, 0, plan.q_bytes, plan.qpad)
             else:
-                made = _padded_output(q_cache, qshape, (ph, pw), dtype, dev)
+                made = _padded_output(q_cache, plan.qshape, plan.qpad, emit[3], dev)
             q, kept = made
             del made
-            qb |= kept
-    M = prepared.rows or pixels
+            if kept:
+                ints = plan.kept(kept)
     keep = (prepared.data, blob, bias, y, out, q, scale, shift, residual)
 
     def launch():
-        if pool is not None:
-            _lib.call("ds_mfma_conv2d_pool", *[_lib.ptr(t) for t in keep[:3] + keep[4:8]], Nb, C, Hp, Wp, O, FH, FW, sh, sw,
-                      *prepared.filter, max_shift, prepared.x_bytes, int(fraction_bits_in), int(bool(relu)), int(I), int(Fq),
-                      ph, pw, qb, *qfilter, int(prepared.written_by_conv is not None), *(prepared.written_by_conv or (0, 0)),
-                      *pool, _lib.current_stream(dev))
-            return
-        _lib.call("ds_mfma_conv2d", *[_lib.ptr(t) for t in keep], Nb, C, Hp, Wp, O, FH, FW, sh, sw, ch, cw,
-                  prepared.filter[0], prepared.filter[1], prepared.rows, max_shift, prepared.x_bytes,
-                  int(fraction_bits_in or 0), int(bool(relu)), int(I), int(Fq), ph, pw, qb, *qfilter,
-                  int(prepared.written_by_conv is not None), *(prepared.written_by_conv or (0, 0)),
-                  _lib.current_stream(dev))
+        _lib.call("ds_mfma_conv2d_packed", _POINTERS(*[0 if t is None else t.data_ptr() for t in keep]), ints,
+                  _lib.stream_handle(dev))
 
-    kind = "linear" if prepared.rows else "conv"
-    with _Timed(kind, M, C * FH * FW, O, dev):
+    if _TIMING_SINK is None and _REPLAY_SINK is None:
         launch()
-    if _REPLAY_SINK is not None and fraction_bits_in is not None:
-        _REPLAY_SINK.append((kind, M, C * FH * FW, O, launch))
-    return y if fraction_bits_in is None else (out, q if handed is None else handed)
+    else:
+        kind = "linear" if prepared.rows else "conv"
+        with _Timed(kind, plan.pixels, plan.terms, O, dev):
+            launch()
+        if _REPLAY_SINK is not None and not sums_only:
+            _REPLAY_SINK.append((kind, plan.pixels, plan.terms, O, launch))
+    return y if sums_only else (out, q if handed is None else handed)
+
+
+_POINTERS = struct.Struct("=9Q").pack
+_INTS = struct.Struct("=31i").pack
+
+
+class _ConvPlan:
+    """What :func:`mfma_conv2d` derives from sizes and options alone."""
+
+    __slots__ = ("shape", "pixels", "terms", "qshape", "qpad", "qfilter", "q_bytes", "ints", "_values", "_kept")
+
+    def kept(self, flags):
+        """The integer arguments for a hand-off buffer with these ``DS_Q_*`` flags."""
+        ints = self._kept.get(flags)
+        if ints is None:
+            values = list(self._values)
+            values[_Q_BYTES_AT] |= flags
+            ints = self._kept[flags] = _INTS(*values)
+        return ints
+
+
+_Q_BYTES_AT = 22   # among the integers of ds_mfma_conv2d
+
+
+@functools.lru_cache(_SIZES)
+def _conv_plan(dims, prep_filter, rows, x_bytes, written_by_conv, O, kernel_size, stride, crop, max_shift, F_in, relu, emit,
+               qfilter, pool):
+    Nb, C, Hp, Wp = dims
+    (FH, FW), (sh, sw), (ch, cw) = kernel_size, stride, crop
+    OH, OW = (Hp - 2 * ch - FH) // sh + 1, (Wp - 2 * cw - FW) // sw + 1
+    plan = _ConvPlan()
+    plan.pixels, plan.terms = rows or Nb * OH * OW, C * FH * FW
+    if pool is not None:
+        if rows or ch or cw or F_in is None:
+            raise ValueError("a pooled layer has images, a float result, and no crop")
+        pk, ps, pp = pool
+        OH, OW = (OH + 2 * pp - pk) // ps + 1, (OW + 2 * pp - pk) // ps + 1
+    plan.shape = (rows, O) if rows else (Nb, O, OH, OW)
+    (ph, pw), I, Fq, bytes_of = ((0, 0), 16, 16, 4) if emit is None or F_in is None else (emit[0], emit[1], emit[2], 1 if emit[3] else 4)
+    plan.qshape, plan.qpad, plan.qfilter, plan.q_bytes = (Nb, O, OH + 2 * ph, OW + 2 * pw), (ph, pw), qfilter, bytes_of
+    qf = qfilter if emit is not None and qfilter is not None else (1, 1)
+    plan._values = (Nb, C, Hp, Wp, O, FH, FW, sh, sw, ch, cw, *prep_filter, rows, max_shift, x_bytes, F_in or 0, int(relu), I, Fq,
+                    ph, pw, bytes_of, *qf, int(written_by_conv is not None), *(written_by_conv or (0, 0)), *(pool or (0, 0, 0)))
+    plan._kept = {}
+    plan.ints = _INTS(*plan._values)
+    return plan
 
 
 def conv2d(input, shift, sign, bias=None, conc_weight=None, stride=1, padding=0, dilation=1,

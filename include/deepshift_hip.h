@@ -432,6 +432,9 @@ int ds_mfma_conv2d_pool(const void *prepared, const void *blob, const int32_t *b
                         int sh, int sw, int prep_FH, int prep_FW, int max_shift, int x_bytes, int F_in, int relu, int I,
                         int F, int ph, int pw, int q_bytes, int q_FH, int q_FW, int prep_tiles, int prep_ph, int prep_pw,
                         int pool_k, int pool_s, int pool_p, ds_stream_t stream);
+/* The same two with their arguments in arrays, for callers to whom forty arguments cost more than the launch: pointers, the
+ * nine of ds_mfma_conv2d in its order; ints, its 28 integers in its order, then pool_k (0: no pooling), pool_s, pool_p. */
+int ds_mfma_conv2d_packed(const void *const *pointers, const int32_t *ints, ds_stream_t stream);
 
 /* ---- fixed-point conversion ------------------------------------------------------------ */
 
