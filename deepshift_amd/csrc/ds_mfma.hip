@@ -884,8 +884,9 @@ __device__ __forceinline__ void digit4(const MfmaArgs &a, int32_t (*slot)[64], i
 
 // The sums of one wave's tile over blocks kb0 .. kb1 - 1.  Two sets of operands, the loads of a block in flight during the
 // products of the one before; with digit d3, whose sums leave no room for them (14 VGPRs went to scratch and back in every
-// block), one set, loaded again once the last operands of a block are formed and behind its last products.
-template <int MODE, int CT, int NT, bool HIGH, bool ONE_SET = HIGH>
+// block), and for 64 pixels (17 VGPRs; 32 channels of 16 x 16, 256 images: 15.8 us, so 14.7), one set, loaded again once the
+// last operands of a block are formed and behind its last products.
+template <int MODE, int CT, int NT, bool HIGH, bool ONE_SET = HIGH || (NT == 2 && !mode_i8(MODE))>
 __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT], const int8_t *w, int kb0, int kb1,
                                          const uint32_t (&px)[NT], const uint32_t (&px01)[NT], const PixelAt (&at)[NT], int lane)
 {
@@ -1496,39 +1497,42 @@ static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
     return launch_status();
 }
 
-// Waves that share a tile's reduction, of `blocks` blocks.  A part pays for the start of its loads, its share of an
-// epilogue and the meeting in LDS, so short reductions are cut only where most wave slots would stay empty, longer ones
-// as long as the parts fill slots that whole tiles leave empty, and in two where a few tiles would need a second round.
-// Measured with 1, 2 and 4 parts, int32 activations, shifts to 14 (us; 2048 wave slots):
-//   blocks    512 tiles         1024              1536              2048              2560              4096
-//     4       10.6 10.2  9.6    12.1 13.6 17.1    16.0 20.4 23.8    17.2 24.1 31.2                      29.0 43.1 56.3
-//     9       14.2 12.5 11.2    15.7 16.7 20.6    22.5 25.6 28.5    23.8 30.4 36.4                      41.7 54.5 67.2
-//    18       21.8 16.7 14.9    23.6 23.4 25.5    34.8 33.4 34.6    37.4 41.1 45.4    51.1 50.7 54.4    68.2 73.0 83.6
-//    36       34.3 23.2 20.7    37.8 35.8 36.4    56.8 50.9 52.4    60.0 63.9 67.5    83.3 77.5 82.9   118.7  123  132
-//   144        114 65.6 64.0     116  112  114     194  164  168     211  216  222     304  266  279
-// The second walk for digits 3 and 4 lengthens some tiles only, which two parts even out: 3584 tiles of 72 blocks 317,
-// 295, 300.  8-bit activations (3072 slots) have none, and turn at about the same fill otherwise.
-// Cutting up to three tiles a slot, whatever the length, left layers of few channels behind the vector kernels: 17 -> 64
-// channels, 3 x 3, 64 images of 32 x 32, with the layout pass: 55 us against 45 there and 42 with this rule; 9 -> 128: 62
-// against 52 and 47.
-static int reduction_parts(long tiles, long waves, int blocks, bool i8)
+// Waves that share a tile's reduction, of `blocks` blocks.  Waves in one workgroup also share a tile's epilogue, which is most
+// of a short reduction's time, so few tiles always take four; more tiles take as many as fit a workgroup a CU (two, three
+// with the registers of 8-bit activations), if the reduction pays for its parts' start and their meeting in LDS; and a long
+// one is cut in two while that fills slots which whole tiles leave empty.  Measured with 1, 2 and 4 parts, hand-off to the
+// next layer (us; 256 CUs, tiles of 64 channels x 32 pixels):
+//   int32, blocks  512 tiles        768               1024              1536              2560              4096
+//     2            10.6  9.3  8.5*  10.9 11.1 14.2                                                          (*: 384)
+//     4            11.8 10.2  9.4   12.0 12.2 14.6    12.4 12.5 16.7    16.6 19.3 23.8    23.9 28.2 37.5    29.9 41.3 57.3
+//     9            14.4 11.6 10.9   14.7 14.7 16.9    15.2 15.4 19.6    21.6 23.1 28.0    30.3 34.0 43.8    39.4 50.0 67.4
+//     18           19.4 14.6 13.3   20.8 19.5 20.3    21.6 20.6 24.1    30.1 29.5 33.8    43.7 44.2 53.2    62.2 71.9 88.2
+//     36           30.4 20.7 18.7   31.1 28.4 26.6    32.3 29.7 32.8    47.8 43.8 46.4    84.1 80.8 86.5     121  133  143
+//   8-bit
+//     4             7.4  7.5  6.7    7.5  8.2  7.6     7.6  8.4 11.0     9.2  9.4 13.2    11.4 15.0 20.5    15.1 21.2 29.8
+//     9             8.7  8.2  7.5    8.8  9.4  8.3     8.9  9.5 11.9    11.4 11.3 14.5    14.9 17.6 22.4    19.3 25.7 34.1
+//     18           11.2  9.4  8.6   11.4 11.3 10.1    11.5 11.6 13.5    15.9 15.2 17.2    21.4 22.1 26.9    27.4 32.3 40.8
+//     36           16.3 11.9 10.6   16.6 15.6 13.1    17.7 16.6 17.4    24.4 21.2 22.8    33.3 32.0 35.8    44.3 48.0 55.0
+// Very long ones take four up to seven tiles a CU, unless their activations are read once, from memory (256 -> 256 channels,
+// 3 x 3, 64 images of 14 x 14, 1568 tiles of 72 blocks: 77.6, 79.1, 73.6; 2304 -> 64, 1 x 1, as many: 96, 102, 105).
+static int reduction_parts(long tiles, long cus, int blocks, bool i8, bool rereads)
 {
-    if (tiles * 8 <= waves * (blocks < 16 ? 2 : blocks < 32 ? 6 : 7)) return blocks >= 4 ? 4 : 1;
-    return !i8 && blocks >= 32 && tiles > waves && tiles < 2 * waves ? 2 : 1;
+    if (tiles <= 2 * cus || (tiles <= 3 * cus && blocks >= (i8 ? 9 : 32))) return 4;
+    if (tiles <= 6 * cus) return blocks >= 16 ? 2 : 1;
+    if (tiles <= 7 * cus && blocks >= 64 && rereads) return 4;
+    return !i8 && blocks >= 32 && tiles > 8 * cus && tiles < 16 * cus ? 2 : 1;
 }
 
 template <int MODE>
 static int launch_mfma(MfmaArgs &a, hipStream_t st)
 {
-    const long waves = (long)device_cus() * (mode_i8(MODE) ? 12 : 8);   // wave slots
+    const long cus = device_cus();
     const bool pair = a.N > 32;
     const long tiles = pair ? (long)ceil_div(a.N, 64) * ceil_div((int)a.pixels, 32) : (long)ceil_div((int)a.pixels, 64);
-    // Few tiles and a long reduction leave the chip idle behind one wave's serial chain: half the tile, and the
-    // reduction in eight parts (one image, 512 channels of 7 x 7, 16 tiles: 34 -> 22 us; 256 of 14 x 14, 32 tiles:
-    // 21 -> 16; 112 tiles: 38 -> 26).  Past a sixteenth of the slots the extra epilogues cost more than the shorter
-    // chain gives (200 tiles: 23.6 -> 25.1; 392 tiles: 18.6 -> 23), as they do on short reductions (18 blocks: even).
-    if (tiles <= waves / 16 && a.KB >= 32) return launch_tiles<MODE, 1, 1, 8>(a, 8, st);
-    const int ks = reduction_parts(tiles, waves, a.KB, mode_i8(MODE));
+    // Fewer than a tile for every other CU: half the tile, and the reduction in eight parts (64 and 128 tiles, us with four
+    // parts and these: 4 blocks 8.0, 7.8; 18: 9.9, 9.1; 36: 11.9, 10.5; 144: 28.4, 21.0; 256 tiles: 30.9, 41.2).
+    if (tiles <= cus / 2) return launch_tiles<MODE, 1, 1, 8>(a, 8, st);
+    const int ks = reduction_parts(tiles, cus, a.KB, mode_i8(MODE), a.N > 64 || a.FH * a.fwg > 1);
     return pair ? launch_tiles<MODE, 2, 1, 4>(a, ks, st) : launch_tiles<MODE, 1, 2, 4>(a, ks, st);
 }
 
