@@ -426,6 +426,9 @@ struct MfmaArgs {
     int relu, q_bytes, qHp, qWp, qph, qpw;
     int qscattered;             // a unit's pixels are not 32 in a row of the output: its flags are shared with other units
     float inv;
+    // the shorter epilogue: 2^F of the sums, 2^F of q if nothing else is written
+    float unfold, qfold;
+    int q_only;
     QuantSpec qspec;
     FastDiv by_image, by_row, by_ctiles;
 };
@@ -886,9 +889,10 @@ __device__ __forceinline__ void digit4(const MfmaArgs &a, int32_t (*slot)[64], i
 // products of the one before; with digit d3, whose sums leave no room for them (14 VGPRs went to scratch and back in every
 // block), and for 64 pixels (17 VGPRs; 32 channels of 16 x 16, 256 images: 15.8 us, so 14.7), one set, loaded again once the
 // last operands of a block are formed and behind its last products.
-template <int MODE, int CT, int NT, bool HIGH, bool ONE_SET = HIGH || (NT == 2 && !mode_i8(MODE))>
+template <int MODE, int CT, int NT, bool HIGH, bool ONE_SET = HIGH || (NT == 2 && !mode_i8(MODE)), typename Asked>
 __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT], const int8_t *w, int kb0, int kb1,
-                                         const uint32_t (&px)[NT], const uint32_t (&px01)[NT], const PixelAt (&at)[NT], int lane)
+                                         const uint32_t (&px)[NT], const uint32_t (&px01)[NT], const PixelAt (&at)[NT], int lane,
+                                         Asked first_asked)
 {
     typedef Operands<MODE, CT, NT, HIGH> Ops;
     Sums<CT, NT, HIGH> t = {};
@@ -906,6 +910,7 @@ __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT
             block_s7<MODE, CT, NT, HIGH>(o, t, reload);
     };
     load(o0);
+    first_asked();
     if constexpr (ONE_SET) {
         bool more;
 #pragma unroll 1
@@ -969,15 +974,46 @@ template <int CHANNELS>
 struct ChannelTails {
     int32_t add[CHANNELS];
     float scale[CHANNELS], shift[CHANNELS];
+    float scale1[CHANNELS], shift1[CHANNELS];   // the same for the shorter epilogue
+    int odd[4];                                 // per wave: whether one of its channels has no exact shorter form
 };
-template <int CHANNELS>
-__device__ __forceinline__ void stage_tails(const MfmaArgs &a, ChannelTails<CHANNELS> &t, int first, int count)
+// A thread's channel of these, asked for first and stored once the first operands have been asked for too: one latency, not
+// two, before the first product, which short reductions are made of (8-bit, 64 -> 256 channels,
+// 1 x 1, 128 images of 56 x 56: 97 -> 89 us; 256 -> 64: 39.4 -> 37.4; one image of 512 x 7 x 7, 3 x 3, int32: 18.9 -> 17.1).
+struct TailOfThread {
+    int32_t add;
+    float scale, shift;
+};
+__device__ __forceinline__ TailOfThread ask_tail(const MfmaArgs &a, int first, int count)
 {
-    const int i = threadIdx.x, ch = first + i, c = ch < a.N ? ch : a.N - 1;
-    if (i >= count) return;
-    t.add[i] = (a.bias ? a.bias[c] : 0) - (a.corr ? a.corr[c] : 0);
-    t.scale[i] = a.scale ? a.scale[c] : 1.0f;
-    t.shift[i] = a.shift ? a.shift[c] : 0.0f;
+    TailOfThread r{0, 1.0f, 0.0f};
+    const int i = threadIdx.x, c = first + i < a.N ? first + i : a.N - 1;
+    if (i >= count) return r;
+    r.add = (a.bias ? a.bias[c] : 0) - (a.corr ? a.corr[c] : 0);
+    r.scale = a.scale ? a.scale[c] : 1.0f;
+    r.shift = a.shift ? a.shift[c] : 0.0f;
+    return r;
+}
+// The shorter epilogue: powers of two -- 2^-F of the sums, and 2^F of the next layer's grid where only its input is written --
+// are multiplied into scale and shift, which changes no rounding while nothing leaves the range of normal numbers.  That is
+// looked at here, per channel: a factor that loses bits, a scale or shift past any use take the other way.  For int32
+// activations: 8-bit launches, whose registers are a third fewer, spill over it (block ends 195 -> 208 us) and gain nothing.
+// 64 channels of 56 x 56, 3 x 3, 64 images: 87.6 -> 84.3 us; 16 of 32 x 32, 256 images: 30.0 -> 29.2; 64 -> 256, 1 x 1: 278 -> 258.
+template <int CHANNELS>
+__device__ __forceinline__ void stage_tails(const MfmaArgs &a, ChannelTails<CHANNELS> &t, const TailOfThread &r, int count)
+{
+    const int i = threadIdx.x;
+    const float folded = r.scale * a.inv;
+    const bool plain = folded * a.unfold == r.scale && fabsf(r.scale) < 0x1p60f && fabsf(r.shift) < 0x1p60f;
+    if (i < count) {
+        t.add[i] = r.add;
+        t.scale[i] = r.scale;
+        t.shift[i] = r.shift;
+        t.scale1[i] = folded * a.qfold;
+        t.shift1[i] = r.shift * a.qfold;
+    }
+    const int odd = __any(i < count && !plain) ? 1 : 0;
+    if ((i & 63) == 0 && i < 256) t.odd[i >> 6] = odd;
 }
 struct ChannelTail {
     int32_t add[kUnit];
@@ -1115,37 +1151,9 @@ __device__ __forceinline__ void quantize_all(const float (&f)[kUnit], int32_t (&
         for (int i = 0; i < kUnit; ++i) q[i] = quantize_one(f[i], s);
     }
 }
-__device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail &t, const int32_t (&sum)[kUnit],
-                                           const float (&res)[kUnit], int ch0, const OutAt &o)
+// The next layer's input of a unit, quantised.
+__device__ __forceinline__ void store_q(const MfmaArgs &a, int32_t (&qv)[kUnit], int ch0, const OutAt &o)
 {
-    int32_t v[kUnit];
-#pragma unroll
-    for (int i = 0; i < kUnit; ++i) v[i] = sum[i] + t.add[i];
-    if (a.y) {
-        store_channels(a.y + o.i, v, ch0, a.ostride_c, a.N, o.in);
-        return;
-    }
-    float f[kUnit];
-    if (a.residual) {
-#pragma unroll
-        for (int i = 0; i < kUnit; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], &res[i], 0);
-    } else {
-#pragma unroll
-        for (int i = 0; i < kUnit; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], nullptr, 0);
-    }
-    if (a.relu)
-#pragma unroll
-        for (int i = 0; i < kUnit; ++i) f[i] = fmaxf(f[i], 0.0f);
-    if (a.out) store_channels(a.out + o.i, f, ch0, a.ostride_c, a.N, o.in);
-    if (!a.q) return;
-    int32_t qv[kUnit];
-    if (a.relu && a.qspec.I != 1) {
-        // neither negative nor NaN: the conversion's truncation is the floor, the lower bound is met
-#pragma unroll
-        for (int i = 0; i < kUnit; ++i) qv[i] = f2i_sat(fminf(f[i] * a.qspec.scale, a.qspec.hi));
-    } else {
-        quantize_all(f, qv, a.qspec);
-    }
     if (a.qflags) {
         if ((ch0 & ~15) + 2 * kUnit > a.N)
 #pragma unroll
@@ -1160,6 +1168,59 @@ __device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail 
     } else {
         store_channels((int32_t *)a.q + o.j, qv, ch0, a.qHp * a.qWp, a.N, o.in);
     }
+}
+// What follows the affine step.
+__device__ __forceinline__ void store_values(const MfmaArgs &a, float (&f)[kUnit], const float (&res)[kUnit], int ch0, const OutAt &o)
+{
+    if (a.residual)
+#pragma unroll
+        for (int i = 0; i < kUnit; ++i) f[i] += res[i];
+    if (a.relu)
+#pragma unroll
+        for (int i = 0; i < kUnit; ++i) f[i] = fmaxf(f[i], 0.0f);
+    if (a.out) store_channels(a.out + o.i, f, ch0, a.ostride_c, a.N, o.in);
+    if (!a.q) return;
+    int32_t qv[kUnit];
+    if (a.relu && a.qspec.I != 1) {
+        // neither negative nor NaN: the conversion's truncation is the floor, the lower bound is met
+#pragma unroll
+        for (int i = 0; i < kUnit; ++i) qv[i] = f2i_sat(fminf(f[i] * a.qspec.scale, a.qspec.hi));
+    } else {
+        quantize_all(f, qv, a.qspec);
+    }
+    store_q(a, qv, ch0, o);
+}
+__device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail &t, const int32_t (&sum)[kUnit],
+                                           const float (&res)[kUnit], int ch0, const OutAt &o)
+{
+    int32_t v[kUnit];
+#pragma unroll
+    for (int i = 0; i < kUnit; ++i) v[i] = sum[i] + t.add[i];
+    if (a.y) {
+        store_channels(a.y + o.i, v, ch0, a.ostride_c, a.N, o.in);
+        return;
+    }
+    float f[kUnit];
+#pragma unroll
+    for (int i = 0; i < kUnit; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], nullptr, 0);
+    store_values(a, f, res, ch0, o);
+}
+// The shorter epilogue (stage_tails): sum is complete, scale and shift of t are the folded ones.
+__device__ __forceinline__ void store_tail_folded(const MfmaArgs &a, const ChannelTail &t, const int32_t (&sum)[kUnit],
+                                                  const float (&res)[kUnit], int ch0, const OutAt &o)
+{
+    float f[kUnit];
+#pragma unroll
+    for (int i = 0; i < kUnit; ++i) f[i] = affine_one(sum[i], 1.0f, t.scale[i], t.shift[i], nullptr, 0);
+    if (!a.q_only) {
+        store_values(a, f, res, ch0, o);
+        return;
+    }
+    // ReLU, the upper bound and the floor in two instructions a value
+    int32_t qv[kUnit];
+#pragma unroll
+    for (int i = 0; i < kUnit; ++i) qv[i] = f2i_sat(__builtin_amdgcn_fmed3f(f[i], 0.0f, a.qspec.hi));
+    store_q(a, qv, ch0, o);
 }
 
 // Four or eight waves per workgroup; a wave owns CT * 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
@@ -1196,31 +1257,36 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
         px01[p] = row + col * a.lay.px01 + (lane >> 5) * a.lay.half01;
     }
     const int tail0 = t % a.tc * (CT * 32) + 4 * (lane >> 5);   // the lane's first channel there
-    stage_tails(a, tails, ct * a.tc * (CT * 32), a.tc * (CT * 32));
-    __syncthreads();
+    const TailOfThread tail = ask_tail(a, ct * a.tc * (CT * 32), a.tc * (CT * 32));
+    // every wave comes here once, wherever its tile takes it
+    const auto staged = [&] {
+        stage_tails(a, tails, tail, a.tc * (CT * 32));
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
     v16i total[CT][NT] = {};
     if (live && kb0 < kb1) {
         const int8_t *w = a.blob + (size_t)(c0 >> 5) * (a.KB * mode_block(MODE));
-        if constexpr (mode_i8(MODE)) {
-            contract<MODE, CT, NT, false>(a, total, w, kb0, kb1, px, px01, at, lane);
-        } else {
+        int high = 0;
+        if constexpr (!mode_i8(MODE)) {
             const uint32_t last = p0 + NT * 32 - 1;
-            const int high = any_high(a, p0, last < a.pixels ? last : a.pixels - 1, lane);
-            if (high) {
-                if (high & 2) digit4<MODE, CT, NT>(a, part[wave], lane, w, kb0, kb1, px, at);
-                contract<MODE, CT, NT, true>(a, total, w, kb0, kb1, px, px01, at, lane);
-                if (high & 2)
+            high = any_high(a, p0, last < a.pixels ? last : a.pixels - 1, lane);
+            if (high & 2) digit4<MODE, CT, NT>(a, part[wave], lane, w, kb0, kb1, px, at);
+            if (high) contract<MODE, CT, NT, true>(a, total, w, kb0, kb1, px, px01, at, lane, staged);
+            if (high & 2)
 #pragma unroll
-                    for (int c = 0; c < CT; ++c)
+                for (int c = 0; c < CT; ++c)
 #pragma unroll
-                        for (int p = 0; p < NT; ++p)
+                    for (int p = 0; p < NT; ++p)
 #pragma unroll
-                            for (int i = 0; i < 16; ++i) total[c][p][i] += part[wave][(c * NT + p) * 16 + i][lane];
-            } else {
-                contract<MODE, CT, NT, false>(a, total, w, kb0, kb1, px, px01, at, lane);
-            }
+                        for (int i = 0; i < 16; ++i) total[c][p][i] += part[wave][(c * NT + p) * 16 + i][lane];
         }
+        if (!high) contract<MODE, CT, NT, false>(a, total, w, kb0, kb1, px, px01, at, lane, staged);
+    } else {
+        staged();
     }
+    const bool folded = !mode_i8(MODE) && WAVES == 4 && a.ks == 1 && !a.y && !(tails.odd[0] | tails.odd[1]);
     const int chl = c0 + 4 * (lane >> 5);
     if (a.ks == 1) {
         if (!live) return;
@@ -1232,6 +1298,28 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
         if (a.residual)
 #pragma unroll
             for (int u = 0; u < CT * 2 * NT; ++u) load_residual(a, res[u], chl + u / NT * 16, o[u % NT]);
+        if (folded) {
+#pragma unroll
+            for (int c = 0; c < CT * 2; ++c) {
+                asm volatile("" ::: "memory");   // the constants of one unit at a time
+                ChannelTail tl;
+#pragma unroll
+                for (int i = 0; i < kUnit; ++i) {
+                    const int ch = tail0 + c * 16 + 8 * (i >> 2) + (i & 3);
+                    tl.add[i] = tails.add[ch];
+                    tl.scale[i] = tails.scale1[ch];
+                    tl.shift[i] = tails.shift1[ch];
+                }
+#pragma unroll
+                for (int p = 0; p < NT; ++p) {
+                    int32_t v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = total[c >> 1][p][(c & 1) * 8 + i] + tl.add[i];
+                    store_tail_folded(a, tl, v, res[c * NT + p], chl + c * 16, o[p]);
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int c = 0; c < CT * 2; ++c) {
             ChannelTail tl;
@@ -1312,7 +1400,7 @@ __global__ __launch_bounds__(256, 2) void mfma_pool_kernel(MfmaArgs a, MfmaPool 
     const int h0 = (int)(tiles - n * m.tiles_h) * m.th;
     const int r0 = h0 * m.ps - m.pp, q0 = w0 * m.ps - m.pp;   // the rectangle's first row and column
     const int pixels = m.PH * m.PW;
-    stage_tails(a, tails, c0, 64);
+    stage_tails(a, tails, ask_tail(a, c0, 64), 64);
     if (threadIdx.x < 64) flips[threadIdx.x] = tails.scale[threadIdx.x] < 0.0f ? -1 : 0;
     __syncthreads();
     const int8_t *w = a.blob + (size_t)(c0 >> 5) * (a.KB * mode_block(MODE));
@@ -1332,19 +1420,20 @@ __global__ __launch_bounds__(256, 2) void mfma_pool_kernel(MfmaArgs a, MfmaPool 
         const uint32_t px[1] = {row + col * a.lay.cp + (lane >> 5) * 16};
         const uint32_t px01[1] = {row + col * a.lay.px01 + (lane >> 5) * a.lay.half01};
         v16i total[2][1];
+        const auto none = [] {};
         int32_t (*slot)[64] = (int32_t (*)[64])(sums + t * 32 * kPoolStride);   // this tile's own place, before its sums
         if constexpr (mode_i8(MODE)) {
-            contract<MODE, 2, 1, false>(a, total, w, 0, a.KB, px, px01, at, lane);
+            contract<MODE, 2, 1, false>(a, total, w, 0, a.KB, px, px01, at, lane, none);
         } else if (high) {
             if (high & 2) digit4<MODE, 2, 1>(a, slot, lane, w, 0, a.KB, px, at);
-            contract<MODE, 2, 1, true>(a, total, w, 0, a.KB, px, px01, at, lane);
+            contract<MODE, 2, 1, true>(a, total, w, 0, a.KB, px, px01, at, lane, none);
             if (high & 2)
 #pragma unroll
                 for (int c = 0; c < 2; ++c)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) total[c][0][i] += slot[c * 16 + i][lane];
         } else {
-            contract<MODE, 2, 1, false, true>(a, total, w, 0, a.KB, px, px01, at, lane);
+            contract<MODE, 2, 1, false, true>(a, total, w, 0, a.KB, px, px01, at, lane, none);
         }
         asm volatile("" ::: "memory");   // the constants are read here, not kept in 96 registers through the loop
 #pragma unroll
@@ -1768,6 +1857,9 @@ static int mfma_conv2d_any(const void *prepared, const void *blob, const int32_t
     a.qWp = columns + 2 * pw;
     if (q && (double)a.qHp * a.qWp > 2147483647.0) return DS_EINVAL;
     a.inv = ldexpf(1.0f, -F_in);
+    a.unfold = ldexpf(1.0f, F_in);
+    a.q_only = q && !out && !residual && relu && I != 1;
+    a.qfold = a.q_only ? ldexpf(1.0f, F) : 1.0f;
     a.qspec = make_spec(I, F, DS_Q_ROUND_TO_FIXED);
     a.by_image = fast_div((uint32_t)(a.OH * a.OW));
     a.by_row = fast_div((uint32_t)a.OW);

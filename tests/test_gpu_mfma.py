@@ -389,3 +389,31 @@ def test_windows_without_a_form_keep_their_pass():
     assert serves(8, 8, 3, 2, 1) == 1 and serves(1, 1, 1, 1, 0) == 1 and serves(11, 11, 11, 1, 0) == 1
     assert serves(8, 8, 12, 1, 0) == 0 and serves(8, 8, 3, 2, 2) == 0 and serves(2, 8, 3, 1, 0) == 0 and serves(8, 8, 3, 0, 1) == 0
     assert not kernels.mfma_pool_serves(1, 8, 8, 32, (3, 2, 1)) and not kernels.mfma_pool_serves(64, 1024, 1024, 64, (3, 2, 1))
+
+
+@pytest.mark.parametrize("x_bytes", [4, 1])
+@pytest.mark.parametrize("O", [64, 40])
+def test_scales_without_a_shorter_epilogue(rng, x_bytes, O):
+    """Constants that powers of two cannot be multiplied into -- a scale next to the smallest floats, one whose product with
+    2^-F has no normal form, huge and infinite ones, NaN -- beside ordinary ones, in launches with many tiles, whose epilogue
+    multiplies them in where it can: float and quantised results against the separate pass."""
+    C, Nb, H, k = 32, 33, 33, 1
+    F_in, I, F, dtype = (16, 16, 16, torch.int32) if x_bytes == 4 else (5, 3, 5, torch.int8)
+    s, sign, cw = _weights(rng, (O, C, k, k), 6, ternary=False)
+    x = _dev(_activations(rng, (Nb, C, H, H), x_bytes, 1 << 18))
+    prepared, blob, top = kernels.mfma_route(x, 0, cw, O, (k, k), x_bytes)
+    y = kernels.mfma_conv2d(prepared, blob, None, O, (k, k), 1, top)
+    for at, scale_at, shift_at in ((None, None, None), (3, 2.0 ** -120 * 1.2345678, 0.5), (5, 1.1e-38, 0.0), (7, 1e-45, 1e-45),
+                                   (9, float("inf"), 0.0), (1, float("nan"), 1.0), (2, 3e38, -3e38), (0, 0.0, float("nan")),
+                                   (4, -2.0 ** 70, 2.0 ** 70), (6, 1.0, float("inf"))):
+        scale, shift = torch.rand(O, device=DEV) + 0.5, torch.randn(O, device=DEV)
+        if at is not None:
+            scale[at], shift[at] = scale_at, shift_at
+        for relu in (True, False):
+            f, q = kernels.requantize_affine_pad(y, F_in, scale, shift, None, relu, (1, 1), I, F, True, dtype)
+            args = (prepared, blob, None, O, (k, k), 1, top, 0, F_in, scale, shift, None, relu, ((1, 1), I, F, dtype))
+            out, got = kernels.mfma_conv2d(*args, True)
+            assert torch.equal(out.view(torch.int32), f.view(torch.int32)) or torch.equal(torch.nan_to_num(out, nan=7.0),
+                                                                                        torch.nan_to_num(f, nan=7.0))
+            assert torch.equal(got, q)
+            assert torch.equal(kernels.mfma_conv2d(*args, False)[1], q)
