@@ -417,7 +417,8 @@ struct MfmaArgs {
     int N, KB, FH, fwg, tapstep, tapstep01;
     int OH, OW, sh, sw, crop_h, crop_w;
     uint32_t pixels;
-    int ks, tc, ctiles, ptiles;   // K parts, channel tiles per workgroup, workgroups along channels and pixels
+    int ks, tc, ctiles;         // K parts, channel tiles per workgroup, workgroups along channels
+    uint32_t whole, tail_tile;  // workgroups that this holds for; the others share tiles of pixels from tail_tile on four ways
     long ostride_n;
     int ostride_c;
     int matrix;                 // pixels are matrix rows
@@ -1234,16 +1235,23 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroups are dealt to the eight XCDs in turn: give each XCD neighbouring tiles
-    uint32_t wg = blockIdx.x;
-    const uint32_t per = gridDim.x >> 3;
-    if (wg < per * 8) wg = (wg & 7) * per + (wg >> 3);
+    uint32_t wg = blockIdx.x, tile0 = 0;
+    const uint32_t per = a.whole >> 3;
+    int ks = a.ks;
+    if (wg >= a.whole) {
+        wg -= a.whole;
+        tile0 = a.tail_tile;
+        ks = 4;
+    } else if (wg < per * 8) {
+        wg = (wg & 7) * per + (wg >> 3);
+    }
     const uint32_t pt = div_by_uniform(wg, a.by_ctiles);
     const int ct = (int)(wg - pt * a.ctiles);
-    const int kpart = wave % a.ks, t = wave / a.ks;
-    const int pw = WAVES / a.ks / a.tc;   // pixel tiles per workgroup
+    const int kpart = wave % ks, t = wave / ks;
+    const int pw = WAVES / ks / a.tc;   // pixel tiles per workgroup
     const int c0 = (ct * a.tc + t % a.tc) * (CT * 32);
-    const uint32_t p0 = ((uint32_t)pt * pw + t / a.tc) * (NT * 32);
-    const int kb0 = (int)((long)a.KB * kpart / a.ks), kb1 = (int)((long)a.KB * (kpart + 1) / a.ks);
+    const uint32_t p0 = (tile0 + pt * pw + t / a.tc) * (NT * 32);
+    const int kb0 = (int)((long)a.KB * kpart / ks), kb1 = (int)((long)a.KB * (kpart + 1) / ks);
 
     const bool live = c0 < a.N && p0 < a.pixels;
     uint32_t pix[NT], px[NT], px01[NT];
@@ -1286,9 +1294,9 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
     } else {
         staged();
     }
-    const bool folded = !mode_i8(MODE) && WAVES == 4 && a.ks == 1 && !a.y && !(tails.odd[0] | tails.odd[1]);
+    const bool folded = !mode_i8(MODE) && WAVES == 4 && ks == 1 && !a.y && !(tails.odd[0] | tails.odd[1]);
     const int chl = c0 + 4 * (lane >> 5);
-    if (a.ks == 1) {
+    if (ks == 1) {
         if (!live) return;
         // units of 16 channels x 32 pixels; every residual is on its way before the first value is stored
         OutAt o[NT];
@@ -1344,7 +1352,7 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
     if (!live) return;
     // the ks waves of a tile share its epilogue, in halves of 32 x 32 values
     constexpr int all = CT * NT * 2;
-    const int units = all > a.ks ? all / a.ks : 1;
+    const int units = all > ks ? all / ks : 1;
     for (int u = kpart * units; u < (kpart + 1) * units && u < all; ++u) {
         const int ch = chl + (u >> 1) / NT * 32 + (u & 1) * 16;
         const uint32_t pp = p0 + (u >> 1) % NT * 32 + (lane & 31);
@@ -1357,7 +1365,7 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             v[i] = 0;
-            for (int s = 0; s < a.ks; ++s) v[i] += part[t * a.ks + s][u * 8 + i][lane];
+            for (int s = 0; s < ks; ++s) v[i] += part[t * ks + s][u * 8 + i][lane];
         }
         store_tail(a, tl, v, res, ch, o);
     }
@@ -1573,17 +1581,43 @@ __global__ __launch_bounds__(256) void mfma_operand_border_kernel(int8_t *__rest
     }
 }
 
+// ks waves to a tile; with `groups` (ks 1, CT 2), whole tiles for that many groups of four pixel tiles, and the pixel tiles
+// that are left shared four ways.
 template <int MODE, int CT, int NT, int WAVES>
-static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
+static int launch_tiles(MfmaArgs &a, int ks, long groups, hipStream_t st)
 {
-    const int ctiles = ceil_div(a.N, CT * 32);
+    const int ctiles = ceil_div(a.N, CT * 32), tiles = ceil_div((int)a.pixels, NT * 32);
     a.ks = ks;
     a.tc = CT == 1 && WAVES / a.ks >= 2 && ctiles > 1 ? 2 : 1;
     a.ctiles = ceil_div(ctiles, a.tc);
-    a.ptiles = ceil_div((int)a.pixels, NT * 32 * (WAVES / a.ks / a.tc));
     a.by_ctiles = fast_div((uint32_t)a.ctiles);
-    hipLaunchKernelGGL((mfma_kernel<MODE, CT, NT, WAVES>), dim3((unsigned)(a.ctiles * a.ptiles)), dim3(WAVES * 64), 0, st, a);
+    const int pw = WAVES / a.ks / a.tc;
+    long grid = (long)a.ctiles * ceil_div(tiles, pw);
+    a.whole = (uint32_t)grid;
+    if (groups > 0) {
+        a.whole = (uint32_t)(groups * a.ctiles);
+        a.tail_tile = (uint32_t)(groups * pw);
+        grid = a.whole + (tiles - groups * pw) * (long)a.ctiles;
+    }
+    hipLaunchKernelGGL((mfma_kernel<MODE, CT, NT, WAVES>), dim3((unsigned)grid), dim3(WAVES * 64), 0, st, a);
     return launch_status();
+}
+
+// Whole tiles would give some CUs a workgroup more than others: all get the same number, and the tiles that are left, which
+// a fraction of the chip would work on alone, are shared four ways.  Groups of four pixel tiles that stay whole; 0: not so.
+// What is left may be more the longer the reduction is (it pays for four starts and the meeting), and short reductions gain
+// only where a round is a good part of the launch.  us without and with, 64 channels, hand-off (left in tiles a CU):
+//   1280 tiles (1)     blocks 4: 15.4 12.5   9: 19.9 15.6   18: 28.2 21.4   36: 41.7 33.3   72: 81.2 71.1
+//   1536 and 2560 (2)  4: 15.6 18.3, 21.9 22.6   9: 20.0 24.0, 28.2 28.2   18: 28.6 27.5, 41.5 38.6   36: 43.8 40.1, 79.8 69.8
+//   1792 (3)           9: 20.3 24.2   18: 28.8 31.4   36: 48.2 48.1   72: 101 98
+// ResNet layers, 3 x 3, 64 images, of 64, 128, 256 channels, whose tiles are 49 times a power of two: 89 80, 80 66, 74 71; 8-bit
+// 42 38, 41 33, 37 34; 128 images of 256 channels of 14 x 14 134 117, 8-bit 68 54; 1024 -> 256, 1 x 1, 8-bit: 37 30.
+static long even_groups(const MfmaArgs &a, long cus)
+{
+    const long ctiles = ceil_div(a.N, 64), tiles = ceil_div((int)a.pixels, 32), grid = ctiles * ((tiles + 3) / 4);
+    if (grid <= cus || (a.KB < 8 && grid > 4 * cus)) return 0;
+    const long groups = grid / cus * cus / ctiles, left = (tiles - groups * 4) * ctiles;
+    return left > 0 && left <= (a.KB >= 32 ? 3 : a.KB >= 16 ? 2 : 1) * cus ? groups : 0;
 }
 
 // Waves that share a tile's reduction, of `blocks` blocks.  Waves in one workgroup also share a tile's epilogue, which is most
@@ -1602,13 +1636,10 @@ static int launch_tiles(MfmaArgs &a, int ks, hipStream_t st)
 //     9             8.7  8.2  7.5    8.8  9.4  8.3     8.9  9.5 11.9    11.4 11.3 14.5    14.9 17.6 22.4    19.3 25.7 34.1
 //     18           11.2  9.4  8.6   11.4 11.3 10.1    11.5 11.6 13.5    15.9 15.2 17.2    21.4 22.1 26.9    27.4 32.3 40.8
 //     36           16.3 11.9 10.6   16.6 15.6 13.1    17.7 16.6 17.4    24.4 21.2 22.8    33.3 32.0 35.8    44.3 48.0 55.0
-// Very long ones take four up to seven tiles a CU, unless their activations are read once, from memory (256 -> 256 channels,
-// 3 x 3, 64 images of 14 x 14, 1568 tiles of 72 blocks: 77.6, 79.1, 73.6; 2304 -> 64, 1 x 1, as many: 96, 102, 105).
-static int reduction_parts(long tiles, long cus, int blocks, bool i8, bool rereads)
+static int reduction_parts(long tiles, long cus, int blocks, bool i8)
 {
     if (tiles <= 2 * cus || (tiles <= 3 * cus && blocks >= (i8 ? 9 : 32))) return 4;
     if (tiles <= 6 * cus) return blocks >= 16 ? 2 : 1;
-    if (tiles <= 7 * cus && blocks >= 64 && rereads) return 4;
     return !i8 && blocks >= 32 && tiles > 8 * cus && tiles < 16 * cus ? 2 : 1;
 }
 
@@ -1620,9 +1651,10 @@ static int launch_mfma(MfmaArgs &a, hipStream_t st)
     const long tiles = pair ? (long)ceil_div(a.N, 64) * ceil_div((int)a.pixels, 32) : (long)ceil_div((int)a.pixels, 64);
     // Fewer than a tile for every other CU: half the tile, and the reduction in eight parts (64 and 128 tiles, us with four
     // parts and these: 4 blocks 8.0, 7.8; 18: 9.9, 9.1; 36: 11.9, 10.5; 144: 28.4, 21.0; 256 tiles: 30.9, 41.2).
-    if (tiles <= cus / 2) return launch_tiles<MODE, 1, 1, 8>(a, 8, st);
-    const int ks = reduction_parts(tiles, cus, a.KB, mode_i8(MODE), a.N > 64 || a.FH * a.fwg > 1);
-    return pair ? launch_tiles<MODE, 2, 1, 4>(a, ks, st) : launch_tiles<MODE, 1, 2, 4>(a, ks, st);
+    if (tiles <= cus / 2) return launch_tiles<MODE, 1, 1, 8>(a, 8, 0, st);
+    const long groups = pair ? even_groups(a, cus) : 0;
+    const int ks = groups ? 1 : reduction_parts(tiles, cus, a.KB, mode_i8(MODE));
+    return pair ? launch_tiles<MODE, 2, 1, 4>(a, ks, groups, st) : launch_tiles<MODE, 1, 2, 4>(a, ks, 0, st);
 }
 
 // The rectangle of pooled pixels of a workgroup, whose convolution takes at most `limit` pixels: the one with the fewest tiles

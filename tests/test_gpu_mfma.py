@@ -417,3 +417,35 @@ def test_scales_without_a_shorter_epilogue(rng, x_bytes, O):
                                                                                         torch.nan_to_num(f, nan=7.0))
             assert torch.equal(got, q)
             assert torch.equal(kernels.mfma_conv2d(*args, False)[1], q)
+
+
+# (tiles of 64 channels x 32 pixels per CU at least, x_bytes, C, O, images of H x W): launches whose whole tiles end with
+# workgroups on some CUs only, by how much is left and how long the reduction is; the last tiles end inside one
+UNEVEN = [(4, 4, 32, 64, (5, 91, 91)), (4, 1, 40, 70, (3, 85, 83)), (5, 4, 70, 128, (6, 61, 61)), (6, 1, 128, 256, (49, 15, 17)),
+          (6, 4, 128, 100, (7, 59, 60)), (4, 4, 320, 640, (1, 61, 71))]
+
+
+@pytest.mark.parametrize("x_bytes,C,O,images", [c[1:] for c in UNEVEN], ids=lambda v: str(v).replace(" ", ""))
+def test_tiles_that_are_left_are_shared(oracle, rng, x_bytes, C, O, images):
+    """Sums against the oracle, and the epilogue of whole and shared tiles against the separate pass, with digits 3 and 4 in
+    the shared ones."""
+    Nb, H, W = images
+    tiles = -(-Nb * H * W // 32) * -(-O // 64)
+    assert tiles > 1024
+    s, sign, cw = _weights(rng, (O, C, 3, 3), 14, ternary=False)
+    x = _activations(rng, (Nb, C, H, W), x_bytes, 1 << 18)
+    if x_bytes == 4:
+        x[-1, :, -2:] <<= 6
+        x[-1, ..., -1] = -2 ** 31
+    bias = rng.integers(-2 ** 20, 2 ** 20, size=O).astype(np.int32)
+    prepared, blob, top = kernels.mfma_route(_dev(x), 1, cw, O, (3, 3), x_bytes)
+    y = kernels.mfma_conv2d(prepared, blob, _dev(bias), O, (3, 3), 1, top)
+    xp = np.pad(x.astype(np.int32), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    np.testing.assert_array_equal(y.cpu().numpy(), oracle.conv2d(xp, -s.astype(np.int32), sign.astype(np.int32), bias, (1, 1),
+                                                                 nthreads=16))
+    F_in, I, F, dtype = (16, 16, 16, torch.int32) if x_bytes == 4 else (5, 3, 5, torch.int8)
+    scale, shift, res = (torch.rand(O, device=DEV) + 0.5), torch.randn(O, device=DEV), torch.randn(y.shape, device=DEV)
+    f, q = kernels.requantize_affine_pad(y, F_in, scale, shift, res, True, (1, 1), I, F, True, dtype)
+    args = (prepared, blob, _dev(bias), O, (3, 3), 1, top, 0, F_in, scale, shift, res, True, ((1, 1), I, F, dtype, (3, 3)))
+    out, handed = kernels.mfma_conv2d(*args, True)
+    assert torch.equal(out, f) and torch.equal(handed.padded(), q)
