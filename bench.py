@@ -32,12 +32,12 @@ LANE_OPS = CU_COUNT * LANES_PER_CU * CLOCK_HZ  # 39.3e12 int32 lane-operations p
 # operand can be shared between output channels, which is what the shift-plane kernels do), so no int32
 # vector kernel can exceed 39.3 Tpair/s.
 PEAK_PAIRS = LANE_OPS / 1.0
-# The matrix-core kernels spend a fixed number of int8 products per pair (1024 per clock and SIMD): 18 for shifts up
-# to 14 on int32 activations, one per distinct shift (8 or 3 here) on 8-bit activations.
+# The matrix-core kernels spend a fixed number of sparse int8 products per pair (1024 per clock and SIMD that count, of
+# 2048 places): 10 for shifts up to 14 on int32 activations, 4 (2 for shifts up to 3) on 8-bit activations.
 MFMA_PRODUCTS = CU_COUNT * 4 * 1024 * CLOCK_HZ
-PEAK_PAIRS_MFMA = MFMA_PRODUCTS / 18
-PEAK_PAIRS_MFMA_ACT8 = MFMA_PRODUCTS / 8
-PEAK_PAIRS_MFMA_ACT8_2BIT = MFMA_PRODUCTS / 3
+PEAK_PAIRS_MFMA = MFMA_PRODUCTS / 10
+PEAK_PAIRS_MFMA_ACT8 = MFMA_PRODUCTS / 4
+PEAK_PAIRS_MFMA_ACT8_2BIT = MFMA_PRODUCTS / 2
 # secondary figure: a kernel that shifts and accumulates every pair separately (v_ashrrev_i32 + v_xad_u32)
 PEAK_PAIRS_TWO_INSTR = LANE_OPS / 2.0
 HBM_PEAK = 8.0e12
@@ -46,7 +46,7 @@ BATCH = 64
 CHW = (3, 224, 224)
 
 # the kernel behind the 3x3 convolutions of the headline network, as rocprofv3 names it
-DOMINANT_KERNEL = "ds::mfma_kernel<0, 2, 4>"
+DOMINANT_KERNEL = "ds::mfma_kernel<0, 2, 1, 4>"
 
 
 def log(*a):
@@ -386,7 +386,7 @@ def graph_replay_timing(fused, x, steps):
 
 def config5(device, steps=5):
     """Benchmark configuration 5: ResNet-50, batch 128, weight_bits 3 (2-bit shift fields), activations
-    3.5 (8 bits): the convolutions on the matrix-core kernels, three int8 products per pair."""
+    3.5 (8 bits): the convolutions on the matrix-core kernels, two sparse int8 products per pair."""
     from deepshift_amd import workloads
     return fused_model_timing(device, workloads.ResNet50, 128, 3, 3, 5,
                               "ResNet-50, batch 128 x 3x224x224, weight_bits 3, activations 3.5", steps,
@@ -395,7 +395,7 @@ def config5(device, steps=5):
 
 def config4_act8(device, steps=5):
     """The headline network with the reference's 8-bit activation format (`-ab 3 5`, weight_bits 5):
-    the convolutions on the matrix-core kernels, eight int8 products per pair."""
+    the convolutions on the matrix-core kernels, four sparse int8 products per pair."""
     from deepshift_amd import workloads
     return fused_model_timing(device, workloads.ResNet18, BATCH, 5, 3, 5,
                               "ResNet-18, batch 64 x 3x224x224, weight_bits 5, activations 3.5", steps,
@@ -886,8 +886,8 @@ def main():
         "shift_gops": 2 * pairs / kernel_s / 1e9,
         "shift_layers_images_per_s": BATCH / kernel_s,
         "roofline": {
-            # Bound: matrix cores.  peak = 256 CUs x 4 SIMDs x 1024 int8 products per clock x 2.4 GHz / 18 products
-            # per pair = 139.8 Tpair/s.  achieved = the pairs of the dominant kernel's launches / their duration in
+            # Bound: matrix cores.  peak = 256 CUs x 4 SIMDs x 1024 int8 products per clock x 2.4 GHz / 10 products
+            # per pair = 251.7 Tpair/s.  achieved = the pairs of the dominant kernel's launches / their duration in
             # this run, timed with HIP events around runs of those launches (replay_timing);
             # avg_launch_us_in_step: an event pair around each one.
             "bound": "mfma",
