@@ -1044,9 +1044,9 @@ def mfma_pool_serves(Nb, OH, OW, O, pool):
 
 def _layout_pass_pays(Nb, H, W, K, O, stride, one_tap):
     """Whether the matrix cores win by more than their layout pass against kernels that read an unpadded int32 input as it
-    is, in one launch.  Us there and here, 128 x 56 x 56 images, 1 x 1: 4 -> 64 channels 24, 68; 24 -> 128: 84, 103;
-    32 -> 64: 63, 66; 32 -> 128: 117, 103; 64 -> 16: 46, 69; 3 x 3: 4 -> 64: 60, 67.  Small images, where two launches
-    cost the host 23: K = 24: 15, K = 32 and 36: 17 to 22, K = 64: 25."""
+    is, in one launch.  Us there and here, 128 x 56 x 56 images, 1 x 1: 4 -> 64 channels 25, 62; 24 -> 128: 91, 92;
+    32 -> 64: 63, 57; 32 -> 128: 116, 92; 40 -> 64: 72, 76; 64 -> 16: 44, 64; 64 -> 64: 98, 85; 3 x 3: 4 -> 64: 59, 51.
+    8 x 14 x 14 images, where two launches cost the host 17: K = 24: 14, K = 32 and 36: 17, K = 64: 25."""
     sh, sw = _pair(stride)
     pixels = Nb * (H // sh) * (W // sw)
     if K <= 40:
