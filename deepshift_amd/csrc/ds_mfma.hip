@@ -197,7 +197,7 @@ struct PrepArgs {
     MfmaX lay;
     int C, H, W, ph, pw;
     int M, K;        // rows of a matrix: image n holds rows 64 n .. 64 n + 63, C = K
-    int vec;         // a matrix whose rows can be read four values at a time
+    int vec;         // a matrix of 32-bit values whose rows can be read four at a time
     int per, rpw;    // items of a row's part, rows per workgroup
     FastDiv by_per, by_wp, by_hp;
     QuantSpec spec;
@@ -250,7 +250,10 @@ __device__ __forceinline__ void prep_values(const PrepArgs &a, int n, int h, int
         const int m = n * 64 + wp;
         in = m < a.M;
         const size_t base = (size_t)(in ? m : 0) * a.K;
-        if (a.vec) {
+        if (SRC == kSrcI8) {
+#pragma unroll
+            for (int i = 0; i < CH; ++i) raw[i] = ((const int8_t *)a.x)[base + (c0 + i < a.K ? c0 + i : 0)];
+        } else if (a.vec) {
             // rows and base aligned: four values per load
 #pragma unroll
             for (int q = 0; q < CH / 4; ++q) {

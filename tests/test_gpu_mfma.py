@@ -82,6 +82,27 @@ def test_matrices_match_the_oracle(oracle, rng, M, K, N):
         np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("M,K,N", [(1, 7, 3), (63, 33, 31), (64, 64, 64), (65, 129, 70), (130, 1001, 33)])
+def test_8_bit_matrices_match_the_oracle(oracle, rng, M, K, N):
+    """Bytes are read as bytes, at any address, four times as many to a word as the other sources have: rows, columns and
+    channels at the edges of 64, 32 and 4, and the prepared bytes themselves against those of the same values from float."""
+    for top in (14, 3):
+        s, sign, cw = _weights(rng, (N, K), top, ternary=False)
+        x = _activations(rng, (M, K), 1, 128)
+        want = oracle.linear(x.astype(np.int32), -s.astype(np.int32), sign.astype(np.int32), None)
+        base = torch.empty(M * K + 1, dtype=torch.int8, device=DEV)
+        base[1:] = _dev(x).reshape(-1)
+        blob = kernels._mfma_of(cw, top, 1, N, K, 1, 1)
+        floats = kernels.mfma_prepare(_dev(x).clamp(max=96).float() / 32, 0, (1, 1), 1, 3, 5)
+        same = kernels.mfma_prepare(_dev(x).clamp(max=96), 0, (1, 1), 1)
+        used = (M + 63) // 64 * ((K + 31) // 32) * 64 * 32
+        assert torch.equal(same.data[:used], floats.data[:used])
+        for xd in (_dev(x), base[1:].view(M, K)):
+            prepared = kernels.mfma_prepare(xd, 0, (1, 1), 1)
+            got = kernels.mfma_conv2d(prepared, blob, None, N, (1, 1), 1, top)
+            np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("x_bytes", [4, 1])
 @pytest.mark.parametrize("Nb,C,H,O,k,st", [(2, 32, 14, 40, 3, 1), (1, 64, 7, 96, 1, 1), (40, 32, 28, 64, 3, 2)])
 def test_epilogue_matches_the_separate_passes(rng, x_bytes, Nb, C, H, O, k, st):
