@@ -91,6 +91,7 @@ SIGNATURES = {
     "ds_mfma_prepare": (_c_int, [_ptr, _c_int, _ptr] + [_c_int] * 13 + [_ptr]),
     "ds_mfma_conv2d": (_c_int, [_ptr] * 9 + [_c_int] * 28 + [_ptr]),
     "ds_mfma_pool_serves": (_c_int, [_c_int] * 5),
+    "ds_mfma_pool_pays": (_c_int, [_c_int] * 12),
     "ds_mfma_conv2d_packed": (_c_int, [ctypes.c_char_p, ctypes.c_char_p, _ptr]),
     "ds_mfma_conv2d_pool": (_c_int, [_ptr] * 7 + [_c_int] * 28 + [_ptr]),
     "ds_quantize_f32_i32": (_c_int, [_ptr, _ptr, _c_i64, _c_int, _c_int, _c_int, _ptr]),

@@ -1660,28 +1660,74 @@ static int launch_mfma(MfmaArgs &a, hipStream_t st)
     return pair ? launch_tiles<MODE, 2, 1, 4>(a, ks, groups, st) : launch_tiles<MODE, 1, 2, 4>(a, ks, 0, st);
 }
 
-// The rectangle of pooled pixels of a workgroup, whose convolution takes at most `limit` pixels: the one with the fewest tiles
-// of 32 pixels over an image.
-static bool pool_tile(MfmaPool &m, int limit)
+// Workgroups of a fused pooling launch, two a CU, one after another: how long it takes, in rounds -- one tile of 32 pixels for
+// each of a workgroup's four waves -- of a CU that has two of them.  A round without a second workgroup takes 0.8 of that.
+static double pool_rounds(long workgroups, int tiles, long cus)
 {
-    long best = 0;
-    for (int th = 1; th <= m.POH; ++th) {
-        const long PH = (long)(th - 1) * m.ps + m.pk;
-        if (PH * m.pk > limit) break;
-        long tw = (limit / PH - m.pk) / m.ps + 1;   // the widest, then as wide as that many in a row need to be
-        if (tw > m.POW) tw = m.POW;
-        const int across = ceil_div(m.POW, (int)tw);
-        tw = ceil_div(m.POW, across);
-        const long PW = (tw - 1) * m.ps + m.pk;
-        const long spent = (long)ceil_div(m.POH, th) * across * ((PH * PW + 31) / 32);
-        if (best && spent >= best) continue;
-        best = spent;
-        m.th = th;
-        m.tw = (int)tw;
-        m.PH = (int)PH;
-        m.PW = (int)PW;
-    }
-    return best > 0;
+    const long rest = workgroups % (2 * cus);
+    return ceil_div(tiles, 4) * (workgroups / (2 * cus) + (rest == 0 ? 0.0 : rest <= cus ? 0.8 : 1.0));
+}
+
+// The rectangle of pooled pixels of a workgroup, whose convolution takes at most kPoolPixels: the one whose launch takes the
+// fewest rounds, of these the one with the fewest tiles, and the largest of those.  Returns the rounds.
+static double pool_tile(MfmaPool &m, long images, long cus)
+{
+    double best = 0;
+    long least = 0, fewest = 0;
+    for (int limit = kPoolPixels; limit >= 128; limit /= 2)
+        for (int th = 1; th <= m.POH; ++th) {
+            const long PH = (long)(th - 1) * m.ps + m.pk;
+            if (PH * m.pk > limit) break;
+            long tw = (limit / PH - m.pk) / m.ps + 1;   // the widest, then as wide as that many in a row need to be
+            if (tw > m.POW) tw = m.POW;
+            const int down = ceil_div(m.POH, th), across = ceil_div(m.POW, (int)tw);
+            tw = ceil_div(m.POW, across);
+            const long PW = (tw - 1) * m.ps + m.pk, rectangles = (long)down * across;
+            const int tiles = (int)((PH * PW + 31) / 32);
+            const double rounds = pool_rounds(images * rectangles, tiles, cus);
+            const long spent = rectangles * tiles;
+            if (best > 0 && (rounds > best || (rounds == best && (spent > least || (spent == least && rectangles >= fewest))))) continue;
+            best = rounds;
+            least = spent;
+            fewest = rectangles;
+            m.th = th;
+            m.tw = (int)tw;
+            m.PH = (int)PH;
+            m.PW = (int)PW;
+            m.tiles_h = down;
+            m.tiles_w = across;
+        }
+    return best;
+}
+
+// Whether a convolution and the max pooling behind it take less time as one launch than as sums, a pooling pass and, as a
+// rule, a layout pass for the layer that reads the result: an estimate of both, in us, fitted to 240 shapes and 160 drawn ones.
+// The single launch multiplies pixels that rectangles share more than once, leaves waves idle in rectangles of odd sizes, and
+// never cuts a reduction: a round (pool_rounds) takes `block` per block of the reduction and 4.  The separate one writes and
+// reads the sums, 4 ns a tile, reads each as often as windows overlap, 0.4 ps a value more than the single launch does from LDS,
+// and has two more launches: 12, between what they take in a graph (7) and what they take the host (14).  us separate, fused,
+// issued one after another, with the next layer's operands (* fused; 3 x 3 convolutions, 2 x 2 windows unless said otherwise;
+// int32, then 8-bit activations, shifts to 14):
+//   7 x 7 stem of 224 x 224, 3 x 3 stride 2    1 image  24 14*  25 10*     8  40 30*  32 15*     64  224 156*  122 79*
+//   64 -> 64 channels of 224 x 224             1  40 29*  28 14*           8  175 146*  103 70*
+//   64 -> 128 of 112 x 112                     1  28 19*  24 10*           8  95 79*  59 37*     64  726 555*  460 246*
+//   128 -> 256 of 56 x 56                      1  26 29   25 14*           8  83 81*  50 38*     64  579 520*  306 238*
+//   256 -> 512 of 28 x 28                      1  25 50   25 23            8  83 79*  48 37*     64  500 522   260 245*
+//   512 -> 512 of 28 x 28                      1  37 117  24 41            8  144 154  75 74*    64  932 1060  462 479*
+//   512 -> 512 of 14 x 14                      1  25 116  24 39            8  52 115  31 41      64  253 309   130 146
+//   256 -> 256 of 13 x 13, 3 x 3 stride 2      1  25 49   24 23            8  25 49   24 23      64  75 77     44 36*
+//   64 -> 192 of 27 x 27, 5 x 5 then 3 x 3 / 2 1  24 37   24 18            8  38 38   25 18*     64  151 166   84 78
+//   32 images, 64 -> 64 of 32 x 32, stride 1   3 x 3  41 32*  32 15*       5 x 5  63 43*  55 24*     11 x 11  147 105*  138 61*
+//     512 -> 64                                3 x 3  101 159  58 74       5 x 5  124 242  81 95     11 x 11  209 619   166 289
+//   128 images, 64 -> 128 of 16 x 16  44 28*  34 13*       128 -> 256 of 8 x 8  43 42  30 20*       512 -> 512 of 2 x 2  29 228  24 83
+static bool pool_pays(const MfmaPool &m, int mode, int KB, long images, long pixels, int ctiles, long cus)
+{
+    MfmaPool tile = m;
+    const double block = mode == kI32S15 ? 0.95 : mode == kI32S7 ? 0.9 : mode == kI32S4 ? 0.5 : mode == kI8S8 ? 0.36 : 0.23;
+    const double tiles = (pixels + 31) / 32 * (double)ctiles;
+    const double looks = (double)images * ctiles * 64 * m.POH * m.POW * m.pk * m.pk;
+    const double fused = pool_tile(tile, images * ctiles, cus) * (KB * block + 4.0);
+    return fused <= 12.0 + (tiles / (8.0 * cus) + 0.07) * KB * block + tiles * 0.004 + looks * 0.4e-6;
 }
 
 template <int MODE>
@@ -1921,17 +1967,10 @@ static int mfma_conv2d_any(const void *prepared, const void *blob, const int32_t
                                a.qWp, ph, pw);
     }
     if (pool_k) {
-        // rectangles of up to 256 pixels; half of that where they would leave half of the chip without one
         a.ctiles = ceil_div(O, 64);
         a.by_ctiles = fast_div((uint32_t)a.ctiles);
-        long grid = 0;
-        for (int limit = kPoolPixels; limit >= 128; limit /= 2) {
-            if (!pool_tile(m, limit)) break;
-            m.tiles_h = ceil_div(m.POH, m.th);
-            m.tiles_w = ceil_div(m.POW, m.tw);
-            grid = (long)Nb * m.tiles_h * m.tiles_w * a.ctiles;
-            if (grid >= device_cus()) break;
-        }
+        pool_tile(m, (long)Nb * a.ctiles, device_cus());
+        const long grid = (long)Nb * m.tiles_h * m.tiles_w * a.ctiles;
         m.by_pw = fast_div((uint32_t)m.PW);
         m.by_tw = fast_div((uint32_t)m.tw);
         m.by_tiles_w = fast_div((uint32_t)m.tiles_w);
@@ -1987,6 +2026,22 @@ DS_EXPORT int ds_mfma_pool_serves(int OH, int OW, int pool_k, int pool_s, int po
 {
     if (pool_k < 1 || pool_s < 1 || pool_p < 0 || 2 * (long)pool_p > pool_k || pool_k > 11) return 0;
     return OH > 0 && OW > 0 && OH + 2 * (long)pool_p >= pool_k && OW + 2 * (long)pool_p >= pool_k;
+}
+
+DS_EXPORT int ds_mfma_pool_pays(int Nb, int C, int OH, int OW, int O, int FH, int FW, int max_shift, int x_bytes, int pool_k,
+                                int pool_s, int pool_p)
+{
+    if (Nb <= 0 || !ds_mfma_pool_serves(OH, OW, pool_k, pool_s, pool_p)) return 0;
+    if (ds_mfma_weight_bytes(O, C, FH, FW, max_shift, x_bytes) == 0) return 0;
+    const double pixels = (double)Nb * OH * OW;
+    if (pixels * O * 4 >= 2147483648.0) return 0;
+    MfmaPool m{};
+    m.pk = pool_k;
+    m.ps = pool_s;
+    m.pp = pool_p;
+    m.POH = (OH + 2 * pool_p - pool_k) / pool_s + 1;
+    m.POW = (OW + 2 * pool_p - pool_k) / pool_s + 1;
+    return pool_pays(m, mode_of(max_shift, x_bytes), mfma_geom(O, C, FH, FW).kb, Nb, (long)pixels, ceil_div(O, 64), device_cus());
 }
 
 DS_EXPORT int ds_mfma_conv2d_pool(const void *prepared, const void *blob, const int32_t *bias, float *out, void *q,

@@ -1037,9 +1037,22 @@ def _mfma_conv_serves(Nb, C, Hp, Wp, O, kernel_size, stride, x_bytes=4):
 
 
 def mfma_pool_serves(Nb, OH, OW, O, pool):
-    """Whether a convolution on the matrix cores takes the max pooling behind it into its launch: more than 32 channels (half
-    of its tiles of 64 would be padding), and the window and the size before the pooling have a form there."""
+    """Whether a convolution on the matrix cores can take the max pooling behind it into its launch: more than 32 channels
+    (half of its tiles of 64 would be padding), and the window and the size before the pooling have a form there."""
     return O > 32 and Nb * O * OH * OW < 1 << 29 and bool(_lib.lib().ds_mfma_pool_serves(OH, OW, *(int(v) for v in pool)))
+
+
+@functools.lru_cache(_SIZES)
+def _pool_pays(Nb, C, OH, OW, O, FH, FW, max_shift, x_bytes, pool):
+    return mfma_pool_serves(Nb, OH, OW, O, pool) and bool(_lib.lib().ds_mfma_pool_pays(Nb, C, OH, OW, O, FH, FW, max_shift, x_bytes, *pool))
+
+
+def mfma_pool_pays(prepared, O, kernel_size, stride, max_shift, pool):
+    """Whether :func:`mfma_conv2d` with ``pool`` takes less time than the layer's sums and a pass of its own for the pooling."""
+    Nb, C, Hp, Wp = prepared.dims
+    (FH, FW), (sh, sw) = _pair(kernel_size), _pair(stride)
+    return _pool_pays(Nb, C, (Hp - FH) // sh + 1, (Wp - FW) // sw + 1, int(O), FH, FW, int(max_shift), prepared.x_bytes,
+                      tuple(int(v) for v in pool))
 
 
 def _layout_pass_pays(Nb, H, W, K, O, stride, one_tap):

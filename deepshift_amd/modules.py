@@ -352,8 +352,8 @@ def _mfma_forward(module, input, conc_weight, scale, shift, residual, relu, preq
     bias = module._fixed_bias.get(module.bias, I, Fb, round_to_fixed=True)
     fused = _FUSE_EPILOGUE and (x_bytes == 4 or _FUSE_INT8)
     if fused and pool is not None:
-        sums = [(prepared.dims[2 + i] - module.kernel_size[i]) // module.stride[i] + 1 for i in (0, 1)]
-        fused = residual is None and kernels.mfma_pool_serves(Nb, *sums, module.out_channels, pool)
+        fused = residual is None and kernels.mfma_pool_pays(prepared, module.out_channels, module.kernel_size, module.stride,
+                                                            max_shift, pool)
     if not fused:
         out = kernels.mfma_conv2d(prepared, blob, bias, module.out_channels, module.kernel_size, module.stride, max_shift)
         return _separate_pass(out, Fb, scale, shift, residual, relu, pool, emit)

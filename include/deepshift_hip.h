@@ -427,6 +427,10 @@ int ds_mfma_conv2d(const void *prepared, const void *blob, const int32_t *bias, 
  * whether there is a form for that window on an OH x OW result (2 pool_p <= pool_k <= 11; 0 or 1); DS_EINVAL also for
  * results of 2 GB and more before the pooling. */
 int ds_mfma_pool_serves(int OH, int OW, int pool_k, int pool_s, int pool_p);
+/* Whether that launch is the faster one for a layer with these sizes (OH x OW before the pooling): 0 also where there is no
+ * form for it. */
+int ds_mfma_pool_pays(int Nb, int C, int OH, int OW, int O, int FH, int FW, int max_shift, int x_bytes, int pool_k, int pool_s,
+                      int pool_p);
 int ds_mfma_conv2d_pool(const void *prepared, const void *blob, const int32_t *bias, float *out, void *q,
                         const float *scale, const float *shift, int Nb, int C, int Hp, int Wp, int O, int FH, int FW,
                         int sh, int sw, int prep_FH, int prep_FW, int max_shift, int x_bytes, int F_in, int relu, int I,

@@ -405,6 +405,38 @@ def test_pooling_in_the_launch_matches_the_separate_pass(rng, top, x_bytes, shap
         assert torch.equal(got.padded(), q[:, :, 1:-1])
 
 
+# (Nb, C, H, O, k), pool, (I, F), whether the pooling runs in the launch: rectangles of one to eight tiles, with whole and half
+# limits, beside layers whose single launch would leave waves idle
+POOL_ROUTES = [((1, 128, 14, 128, 3), (2, 2, 0), (16, 16), False), ((3, 256, 13, 256, 3), (3, 2, 0), (16, 16), False), ((128, 64, 16, 128, 3), (2, 2, 0), (16, 16), True),
+               ((40, 16, 28, 40, 3), (2, 2, 0), (16, 16), True), ((33, 64, 13, 96, 1), (3, 2, 1), (16, 16), True), ((70, 64, 8, 70, 3), (2, 2, 0), (3, 5), True),
+               ((9, 512, 6, 512, 3), (2, 2, 0), (3, 5), False), ((5, 20, 31, 64, 5), (5, 1, 2), (3, 5), True)]
+
+
+@pytest.mark.parametrize("shape,pool,act,fused", POOL_ROUTES, ids=lambda v: str(v).replace(" ", ""))
+def test_pooled_layers_agree_on_both_routes(monkeypatch, shape, pool, act, fused):
+    """A pooled layer as modules route it -- in one launch, which hands operands on, or as sums and a pass of its own -- against
+    the separate pass."""
+    Nb, C, H, O, k = shape
+    torch.manual_seed(3)
+    layer = modules.Conv2dShift(C, O, k, padding=k // 2, use_kernel=True, act_integer_bits=act[0], act_fraction_bits=act[1]).to(DEV).eval()
+    layer.shift.data = torch.randint(-14, 1, layer.shift.shape, device=DEV).float()
+    layer.shift.data.view(-1)[0] = -14
+    layer.sign.data = torch.randint(0, 2, layer.sign.shape, device=DEV).float() * 2 - 1
+    x = torch.randn(Nb, C, H, H, device=DEV) * (40 if act[0] == 16 else 1)
+    scale, shift = torch.randn(O, device=DEV) * 0.1, torch.randn(O, device=DEV)
+    emit = ((1, 1), *act, True, torch.int8 if act[0] + act[1] <= 8 else torch.int32)
+    with torch.no_grad():
+        def run():
+            return modules.conv_kernel_forward(layer, x, layer.packed_weights(), scale, shift, None, True, False, emit, pool,
+                                               emit_filter=(3, 3))
+
+        f, q = run()
+        assert isinstance(q, kernels.Prepared) == fused
+        monkeypatch.setattr(modules, "_FUSE_EPILOGUE", False)
+        want_f, want_q = run()
+    assert torch.equal(f, want_f) and torch.equal(q.padded() if fused else q, want_q)
+
+
 def test_windows_without_a_form_keep_their_pass():
     serves = kernels._lib.lib().ds_mfma_pool_serves
     assert serves(8, 8, 3, 2, 1) == 1 and serves(1, 1, 1, 1, 0) == 1 and serves(11, 11, 11, 1, 0) == 1

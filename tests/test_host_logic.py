@@ -346,3 +346,20 @@ def test_small_linear_layers_are_routed_once(monkeypatch):
     cw = utils.ConcWeight(None, 0, 4, 0, 14)
     assert kernels.linear_forward(torch.zeros(8, 329), cw, None, 10, 16, 16, False) == "out"
     assert asked == [(8, 329, 10)] and launched == ["tiled"]
+
+
+# (images, channels, rows and columns before the pooling, output channels, filter), window: pooled in the convolution's launch?
+@pytest.mark.parametrize("Nb,C,OH,O,k,pool,int32,int8", [
+    (64, 3, 112, 64, 7, (3, 2, 1), True, True), (1, 3, 112, 64, 7, (3, 2, 1), True, True),     # stems
+    (64, 64, 112, 128, 3, (2, 2, 0), True, True), (128, 64, 16, 128, 3, (2, 2, 0), True, True),
+    (32, 64, 32, 64, 3, (11, 1, 5), True, True),                                               # the pass would look 121 times
+    (64, 512, 14, 512, 3, (2, 2, 0), False, False), (1, 512, 14, 512, 3, (2, 2, 0), False, False),
+    (1, 512, 28, 512, 3, (2, 2, 0), False, False), (1, 256, 13, 256, 3, (3, 2, 0), False, False),
+    (128, 512, 2, 512, 3, (2, 2, 0), False, False),
+    (32, 512, 32, 64, 3, (5, 1, 2), False, False), (32, 512, 16, 256, 5, (11, 1, 5), False, False),   # products twice and more
+    (1, 64, 8, 64, 3, (12, 1, 0), False, False), (1, 64, 8, 32, 3, (2, 2, 0), False, False)])         # no form
+def test_a_pooled_launch_is_taken_where_it_pays(Nb, C, OH, O, k, pool, int32, int8):
+    """Windows that make the single launch multiply pixels more than once, and reductions that it leaves to few waves, keep
+    sums and a pooling pass; layers that are bound by their sums do not."""
+    assert kernels._pool_pays(Nb, C, OH, OH, O, k, k, 14, 4, pool) == int32
+    assert kernels._pool_pays(Nb, C, OH, OH, O, k, k, 14, 1, pool) == int8
