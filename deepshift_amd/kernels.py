@@ -1055,16 +1055,26 @@ def mfma_pool_pays(prepared, O, kernel_size, stride, max_shift, pool):
                       tuple(int(v) for v in pool))
 
 
-def _layout_pass_pays(Nb, H, W, K, O, stride, one_tap):
+def _layout_pass_pays(Nb, H, W, C, taps, O, stride):
     """Whether the matrix cores win by more than their layout pass against kernels that read an unpadded int32 input as it
-    is, in one launch.  Us there and here, 128 x 56 x 56 images, 1 x 1: 4 -> 64 channels 25, 62; 24 -> 128: 91, 92;
-    32 -> 64: 63, 57; 32 -> 128: 116, 92; 40 -> 64: 72, 76; 64 -> 16: 44, 64; 64 -> 64: 98, 85; 3 x 3: 4 -> 64: 59, 51.
-    8 x 14 x 14 images, where two launches cost the host 17: K = 24: 14, K = 32 and 36: 17, K = 64: 25."""
+    is, in one launch.  Us there and here, shifts to 14, 128 x 56 x 56 images, and 8 x 14 x 14, where two launches cost the host
+    17.  Fewer than 32 terms: 24 -> 64 channels, 1 x 1: 51, 56 and 15, 18; 6 -> 64, 2 x 2: 46, 51 and 14, 17.  32 to 40 of
+    several taps: 4 -> 64, 3 x 3: 59, 52 and 17, 17; 8 -> 64, 2 x 2: 59, 51 and 17, 17; but 1 -> 128, 6 x 6: 92, 106 and 17, 17.
+    Of one tap, where channels past 32 fill a second block by little: 32 -> 16: 29, 42 and 18, 18; 32 -> 64: 63, 58 and 17, 19;
+    32 -> 128: 116, 93; 36 -> 32: 48, 59 and 17, 17; 36 -> 64: 64, 75 and 17, 17, of 32 images 34, 29; 40 -> 64: 70, 75 and 19, 17;
+    40 -> 128: 131, 119 and 19, 17.  More: 45 -> 64 (5, 3 x 3): 72, 54 and 20, 17; 48 -> 64: 77, 78 and 20, 17; 48 -> 16: 34, 60 and
+    22, 17; 64 -> 16: 44, 65; 64 -> 64: 98, 85 and 25, 17."""
     sh, sw = _pair(stride)
     pixels = Nb * (H // sh) * (W // sw)
-    if K <= 40:
-        return one_tap and K >= 32 and O >= 128 and pixels >= 1 << 15
-    return O > 16 or pixels < 1 << 18
+    if C * taps < 32:
+        return False
+    if C * taps > 40:
+        return O > 16 or pixels < 1 << 18
+    if taps > 1:
+        return C >= 4 or pixels < 1 << 18
+    if C == 32:
+        return O > 16 and pixels >= 1 << 14
+    return O >= 128 or pixels < (1 << 18 if O >= 64 else 1 << 15)
 
 
 def _mfma_linear(x, conc_weight, bias, N):
@@ -1325,7 +1335,7 @@ def conv2d(input, shift, sign, bias=None, conc_weight=None, stride=1, padding=0,
     if bias is not None:
         bias = _require_device_i32("bias", bias)
     if _mfma_conv_serves(Nb, C, H + 2 * ph, W + 2 * pw, O, (FH, FW), stride) and \
-            (ph or pw or _layout_pass_pays(Nb, H, W, C * FH * FW, O, stride, FH * FW == 1)):
+            (ph or pw or _layout_pass_pays(Nb, H, W, C, FH * FW, O, stride)):
         route = mfma_route(input, (ph, pw), conc_weight, O, (FH, FW), 4)
         if route is not None:
             return mfma_conv2d(route[0], route[1], bias, O, (FH, FW), stride, route[2])

@@ -366,6 +366,24 @@ def test_few_channels_agree_on_both_kernels(rng, C, O, k):
                        kernels.conv2d_tiled(padded, kernels._tiled_of(cw, O, C, k, k), None, O, (k, k), 1, kernels.kernel_bits(cw)))
 
 
+@pytest.mark.parametrize("C,k", [(4, 3), (8, 2), (9, 2), (1, 6), (32, 1), (33, 1), (40, 1)])
+@pytest.mark.parametrize("O", [24, 70])
+def test_short_unpadded_reductions_agree_on_both_routes(monkeypatch, oracle, rng, C, k, O):
+    """32 to 40 terms without padding, with and without the layout pass, whichever the rule takes: strides, an input whose
+    channels are not in order in memory, the whole range of activations."""
+    s, sign, cw = _weights(rng, (O, C, k, k), 14, ternary=True)
+    x = _activations(rng, (3, C, 11, 13), 4, 2 ** 31 - 1)
+    bias = rng.integers(-2 ** 20, 2 ** 20, size=O).astype(np.int32)
+    xd = _dev(x)
+    for stride in ((1, 1), (2, 1)):
+        want = oracle.conv2d(x, -s.astype(np.int32), sign.astype(np.int32), bias, stride)
+        for layout in (True, False):
+            monkeypatch.setattr(kernels, "_layout_pass_pays", lambda *args, v=layout: v)
+            for at in (xd, xd.to(memory_format=torch.channels_last), xd.transpose(2, 3).contiguous().transpose(2, 3)):
+                got = kernels.conv2d(at, _dev(s), _dev(sign), _dev(bias), cw, stride, 0)
+                np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
 # (Nb, C, H, W, O, k, stride, pad), (pool kernel, stride, padding)
 POOLED = [((2, 3, 45, 37, 64, 7, 2, 3), (3, 2, 1)), ((3, 20, 14, 9, 70, 3, 1, 1), (2, 2, 0)), ((1, 64, 9, 12, 33, 1, 1, 0), (3, 1, 1)),
           ((2, 8, 23, 23, 129, 3, 1, 1), (11, 4, 5)), ((40, 3, 64, 64, 40, 3, 2, 1), (3, 2, 0)), ((1, 33, 5, 70, 34, 3, 1, 1), (5, 3, 2)),

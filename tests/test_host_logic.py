@@ -363,3 +363,15 @@ def test_a_pooled_launch_is_taken_where_it_pays(Nb, C, OH, O, k, pool, int32, in
     sums and a pooling pass; layers that are bound by their sums do not."""
     assert kernels._pool_pays(Nb, C, OH, OH, O, k, k, 14, 4, pool) == int32
     assert kernels._pool_pays(Nb, C, OH, OH, O, k, k, 14, 1, pool) == int8
+
+
+# images of H x H, input channels, taps, output channels: us of the kernels that read the input in place, and of the layout pass
+# and the matrix cores
+@pytest.mark.parametrize("Nb,H,C,taps,O,there,here", [
+    (128, 56, 24, 1, 64, 51, 56), (8, 14, 24, 1, 64, 15, 18), (128, 56, 6, 4, 64, 46, 51), (128, 56, 4, 9, 64, 59, 52),
+    (32, 56, 4, 9, 32, 21, 17), (128, 56, 8, 4, 64, 59, 51), (128, 56, 1, 36, 128, 92, 106), (128, 56, 32, 1, 16, 29, 42),
+    (128, 56, 32, 1, 64, 63, 58), (8, 14, 32, 1, 64, 17, 19), (32, 56, 32, 1, 64, 35, 26), (128, 56, 32, 1, 128, 116, 93),
+    (128, 56, 36, 1, 32, 48, 59), (128, 56, 36, 1, 64, 64, 75), (32, 56, 36, 1, 64, 34, 29), (128, 56, 40, 1, 128, 131, 119),
+    (128, 56, 5, 9, 64, 72, 54), (128, 56, 64, 1, 16, 44, 65), (8, 14, 64, 1, 16, 28, 17), (128, 56, 64, 1, 64, 98, 85)])
+def test_the_layout_pass_is_taken_where_it_was_faster(Nb, H, C, taps, O, there, here):
+    assert kernels._layout_pass_pays(Nb, H, H, C, taps, O, 1) == (here < there)
