@@ -137,6 +137,39 @@ def test_matrix_core_entry_points_refuse_the_formats_that_conversions_refuse():
     assert conv(16, 16, 4, -1) == -1 and conv(16, 16, 4, 32) == -1
 
 
+def test_pooled_entry_points_refuse_what_they_have_no_form_for():
+    """ds_mfma_conv2d_pool and the packed call: windows past the form, results of 2 GB, formats, and, in the arrays, what the
+    typed signature has no place for (sums, a residual, a matrix)."""
+    import struct
+    L = _lib.lib()
+    one = ctypes.c_void_p(256)
+
+    def pool(k=3, s=2, p=1, Nb=1, H=64, W=64, O=64, F_in=16, I=16, q_bytes=4, max_shift=14, out=one, q=one):
+        return L.ds_mfma_conv2d_pool(one, one, None, out, q, None, None, Nb, 64, H, W, O, 1, 1, 1, 1, 1, 1, max_shift, 4, F_in, 1, I,
+                                     16, 0, 0, q_bytes, 1, 1, 0, 0, 0, k, s, p, None)
+
+    assert pool(k=0) == -1 and pool(k=-3) == -1 and pool(k=12) == -1 and pool(s=0) == -1 and pool(p=-1) == -1 and pool(p=2) == -1
+    assert pool(H=1, W=64, p=0) == -1                           # no window fits
+    assert pool(out=None, q=None) == -1 and pool(I=17) == -1 and pool(q_bytes=2) == -1 and pool(F_in=32) == -1
+    assert pool(max_shift=15) == -1
+    assert pool(Nb=9, H=1024, W=1024) == -1                     # 2.4 GB of sums
+
+    def packed(y=0, out=256, q=0, residual=0, rows=0, H=64, k=3, s=2, p=1):
+        pointers = struct.pack("=9Q", 256, 256, 0, y, out, q, 0, 0, residual)
+        ints = struct.pack("=31i", 1, 64, H, 64, 64, 1, 1, 1, 1, 0, 0, 1, 1, rows, 14, 4, 16, 1, 16, 16, 0, 0, 4, 1, 1, 0, 0, 0, k, s, p)
+        return L.ds_mfma_conv2d_packed(pointers, ints, None)
+
+    assert packed(y=256, out=0) == -1 and packed(residual=256) == -1 and packed(rows=64, H=1) == -1
+    assert packed(k=12) == -1 and packed(k=-1) == -1 and packed(s=0) == -1
+    assert L.ds_mfma_conv2d_packed(None, b"", None) == -1 and L.ds_mfma_conv2d_packed(b"", None, None) == -1
+    # the choice: no form, no gain
+    assert L.ds_mfma_pool_pays(64, 3, 112, 112, 64, 7, 7, 14, 4, 3, 2, 1) == 1
+    for sizes in [(0, 3, 112, 112, 64, 7, 7, 14, 4, 3, 2, 1), (64, 3, 112, 112, 64, 7, 7, 15, 4, 3, 2, 1),
+                  (64, 3, 112, 112, 64, 7, 7, 14, 4, 12, 2, 1), (64, 3, 2, 2, 64, 7, 7, 14, 4, 3, 2, 0),
+                  (64, 3, 1024, 1024, 64, 7, 7, 14, 4, 3, 2, 1), (64, 3, 112, 112, 0, 7, 7, 14, 4, 3, 2, 1)]:
+        assert L.ds_mfma_pool_pays(*sizes) == 0, sizes
+
+
 def test_error_is_raised_as_exception():
     with pytest.raises(_lib.DeepShiftError) as err:
         _lib.call("ds_quantize_f32_i32", None, None, 10, 0, 16, 0, None)

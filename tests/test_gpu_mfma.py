@@ -455,6 +455,52 @@ def test_pooled_layers_agree_on_both_routes(monkeypatch, shape, pool, act, fused
     assert torch.equal(f, want_f) and torch.equal(q.padded() if fused else q, want_q)
 
 
+@pytest.mark.parametrize("x_bytes", [4, 1])
+def test_the_long_signatures_answer_like_the_packed_one(rng, x_bytes):
+    """ds_mfma_conv2d (sums; float, padded and operand results, from a window of the prepared tensor) and ds_mfma_conv2d_pool, as a
+    caller of the library writes them, against the arrays that the package sends."""
+    lib = kernels._lib
+    Nb, C, H, W, O, top = 2, 40, 13, 11, 70, 6
+    F_in, I, F, dtype = (16, 16, 16, torch.int32) if x_bytes == 4 else (5, 3, 5, torch.int8)
+    stream = lib.stream_handle(torch.device(DEV))
+    _, _, cw = _weights(rng, (O, C, 2, 3), top, ternary=True)
+    _, _, inner = _weights(rng, (O, C, 1, 2), top, ternary=True)
+    bias = _dev(rng.integers(-2 ** 20, 2 ** 20, size=O).astype(np.int32))
+    scale, shift = torch.randn(O, device=DEV), torch.randn(O, device=DEV)
+    prepared, blob, at = kernels.mfma_route(_dev(_activations(rng, (Nb, C, H, W), x_bytes, 1 << 22)), (1, 2), cw, O, (2, 3), x_bytes)
+    inner_blob = kernels._mfma_of(inner, at, x_bytes, O, C, 1, 2)
+    sizes = (Nb, C, H + 2, W + 4, O)
+    OH, OW = (H + 2 - 2) // 2 + 1, W + 4 - 3 + 1
+    y = torch.empty(Nb, O, OH, OW, dtype=torch.int32, device=DEV)
+    lib.call("ds_mfma_conv2d", lib.ptr(prepared.data), lib.ptr(blob), lib.ptr(bias), lib.ptr(y), None, None, None, None, None, *sizes,
+             2, 3, 2, 1, 0, 0, 2, 3, 0, at, x_bytes, 0, 0, 16, 16, 0, 0, 4, 1, 1, 0, 0, 0, stream)
+    assert torch.equal(y, kernels.mfma_conv2d(prepared, blob, bias, O, (2, 3), (2, 1), at))
+    # the centre of the prepared tensor, read by a filter of one row
+    residual = torch.randn(Nb, O, H, (W - 2) // 2 + 1, device=DEV)
+    args = (prepared, inner_blob, bias, O, (1, 2), (1, 2), at, (1, 2), F_in, scale, shift, residual, True)
+    for filt in (None, (3, 3)):
+        want_f, want_q = kernels.mfma_conv2d(*args, ((2, 1), I, F, dtype, filt))
+        out, q = torch.empty_like(want_f), torch.empty_like(want_q if filt is None else want_q.data)
+        lib.call("ds_mfma_conv2d", lib.ptr(prepared.data), lib.ptr(inner_blob), lib.ptr(bias), None, lib.ptr(out), lib.ptr(q),
+                 lib.ptr(scale), lib.ptr(shift), lib.ptr(residual), *sizes, 1, 2, 1, 2, 1, 2, 2, 3, 0, at, x_bytes, F_in, 1, I, F, 2, 1,
+                 x_bytes | (0 if filt is None else lib.DS_Q_OPERANDS), *(filt or (1, 1)), 0, 0, 0, stream)
+        got = q if filt is None else kernels.Prepared(q, want_q.dims, filt, 0, x_bytes, (2, 1)).padded()
+        assert torch.equal(out, want_f) and torch.equal(got, want_q if filt is None else want_q.padded())
+    # operands from a convolution's epilogue, and a max pooling behind the layer that reads them
+    _, _, cw2 = _weights(rng, (64, O, 3, 3), top, ternary=True)
+    blob2, bias2 = kernels._mfma_of(cw2, at, x_bytes, 64, O, 3, 3), _dev(rng.integers(-2 ** 20, 2 ** 20, size=64).astype(np.int32))
+    scale2, shift2 = torch.randn(64, device=DEV), torch.randn(64, device=DEV)
+    args = (want_q, blob2, bias2, 64, (3, 3), (1, 1), at, 0, F_in, scale2, shift2, None, True)
+    for filt in (None, (3, 3)):
+        pooled_f, pooled_q = kernels.mfma_conv2d(*args, ((1, 2), I, F, dtype, filt), True, None, (3, 2, 1))
+        out, q = torch.empty_like(pooled_f), torch.empty_like(pooled_q if filt is None else pooled_q.data)
+        lib.call("ds_mfma_conv2d_pool", lib.ptr(want_q.data), lib.ptr(blob2), lib.ptr(bias2), lib.ptr(out), lib.ptr(q), lib.ptr(scale2),
+                 lib.ptr(shift2), *want_q.dims, 64, 3, 3, 1, 1, 3, 3, at, x_bytes, F_in, 1, I, F, 1, 2,
+                 x_bytes | (0 if filt is None else lib.DS_Q_OPERANDS), *(filt or (1, 1)), 1, 2, 1, 3, 2, 1, stream)
+        got = q if filt is None else kernels.Prepared(q, pooled_q.dims, filt, 0, x_bytes, (1, 2)).padded()
+        assert torch.equal(out, pooled_f) and torch.equal(got, pooled_q if filt is None else pooled_q.padded())
+
+
 def test_windows_without_a_form_keep_their_pass():
     serves = kernels._lib.lib().ds_mfma_pool_serves
     assert serves(8, 8, 3, 2, 1) == 1 and serves(1, 1, 1, 1, 0) == 1 and serves(11, 11, 11, 1, 0) == 1
