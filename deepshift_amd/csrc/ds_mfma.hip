@@ -892,7 +892,9 @@ __device__ __forceinline__ void digit4(const MfmaArgs &a, int32_t (*slot)[64], i
 // The sums of one wave's tile over blocks kb0 .. kb1 - 1.  Two sets of operands, the loads of a block in flight during the
 // products of the one before; with digit d3, whose sums leave no room for them (14 VGPRs went to scratch and back in every
 // block), and for 64 pixels (17 VGPRs; 32 channels of 16 x 16, 256 images: 15.8 us, so 14.7), one set, loaded again once the
-// last operands of a block are formed and behind its last products.
+// last operands of a block are formed and behind its last products.  Launches of 32 channels x 64 pixels still keep VGPRs in
+// scratch, but across a loop, not in one: 6, 16 and 2 (shifts to 14, 6 and 3) are stored before the loop with digit d3 and loaded
+// behind it, 3 and 4 (8-bit activations) before the epilogue's separate pieces.
 template <int MODE, int CT, int NT, bool HIGH, bool ONE_SET = HIGH || (NT == 2 && !mode_i8(MODE)), typename Asked>
 __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT], const int8_t *w, int kb0, int kb1,
                                          const uint32_t (&px)[NT], const uint32_t (&px01)[NT], const PixelAt (&at)[NT], int lane,
