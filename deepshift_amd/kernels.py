@@ -1057,24 +1057,28 @@ def mfma_pool_pays(prepared, O, kernel_size, stride, max_shift, pool):
 
 def _layout_pass_pays(Nb, H, W, C, taps, O, stride):
     """Whether the matrix cores win by more than their layout pass against kernels that read an unpadded int32 input as it
-    is, in one launch.  Us there and here, shifts to 14, 128 x 56 x 56 images, and 8 x 14 x 14, where two launches cost the host
-    17.  Fewer than 32 terms: 24 -> 64 channels, 1 x 1: 51, 56 and 15, 18; 6 -> 64, 2 x 2: 46, 51 and 14, 17.  32 to 40 of
-    several taps: 4 -> 64, 3 x 3: 59, 52 and 17, 17; 8 -> 64, 2 x 2: 59, 51 and 17, 17; but 1 -> 128, 6 x 6: 92, 106 and 17, 17.
-    Of one tap, where channels past 32 fill a second block by little: 32 -> 16: 29, 42 and 18, 18; 32 -> 64: 63, 58 and 17, 19;
-    32 -> 128: 116, 93; 36 -> 32: 48, 59 and 17, 17; 36 -> 64: 64, 75 and 17, 17, of 32 images 34, 29; 40 -> 64: 70, 75 and 19, 17;
-    40 -> 128: 131, 119 and 19, 17.  More: 45 -> 64 (5, 3 x 3): 72, 54 and 20, 17; 48 -> 64: 77, 78 and 20, 17; 48 -> 16: 34, 60 and
-    22, 17; 64 -> 16: 44, 65; 64 -> 64: 98, 85 and 25, 17."""
+    is, in one launch.  Us there and here, shifts to 14, 128 x 56 x 56 images, and 8 x 14 x 14, where a launch costs the host 17
+    and two 17 to 19.  Fewer than 32 terms: 24 -> 64 channels, 1 x 1: 51, 56 and 15, 18; 6 -> 64, 2 x 2: 46, 51 and 14, 17.
+    32 to 40, where the host decides up to 36000 or 64000 pixels: 4 -> 64, 3 x 3: 59, 52, of 40 x 30 x 30 images 18.6, 19.4, of
+    40 x 40 x 40 22, 20; 4 -> 128: 93, 87 and 22, 20 and 34, 23; 8 -> 64, 2 x 2: 59, 51 and 21, 20 and 22, 20; but 1 -> 128, 6 x 6:
+    92, 106.  Of one tap, where channels past 32 fill a second block by little: 32 -> 16: 29, 42; 32 -> 64: 63, 57 and 22, 20 and
+    23, 19; 32 -> 128: 115, 93 and 30, 20 and 35, 23; 36 -> 24: 46, 58 and 21, 19 and 21, 21; 36 -> 64: 64, 75 and 21, 19 and 22, 23,
+    of 32 x 56 x 56 34, 29; 40 -> 64: 70, 75 and 23, 19 and 24, 22; 36 -> 128: 117, 118 and 29, 23 and 34, 29.
+    More: 45 -> 64 (5, 3 x 3): 72, 54 and 20, 17; 48 -> 64: 77, 78 and 20, 17; 48 -> 16: 34, 60 and 22, 17; 64 -> 16: 44, 65;
+    64 -> 64: 98, 85 and 25, 17."""
     sh, sw = _pair(stride)
     pixels = Nb * (H // sh) * (W // sw)
     if C * taps < 32:
         return False
     if C * taps > 40:
         return O > 16 or pixels < 1 << 18
+    if taps == 1 and O >= 128:
+        return pixels >= 1 << 15
+    if pixels < 3 << 14:
+        return False
     if taps > 1:
-        return C >= 4 or pixels < 1 << 18
-    if C == 32:
-        return O > 16 and pixels >= 1 << 14
-    return O >= 128 or pixels < (1 << 18 if O >= 64 else 1 << 15)
+        return C >= 4
+    return O > 16 if C == 32 else O >= 64 and pixels < 1 << 18
 
 
 def _mfma_linear(x, conc_weight, bias, N):
