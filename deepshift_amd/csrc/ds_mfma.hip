@@ -38,6 +38,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr int kDigits = 5;          // 7-bit digits of an int32 activation
 constexpr int kMfmaMaxK = 1 << 17;  // 64 * 127 * K stays within int32
 constexpr int kMaxRows = 1 << 24;   // ds_mfma_prepare launches 256 threads per row, and a launch has less than 2^32
+constexpr int kMaxParts = 1 << 15;  // of a row in ds_mfma_prepare; a launch has less than 2^16 workgroups along y
 constexpr int kMaxPad = 1 << 28;
 
 // Which products a launch forms (MfmaMode): the widest shift that occurs, and the activations' width.
@@ -180,6 +181,7 @@ inline MfmaX mfma_x(int Nb, int C, int Hp, int Wp, const MfmaGeom &g, bool i8)
     // as many channel blocks of a row per workgroup as its threads take at a go (mfma_prepare_kernel)
     const int per_block = Wp * (g.cp == 32 ? 2 : 1);
     x.cbf = per_block >= 256 ? 1 : 256 / per_block < g.cb ? 256 / per_block : g.cb;
+    if (x.cbf < ceil_div(g.cb, kMaxParts)) x.cbf = ceil_div(g.cb, kMaxParts);
     x.fy = ceil_div(g.cb, x.cbf);
     // a block of several taps may read up to 32 bytes past the last pixel
     x.planes = align_up((size_t)x.rows * x.rstride + 64, 256);

@@ -103,6 +103,17 @@ def test_8_bit_matrices_match_the_oracle(oracle, rng, M, K, N):
             np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
+def test_more_blocks_of_channels_than_a_launch_has_workgroups_along_y():
+    """A row of 2^16 + 3 blocks of 32 channels x 128 pixels: a workgroup of the layout pass takes several of them."""
+    blocks = (1 << 16) + 3
+    x = torch.randint(-128, 128, (1, blocks * 32 - 5, 1, 128), dtype=torch.int8, device=DEV)
+    got = kernels.mfma_prepare(x, 0, (1, 1), 1)
+    want = torch.zeros(blocks * 32, 128, dtype=torch.int8, device=DEV)
+    want[:-5] = x[0, :, 0]
+    want = want.view(blocks, 32, 128).transpose(1, 2).reshape(-1)
+    assert torch.equal(got.data[:want.numel()].view(torch.int8), want)
+
+
 @pytest.mark.parametrize("x_bytes", [4, 1])
 @pytest.mark.parametrize("Nb,C,H,O,k,st", [(2, 32, 14, 40, 3, 1), (1, 64, 7, 96, 1, 1), (40, 32, 28, 64, 3, 2)])
 def test_epilogue_matches_the_separate_passes(rng, x_bytes, Nb, C, H, O, k, st):
