@@ -430,13 +430,13 @@ struct MfmaArgs {
     MfmaX qlay;                 // q in the operand layout of the next layer (qlay.planes != 0)
     uint8_t *qflags;
     int relu, q_bytes, qHp, qWp, qph, qpw;
-    int qscattered;             // a unit's pixels are not 32 in a row of the output: its flags are shared with other units
     float inv;
-    // the shorter epilogue: 2^F of the sums, 2^F of q if nothing else is written
+    // the shorter epilogue: 2^F of the sums, 2^F of q if nothing else is written (q_only)
     float unfold, qfold;
     int q_only;
     QuantSpec qspec;
-    FastDiv by_image, by_row, by_ctiles;
+    // at odd multiples of 4 bytes the layers of 8-bit networks took 0.7 % more, those of ResNet-20 0.6 %
+    alignas(8) FastDiv by_image, by_row, by_ctiles;
 };
 
 __device__ __forceinline__ v4i perm4(uint32_t neg, uint32_t pos, v4i sel)
@@ -896,7 +896,7 @@ __device__ __forceinline__ void digit4(const MfmaArgs &a, int32_t (*slot)[64], i
 // block), and for 64 pixels (17 VGPRs; 32 channels of 16 x 16, 256 images: 15.8 us, so 14.7), one set, loaded again once the
 // last operands of a block are formed and behind its last products.  Launches of 32 channels x 64 pixels still keep VGPRs in
 // scratch, but across a loop, not in one: 6, 16 and 2 (shifts to 14, 6 and 3) are stored before the loop with digit d3 and loaded
-// behind it, 3 and 4 (8-bit activations) before the epilogue's separate pieces.
+// behind it, 3 (8-bit activations) before the epilogue's separate pieces.
 template <int MODE, int CT, int NT, bool HIGH, bool ONE_SET = HIGH || (NT == 2 && !mode_i8(MODE)), typename Asked>
 __device__ __forceinline__ void contract(const MfmaArgs &a, v16i (&total)[CT][NT], const int8_t *w, int kb0, int kb1,
                                          const uint32_t (&px)[NT], const uint32_t (&px01)[NT], const PixelAt (&at)[NT], int lane,
@@ -1057,7 +1057,9 @@ __device__ __forceinline__ OutAt out_at(const MfmaArgs &a, const PixelAt &at, ui
 }
 // Eight values per lane (channels ch0 + 8 g + 0..3, ch0 = 16 u + 4 (lane >> 5)) into the next layer's operand layout: the
 // halves of a wave swap words, so that a lane holds eight channels side by side and the 32 pixels of a digit are stored
-// in a row.  Digits d3 and d4 only, with a flag, where the 32 pixels x 16 channels have any.
+// in a row.  Digits d3 and d4 only, with a flag, where the 32 pixels x 16 channels have any.  SCATTERED: a unit's pixels are not
+// 32 in a row of the output, so its flags are shared with other units.
+template <bool SCATTERED>
 __device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t (&qv)[kUnit], int ch0, const OutAt &o)
 {
     const int half = (ch0 >> 2) & 1, u16 = ch0 >> 4;   // half = lane >> 5: ch0 is a multiple of 16 plus 0 or 4
@@ -1091,11 +1093,23 @@ __device__ __forceinline__ void store_operands(const MfmaArgs &a, const int32_t 
     }
     const uint32_t high4 = w[4][0] | w[4][1], high = w[3][0] | w[3][1] | high4;
     bool any = true;
-    if (a.qscattered) {
-        // d3 and d4 are always there; flags, zero before the launch, gather what their 32 pixels have
-        if (u16 < L.c16 && o.in && high) {
-            const size_t at = (size_t)(o.p >> 5) * L.c16 + u16;
-            atomicOr((uint32_t *)a.qflags + (at >> 2), (high4 ? 3u : 1u) << (8 * (at & 3)));
+    if constexpr (SCATTERED) {
+        // d3 and d4 are always there; flags, zero before the launch, gather what their 32 pixels have.  One atomic for each flag
+        // that the wave meets, some four or eight of them: one for each lane queued at the same words wherever most results are
+        // past 16 (16.16; 3 x 3, us then and now, 64 images of 64 -> 128 channels of 112 x 112, 2 x 2 windows: 1060 and 625, as
+        // sums and a pass 810; 64 of 512 of 28 x 28: 1590 and 1112; 32 of 64 of 32 x 32, 3 x 3 stride 1: 117 and 44, 49)
+        const uint32_t flag = o.p >> 5;
+        const bool set = u16 < L.c16 && o.in && high;
+        for (uint64_t left = __ballot(set); left;) {
+            const int first = __ffsll((unsigned long long)left) - 1;
+            const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)flag, first);
+            const bool same = set && flag == f;
+            const bool four = __any(same && high4);
+            left &= ~__ballot(same);
+            if ((int)(threadIdx.x & 63) == first) {
+                const size_t at = (size_t)f * L.c16 + u16;
+                atomicOr((uint32_t *)a.qflags + (at >> 2), (four ? 3u : 1u) << (8 * (at & 3)));
+            }
         }
     } else {
         any = __any(o.in && high != 0);
@@ -1160,6 +1174,7 @@ __device__ __forceinline__ void quantize_all(const float (&f)[kUnit], int32_t (&
     }
 }
 // The next layer's input of a unit, quantised.
+template <bool SCATTERED>
 __device__ __forceinline__ void store_q(const MfmaArgs &a, int32_t (&qv)[kUnit], int ch0, const OutAt &o)
 {
     if (a.qflags) {
@@ -1167,7 +1182,7 @@ __device__ __forceinline__ void store_q(const MfmaArgs &a, int32_t (&qv)[kUnit],
 #pragma unroll
             for (int i = 0; i < kUnit; ++i)
                 if (ch0 + 8 * (i >> 2) + (i & 3) >= a.N) qv[i] = 0;
-        store_operands(a, qv, ch0, o);
+        store_operands<SCATTERED>(a, qv, ch0, o);
     } else if (a.q_bytes == 1) {
         int8_t b[kUnit];
 #pragma unroll
@@ -1178,6 +1193,7 @@ __device__ __forceinline__ void store_q(const MfmaArgs &a, int32_t (&qv)[kUnit],
     }
 }
 // What follows the affine step.
+template <bool SCATTERED>
 __device__ __forceinline__ void store_values(const MfmaArgs &a, float (&f)[kUnit], const float (&res)[kUnit], int ch0, const OutAt &o)
 {
     if (a.residual)
@@ -1196,8 +1212,9 @@ __device__ __forceinline__ void store_values(const MfmaArgs &a, float (&f)[kUnit
     } else {
         quantize_all(f, qv, a.qspec);
     }
-    store_q(a, qv, ch0, o);
+    store_q<SCATTERED>(a, qv, ch0, o);
 }
+template <bool SCATTERED>
 __device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail &t, const int32_t (&sum)[kUnit],
                                            const float (&res)[kUnit], int ch0, const OutAt &o)
 {
@@ -1211,7 +1228,7 @@ __device__ __forceinline__ void store_tail(const MfmaArgs &a, const ChannelTail 
     float f[kUnit];
 #pragma unroll
     for (int i = 0; i < kUnit; ++i) f[i] = affine_one(v[i], a.inv, t.scale[i], t.shift[i], nullptr, 0);
-    store_values(a, f, res, ch0, o);
+    store_values<SCATTERED>(a, f, res, ch0, o);
 }
 // The shorter epilogue (stage_tails): sum is complete, scale and shift of t are the folded ones.
 __device__ __forceinline__ void store_tail_folded(const MfmaArgs &a, const ChannelTail &t, const int32_t (&sum)[kUnit],
@@ -1221,14 +1238,14 @@ __device__ __forceinline__ void store_tail_folded(const MfmaArgs &a, const Chann
 #pragma unroll
     for (int i = 0; i < kUnit; ++i) f[i] = affine_one(sum[i], 1.0f, t.scale[i], t.shift[i], nullptr, 0);
     if (!a.q_only) {
-        store_values(a, f, res, ch0, o);
+        store_values<false>(a, f, res, ch0, o);
         return;
     }
     // ReLU, the upper bound and the floor in two instructions a value
     int32_t qv[kUnit];
 #pragma unroll
     for (int i = 0; i < kUnit; ++i) qv[i] = f2i_sat(__builtin_amdgcn_fmed3f(f[i], 0.0f, a.qspec.hi));
-    store_q(a, qv, ch0, o);
+    store_q<false>(a, qv, ch0, o);
 }
 
 // Four or eight waves per workgroup; a wave owns CT * 32 channels x NT * 32 pixels and one of ks parts of the reduction (the
@@ -1344,7 +1361,7 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
                 int32_t v[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] = total[c >> 1][p][(c & 1) * 8 + i];
-                store_tail(a, tl, v, res[c * NT + p], chl + c * 16, o[p]);
+                store_tail<false>(a, tl, v, res[c * NT + p], chl + c * 16, o[p]);
             }
         }
         return;
@@ -1374,7 +1391,7 @@ __global__ __launch_bounds__(WAVES * 64, mode_i8(MODE) && WAVES == 4 ? 3 : 2) vo
             v[i] = 0;
             for (int s = 0; s < ks; ++s) v[i] += part[t * ks + s][u * 8 + i][lane];
         }
-        store_tail(a, tl, v, res, ch, o);
+        store_tail<false>(a, tl, v, res, ch, o);
     }
 }
 
@@ -1525,7 +1542,7 @@ __global__ __launch_bounds__(256, 2) void mfma_pool_kernel(MfmaArgs a, MfmaPool 
             best[i] ^= flips[ch + 8 * (i >> 2) + (i & 3)];
             plain.add[i] = 0;   // it is in the sums
         }
-        store_tail(a, plain, best, res, c0 + ch, o);
+        store_tail<true>(a, plain, best, res, c0 + ch, o);
     }
 }
 
@@ -1979,7 +1996,6 @@ static int mfma_conv2d_any(const void *prepared, const void *blob, const int32_t
         m.by_tw = fast_div((uint32_t)m.tw);
         m.by_tiles_w = fast_div((uint32_t)m.tiles_w);
         m.by_tiles_h = fast_div((uint32_t)m.tiles_h);
-        a.qscattered = 1;
         if (operands && q_bytes == 4) {
             const long words = (long)(align_up(((size_t)Nb * rows * columns / 32 + 1) * a.qlay.c16, 4) / 4);
             hipLaunchKernelGGL(mfma_clear_kernel, dim3((unsigned)(words / 256 < 1024 ? words / 256 + 1 : 1024)), dim3(256), 0, st,

@@ -434,6 +434,34 @@ def test_pooling_in_the_launch_matches_the_separate_pass(rng, top, x_bytes, shap
         assert torch.equal(got.padded(), q[:, :, 1:-1])
 
 
+@pytest.mark.parametrize("shape,pool", [((3, 16, 21, 40, 40), (2, 2, 0)), ((2, 16, 9, 131, 129), (3, 1, 1)), ((5, 16, 70, 1, 64), (1, 1, 0)),
+                                        ((1, 16, 80, 12, 80), (5, 1, 2))], ids=lambda v: str(v).replace(" ", ""))
+def test_each_flag_of_a_pooled_hand_off_says_what_its_values_have(rng, shape, pool):
+    """Digits d3 and d4 in few places: waves whose windows lie in one flag's 32 pixels, in several, and in none that is set;
+    each flag is that of its pixels and channels, no other's."""
+    Nb, C, H, W, O = shape
+    s, sign, cw = _weights(rng, (O, C, 1, 1), 14, ternary=False)
+    x = rng.integers(-2 ** 8, 2 ** 8, size=(Nb, C, H, W)).astype(np.int32)
+    for top in (2 ** 19, 2 ** 26):
+        x[rng.integers(0, Nb, 3), :, rng.integers(0, H, 3), rng.integers(0, W, 3)] = rng.integers(-top, top, size=(3, C))
+    prepared, blob, at = kernels.mfma_route(_dev(x), 0, cw, O, (1, 1), 4)
+    scale, shift = torch.ones(O, device=DEV), torch.zeros(O, device=DEV)
+    scale[::3] = 4
+    y = kernels.mfma_conv2d(prepared, blob, None, O, (1, 1), 1, at)
+    _, q = kernels.requantize_affine_maxpool(y, 16, scale, shift, True, pool, (1, 1), 16, 16, False, torch.int32)
+    _, got = kernels.mfma_conv2d(prepared, blob, None, O, (1, 1), 1, at, 0, 16, scale, shift, None, True,
+                                 ((1, 1), 16, 16, torch.int32, (3, 3)), False, None, pool)
+    assert torch.equal(got.padded(), q)
+    c16, pixels = (O + 15) // 16, Nb * (q.shape[2] - 2) * (q.shape[3] - 2)
+    level = (q >= 2 ** 20).to(torch.uint8) + 2 * (q >= 2 ** 27 - 2 ** 20).to(torch.uint8)
+    level = level[:, :, 1:-1, 1:-1].permute(0, 2, 3, 1).reshape(pixels, O)
+    level = torch.nn.functional.pad(level, (0, c16 * 16 - O, 0, -pixels % 32)).view(-1, 32, c16, 16)
+    want = level.amax((1, 3))
+    assert 0 < int((want > 0).sum()) < want.numel() and int(want.max()) == 3
+    planes = (q.shape[0] * q.shape[2] * q.shape[3] * ((O + 31) // 32 * 32) * 5 + 64 + 255) // 256 * 256
+    assert torch.equal(got.data[planes:planes + want.numel()].view_as(want), want)
+
+
 # (Nb, C, H, O, k), pool, (I, F), whether the pooling runs in the launch: rectangles of one to eight tiles, with whole and half
 # limits, beside layers whose single launch would leave waves idle
 POOL_ROUTES = [((1, 128, 14, 128, 3), (2, 2, 0), (16, 16), False), ((3, 256, 13, 256, 3), (3, 2, 0), (16, 16), False), ((128, 64, 16, 128, 3), (2, 2, 0), (16, 16), True),
