@@ -118,11 +118,10 @@ def _split_result(fused_mod, result):
 
 def parity_gate(fused, x, images=None):
     """Before any timing: one forward pass of the FUSED model that is about to be timed, with a hook on every
-    fused shift-convolution launch it issues (ds_conv2d_tiled_fused_i32, ds_conv2d_tiled_fused_pair_i32, the
-    stem's ds_conv2d_tiled_i32 + pooling pass); each launch's own inputs and outputs -- the tensors the
-    timed launches read and write -- are then compared, for the first and the last image, bit for bit with
-    the oracle's restatement of the reference chain on the same inputs.  Returns the number of launches
-    checked."""
+    fused shift-convolution module (a convolution, the stem's with its max pooling, or a convolution and the
+    shortcut beside it); each module's own inputs and outputs -- the tensors the timed launches read and
+    write -- are then compared, for the first and the last image, bit for bit with the oracle's restatement of
+    the reference chain on the same inputs.  Returns the number of modules checked."""
     from deepshift_amd import fuse
     from oracle import shift_oracle as so
     oracle = so.get()
@@ -796,7 +795,7 @@ def main():
     if not torch.allclose(got, want, rtol=0, atol=2e-3 * float(want.abs().max()) + 1e-4):
         raise SystemExit("fused pipeline diverges from the plain converted model")
     checked = parity_gate(fused, x)
-    log("parity gate passed on the %d convolution launches of the timed model; %d conv + 1 fc shift layers"
+    log("parity gate passed on the %d fused convolution modules of the timed model; %d conv + 1 fc shift layers"
         % (checked, n_conv))
     sec_unfused = time_steps(model, x, max(2, args.steps // 2), args.warmup)
     sec_per_step = time_steps(fused, x, args.steps, args.warmup)
@@ -877,7 +876,7 @@ def main():
                                "(benchmark configuration 4); weight_bits 5 (4-bit shift + sign, 6 codes per "
                                "word), activations 16.16; BatchNorm, residual, ReLU and the next layer's "
                                "fixed-point conversion in each convolution's epilogue, the stem's max "
-                               "pooling in one conversion pass, global average pooling fp32 PyTorch",
+                               "pooling in its convolution's launch, global average pooling fp32 PyTorch",
                    "batch": BATCH, "shift_layers": 21, "shift_launches": len(layers), "pairs_per_step": pairs},
         "unfused_images_per_s": BATCH / sec_unfused,
         # the same step replayed from a captured HIP graph: an extra beside `value`, which is the eager step
@@ -901,8 +900,9 @@ def main():
             "avg_launch_us_in_step": dom_s_bracketed / len(dominant) * 1e6,
             "frac_in_step": dom_pairs / dom_s_bracketed / PEAK_PAIRS_MFMA,
             "pairs_per_launch": dom_pairs / len(dominant),
-            # the whole step (all 21 shift launches; the layout passes in front of the stem and behind the pooling,
-            # and the pooling pass, are not among them) against the same bound
+            # the whole step (all 21 shift launches; the stem's pools its result too, and multiplies the pixels that its
+            # rectangles share once more, which are not counted; the layout pass in front of it is not among them)
+            # against the same bound
             "step_achieved": pairs / kernel_s / 1e12,
             "step_frac": pairs / kernel_s / PEAK_PAIRS_MFMA,
             # secondary: against a kernel that spends two vector instructions on every pair
