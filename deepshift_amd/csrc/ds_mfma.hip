@@ -1730,21 +1730,25 @@ static double pool_tile(MfmaPool &m, long images, long cus)
 // The single launch multiplies pixels that rectangles share more than once, leaves waves idle in rectangles of odd sizes, and
 // never cuts a reduction: a round (pool_rounds) takes `block` per block of the reduction and 4.  The separate one writes and
 // reads the sums, 4 ns a tile, reads each as often as windows overlap, 0.4 ps a value more than the single launch does from LDS,
-// and has two more launches: 12, between what they take in a graph (7) and what they take the host (14).  us separate, fused,
+// and has two more launches: 12, between what they take in a graph (7) and what they take the host (14).  Nor is it done before
+// the host has issued all of it, kPoolHost: 24 on the host of the table below, 37 on a slower one, where one launch takes 25 (us
+// there, 1 image: 32 -> 96 channels of 13 x 13, 5 x 5: 39 28; 512 -> 256, 1 x 1, 3 x 3 windows stride 1: 40 31; 64 -> 96 of 16 x 16,
+// 5 x 5 stride 1: 38 29; 8-bit 128 -> 40 of 27 x 27, 3 x 3 / 2: 38 26; 2 images 256 -> 96 of 6 x 6: 38 27).  us separate, fused,
 // issued one after another, with the next layer's operands (* fused; 3 x 3 convolutions, 2 x 2 windows unless said otherwise;
 // int32, then 8-bit activations, shifts to 14):
 //   7 x 7 stem of 224 x 224, 3 x 3 stride 2    1 image  24 14*  25 10*     8  40 30*  32 15*     64  224 156*  122 79*
 //   64 -> 64 channels of 224 x 224             1  40 29*  28 14*           8  175 146*  103 70*
 //   64 -> 128 of 112 x 112                     1  28 19*  24 10*           8  95 79*  59 37*     64  726 555*  460 246*
 //   128 -> 256 of 56 x 56                      1  26 29   25 14*           8  83 81*  50 38*     64  579 520*  306 238*
-//   256 -> 512 of 28 x 28                      1  25 50   25 23            8  83 79*  48 37*     64  500 522   260 245*
+//   256 -> 512 of 28 x 28                      1  25 50   25 23*           8  83 79*  48 37*     64  500 522   260 245*
 //   512 -> 512 of 28 x 28                      1  37 117  24 41            8  144 154  75 74*    64  932 1060  462 479*
 //   512 -> 512 of 14 x 14                      1  25 116  24 39            8  52 115  31 41      64  253 309   130 146
-//   256 -> 256 of 13 x 13, 3 x 3 stride 2      1  25 49   24 23            8  25 49   24 23      64  75 77     44 36*
-//   64 -> 192 of 27 x 27, 5 x 5 then 3 x 3 / 2 1  24 37   24 18            8  38 38   25 18*     64  151 166   84 78
+//   256 -> 256 of 13 x 13, 3 x 3 stride 2      1  25 49   24 23*           8  25 49   24 23*     64  75 77     44 36*
+//   64 -> 192 of 27 x 27, 5 x 5 then 3 x 3 / 2 1  24 37   24 18*           8  38 38   25 18*     64  151 166   84 78
 //   32 images, 64 -> 64 of 32 x 32, stride 1   3 x 3  41 32*  32 15*       5 x 5  63 43*  55 24*     11 x 11  147 105*  138 61*
 //     512 -> 64                                3 x 3  101 159  58 74       5 x 5  124 242  81 95     11 x 11  209 619   166 289
 //   128 images, 64 -> 128 of 16 x 16  44 28*  34 13*       128 -> 256 of 8 x 8  43 42  30 20*       512 -> 512 of 2 x 2  29 228  24 83
+constexpr double kPoolHost = 24.0;
 static bool pool_pays(const MfmaPool &m, int mode, int KB, long images, long pixels, int ctiles, long cus)
 {
     MfmaPool tile = m;
@@ -1752,7 +1756,8 @@ static bool pool_pays(const MfmaPool &m, int mode, int KB, long images, long pix
     const double tiles = (pixels + 31) / 32 * (double)ctiles;
     const double looks = (double)images * ctiles * 64 * m.POH * m.POW * m.pk * m.pk;
     const double fused = pool_tile(tile, images * ctiles, cus) * (KB * block + 4.0);
-    return fused <= 12.0 + (tiles / (8.0 * cus) + 0.07) * KB * block + tiles * 0.004 + looks * 0.4e-6;
+    const double separate = 12.0 + (tiles / (8.0 * cus) + 0.07) * KB * block + tiles * 0.004 + looks * 0.4e-6;
+    return fused <= (separate > kPoolHost ? separate : kPoolHost);
 }
 
 template <int MODE>

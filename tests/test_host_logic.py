@@ -352,9 +352,11 @@ def test_small_linear_layers_are_routed_once(monkeypatch):
 @pytest.mark.parametrize("Nb,C,OH,O,k,pool,int32,int8", [
     (64, 3, 112, 64, 7, (3, 2, 1), True, True), (1, 3, 112, 64, 7, (3, 2, 1), True, True),     # stems
     (64, 64, 112, 128, 3, (2, 2, 0), True, True), (128, 64, 16, 128, 3, (2, 2, 0), True, True),
+    (1, 32, 13, 96, 5, (2, 2, 0), True, True), (1, 512, 13, 256, 1, (3, 1, 1), True, True),   # done before the host issues the rest
+    (1, 64, 27, 192, 5, (3, 2, 0), False, True), (1, 64, 16, 96, 3, (5, 1, 2), True, True),
     (32, 64, 32, 64, 3, (11, 1, 5), True, True),                                               # the pass would look 121 times
     (64, 512, 14, 512, 3, (2, 2, 0), False, False), (1, 512, 14, 512, 3, (2, 2, 0), False, False),
-    (1, 512, 28, 512, 3, (2, 2, 0), False, False), (1, 256, 13, 256, 3, (3, 2, 0), False, False),
+    (1, 512, 28, 512, 3, (2, 2, 0), False, False), (1, 256, 13, 256, 3, (3, 2, 0), False, True),   # 8-bit: 24 us apart, 23 in one
     (128, 512, 2, 512, 3, (2, 2, 0), False, False),
     (32, 512, 32, 64, 3, (5, 1, 2), False, False), (32, 512, 16, 256, 5, (11, 1, 5), False, False),   # products twice and more
     (1, 64, 8, 64, 3, (12, 1, 0), False, False), (1, 64, 8, 32, 3, (2, 2, 0), False, False)])         # no form
